@@ -2037,7 +2037,7 @@ int jitnn_hip_llama_embed_dev(jitnn_hip_llama *m, const int *tokens_dev, int cou
 
 int jitnn_hip_llama_argmax_dev(jitnn_hip_llama *m, const float *logits_dev, int *token_dev, void *stream) {
     if (!m || !logits_dev || !token_dev) return fail(JITNN_HIP_EINVAL, "NULL argument");
-    hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, logits_dev, m->vocab, token_dev);
+    hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(ARG_THREADS), 0, (hipStream_t)stream, logits_dev, m->vocab, token_dev);
     HIP_TRY(hipGetLastError());
     return JITNN_HIP_OK;
 }

@@ -344,3 +344,28 @@ def test_generate_argument_checks():
     assert _lib.lib.jitnn_hip_llama_set_embedding(None, 0, None, 0) == _lib.EINVAL
     with pytest.raises(ValueError):
         jitnn_amd.Tokenizer("wordpiece", ["a"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [1, 3, 6, 4096, 32767, 32768, 32775, 128256])
+def test_argmax_kernel_sizes_and_alignment(vocab):
+    """The 16-byte loads' edges: fewer values than a quad, ragged heads and tails (logits at every 4-byte offset), one trip of the
+    workgroup (1024 threads x 8 quads) less, exactly and more - the maximum at the ends and in between, twice where it fits."""
+    import ctypes as C
+    import torch
+    import jitnn_amd
+    from jitnn_amd import _lib
+    dec = jitnn_amd.LlamaDecoder(1, 256, 4, 2, 64, 512, vocab, 8)
+    buf = torch.randn(vocab + 3, device="cuda", generator=torch.Generator(device="cuda").manual_seed(vocab))
+    out = torch.empty(1, dtype=torch.int32, device="cuda")
+    for off in range(4):
+        x = buf[off:off + vocab]
+        for at in {0, vocab // 2, vocab - 1}:
+            keep = x[[at, vocab - 1]].clone()
+            x[at] = x[vocab - 1] = 50.0
+            _lib.check(_lib.lib.jitnn_hip_llama_argmax_dev(dec.handle, C.c_void_p(x.data_ptr()), C.c_void_p(out.data_ptr()), None), "argmax")
+            torch.cuda.synchronize()
+            assert int(out.item()) == at, (off, at)
+            x[vocab - 1] = keep[1]
+            x[at] = keep[0]
+    dec.close()
