@@ -736,6 +736,108 @@ int stage_reserve(size_t pinned_bytes, size_t dev_bytes) {
     return JITNN_HIP_OK;
 }
 
+// ---- thousands of rows: weights dequantised into operand order first, then a plain FP16 product (prefill_wide.h)
+
+// The weight rows of a tile (32 rt) and the microseconds the product should take: whole rounds of one tile per CU, each
+// `step` per 32 values of K and `fixed` for its prologue and epilogue (measured on whole rounds: 4096 x 4096 x 4096 tokens
+// takes 110 us with rt 8, one round, and 125 with rt 4, two; 6144 x 4096 x 4096 takes 174 with rt 6 against 197 with rt 8).
+struct WidePlan {
+    int rt = 0, tiles_n = 0;
+    double us = 0;
+};
+WidePlan wide_plan(const int *n, int count, int k, int mtiles, bool dual) {
+    static const struct { int rt; double step, fixed; } kinds[] = {{8, 0.78, 10.0}, {6, 0.59, 8.0}, {4, 0.44, 5.0}};
+    WidePlan best;
+    const int nst = pf_ksteps(k) / 2;
+    for (const auto &kind : kinds) {
+        if (dual && kind.rt != 8) break;
+        const int tn = dual ? 16 * kind.rt : 32 * kind.rt;
+        int tiles = 0;
+        for (int i = 0; i < count; ++i) tiles += (n[i] + tn - 1) / tn;
+        const int rounds = (int)(((long long)tiles * mtiles + g.cus - 1) / g.cus);
+        const double us = rounds * (kind.step * nst + kind.fixed);
+        if (!best.rt || us < best.us) best = {kind.rt, tiles, us};
+    }
+    return best;
+}
+
+// Dequantised weights beyond this stay on the kernel that decodes as it goes.
+constexpr size_t WIDE_MAX_BYTES = (size_t)512 << 20;
+size_t wide_weight_bytes(const WidePlan &p, int k) { return (size_t)p.tiles_n * p.rt * pf_ksteps(k) * 1024; }
+size_t wide_scratch_bytes(const WidePlan &p, int k, int rows) {
+    const size_t mblocks = (size_t)(rows + PF_BM - 1) / PF_BM * (PF_BM / 32);
+    return mblocks * pf_ksteps(k) * 1024 + (((size_t)rows * 8 + 255) & ~(size_t)255) + wide_weight_bytes(p, k);
+}
+
+// Whether `count` weights of one row length (dual: a gate and an up weight) are worth dequantising first for `rows` rows:
+// the estimate of both passes against that of prefill_mfma_kernel, which takes rounds of 128-row tiles (dual: 64 rows of each
+// weight) by 256 tokens at `step` us per 64 values of K.  Measured, both routes, activation preparation included (us):
+// 14336 x 4096 Q4_K, 1024 / 2048 / 4096 rows 139 / 268 / 496 there and 137 / 256 / 484 here; 4096 x 14336 Q6_K 169 / 298 / 612
+// and 228 / 292 / 486; 11008 x 4096 Q4_0 162 / 245 / 488 and 111 / 194 / 361; 4096 x 4096 Q4_K 58 / 85 / 160 and 65 / 84 / 139;
+// Q8_0 64 / 94 / 179 and 65 / 85 / 140.  Two tiles of tokens or fewer, short rows of K and launches that split K lose
+// here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
+// estimate is good to a tenth on short launches: the margins.
+bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual, WidePlan *plan) {
+    if (count > 3 || rows <= 2 * PF_BM || ws[0]->k < 1024) return false;
+    const int k = ws[0]->k, mtiles = (rows + PF_BM - 1) / PF_BM, nsteps = (k + PF_BK - 1) / PF_BK;
+    int n[3] = {0, 0, 0}, tiles = 0;
+    double dequant = 0, step = 0;
+    for (int i = 0; i < count; ++i) {
+        const int f = ws[i]->fmt;
+        if (ws[i]->k != k || !has_many_row_kernel(f)) return false;
+        if (i == 0 || !dual) n[i] = ws[i]->n;
+        tiles += (ws[i]->n + PF_BN - 1) / PF_BN;
+        dequant += 3.0 + (f == F_Q6_K ? 0.62e-6 : 0.45e-6) * ws[i]->n * (double)k;
+        step = std::max(step, f == F_Q4_K ? 0.87 : f == F_Q6_K ? 1.17 : 1.06);
+    }
+    *plan = wide_plan(n, dual ? 1 : count, k, mtiles, dual);
+    if (wide_weight_bytes(*plan, k) > WIDE_MAX_BYTES) return false;
+    if ((long long)tiles * mtiles * 2 <= g.cus) return false;
+    const double decoding = (double)(((long long)tiles * mtiles + g.cus - 1) / g.cus) * (step * nsteps + 10.0);
+    return plan->us + dequant < (decoding > 150.0 ? 0.95 : rows > 1024 ? 0.9 : 0.8) * decoding;
+}
+
+// The arguments are those of launch_prefill_group; dual: ws is a gate and an up weight, ys[0] = silu(x gate^T) * (x up^T).
+int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws, float *const *ys, int count, bool dual, const float *x, int rows,
+                        const float *bias, const float *norm_w, float eps, hipStream_t stream, const float *residual, const float *swiglu_up,
+                        const PfPending *pend) {
+    const KernelRef kr = prefill_wide_kernel_ref(dual, plan.rt);
+    if (!kr.fn) return fail(JITNN_HIP_EUNSUPPORTED, "no wide kernel of %d row blocks", plan.rt);
+    if (int rc = allow_lds(kr.fn, kr.lds)) return rc;
+    const int k = ws[0]->k, ksteps = pf_ksteps(k), tn = dual ? 16 * plan.rt : 32 * plan.rt;
+    PwArgs a{};
+    a.tiles_m = (rows + PF_BM - 1) / PF_BM;
+    a.tiles_n = plan.tiles_n;
+    a.m = rows;
+    a.ksteps = ksteps;
+    const int mblocks = a.tiles_m * (PF_BM / 32);
+    const size_t xo_bytes = (size_t)mblocks * ksteps * 1024, scale_bytes = ((size_t)rows * 8 + 255) & ~(size_t)255;
+    void *wsp = nullptr;
+    if (int rc = workspace(wide_scratch_bytes(plan, k, rows), stream, &wsp)) return rc;
+    _Float16 *xo = (_Float16 *)wsp, *wo = (_Float16 *)((uint8_t *)wsp + xo_bytes + scale_bytes);
+    float *scale = (float *)((uint8_t *)wsp + xo_bytes), *inv = scale + rows;
+    a.wo = wo;
+    a.xo = xo;
+    a.inv_scale = inv;
+    a.bias = bias;
+    a.res = residual;
+    int tile = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.tile0[i] = tile;
+        if (i >= (dual ? 1 : count)) continue;
+        a.y[i] = ys[i];
+        a.n[i] = a.ld[i] = ws[i]->n;
+        _Float16 *dst = wo + (size_t)tile * plan.rt * ksteps * 512;
+        wide_dequant_launch(ws[i]->fmt, stream, ws[i]->dev, dst, ws[i]->n, k, dual ? 0 : -1);
+        if (dual) wide_dequant_launch(ws[1]->fmt, stream, ws[1]->dev, dst, ws[1]->n, k, 1);
+        tile += (ws[i]->n + tn - 1) / tn;
+    }
+    prefill_prepare_launch(x, scale, inv, xo, rows, k, mblocks, norm_w, eps, swiglu_up, stream, pend);
+    prefill_wide_launch(dual, plan.rt, stream, a);
+    HIP_TRY(hipGetLastError());
+    return workspace_done(stream);
+}
+
 // More rows than the GEMV kernels take: FP16 activations in operand order + dequantise-to-LDS MFMA kernel.
 // `count` weights of one row length share the activations x [rows, k] (prepared once): ys[i] = x ws[i]^T (+ bias, one
 // weight only).  norm_w != nullptr: the RMSNorm in front of the linears is fused into the preparation (rows of at most
@@ -762,6 +864,12 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     if (count < 1 || count > 4) return fail(JITNN_HIP_EINVAL, "%d weights on one activation", count);
     if (residual && (count != 1 || bias || ws[0]->n % 4 != 0)) return fail(JITNN_HIP_EINVAL, "a residual needs one weight, no bias and rows of whole quads");
     const int k = ws[0]->k;
+    WidePlan plan;
+    if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, &plan)) {
+        const int rc = launch_prefill_wide(plan, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
+        if (rc != JITNN_HIP_ENOMEM) return rc;
+        (void)hipGetLastError();  // (no room for the dequantised weights: the kernel that decodes them as it goes needs none)
+    }
     const int mtiles = (rows + PF_BM - 1) / PF_BM, mblocks = mtiles * (PF_BM / 32);  // operands padded to whole tiles of tokens
     const int nsteps = (k + PF_BK - 1) / PF_BK;
     auto kq = [](const jitnn_hip_weight *w) { return block_values(w->fmt) == 256; };
@@ -892,6 +1000,13 @@ bool prefill_dual_ok(const jitnn_hip_weight *gate, const jitnn_hip_weight *up) {
 
 int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up, float *h, const float *x, int rows, const float *norm_w, float eps,
                         hipStream_t stream, const PfPending *pend) {
+    const jitnn_hip_weight *const pair[2] = {gate, up};
+    WidePlan plan;
+    if (wide_pays(pair, 2, rows, true, &plan)) {
+        const int rc = launch_prefill_wide(plan, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
+        if (rc != JITNN_HIP_ENOMEM) return rc;
+        (void)hipGetLastError();
+    }
     const bool kq = block_values(gate->fmt) == 256;
     const KernelRef kr = kq ? prefill_kernel_dual_k(gate->fmt) : prefill_kernel_dual_q32(gate->fmt);
     if (!kr.fn) return fail(JITNN_HIP_EUNSUPPORTED, "no many-row kernel for format %d", gate->fmt);
@@ -1684,6 +1799,25 @@ int ensure_prefill(jitnn_hip_llama *m, int tokens) {
     return JITNN_HIP_OK;
 }
 
+// Grows the thread's scratch once, to what the largest launch of a prompt pass over dequantised weights takes, instead of
+// step by step along the first layer (every growth waits for the device).
+void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
+    if (tokens <= g.gemv_max_rows) return;
+    size_t most = 0;
+    WidePlan p;
+    for (int l = 0; l < m->layers; ++l) {
+        const jitnn_hip_weight *const *w = m->w + (size_t)l * 7;
+        const struct { int which, count; bool dual; } launches[] = {
+            {JITNN_HIP_W_ATTN_Q, 3, false}, {JITNN_HIP_W_ATTN_O, 1, false}, {JITNN_HIP_W_FFN_GATE, 2, true}, {JITNN_HIP_W_FFN_DOWN, 1, false}};
+        for (const auto &c : launches) {
+            if (c.dual && !prefill_dual_ok(w[c.which], w[c.which + 1])) continue;
+            if (wide_pays(w + c.which, c.count, tokens, c.dual, &p)) most = std::max(most, wide_scratch_bytes(p, w[c.which]->k, tokens));
+        }
+    }
+    void *unused;
+    if (most && workspace(most, st, &unused)) (void)hipGetLastError();  // (no room: the launches ask again, each for its own)
+}
+
 template <int D>
 int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, const float *q, float *att, hipStream_t st) {
     const int group = m->heads / m->kv;
@@ -1916,6 +2050,7 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
     count_op(ST_PREFILL, model_weight_bytes(m) + 4ll * m->layers * 2 * (pos0 + tokens) * m->kv * m->hd + 4ll * ((long long)tokens * m->d + (logits_dev ? m->vocab : 0)));
     StatNest nest;
     const int d = m->d, T = tokens, qd = m->heads * m->hd;
+    prefill_reserve(m, T, st);
     float *xn = m->pf[0], *q = m->pf[1], *k = m->pf[2], *v = m->pf[3], *att = m->pf[4], *xa = m->pf[5], *xb = m->pf[6], *gate = m->pf[7],
           *up = m->pf[8], *h = m->pf[9];
     const float *x = x_dev;

@@ -73,6 +73,23 @@ void prefill_join_launch(const float *part, const float *bias, const float *res,
 // the join of a launch of several segments: part = per segment splits[i] arrays [m, n[i]], one segment after the other
 void prefill_join_group_launch(const float *part, const PfSegments &sg, int m, unsigned blocks, hipStream_t s);
 
+// ---- prefill_wide.hip: the product of thousands of rows, on weights dequantised into matrix-core operand order beforehand.
+// Up to three weights of one activation (or a gate / up pair) stand in wo one after the other, each padded to whole tiles of
+// 32 rt rows.
+struct PwArgs {
+    const _Float16 *wo, *xo;  // operands: [32-row block][K step of 16][512]
+    const float *inv_scale;   // [m]
+    const float *bias, *res;  // [n], [m, ld]; one segment only, not DUAL
+    float *y[3];              // [m, ld]
+    int n[3], ld[3];          // rows of the weight here, floats from one output row to the next
+    int tile0[3];             // first row tile of the segment (segments that do not exist: tiles_n)
+    int tiles_n, tiles_m, m, ksteps;
+};
+KernelRef prefill_wide_kernel_ref(bool dual, int rt);  // rt 8, 6 or 4; dual: 8
+void prefill_wide_launch(bool dual, int rt, hipStream_t s, const PwArgs &a);
+// rows of W [n, k] as operands to wo; half 0 / 1: the gate / up rows of a dual product, whose row blocks alternate in pairs
+void wide_dequant_launch(int fmt, hipStream_t s, const uint8_t *W, _Float16 *wo, int n, int k, int half);
+
 // ---- gemv_mfma.hip: gemv_mfma_kernel<fmt>
 KernelRef gemv_mfma_kernel_ref(int fmt);
 void gemv_mfma_launch(int fmt, unsigned blocks, hipStream_t s, const uint8_t *W, const float *x, const float *bias, float *y, int n, int k, int rows);

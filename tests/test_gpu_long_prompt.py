@@ -1,0 +1,62 @@
+"""The routes of long prompts - weights dequantised first, then a plain FP16 product - at the sizes where their tiles can go
+wrong, against the oracle's dequantised values in FP64 and against the same prompt in short passes."""
+import numpy as np
+import pytest
+
+from helpers import GGML_ID, norm_err, random_valid_blocks
+from test_gpu_decode import build
+
+pytestmark = pytest.mark.gpu
+
+MFMA_BAR = 2e-3  # FP16 operands, FP32 accumulation: the bar of the many-row path
+
+
+@pytest.fixture(scope="module")
+def jn():
+    import jitnn_amd
+    jitnn_amd.init()
+    return jitnn_amd
+
+
+# ragged rows, tokens and K steps (32 past a whole 64) for tiles of 192 rows, then tiles of 256 and of 128 rows; row counts that
+# are no multiple of four
+CASES = [("Q4_0", 11003, 1056, 513), ("Q4_1", 11005, 1120, 600), ("Q8_0", 11004, 1024, 768), ("Q5_1", 10930, 1184, 515),
+         ("Q4_K", 11001, 1024, 513), ("Q5_K", 11003, 1280, 600), ("Q6_K", 11136, 1024, 701), ("Q2_K", 11007, 1024, 514),
+         ("Q8_0", 12803, 1056, 1025), ("Q8_0", 2101, 4096, 3900)]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("fmt,n,k,rows", CASES)
+def test_linear_many_rows(jn, fmt, n, k, rows, bias):
+    from oracle import oracle
+    rng = np.random.default_rng(n + k + rows)
+    raw = random_valid_blocks(rng, fmt, n, k)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[0] *= 1e4
+    x[1] *= 1e-6
+    b = rng.standard_normal(n).astype(np.float32) if bias else None
+    y = jn.Gguf.linear(jn.Tensor.of(x), jn.Tensor.quantized(jn.DType[fmt], raw, n, k), jn.Tensor.of(b) if bias else None).numpy()
+    w = oracle.dequantize(GGML_ID[fmt], raw, n * k).reshape(n, k).astype(np.float64)
+    ref = x.astype(np.float64) @ w.T
+    wnorm = float(np.sqrt((w ** 2).sum() / n))
+    got = y.astype(np.float64) - (b if bias else 0.0)
+    for r in range(rows):  # row by row, against the larger of its biggest output and |x_r| * rms row norm of W
+        scale = max(float(np.abs(ref[r]).max()), float(np.linalg.norm(x[r].astype(np.float64))) * wnorm, 1e-30)
+        assert np.abs(got[r] - ref[r]).max() <= MFMA_BAR * scale + (1e-6 * np.abs(b).max() if bias else 0.0), (fmt, r)
+
+
+def test_long_prompt_equals_short_passes(jn):
+    """2900 tokens through one layer, whose q, k | v, gate | up and down launches all take the dequantised route, against the
+    same tokens in passes of 256, where none does.  Both round the same operands to FP16 and add up in FP32, in another order;
+    what differs before one rounding (2^-11) differs by one after it: the bar of one linear."""
+    cfg = dict(layers=1, d_model=1024, heads=32, kv_heads=8, head_dim=64, ffn=1536, vocab=512, max_ctx=2900, rms_eps=1e-5, rope_theta=1e4)
+    dec, *_ = build(jn, cfg, 4)
+    x = np.random.default_rng(6).standard_normal((2900, cfg["d_model"])).astype(np.float32)
+    whole = dec.prefill(x, 0)
+    k1, v1 = dec.kv_read(0, 0, 2900)
+    for p in range(0, 2900, 256):
+        parts = dec.prefill(x[p:p + 256], p)
+    k2, v2 = dec.kv_read(0, 0, 2900)
+    for a, b in ((k1, k2), (v1, v2), (whole, parts)):
+        assert np.isfinite(a).all() and norm_err(a, b) <= MFMA_BAR, norm_err(a, b)
+    dec.close()
