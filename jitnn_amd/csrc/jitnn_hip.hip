@@ -842,13 +842,13 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
 // `count` weights of one row length share the activations x [rows, k] (prepared once): ys[i] = x ws[i]^T (+ bias, one
 // weight only).  norm_w != nullptr: the RMSNorm in front of the linears is fused into the preparation (rows of at most
 // XP_MAXK values; the caller checks with prefill_prepare_fuses_norm).
-// residual != nullptr (one weight only, no bias): y = residual + x w^T, added by the join of the K slices, or, in a launch that
-// does not split K, by the kernel as it stores.
+// residual != nullptr (one weight only): y = residual + x w^T, added by the join of the K slices, or, for a launch that
+// does not split K, by a pass of its own over the product left in `tmp` [rows, n].
 // part_ext / defer (one weight with a residual): the K slices go to part_ext ([8][rows, n] floats, the caller's) and, when the
 // launch does split K, their join is left to the caller - *defer describes it, and the activation preparation of the next
 // linears can do it on the way (pend: this call's activations are that pending row, not x).
 int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, int count, const float *x, int rows, const float *bias,
-                         const float *norm_w, float eps, hipStream_t stream, const float *residual = nullptr,
+                         const float *norm_w, float eps, hipStream_t stream, const float *residual = nullptr, float *tmp = nullptr,
                          const float *swiglu_up = nullptr, ScratchSource src = SCRATCH_THREAD, float *part_ext = nullptr, PfPending *defer = nullptr,
                          const PfPending *pend = nullptr, PfGroupPending *gdefer = nullptr) {
     // (the kernels live in prefill_k.hip, prefill_q32.hip and prefill_mixed.hip)
@@ -862,7 +862,7 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     } launch[4];
     int nlaunch = 0;
     if (count < 1 || count > 4) return fail(JITNN_HIP_EINVAL, "%d weights on one activation", count);
-    if (residual && (count != 1 || bias || ws[0]->n % 4 != 0)) return fail(JITNN_HIP_EINVAL, "a residual needs one weight, no bias and rows of whole quads");
+    if (residual && (count != 1 || !tmp || ws[0]->n % 4 != 0)) return fail(JITNN_HIP_EINVAL, "a residual needs one weight, rows of whole quads and a buffer");
     const int k = ws[0]->k;
     WidePlan plan;
     if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, &plan)) {
@@ -952,18 +952,18 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
             sg.tiles[q] = tiles_of(wq);
             sg.splits[q] = l.splits[q];
             sg.split_steps[q] = l.split_steps[q];
-            sg.y[q] = split ? part + before : ys[l.first + q];
+            sg.y[q] = split ? part + before : (residual ? tmp : ys[l.first + q]);
             before += (size_t)l.splits[q] * rows * wq->n;
             gx += (unsigned)(sg.tiles[q] * sg.splits[q]);
             out.y[q] = ys[l.first + q];
             out.n[q] = wq->n;
             out.splits[q] = l.splits[q];
         }
-        const float *b1 = split ? nullptr : bias, *r1 = split ? nullptr : residual;  // (a residual: one weight, one format)
+        const float *b1 = split ? nullptr : bias;
         const dim3 grid(gx, mtiles);
         if (l.first_b < l.count) prefill_launch_mixed(w->fmt, ws[l.first + l.first_b]->fmt, l.first_b, grid, stream, sg, xo, inv, rows, k);
-        else if (kq(w)) prefill_launch_k(w->fmt, grid, stream, sg, xo, inv, b1, r1, rows, k);
-        else prefill_launch_q32(w->fmt, grid, stream, sg, xo, inv, b1, r1, rows, k);
+        else if (kq(w)) prefill_launch_k(w->fmt, grid, stream, sg, xo, inv, b1, rows, k);
+        else prefill_launch_q32(w->fmt, grid, stream, sg, xo, inv, b1, rows, k);
         if (split && l.count > 1 && gdefer && nlaunch == 1) {
             // the caller's next kernel adds the slices up as it reads them (they stay in this thread's scratch until its
             // next many-row call)
@@ -984,6 +984,11 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
             const size_t count4 = (size_t)rows * w->n / 4;
             const unsigned blocks = (unsigned)std::min<size_t>((count4 + 255) / 256, (size_t)g.cus * 8);
             prefill_join_launch(part, bias, residual, ys[l.first], count4, w->n, l.splits[0], blocks, stream);
+        } else if (residual) {
+            const size_t count4 = (size_t)rows * w->n / 4;
+            const unsigned blocks = (unsigned)std::min<size_t>((count4 + 255) / 256, (size_t)g.cus * 8);
+            hipLaunchKernelGGL(add_rows_kernel, dim3(blocks), dim3(256), 0, stream, reinterpret_cast<const float4 *>(tmp),
+                               reinterpret_cast<const float4 *>(residual), reinterpret_cast<float4 *>(ys[l.first]), count4);
         }
     }
     HIP_TRY(hipGetLastError());
@@ -1029,7 +1034,7 @@ int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up
 
 int launch_prefill(const jitnn_hip_weight *w, const float *x, int rows, const float *bias, float *y, hipStream_t stream,
                    ScratchSource src = SCRATCH_THREAD) {
-    return launch_prefill_group(&w, &y, 1, x, rows, bias, nullptr, 0.f, stream, nullptr, nullptr, src);
+    return launch_prefill_group(&w, &y, 1, x, rows, bias, nullptr, 0.f, stream, nullptr, nullptr, nullptr, src);
 }
 
 template <int FMT>
@@ -1721,7 +1726,7 @@ int normed_linears_rows(const jitnn_hip_llama *m, const jitnn_hip_weight *const 
     for (int i = 0; i < count; ++i) group = group && has_many_row_kernel(ws[i]->fmt);
     if (group) {
         const bool fused = pend && pend->part && pend->out == x && pend->n == m->d;
-        const int rc = launch_prefill_group(ws, ys, count, x, rows, nullptr, nw, m->eps, st, nullptr, nullptr, SCRATCH_THREAD, nullptr, nullptr,
+        const int rc = launch_prefill_group(ws, ys, count, x, rows, nullptr, nw, m->eps, st, nullptr, nullptr, nullptr, SCRATCH_THREAD, nullptr, nullptr,
                                             fused ? pend : nullptr, gdefer);
         if (fused) *pend = PfPending{};
         else if (pend) flush_pending(*pend, rows, st);  // (never both: a pending join is flushed before anybody reads its row)
@@ -1749,7 +1754,7 @@ int residual_linear_rows(const jitnn_hip_weight *w, const float *x, int rows, co
                          const float *up = nullptr, float *h = nullptr, float *part = nullptr, PfPending *defer = nullptr) {
     const bool many = rows > g.gemv_max_rows && has_many_row_kernel(w->fmt) && w->n % 4 == 0;
     if (many && (!up || prefill_prepare_fuses_norm(w->k))) {
-        return launch_prefill_group(&w, &y, 1, x, rows, nullptr, nullptr, 0.f, st, res, up, SCRATCH_THREAD, part, defer);
+        return launch_prefill_group(&w, &y, 1, x, rows, nullptr, nullptr, 0.f, st, res, tmp, up, SCRATCH_THREAD, part, defer);
     }
     if (up && rows_path(w, rows)) {  // silu(x) * up is formed by the preparation of the one-pass kernel
         count_op(ST_GEMV, (long long)w->nbytes + 4ll * rows * ((long long)w->k + w->n));
@@ -1760,7 +1765,7 @@ int residual_linear_rows(const jitnn_hip_weight *w, const float *x, int rows, co
         const unsigned blocks = (unsigned)std::min<long long>((count + 1023) / 1024, (long long)g.cus * 16);
         hipLaunchKernelGGL(swiglu_kernel, dim3(blocks), dim3(256), 0, st, x, up, h, (int)count);
         x = h;
-        if (many) return launch_prefill_group(&w, &y, 1, x, rows, nullptr, nullptr, 0.f, st, res);
+        if (many) return launch_prefill_group(&w, &y, 1, x, rows, nullptr, nullptr, 0.f, st, res, tmp);
     }
     if (rows_path(w, rows)) {  // the one-pass kernel adds the residual as it stores
         count_op(ST_GEMV, (long long)w->nbytes + 4ll * rows * ((long long)w->k + w->n));

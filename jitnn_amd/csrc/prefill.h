@@ -541,9 +541,8 @@ __device__ __forceinline__ void pf_load_lds(PfRaw<FMT> &r, const uint8_t *b, int
 // w % 2 and w % 2 + 2 - a gate and its up block when DUAL - x tokens [64 (w / 2), +64): half the products per wave and step.
 template <int FMT, bool DUAL = false, int RT = 4>
 __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W, const _Float16 *__restrict__ xo, const float *__restrict__ inv_scale,
-                                                  const float *__restrict__ bias, float *y, const int m, const int n, const int k,
-                                                  const int split_steps, const int tile, const int slice, const uint8_t *__restrict__ W2 = nullptr,
-                                                  const float *res = nullptr) {  // (res may be y)
+                                                  const float *__restrict__ bias, float *__restrict__ y, const int m, const int n, const int k,
+                                                  const int split_steps, const int tile, const int slice, const uint8_t *__restrict__ W2 = nullptr) {
     using Stage = PfStage<FMT>;
     constexpr bool STAGED = Stage::ON;
     extern __shared__ __align__(16) uint8_t pf_smem[];  // pf_lds_bytes<FMT>()
@@ -758,32 +757,6 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
             bv[i] = bias ? b : 0.f;
         }
     }
-    if (res) {
-        // y = res + x W^T (a residual [m, n] of a model's layer).  All of the lane's residuals are read before the first
-        // store (see above); the registers of the operands are free by now.  A pass of its own over the stored product cost
-        // 31 us per 4096 x 4096 launch.
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-            const float *rp = res + min(n0 + 32 * rblock(i) + (lane & 31), n - 1);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[i][j][r] = (acc[i][j][r] * isc[j][r] + bv[i]) + rp[(size_t)min(tok0 + 32 * j + 8 * (r >> 2) + (r & 3), m - 1) * n];
-        }
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-            const int row = n0 + 32 * rblock(i) + (lane & 31);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int tok = tok0 + 32 * j + 8 * (r >> 2) + (r & 3);
-                    if (row < n && tok < m) y[(size_t)tok * n + row] = acc[i][j][r];
-                }
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
         const int row = n0 + 32 * rblock(i) + (lane & 31);
@@ -817,15 +790,15 @@ __device__ __forceinline__ void pf_locate(const PfSegments &sg, int &seg, int &t
 
 // grid: (row tiles x K slices of all segments, token tiles); 256 threads; pf_lds_bytes<FMT>() of dynamic LDS.
 //   sg.y[i]: [m, n[i]], or for a segment that splits K the first slice's array of partial sums (slice z at + z m n[i]);
-//   bias, res [m, n]: one segment that does not split K only.
+//   bias: one segment only.
 template <int FMT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) prefill_mfma_kernel(const PfSegments sg, const _Float16 *__restrict__ xo,
                                                             const float *__restrict__ inv_scale, const float *__restrict__ bias,
-                                                            const float *res, int m, int k) {
+                                                            int m, int k) {
     int seg, tile, slice;
     pf_locate(sg, seg, tile, slice);
-    if (m <= PF_NARROW_ROWS) prefill_mfma_body<FMT, false, 2>(sg.W[seg], xo, inv_scale, bias, sg.y[seg], m, sg.n[seg], k, sg.split_steps[seg], tile, slice, nullptr, res);
-    else prefill_mfma_body<FMT>(sg.W[seg], xo, inv_scale, bias, sg.y[seg], m, sg.n[seg], k, sg.split_steps[seg], tile, slice, nullptr, res);
+    if (m <= PF_NARROW_ROWS) prefill_mfma_body<FMT, false, 2>(sg.W[seg], xo, inv_scale, bias, sg.y[seg], m, sg.n[seg], k, sg.split_steps[seg], tile, slice);
+    else prefill_mfma_body<FMT>(sg.W[seg], xo, inv_scale, bias, sg.y[seg], m, sg.n[seg], k, sg.split_steps[seg], tile, slice);
 }
 
 // The same for weights of two formats (a Q4_K_M layer keeps q and k as Q4_K and v as Q6_K): segments below first_b are

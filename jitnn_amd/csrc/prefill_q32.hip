@@ -14,12 +14,12 @@ KernelRef prefill_kernel_q32(int fmt) {
     }
 }
 
-void prefill_launch_q32(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, const float *res, int m, int k) {
+void prefill_launch_q32(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, int m, int k) {
     switch (fmt) {
-    case F_Q4_0: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q4_0>, grid, dim3(256), pf_lds_bytes<F_Q4_0>(), s, sg, xo, inv_scale, bias, res, m, k); break;
-    case F_Q4_1: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q4_1>, grid, dim3(256), pf_lds_bytes<F_Q4_1>(), s, sg, xo, inv_scale, bias, res, m, k); break;
-    case F_Q8_0: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q8_0>, grid, dim3(256), pf_lds_bytes<F_Q8_0>(), s, sg, xo, inv_scale, bias, res, m, k); break;
-    case F_Q5_1: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q5_1>, grid, dim3(256), pf_lds_bytes<F_Q5_1>(), s, sg, xo, inv_scale, bias, res, m, k); break;
+    case F_Q4_0: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q4_0>, grid, dim3(256), pf_lds_bytes<F_Q4_0>(), s, sg, xo, inv_scale, bias, m, k); break;
+    case F_Q4_1: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q4_1>, grid, dim3(256), pf_lds_bytes<F_Q4_1>(), s, sg, xo, inv_scale, bias, m, k); break;
+    case F_Q8_0: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q8_0>, grid, dim3(256), pf_lds_bytes<F_Q8_0>(), s, sg, xo, inv_scale, bias, m, k); break;
+    case F_Q5_1: hipLaunchKernelGGL(prefill_mfma_kernel<F_Q5_1>, grid, dim3(256), pf_lds_bytes<F_Q5_1>(), s, sg, xo, inv_scale, bias, m, k); break;
     default: break;
     }
 }

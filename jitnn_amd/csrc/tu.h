@@ -34,9 +34,9 @@ struct PfSegments {
 KernelRef prefill_kernel_k(int fmt);
 KernelRef prefill_kernel_q32(int fmt);
 KernelRef prefill_kernel_mixed(int fmt_a, int fmt_b);  // fn == nullptr: this pair has no kernel
-void prefill_launch_k(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, const float *res, int m, int k);
-void prefill_launch_q32(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, const float *res,
-                        int m, int k);
+void prefill_launch_k(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, int m, int k);
+void prefill_launch_q32(int fmt, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale, const float *bias, int m,
+                        int k);
 void prefill_launch_mixed(int fmt_a, int fmt_b, int first_b, dim3 grid, hipStream_t s, const PfSegments &sg, const _Float16 *xo, const float *inv_scale,
                           int m, int k);
 // prefill_dual_k.hip, prefill_dual_q32.hip: prefill_mfma_dual_kernel<fmt>, y [m, n] = silu(x W^T) * (x W2^T) for two weights
