@@ -651,6 +651,14 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     return JITNN_HIP_OK;
 }
 
+// Whether workspace() can hand out `bytes` now: it cannot grow under a stream capture, which an allocation would invalidate.
+bool workspace_fits(size_t bytes, hipStream_t stream) {
+    if (bytes <= g_ws.cap) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) (void)hipGetLastError();
+    return st == hipStreamCaptureStatusNone;
+}
+
 int workspace_done(hipStream_t stream, ScratchSource src = SCRATCH_THREAD) {
     if (src == SCRATCH_STATIC) return JITNN_HIP_OK;
     Workspace &w = g_ws;
@@ -813,7 +821,9 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
     const int mblocks = a.tiles_m * (PF_BM / 32);
     const size_t xo_bytes = (size_t)mblocks * ksteps * 1024, scale_bytes = ((size_t)rows * 8 + 255) & ~(size_t)255;
     void *wsp = nullptr;
-    if (int rc = workspace(wide_scratch_bytes(plan, k, rows), stream, &wsp)) return rc;
+    const size_t scratch = wide_scratch_bytes(plan, k, rows);
+    if (!workspace_fits(scratch, stream)) return JITNN_HIP_ENOMEM;
+    if (int rc = workspace(scratch, stream, &wsp)) return rc;
     _Float16 *xo = (_Float16 *)wsp, *wo = (_Float16 *)((uint8_t *)wsp + xo_bytes + scale_bytes);
     float *scale = (float *)((uint8_t *)wsp + xo_bytes), *inv = scale + rows;
     a.wo = wo;
@@ -1820,7 +1830,7 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
         }
     }
     void *unused;
-    if (most && workspace(most, st, &unused)) (void)hipGetLastError();  // (no room: the launches ask again, each for its own)
+    if (most && workspace_fits(most, st) && workspace(most, st, &unused)) (void)hipGetLastError();  // (no room: the launches ask again, each for its own)
 }
 
 template <int D>

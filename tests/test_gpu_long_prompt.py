@@ -60,3 +60,51 @@ def test_long_prompt_equals_short_passes(jn):
     for a, b in ((k1, k2), (v1, v2), (whole, parts)):
         assert np.isfinite(a).all() and norm_err(a, b) <= MFMA_BAR, norm_err(a, b)
     dec.close()
+
+
+def test_capture_without_room_for_the_dequantised_weights(jn):
+    """Scratch that fits the operands of the kernel that decodes as it goes, but not dequantised weights beside them, cannot
+    grow under a stream capture: the launch takes the former kernel.  In a thread of its own, whose scratch starts empty."""
+    import ctypes as C
+    import threading
+    import torch
+    from jitnn_amd import _lib as lib
+
+    rows, n, k = 3900, 2101, 4096  # (the Q8_0 case above: dequantised first when called eagerly)
+    rng = np.random.default_rng(8)
+    small = jn.Tensor.quantized(jn.DType.Q8_0, random_valid_blocks(rng, "Q8_0", 32, k), 32, k)
+    w = jn.Tensor.quantized(jn.DType.Q8_0, random_valid_blocks(rng, "Q8_0", n, k), n, k)
+    x = torch.randn(rows, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(8))
+    eager, y = torch.empty(rows, n, device="cuda"), torch.empty(rows, n, device="cuda")
+
+    def call(weight, out, stream):
+        lib.check(lib.lib.jitnn_hip_linear_dev(weight.handle, C.c_void_p(x.data_ptr()), rows, None, C.c_void_p(out.data_ptr()), C.c_void_p(stream.cuda_stream)), "linear")
+
+    call(w, eager, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    failed = []
+
+    def work():
+        try:
+            side = torch.cuda.Stream()
+            with torch.cuda.stream(side):
+                call(small, torch.empty(rows, 32, device="cuda"), side)  # the activations' operands: 32 MiB of scratch
+                side.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    call(w, y, side)
+                for i in range(3):
+                    y.fill_(float("nan"))
+                    graph.replay()
+                    side.synchronize()
+                    err = float((y - eager).abs().max() / eager.abs().max())
+                    assert err <= 1e-4, (i, err)  # the same FP16 operands, 4096 products added up in FP32 in another order
+                del graph
+        except BaseException as e:  # noqa: BLE001 (handed to the test's thread)
+            failed.append(e)
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    if failed:
+        raise failed[0]
