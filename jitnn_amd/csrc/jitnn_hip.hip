@@ -785,7 +785,9 @@ size_t wide_scratch_bytes(const WidePlan &p, int k, int rows) {
 // Q8_0 64 / 94 / 179 and 65 / 85 / 140.  Two tiles of tokens or fewer, short rows of K and launches that split K lose
 // here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
 // estimate is good to a tenth on short launches: the margins.
-bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual, WidePlan *plan) {
+// residual: prefill_mfma_kernel leaves it to add_rows_kernel (12 bytes per output at 6.5 TB/s: 31 us for 4096 x 4096), the wide
+// kernel adds it as it stores: 4096 x 4096 Q4_K at 4096 rows 143 + 31 us there, 127 + 8 here.
+bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual, bool residual, WidePlan *plan) {
     if (count > 3 || rows <= 2 * PF_BM || ws[0]->k < 1024) return false;
     const int k = ws[0]->k, mtiles = (rows + PF_BM - 1) / PF_BM, nsteps = (k + PF_BK - 1) / PF_BK;
     int n[3] = {0, 0, 0}, tiles = 0;
@@ -801,7 +803,7 @@ bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual
     *plan = wide_plan(n, dual ? 1 : count, k, mtiles, dual);
     if (wide_weight_bytes(*plan, k) > WIDE_MAX_BYTES) return false;
     if ((long long)tiles * mtiles * 2 <= g.cus) return false;
-    const double decoding = (double)(((long long)tiles * mtiles + g.cus - 1) / g.cus) * (step * nsteps + 10.0);
+    const double decoding = (double)(((long long)tiles * mtiles + g.cus - 1) / g.cus) * (step * nsteps + 10.0) + (residual ? 12.0 / 6.5e6 * rows * n[0] : 0.0);
     return plan->us + dequant < (decoding > 150.0 ? 0.95 : rows > 1024 ? 0.9 : 0.8) * decoding;
 }
 
@@ -875,7 +877,7 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     if (residual && (count != 1 || !tmp || ws[0]->n % 4 != 0)) return fail(JITNN_HIP_EINVAL, "a residual needs one weight, rows of whole quads and a buffer");
     const int k = ws[0]->k;
     WidePlan plan;
-    if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, &plan)) {
+    if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, residual != nullptr, &plan)) {
         const int rc = launch_prefill_wide(plan, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
         if (rc != JITNN_HIP_ENOMEM) return rc;
         (void)hipGetLastError();  // (no room for the dequantised weights: the kernel that decodes them as it goes needs none)
@@ -1017,7 +1019,7 @@ int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up
                         hipStream_t stream, const PfPending *pend) {
     const jitnn_hip_weight *const pair[2] = {gate, up};
     WidePlan plan;
-    if (wide_pays(pair, 2, rows, true, &plan)) {
+    if (wide_pays(pair, 2, rows, true, false, &plan)) {
         const int rc = launch_prefill_wide(plan, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
         if (rc != JITNN_HIP_ENOMEM) return rc;
         (void)hipGetLastError();
@@ -1822,11 +1824,11 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
     WidePlan p;
     for (int l = 0; l < m->layers; ++l) {
         const jitnn_hip_weight *const *w = m->w + (size_t)l * 7;
-        const struct { int which, count; bool dual; } launches[] = {
-            {JITNN_HIP_W_ATTN_Q, 3, false}, {JITNN_HIP_W_ATTN_O, 1, false}, {JITNN_HIP_W_FFN_GATE, 2, true}, {JITNN_HIP_W_FFN_DOWN, 1, false}};
+        const struct { int which, count; bool dual, residual; } launches[] = {
+            {JITNN_HIP_W_ATTN_Q, 3, false, false}, {JITNN_HIP_W_ATTN_O, 1, false, true}, {JITNN_HIP_W_FFN_GATE, 2, true, false}, {JITNN_HIP_W_FFN_DOWN, 1, false, true}};
         for (const auto &c : launches) {
             if (c.dual && !prefill_dual_ok(w[c.which], w[c.which + 1])) continue;
-            if (wide_pays(w + c.which, c.count, tokens, c.dual, &p)) most = std::max(most, wide_scratch_bytes(p, w[c.which]->k, tokens));
+            if (wide_pays(w + c.which, c.count, tokens, c.dual, c.residual, &p)) most = std::max(most, wide_scratch_bytes(p, w[c.which]->k, tokens));
         }
     }
     void *unused;
