@@ -48,6 +48,7 @@ def _bind() -> C.CDLL:
         "jitnn_hip_linear_noalloc_dev": (i, [vp, vp, i, vp, vp, vp]),
         "jitnn_hip_noalloc_scratch_bytes": (ll, []),
         "jitnn_hip_thread_release": (i, []),
+        "jitnn_hip_thread_scratch": (i, [C.POINTER(ll), C.POINTER(ll), C.POINTER(i)]),
         "jitnn_hip_quantize_q8_0": (i, [vp, ll, vp]),
         "jitnn_hip_quantize_q8_0_dev": (i, [vp, ll, vp, vp]),
         "jitnn_hip_probe_read_dev": (i, [vp, ll, vp]),
@@ -123,6 +124,13 @@ def device_info() -> dict:
     cus, hbm = C.c_int(), C.c_longlong()
     check(lib.jitnn_hip_device_info(name, 256, C.byref(cus), C.byref(hbm)), "jitnn_hip_device_info")
     return {"name": name.value.decode(), "compute_units": cus.value, "hbm_bytes": hbm.value}
+
+
+def thread_scratch() -> tuple[int, int, int]:
+    """The calling thread's many-row scratch: bytes in use, bytes kept for recorded graphs, allocations made for it."""
+    held, kept, count = C.c_longlong(), C.c_longlong(), C.c_int()
+    check(lib.jitnn_hip_thread_scratch(C.byref(held), C.byref(kept), C.byref(count)), "jitnn_hip_thread_scratch")
+    return held.value, kept.value, count.value
 
 
 class _Stat(C.Structure):

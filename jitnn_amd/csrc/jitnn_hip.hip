@@ -26,6 +26,7 @@
 #include "gguf_file.h"
 #include "glue.h"
 #include "prefill.h"
+#include "scratch.h"
 #include "tu.h"
 
 using namespace jitnn;
@@ -608,17 +609,38 @@ int launch_gemv(const jitnn_hip_weight *w, const float *x, int rows, const float
     return JITNN_HIP_OK;
 }
 
-// Per-thread device scratch for the many-row path (FP16 activations and their row scales).  It only grows; a call
-// on another stream than the last one first waits for the previous user, so concurrent streams of one thread
-// cannot overwrite each other's activations.
+// Per-thread device scratch for the many-row path.  It only grows; a call on another stream than the last one first waits
+// for the previous user, so concurrent streams of one thread cannot overwrite each other's activations.  What a call needs
+// of `operands` depends on its activations (and, where it splits K, on its outputs); dequantised weights, whose size also
+// depends on the weight and whose use depends on the route, have a block of their own, so that neither moves the other.
+// A block that a stream capture was given outlives its growth (scratch.h): a recorded graph keeps its address.
+struct DeviceMem {
+    static void *alloc(size_t bytes) {
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static bool release(void *p) {
+        if (hipFree(p) == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
+    }
+};
 struct Workspace {
-    void *ptr = nullptr;
-    size_t cap = 0;
+    ScratchBlock<DeviceMem> operands;  // FP16 activations and their row scales, partial sums of K slices
+    ScratchBlock<DeviceMem> weights;   // dequantised weights of long prompts
     hipStream_t last = nullptr;
     hipEvent_t ev = nullptr;
     bool used = false;
 };
 thread_local Workspace g_ws;
+
+bool stream_recording(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) (void)hipGetLastError();
+    return st != hipStreamCaptureStatusNone;
+}
 
 // Where a many-row launch takes its scratch from: the calling thread's grow-only buffer (may allocate), or the
 // library's static array (never allocates; the caller keeps calls on one GPU from overlapping).
@@ -636,27 +658,27 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     Workspace &w = g_ws;
     touch_thread_state();  // a thread that only ever calls the device-pointer entry points must give its scratch back too
     if (!w.ev) HIP_TRY(hipEventCreateWithFlags(&w.ev, hipEventDisableTiming));
-    if (bytes > w.cap) {
-        if (w.ptr) HIP_TRY(hipFree(w.ptr));  // waits for the device: nobody is still reading the old block
-        w.ptr = nullptr;
-        w.cap = 0;
-        const size_t want = (bytes + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
-        hipError_t e = hipMalloc(&w.ptr, want);
-        if (e != hipSuccess) return fail(JITNN_HIP_ENOMEM, "hipMalloc of %zu bytes of scratch: %s", want, hipGetErrorString(e));
-        w.cap = want;
-        w.used = false;
-    }
+    bool waited = false;
+    void *p = w.operands.get(bytes, stream_recording(stream), &waited);
+    if (!p) return fail(JITNN_HIP_ENOMEM, "no %zu bytes of device memory for scratch", bytes);
+    if (waited) w.used = false;
     if (w.used && w.last != stream) HIP_TRY(hipStreamWaitEvent(stream, w.ev, 0));
-    *out = w.ptr;
+    *out = p;
     return JITNN_HIP_OK;
 }
 
-// Whether workspace() can hand out `bytes` now: it cannot grow under a stream capture, which an allocation would invalidate.
-bool workspace_fits(size_t bytes, hipStream_t stream) {
-    if (bytes <= g_ws.cap) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &st) != hipSuccess) (void)hipGetLastError();
-    return st == hipStreamCaptureStatusNone;
+// Room for `bytes` of dequantised weights, or nullptr: the caller then takes the kernel that decodes them as it goes, which
+// needs none.  Not grown under a stream capture, which an allocation would invalidate.  Followed by workspace() and, after
+// the launches, workspace_done(), which order the two blocks together.
+_Float16 *weight_room(size_t bytes, hipStream_t stream) {
+    Workspace &w = g_ws;
+    touch_thread_state();
+    const bool recording = stream_recording(stream);
+    if (bytes > w.weights.capacity() && recording) return nullptr;
+    bool waited = false;
+    void *p = w.weights.get(bytes, recording, &waited);
+    if (waited) w.used = false;
+    return (_Float16 *)p;
 }
 
 int workspace_done(hipStream_t stream, ScratchSource src = SCRATCH_THREAD) {
@@ -695,7 +717,8 @@ struct HostStage {
 };
 void release_workspace() {
     Workspace &w = g_ws;
-    if (w.ptr) (void)hipFree(w.ptr);
+    w.operands.release_all();
+    w.weights.release_all();
     if (w.ev) (void)hipEventDestroy(w.ev);
     w = Workspace{};
 }
@@ -772,10 +795,9 @@ WidePlan wide_plan(const int *n, int count, int k, int mtiles, bool dual) {
 // Dequantised weights beyond this stay on the kernel that decodes as it goes.
 constexpr size_t WIDE_MAX_BYTES = (size_t)512 << 20;
 size_t wide_weight_bytes(const WidePlan &p, int k) { return (size_t)p.tiles_n * p.rt * pf_ksteps(k) * 1024; }
-size_t wide_scratch_bytes(const WidePlan &p, int k, int rows) {
-    const size_t mblocks = (size_t)(rows + PF_BM - 1) / PF_BM * (PF_BM / 32);
-    return mblocks * pf_ksteps(k) * 1024 + (((size_t)rows * 8 + 255) & ~(size_t)255) + wide_weight_bytes(p, k);
-}
+// what the activations of a many-row linear take as operands, and their row scales behind them
+size_t operand_bytes(int rows, int k) { return (size_t)(rows + PF_BM - 1) / PF_BM * (PF_BM / 32) * pf_ksteps(k) * 1024; }
+size_t row_scale_bytes(int rows) { return ((size_t)rows * 8 + 255) & ~(size_t)255; }
 
 // Whether `count` weights of one row length (dual: a gate and an up weight) are worth dequantising first for `rows` rows:
 // the estimate of both passes against that of prefill_mfma_kernel, which takes rounds of 128-row tiles (dual: 64 rows of each
@@ -807,8 +829,9 @@ bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual
     return plan->us + dequant < (decoding > 150.0 ? 0.95 : rows > 1024 ? 0.9 : 0.8) * decoding;
 }
 
-// The arguments are those of launch_prefill_group; dual: ws is a gate and an up weight, ys[0] = silu(x gate^T) * (x up^T).
-int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws, float *const *ys, int count, bool dual, const float *x, int rows,
+// The arguments are those of launch_prefill_group; wo: weight_room of wide_weight_bytes; dual: ws is a gate and an up weight,
+// ys[0] = silu(x gate^T) * (x up^T).
+int launch_prefill_wide(const WidePlan &plan, _Float16 *wo, const jitnn_hip_weight *const *ws, float *const *ys, int count, bool dual, const float *x, int rows,
                         const float *bias, const float *norm_w, float eps, hipStream_t stream, const float *residual, const float *swiglu_up,
                         const PfPending *pend) {
     const KernelRef kr = prefill_wide_kernel_ref(dual, plan.rt);
@@ -821,12 +844,10 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
     a.m = rows;
     a.ksteps = ksteps;
     const int mblocks = a.tiles_m * (PF_BM / 32);
-    const size_t xo_bytes = (size_t)mblocks * ksteps * 1024, scale_bytes = ((size_t)rows * 8 + 255) & ~(size_t)255;
+    const size_t xo_bytes = operand_bytes(rows, k);
     void *wsp = nullptr;
-    const size_t scratch = wide_scratch_bytes(plan, k, rows);
-    if (!workspace_fits(scratch, stream)) return JITNN_HIP_ENOMEM;
-    if (int rc = workspace(scratch, stream, &wsp)) return rc;
-    _Float16 *xo = (_Float16 *)wsp, *wo = (_Float16 *)((uint8_t *)wsp + xo_bytes + scale_bytes);
+    if (int rc = workspace(xo_bytes + row_scale_bytes(rows), stream, &wsp)) return rc;
+    _Float16 *xo = (_Float16 *)wsp;
     float *scale = (float *)((uint8_t *)wsp + xo_bytes), *inv = scale + rows;
     a.wo = wo;
     a.xo = xo;
@@ -878,9 +899,8 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     const int k = ws[0]->k;
     WidePlan plan;
     if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, residual != nullptr, &plan)) {
-        const int rc = launch_prefill_wide(plan, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
-        if (rc != JITNN_HIP_ENOMEM) return rc;
-        (void)hipGetLastError();  // (no room for the dequantised weights: the kernel that decodes them as it goes needs none)
+        if (_Float16 *wo = weight_room(wide_weight_bytes(plan, k), stream))
+            return launch_prefill_wide(plan, wo, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
     }
     const int mtiles = (rows + PF_BM - 1) / PF_BM, mblocks = mtiles * (PF_BM / 32);  // operands padded to whole tiles of tokens
     const int nsteps = (k + PF_BK - 1) / PF_BK;
@@ -941,8 +961,7 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     }
     size_t part_max = 0;
     for (int i = 0; i < nlaunch; ++i) part_max = std::max(part_max, launch[i].part_bytes);
-    const size_t xo_bytes = (size_t)mblocks * pf_ksteps(k) * 1024;
-    const size_t scale_bytes = ((size_t)rows * 8 + 255) & ~(size_t)255;
+    const size_t xo_bytes = operand_bytes(rows, k), scale_bytes = row_scale_bytes(rows);
     void *wsp = nullptr;
     if (int rc = workspace(xo_bytes + scale_bytes + part_max, stream, &wsp, src)) return rc;
     _Float16 *xo = (_Float16 *)wsp;
@@ -1020,9 +1039,8 @@ int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up
     const jitnn_hip_weight *const pair[2] = {gate, up};
     WidePlan plan;
     if (wide_pays(pair, 2, rows, true, false, &plan)) {
-        const int rc = launch_prefill_wide(plan, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
-        if (rc != JITNN_HIP_ENOMEM) return rc;
-        (void)hipGetLastError();
+        if (_Float16 *wo = weight_room(wide_weight_bytes(plan, gate->k), stream))
+            return launch_prefill_wide(plan, wo, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
     }
     const bool kq = block_values(gate->fmt) == 256;
     const KernelRef kr = kq ? prefill_kernel_dual_k(gate->fmt) : prefill_kernel_dual_q32(gate->fmt);
@@ -1030,8 +1048,7 @@ int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up
     if (int rc = allow_lds(kr.fn, kr.lds)) return rc;
     const int k = gate->k, n = gate->n;
     const int mtiles = (rows + PF_BM - 1) / PF_BM, mblocks = mtiles * (PF_BM / 32);
-    const size_t xo_bytes = (size_t)mblocks * pf_ksteps(k) * 1024;
-    const size_t scale_bytes = ((size_t)rows * 8 + 255) & ~(size_t)255;
+    const size_t xo_bytes = operand_bytes(rows, k), scale_bytes = row_scale_bytes(rows);
     void *wsp = nullptr;
     if (int rc = workspace(xo_bytes + scale_bytes, stream, &wsp, SCRATCH_THREAD)) return rc;
     _Float16 *xo = (_Float16 *)wsp;
@@ -1458,6 +1475,13 @@ int jitnn_hip_quantize_q8_0(const float *x_host, long long numel, void *blocks_h
     return JITNN_HIP_OK;
 }
 
+int jitnn_hip_thread_scratch(long long *held, long long *kept_for_graphs, int *allocations) {
+    if (held) *held = (long long)(g_ws.operands.capacity() + g_ws.weights.capacity());
+    if (kept_for_graphs) *kept_for_graphs = (long long)(g_ws.operands.retired_bytes() + g_ws.weights.retired_bytes());
+    if (allocations) *allocations = g_ws.operands.growths() + g_ws.weights.growths();
+    return JITNN_HIP_OK;
+}
+
 int jitnn_hip_thread_release(void) {
     if (!g.ready) return JITNN_HIP_OK;
     (void)hipDeviceSynchronize();
@@ -1819,8 +1843,8 @@ int ensure_prefill(jitnn_hip_llama *m, int tokens) {
 // Grows the thread's scratch once, to what the largest launch of a prompt pass over dequantised weights takes, instead of
 // step by step along the first layer (every growth waits for the device).
 void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
-    if (tokens <= g.gemv_max_rows) return;
-    size_t most = 0;
+    if (tokens <= g.gemv_max_rows || stream_recording(st)) return;
+    size_t most_weights = 0, most_operands = 0;
     WidePlan p;
     for (int l = 0; l < m->layers; ++l) {
         const jitnn_hip_weight *const *w = m->w + (size_t)l * 7;
@@ -1828,11 +1852,19 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
             {JITNN_HIP_W_ATTN_Q, 3, false, false}, {JITNN_HIP_W_ATTN_O, 1, false, true}, {JITNN_HIP_W_FFN_GATE, 2, true, false}, {JITNN_HIP_W_FFN_DOWN, 1, false, true}};
         for (const auto &c : launches) {
             if (c.dual && !prefill_dual_ok(w[c.which], w[c.which + 1])) continue;
-            if (wide_pays(w + c.which, c.count, tokens, c.dual, c.residual, &p)) most = std::max(most, wide_scratch_bytes(p, w[c.which]->k, tokens));
+            if (!wide_pays(w + c.which, c.count, tokens, c.dual, c.residual, &p)) continue;
+            const int k = w[c.which]->k;
+            most_weights = std::max(most_weights, wide_weight_bytes(p, k));
+            most_operands = std::max(most_operands, operand_bytes(tokens, k) + row_scale_bytes(tokens));
         }
     }
-    void *unused;
-    if (most && workspace_fits(most, st) && workspace(most, st, &unused)) (void)hipGetLastError();  // (no room: the launches ask again, each for its own)
+    bool waited = false;  // (where there is no room the launches ask again, each for its own)
+    if (most_weights) {
+        touch_thread_state();
+        (void)g_ws.weights.get(most_weights, false, &waited);
+        (void)g_ws.operands.get(most_operands, false, &waited);
+    }
+    if (waited) g_ws.used = false;
 }
 
 template <int D>

@@ -1,0 +1,80 @@
+// A thread's grow-only block of device memory, as a policy over an allocator: host code without any HIP, so that it can be
+// driven on a machine that has no GPU (tests/scratch_block_test.cpp).
+#pragma once
+#include <algorithm>
+#include <cstddef>
+#include <new>
+
+namespace jitnn {
+
+// Mem::alloc(bytes) -> address or nullptr; Mem::release(address) waits for the device, false: refused, the memory is still held.
+// The destructor frees nothing (thread_local objects outlive the runtime on the process's first thread): release_all() does.
+template <class Mem>
+class ScratchBlock {
+    struct Retired {
+        void *ptr;
+        size_t bytes;
+        Retired *next;
+    };
+    void *ptr_ = nullptr;
+    size_t cap_ = 0;
+    bool recorded_ = false;  // a stream capture has been given this block: a graph may hold its address
+    Retired *retired_ = nullptr;
+    size_t retired_bytes_ = 0;
+    int growths_ = 0;
+
+    static size_t round_up(size_t b) { return (b + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1); }
+
+    // Moves to a block of `want` bytes.  A block a graph may hold is retired, not freed: it lives until release_all().
+    bool grow(size_t want, bool *waited) {
+        Retired *node = ptr_ ? new (std::nothrow) Retired : nullptr;
+        if (ptr_ && !node) return false;
+        if (ptr_ && !recorded_ && Mem::release(ptr_)) {
+            ptr_ = nullptr;
+            cap_ = 0;
+            *waited = true;
+        }
+        void *p = Mem::alloc(want);
+        if (!p) {
+            delete node;
+            return false;
+        }
+        if (ptr_) {
+            *node = {ptr_, cap_, retired_};
+            retired_ = node;
+            retired_bytes_ += cap_;
+        } else {
+            delete node;
+        }
+        ptr_ = p;
+        cap_ = want;
+        recorded_ = false;
+        ++growths_;
+        return true;
+    }
+
+public:
+    // The block, of at least `bytes`, or nullptr.  recording: the caller's stream is capturing.  *waited is set where the old
+    // block was freed, which waits for the device: nothing enqueued before still runs.
+    void *get(size_t bytes, bool recording, bool *waited) {
+        // (a block that leaves a retired one behind is at least twice as large, so that the retired ones add up to less than it)
+        if (bytes > cap_ && !(recorded_ && grow(round_up(std::max(bytes, 2 * cap_)), waited)) && !grow(round_up(bytes), waited)) return nullptr;
+        if (recording) recorded_ = true;
+        return ptr_;
+    }
+    size_t capacity() const { return cap_; }
+    size_t retired_bytes() const { return retired_bytes_; }
+    int growths() const { return growths_; }  // allocations so far
+    void release_all() {
+        if (ptr_) (void)Mem::release(ptr_);
+        while (retired_) {
+            Retired *r = retired_;
+            (void)Mem::release(r->ptr);
+            retired_ = r->next;
+            delete r;
+        }
+        *this = ScratchBlock{};
+    }
+};
+
+}  // namespace jitnn

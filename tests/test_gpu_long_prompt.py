@@ -108,3 +108,78 @@ def test_capture_without_room_for_the_dequantised_weights(jn):
     t.join()
     if failed:
         raise failed[0]
+
+
+def in_thread(work):
+    """Runs work() in a thread of its own, whose scratch starts empty, and raises here what it raises there."""
+    import threading
+    failed = []
+
+    def body():
+        try:
+            work()
+        except BaseException as e:  # noqa: BLE001 (handed to the test's thread)
+            failed.append(e)
+
+    t = threading.Thread(target=body)
+    t.start()
+    t.join()
+    if failed:
+        raise failed[0]
+
+
+@pytest.mark.parametrize("case", ["same_call", "wider_weight", "more_rows"])
+def test_recorded_linear_outlives_scratch_growth(jn, case):
+    """A long linear recorded into a graph, then an eager call on the same thread that needs more scratch: the same call, which
+    only now finds room for dequantised weights; a weight of more rows; more activations.  The recorded block is kept, so a
+    replay after each gives the eager bits."""
+    import ctypes as C
+    import torch
+    from jitnn_amd import _lib as lib
+
+    rng = np.random.default_rng(9)
+    k = 4096
+    raw = {n: random_valid_blocks(rng, "Q8_0", n, k) for n in (32, 2101, 4200)}
+    w = {n: jn.Tensor.quantized(jn.DType.Q8_0, r, n, k) for n, r in raw.items()}
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(3900, k, device="cuda", generator=gen)
+    longer = torch.randn(4700, k, device="cuda", generator=gen)
+
+    def call(n, xs, out, stream):
+        lib.check(lib.lib.jitnn_hip_linear_dev(w[n].handle, C.c_void_p(xs.data_ptr()), xs.shape[0], None, C.c_void_p(out.data_ptr()), C.c_void_p(stream.cuda_stream)), "linear")
+
+    ref = torch.empty(3900, 2101, device="cuda")
+    call(2101, x, ref, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+
+    def work():
+        side = torch.cuda.Stream()
+        y = torch.empty_like(ref)
+        with torch.cuda.stream(side):
+            call(32 if case == "same_call" else 2101, x, torch.empty(3900, 4200, device="cuda"), side)
+            side.synchronize()
+            assert lib.thread_scratch()[1] == 0
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                call(2101, x, y, side)
+            for i in range(3):
+                if case == "same_call":
+                    again = torch.empty_like(ref)
+                    call(2101, x, again, side)
+                elif case == "wider_weight":
+                    call(4200, x, torch.empty(3900, 4200, device="cuda"), side)
+                else:
+                    call(2101, longer, torch.empty(4700, 2101, device="cuda"), side)
+                side.synchronize()
+                held, kept, _ = lib.thread_scratch()
+                # (the same call needs more of the other block only: nothing recorded is outgrown)
+                assert (kept == 0) if case == "same_call" else (0 < kept < held), (held, kept)
+                y.fill_(float("nan"))
+                graph.replay()
+                side.synchronize()
+                assert torch.equal(y, ref), i
+                if case == "same_call":
+                    assert torch.equal(again, ref), i
+            del graph
+
+    in_thread(work)
