@@ -659,7 +659,9 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     touch_thread_state();  // a thread that only ever calls the device-pointer entry points must give its scratch back too
     if (!w.ev) HIP_TRY(hipEventCreateWithFlags(&w.ev, hipEventDisableTiming));
     bool waited = false;
-    void *p = w.operands.get(bytes, stream_recording(stream), &waited);
+    const bool recording = stream_recording(stream);
+    void *p = w.operands.get(bytes, recording, &waited);
+    if (!p && w.weights.give_up(&waited)) p = w.operands.get(bytes, recording, &waited);  // (dequantised weights are a convenience)
     if (!p) return fail(JITNN_HIP_ENOMEM, "no %zu bytes of device memory for scratch", bytes);
     if (waited) w.used = false;
     if (w.used && w.last != stream) HIP_TRY(hipStreamWaitEvent(stream, w.ev, 0));
@@ -667,17 +669,13 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     return JITNN_HIP_OK;
 }
 
-// Room for `bytes` of dequantised weights, or nullptr: the caller then takes the kernel that decodes them as it goes, which
-// needs none.  Not grown under a stream capture, which an allocation would invalidate.  Followed by workspace() and, after
-// the launches, workspace_done(), which order the two blocks together.
+// Room for `bytes` of dequantised weights, or nullptr - without an error, and without a word to the device where that size was
+// refused before: the caller then takes the kernel that decodes them as it goes, which needs none.  Between workspace(), which
+// orders both blocks on the stream (and may give this one up), and the launches.
 _Float16 *weight_room(size_t bytes, hipStream_t stream) {
-    Workspace &w = g_ws;
-    touch_thread_state();
-    const bool recording = stream_recording(stream);
-    if (bytes > w.weights.capacity() && recording) return nullptr;
     bool waited = false;
-    void *p = w.weights.get(bytes, recording, &waited);
-    if (waited) w.used = false;
+    void *p = g_ws.weights.try_get(bytes, stream_recording(stream), &waited);
+    if (waited) g_ws.used = false;
     return (_Float16 *)p;
 }
 
@@ -829,9 +827,10 @@ bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual
     return plan->us + dequant < (decoding > 150.0 ? 0.95 : rows > 1024 ? 0.9 : 0.8) * decoding;
 }
 
-// The arguments are those of launch_prefill_group; wo: weight_room of wide_weight_bytes; dual: ws is a gate and an up weight,
-// ys[0] = silu(x gate^T) * (x up^T).
-int launch_prefill_wide(const WidePlan &plan, _Float16 *wo, const jitnn_hip_weight *const *ws, float *const *ys, int count, bool dual, const float *x, int rows,
+// The arguments are those of launch_prefill_group; dual: ws is a gate and an up weight, ys[0] = silu(x gate^T) * (x up^T).
+// WIDE_NO_ROOM: nothing was launched, there is no memory for the dequantised weights.
+constexpr int WIDE_NO_ROOM = 1;
+int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws, float *const *ys, int count, bool dual, const float *x, int rows,
                         const float *bias, const float *norm_w, float eps, hipStream_t stream, const float *residual, const float *swiglu_up,
                         const PfPending *pend) {
     const KernelRef kr = prefill_wide_kernel_ref(dual, plan.rt);
@@ -847,7 +846,8 @@ int launch_prefill_wide(const WidePlan &plan, _Float16 *wo, const jitnn_hip_weig
     const size_t xo_bytes = operand_bytes(rows, k);
     void *wsp = nullptr;
     if (int rc = workspace(xo_bytes + row_scale_bytes(rows), stream, &wsp)) return rc;
-    _Float16 *xo = (_Float16 *)wsp;
+    _Float16 *xo = (_Float16 *)wsp, *wo = weight_room(wide_weight_bytes(plan, k), stream);
+    if (!wo) return WIDE_NO_ROOM;
     float *scale = (float *)((uint8_t *)wsp + xo_bytes), *inv = scale + rows;
     a.wo = wo;
     a.xo = xo;
@@ -899,8 +899,8 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     const int k = ws[0]->k;
     WidePlan plan;
     if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, residual != nullptr, &plan)) {
-        if (_Float16 *wo = weight_room(wide_weight_bytes(plan, k), stream))
-            return launch_prefill_wide(plan, wo, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
+        const int rc = launch_prefill_wide(plan, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
+        if (rc != WIDE_NO_ROOM) return rc;
     }
     const int mtiles = (rows + PF_BM - 1) / PF_BM, mblocks = mtiles * (PF_BM / 32);  // operands padded to whole tiles of tokens
     const int nsteps = (k + PF_BK - 1) / PF_BK;
@@ -1039,8 +1039,8 @@ int launch_prefill_dual(const jitnn_hip_weight *gate, const jitnn_hip_weight *up
     const jitnn_hip_weight *const pair[2] = {gate, up};
     WidePlan plan;
     if (wide_pays(pair, 2, rows, true, false, &plan)) {
-        if (_Float16 *wo = weight_room(wide_weight_bytes(plan, gate->k), stream))
-            return launch_prefill_wide(plan, wo, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
+        const int rc = launch_prefill_wide(plan, pair, &h, 2, true, x, rows, nullptr, norm_w, eps, stream, nullptr, nullptr, pend);
+        if (rc != WIDE_NO_ROOM) return rc;
     }
     const bool kq = block_values(gate->fmt) == 256;
     const KernelRef kr = kq ? prefill_kernel_dual_k(gate->fmt) : prefill_kernel_dual_q32(gate->fmt);
@@ -1858,11 +1858,13 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
             most_operands = std::max(most_operands, operand_bytes(tokens, k) + row_scale_bytes(tokens));
         }
     }
-    bool waited = false;  // (where there is no room the launches ask again, each for its own)
+    bool waited = false;  // (where there is no room the launches ask, each for its own)
     if (most_weights) {
         touch_thread_state();
-        (void)g_ws.weights.get(most_weights, false, &waited);
-        (void)g_ws.operands.get(most_operands, false, &waited);
+        g_ws.operands.ask_again();
+        g_ws.weights.ask_again();
+        (void)g_ws.operands.try_get(most_operands, false, &waited);
+        (void)g_ws.weights.try_get(most_weights, false, &waited);
     }
     if (waited) g_ws.used = false;
 }

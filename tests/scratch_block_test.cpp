@@ -8,7 +8,7 @@
 static std::map<void *, size_t> live;  // address -> bytes
 static size_t room = (size_t)1 << 40;  // bytes the "device" has
 static bool refuse_release = false;
-static int releases = 0;
+static int asked = 0;
 
 struct BookMem {
     static size_t used() {
@@ -17,6 +17,7 @@ struct BookMem {
         return u;
     }
     static void *alloc(size_t bytes) {
+        ++asked;
         if (used() + bytes > room) return nullptr;
         static size_t next = 0x1000;
         void *p = (void *)next;
@@ -27,7 +28,6 @@ struct BookMem {
     static bool release(void *p) {
         if (refuse_release) return false;
         if (!live.erase(p)) abort();  // freed twice
-        ++releases;
         return true;
     }
 };
@@ -46,7 +46,7 @@ static void fresh() {
     live.clear();
     room = (size_t)1 << 40;
     refuse_release = false;
-    releases = 0;
+    asked = 0;
 }
 
 static void grows_and_reuses() {
@@ -112,11 +112,55 @@ static void refused_release_is_not_lost() {
     CHECK(live.empty());
 }
 
+// A call that can do without: refused, it keeps what is there, and does not ask for that size or a larger one again.
+static void refused_growth_keeps_the_block() {
+    fresh();
+    Block b;
+    bool waited = false;
+    void *p = b.try_get(10 * MiB, false, &waited);
+    CHECK(p);
+    room = 50 * MiB;
+    CHECK(!b.try_get(45 * MiB, false, &waited) && live.count(p) && b.capacity() == 10 * MiB && !waited);
+    const int before = asked;
+    CHECK(!b.try_get(45 * MiB, false, &waited) && !b.try_get(60 * MiB, false, &waited) && asked == before);
+    CHECK(b.try_get(10 * MiB, false, &waited) == p && asked == before);
+    CHECK(b.try_get(20 * MiB, false, &waited) && asked == before + 1 && waited);  // smaller than what was refused
+    room = 200 * MiB;
+    CHECK(!b.try_get(45 * MiB, false, &waited) && asked == before + 1);
+    b.ask_again();
+    CHECK(b.try_get(45 * MiB, false, &waited) && asked == before + 2);
+    CHECK(b.try_get(45 * MiB, true, &waited) && !b.try_get(60 * MiB, true, &waited) && asked == before + 2);  // no growth under a capture
+    b.release_all();
+    room = 10 * MiB;
+    CHECK(!b.try_get(11 * MiB, false, &waited));
+    b.release_all();  // forgets the refusal
+    room = 20 * MiB;
+    CHECK(b.try_get(11 * MiB, false, &waited));
+    b.release_all();
+    CHECK(live.empty());
+}
+
+// A call that cannot do without gives up the old block where there is no room for both, but never one a graph may hold.
+static void needed_growth_gives_up_the_block() {
+    fresh();
+    Block b;
+    bool waited = false;
+    room = 50 * MiB;
+    CHECK(b.get(30 * MiB, false, &waited) && b.get(40 * MiB, false, &waited) && waited && b.capacity() == 40 * MiB && live.size() == 1);
+    CHECK(!b.get(60 * MiB, false, &waited));
+    CHECK(b.get(30 * MiB, true, &waited) && !b.get(40 * MiB, false, &waited) && live.size() == 1 && b.capacity() == 30 * MiB);
+    CHECK(!b.give_up(&waited));
+    b.release_all();
+    CHECK(live.empty() && !b.give_up(&waited));
+}
+
 int main() {
 #define RUN(f) (f(), printf(#f "\n"))
     RUN(grows_and_reuses);
     RUN(recorded_block_outlives_growth);
     RUN(retired_blocks_are_bounded);
     RUN(refused_release_is_not_lost);
+    RUN(refused_growth_keeps_the_block);
+    RUN(needed_growth_gives_up_the_block);
     return 0;
 }
