@@ -1848,15 +1848,16 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
     WidePlan p;
     for (int l = 0; l < m->layers; ++l) {
         const jitnn_hip_weight *const *w = m->w + (size_t)l * 7;
-        const struct { int which, count; bool dual, residual; } launches[] = {
-            {JITNN_HIP_W_ATTN_Q, 3, false, false}, {JITNN_HIP_W_ATTN_O, 1, false, true}, {JITNN_HIP_W_FFN_GATE, 2, true, false}, {JITNN_HIP_W_FFN_DOWN, 1, false, true}};
-        for (const auto &c : launches) {
-            if (c.dual && !prefill_dual_ok(w[c.which], w[c.which + 1])) continue;
-            if (!wide_pays(w + c.which, c.count, tokens, c.dual, c.residual, &p)) continue;
-            const int k = w[c.which]->k;
+        auto want = [&](int which, int count, bool dual, bool residual) {
+            if (!wide_pays(w + which, count, tokens, dual, residual, &p)) return;
+            const int k = w[which]->k;
             most_weights = std::max(most_weights, wide_weight_bytes(p, k));
             most_operands = std::max(most_operands, operand_bytes(tokens, k) + row_scale_bytes(tokens));
-        }
+        };
+        want(JITNN_HIP_W_ATTN_Q, 3, false, false);
+        want(JITNN_HIP_W_ATTN_O, 1, false, true);
+        want(JITNN_HIP_W_FFN_GATE, 2, prefill_dual_ok(w[JITNN_HIP_W_FFN_GATE], w[JITNN_HIP_W_FFN_UP]), false);
+        want(JITNN_HIP_W_FFN_DOWN, 1, false, true);
     }
     bool waited = false;  // (where there is no room the launches ask, each for its own)
     if (most_weights) {

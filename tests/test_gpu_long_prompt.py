@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from helpers import GGML_ID, norm_err, random_valid_blocks
-from test_gpu_decode import build
+from test_gpu_decode import MIX, build
 
 pytestmark = pytest.mark.gpu
 
@@ -183,3 +183,24 @@ def test_recorded_linear_outlives_scratch_growth(jn, case):
             del graph
 
     in_thread(work)
+
+
+# every launch of the layer takes the dequantised route at 3100 tokens
+LONG = dict(layers=1, d_model=1280, heads=16, kv_heads=2, head_dim=128, ffn=1792, vocab=512, max_ctx=3100, rms_eps=1e-5, rope_theta=1e4)
+TWO_FORMATS = {**MIX, "ffn_up": "Q5_K"}  # gate and up in one launch, but not as one product
+
+
+@pytest.mark.parametrize("mix", [MIX, TWO_FORMATS], ids=["one_product", "two_formats"])
+def test_prompt_pass_grows_the_scratch_once(jn, mix):
+    """The largest launch of the layer is gate and up: the scratch is sized for it before the first launch, also where the two
+    have formats of their own.  One allocation for the operands, one for the weights."""
+    from jitnn_amd import _lib as lib
+    dec, *_ = build(jn, LONG, 4, mix)
+    x = np.random.default_rng(6).standard_normal((3100, LONG["d_model"])).astype(np.float32)
+
+    def work():
+        dec.prefill(x, 0)
+        assert lib.thread_scratch()[2] == 2, lib.thread_scratch()
+
+    in_thread(work)
+    dec.close()
