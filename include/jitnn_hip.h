@@ -69,7 +69,9 @@ JITNN_HIP_API int jitnn_hip_sync(void);
 
 /* Frees what the library keeps for the calling thread: the staging buffers and the stream of the host-pointer entry
  * points and the scratch of the many-row path (both grow on demand and are otherwise kept until the thread ends; the
- * process's first thread keeps them until the process ends).  Waits for the device first.  The counterpart of dropping
+ * process's first thread keeps them until the process ends).  That scratch is one block for the activations' operands and K
+ * slices of the largest call and, once a call has dequantised its weights first (jitnn_hip_linear), one of up to 512 MiB for
+ * those (twice that where a graph keeps an earlier one).  Waits for the device first.  The counterpart of dropping
  * a thread's derived copies (core/cpu/Gemm.java:497-515). */
 JITNN_HIP_API int jitnn_hip_thread_release(void);
 
@@ -125,15 +127,20 @@ JITNN_HIP_API int jitnn_hip_dequantize_dev(const jitnn_hip_weight *w, float *y_d
  * core/ops/Quant.java:66-80,147-187).  rows >= 1; bias may be NULL.
  * Up to 64 rows run the GEMV kernels at FP32-grade accuracy (error ~1e-6 of the largest output): FP32 arithmetic for
  * one and two rows, FP16 hi/lo splits of the activations on the matrix cores for more - 3 to 8 rows in one launch, 9 to
- * 64 rows in one pass over the weights (rows of whole 256-value columns; else in passes of 8); more rows (prefill) run the
- * dequantise-to-LDS MFMA kernel (FP16 operands, FP32 accumulation, error < 2e-3).
+ * 64 rows in one pass over the weights (rows of whole 256-value columns; else in passes of 8); more rows (prefill) run on the
+ * matrix cores (FP16 operands, FP32 accumulation, error < 2e-3) in one of two kernels: one decodes the weights on their way
+ * into LDS; the other, for more than 512 rows and at least 1024 values per weight row where an estimate finds it faster,
+ * multiplies weights that a pass before it has dequantised into the calling thread's scratch (at most 512 MiB).  Where that
+ * scratch cannot grow - no memory, or the stream is being captured - the first one runs.  Both round the same values to
+ * FP16 and give the same bits.
  * JITNN_HIP_GEMV_MAX_ROWS in the environment moves the switch. */
 JITNN_HIP_API int jitnn_hip_linear(const jitnn_hip_weight *w, const float *x_host, int rows, const float *bias_host, float *y_host);
 JITNN_HIP_API int jitnn_hip_linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, void *stream);
 
 /* jitnn_hip_linear_dev for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments, same kernels, same results;
- * where jitnn_hip_linear_dev takes the scratch of a many-row launch (FP16 activations in operand order, their row
+ * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments, same results bit for bit; the
+ * same kernels too, except that weights are never dequantised ahead of the product (long calls can take longer here).  Where
+ * jitnn_hip_linear_dev takes the scratch of a many-row launch (FP16 activations in operand order, their row
  * scales, the partial sums of K slices) from a buffer of the calling thread that it may have to allocate or grow, this
  * entry point takes it from a fixed array of jitnn_hip_noalloc_scratch_bytes() (64 MiB) that the library holds on the
  * GPU for the life of the process, and never calls hipMalloc or hipFree.  A call that needs more scratch (roughly

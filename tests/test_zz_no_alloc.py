@@ -56,6 +56,26 @@ def test_noalloc_linear_matches_linear_dev(jn):
         assert torch.equal(again, ref), (fmt, n, k, rows, "second call")
 
 
+@pytest.mark.parametrize("fmt,n,k,rows", [
+    ("Q4_0", 11003, 1056, 513), ("Q4_1", 11005, 1120, 600), ("Q8_0", 12803, 1056, 1025), ("Q5_1", 10930, 1184, 515), ("Q4_K", 11001, 1024, 513),
+    ("Q5_K", 11003, 1280, 600), ("Q6_K", 4001, 4096, 1300), ("Q2_K", 11007, 1024, 514), ("Q4_0", 4096, 14336, 2048)])
+def test_noalloc_linear_matches_linear_dev_on_dequantised_weights(jn, fmt, n, k, rows):
+    """Calls for which jitnn_hip_linear_dev dequantises the weights first (asserted: the thread's scratch holds them) and this entry
+    point does not: other kernels, the same FP16 operands and FP32 sums - the same bits, also where the activations of a row
+    differ by many orders of magnitude.  Rows, tokens and values per row past whole tiles of every kind."""
+    from jitnn_amd import _lib as lib
+    rng = np.random.default_rng(n + rows)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w = jn.Tensor.quantized(jn.DType[fmt], random_valid_blocks(rng, fmt, n, k), n, k)
+    bias = torch.randn(n, device="cuda", generator=g)
+    x = torch.randn(rows, k, device="cuda", generator=g) * torch.exp(3 * torch.randn(rows, k, device="cuda", generator=g))
+    lib.check(lib.lib.jitnn_hip_thread_release(), "jitnn_hip_thread_release")
+    ref = run(lib, "jitnn_hip_linear_dev", w, x, bias, n)
+    assert lib.thread_scratch()[0] > 2 * n * k  # (the weights, and the activations beside them)
+    got = run(lib, "jitnn_hip_linear_noalloc_dev", w, x, bias, n)
+    assert torch.isfinite(ref).all() and torch.equal(got, ref)
+
+
 def test_noalloc_linear_against_the_oracle_without_allocating_and_under_graph_replay(jn):
     """The entry point against the CPU oracle (not only against its sibling), the property it exists for - a first-ever
     call of a size no earlier call of this process has had leaves the free device memory where it was -, and a many-row
