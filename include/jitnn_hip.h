@@ -151,6 +151,13 @@ JITNN_HIP_API int jitnn_hip_linear_noalloc_dev(const jitnn_hip_weight *w, const 
                                                void *stream);
 JITNN_HIP_API long long jitnn_hip_noalloc_scratch_bytes(void);
 
+/* Which of the two kernels above a launch of more than 64 rows takes: 0 the one that decodes as it goes, otherwise the
+ * weight rows of a tile (256, 192 or 128) of the one that multiplies weights dequantised before it.  `count` (up to three)
+ * weights [n[i], k] on one activation, as the model steps launch q, k and v; gate_up: two weights whose product is formed as
+ * one SwiGLU; residual: one is added.  compute_units 0: the device's; otherwise no device is needed.  What a call then
+ * runs depends on the scratch too (jitnn_hip_linear). */
+JITNN_HIP_API int jitnn_hip_many_row_tile(const int *fmts, const int *n, int count, int k, int rows, int gate_up, int residual, int compute_units);
+
 /* ---- Q8_0 quantiser ----------------------------------------------------------------------------- */
 
 /* FP32 -> Q8_0 blocks (34 bytes per 32 values) with the reference quantiser's arithmetic: F.quantizeQ8 /

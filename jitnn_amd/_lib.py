@@ -47,6 +47,7 @@ def _bind() -> C.CDLL:
         "jitnn_hip_linear_dev": (i, [vp, vp, i, vp, vp, vp]),
         "jitnn_hip_linear_noalloc_dev": (i, [vp, vp, i, vp, vp, vp]),
         "jitnn_hip_noalloc_scratch_bytes": (ll, []),
+        "jitnn_hip_many_row_tile": (i, [C.POINTER(i), C.POINTER(i), i, i, i, i, i, i]),
         "jitnn_hip_thread_release": (i, []),
         "jitnn_hip_thread_scratch": (i, [C.POINTER(ll), C.POINTER(ll), C.POINTER(i)]),
         "jitnn_hip_quantize_q8_0": (i, [vp, ll, vp]),
@@ -131,6 +132,16 @@ def thread_scratch() -> tuple[int, int, int]:
     held, kept, count = C.c_longlong(), C.c_longlong(), C.c_int()
     check(lib.jitnn_hip_thread_scratch(C.byref(held), C.byref(kept), C.byref(count)), "jitnn_hip_thread_scratch")
     return held.value, kept.value, count.value
+
+
+def many_row_tile(weights, k: int, rows: int, gate_up: bool = False, residual: bool = False, compute_units: int = 0) -> int:
+    """Weight rows per tile of the kernel on dequantised weights if a launch of `weights` [(ggml type id, n), ...] on `rows`
+    rows takes it, 0 if it takes the kernel that decodes as it goes."""
+    fmts, n = ((C.c_int * len(weights))(*v) for v in zip(*weights))
+    tile = lib.jitnn_hip_many_row_tile(fmts, n, len(weights), k, rows, gate_up, residual, compute_units)
+    if tile < 0:
+        check(tile, "jitnn_hip_many_row_tile")
+    return tile
 
 
 class _Stat(C.Structure):

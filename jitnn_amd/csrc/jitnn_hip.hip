@@ -774,7 +774,7 @@ struct WidePlan {
     int rt = 0, tiles_n = 0;
     double us = 0;
 };
-WidePlan wide_plan(const int *n, int count, int k, int mtiles, bool dual) {
+WidePlan wide_plan(const int *n, int count, int k, int mtiles, bool dual, int cus) {
     static const struct { int rt; double step, fixed; } kinds[] = {{8, 0.78, 10.0}, {6, 0.59, 8.0}, {4, 0.44, 5.0}};
     WidePlan best;
     const int nst = pf_ksteps(k) / 2;
@@ -783,7 +783,7 @@ WidePlan wide_plan(const int *n, int count, int k, int mtiles, bool dual) {
         const int tn = dual ? 16 * kind.rt : 32 * kind.rt;
         int tiles = 0;
         for (int i = 0; i < count; ++i) tiles += (n[i] + tn - 1) / tn;
-        const int rounds = (int)(((long long)tiles * mtiles + g.cus - 1) / g.cus);
+        const int rounds = (int)(((long long)tiles * mtiles + cus - 1) / cus);
         const double us = rounds * (kind.step * nst + kind.fixed);
         if (!best.rt || us < best.us) best = {kind.rt, tiles, us};
     }
@@ -807,24 +807,34 @@ size_t row_scale_bytes(int rows) { return ((size_t)rows * 8 + 255) & ~(size_t)25
 // estimate is good to a tenth on short launches: the margins.
 // residual: prefill_mfma_kernel leaves it to add_rows_kernel (12 bytes per output at 6.5 TB/s: 31 us for 4096 x 4096), the wide
 // kernel adds it as it stores: 4096 x 4096 Q4_K at 4096 rows 143 + 31 us there, 127 + 8 here.
-bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual, bool residual, WidePlan *plan) {
-    if (count > 3 || rows <= 2 * PF_BM || ws[0]->k < 1024) return false;
-    const int k = ws[0]->k, mtiles = (rows + PF_BM - 1) / PF_BM, nsteps = (k + PF_BK - 1) / PF_BK;
+bool wide_pays(const int *fmt, const int *rows_of, int count, int k, int rows, bool dual, bool residual, int cus, WidePlan *plan) {
+    if (count > 3 || rows <= 2 * PF_BM || k < 1024) return false;
+    const int mtiles = (rows + PF_BM - 1) / PF_BM, nsteps = (k + PF_BK - 1) / PF_BK;
     int n[3] = {0, 0, 0}, tiles = 0;
     double dequant = 0, step = 0;
     for (int i = 0; i < count; ++i) {
-        const int f = ws[i]->fmt;
-        if (ws[i]->k != k || !has_many_row_kernel(f)) return false;
-        if (i == 0 || !dual) n[i] = ws[i]->n;
-        tiles += (ws[i]->n + PF_BN - 1) / PF_BN;
-        dequant += 3.0 + (f == F_Q6_K ? 0.62e-6 : 0.45e-6) * ws[i]->n * (double)k;
+        const int f = fmt[i];
+        if (!has_many_row_kernel(f)) return false;
+        if (i == 0 || !dual) n[i] = rows_of[i];
+        tiles += (rows_of[i] + PF_BN - 1) / PF_BN;
+        dequant += 3.0 + (f == F_Q6_K ? 0.62e-6 : 0.45e-6) * rows_of[i] * (double)k;
         step = std::max(step, f == F_Q4_K ? 0.87 : f == F_Q6_K ? 1.17 : 1.06);
     }
-    *plan = wide_plan(n, dual ? 1 : count, k, mtiles, dual);
+    *plan = wide_plan(n, dual ? 1 : count, k, mtiles, dual, cus);
     if (wide_weight_bytes(*plan, k) > WIDE_MAX_BYTES) return false;
-    if ((long long)tiles * mtiles * 2 <= g.cus) return false;
-    const double decoding = (double)(((long long)tiles * mtiles + g.cus - 1) / g.cus) * (step * nsteps + 10.0) + (residual ? 12.0 / 6.5e6 * rows * n[0] : 0.0);
+    if ((long long)tiles * mtiles * 2 <= cus) return false;
+    const double decoding = (double)(((long long)tiles * mtiles + cus - 1) / cus) * (step * nsteps + 10.0) + (residual ? 12.0 / 6.5e6 * rows * n[0] : 0.0);
     return plan->us + dequant < (decoding > 150.0 ? 0.95 : rows > 1024 ? 0.9 : 0.8) * decoding;
+}
+bool wide_pays(const jitnn_hip_weight *const *ws, int count, int rows, bool dual, bool residual, WidePlan *plan) {
+    int fmt[3], n[3];
+    if (count > 3) return false;
+    for (int i = 0; i < count; ++i) {
+        if (ws[i]->k != ws[0]->k) return false;
+        fmt[i] = ws[i]->fmt;
+        n[i] = ws[i]->n;
+    }
+    return wide_pays(fmt, n, count, ws[0]->k, rows, dual, residual, g.cus, plan);
 }
 
 // The arguments are those of launch_prefill_group; dual: ws is a gate and an up weight, ys[0] = silu(x gate^T) * (x up^T).
@@ -1388,6 +1398,22 @@ int jitnn_hip_linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows
 
 int jitnn_hip_linear_noalloc_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, void *stream) {
     return linear_dev(w, x_dev, rows, bias_dev, y_dev, (hipStream_t)stream, SCRATCH_STATIC);
+}
+
+int jitnn_hip_many_row_tile(const int *fmts, const int *n, int count, int k, int rows, int gate_up, int residual, int compute_units) {
+    if (!fmts || !n || count < 1 || count > 3 || k < 1 || rows < 1 || compute_units < 0) return fail(JITNN_HIP_EINVAL, "no such launch");
+    if (gate_up && (count != 2 || fmts[0] != fmts[1] || n[0] != n[1])) return fail(JITNN_HIP_EINVAL, "gate and up are two weights of one format and shape");
+    if (residual && count != 1) return fail(JITNN_HIP_EINVAL, "a residual goes with one weight");
+    for (int i = 0; i < count; ++i) {
+        const long long need = jitnn_hip_weight_nbytes(fmts[i], n[i], k);
+        if (need < 0) return (int)need;
+    }
+    if (compute_units == 0) {
+        if (int rc = check_ready()) return rc;
+        compute_units = g.cus;
+    }
+    WidePlan plan;
+    return rows > g.gemv_max_rows && wide_pays(fmts, n, count, k, rows, gate_up != 0, residual != 0, compute_units, &plan) ? 32 * plan.rt : 0;
 }
 
 long long jitnn_hip_noalloc_scratch_bytes(void) { return (long long)JITNN_HIP_SCRATCH_BYTES; }

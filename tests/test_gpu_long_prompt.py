@@ -18,17 +18,19 @@ def jn():
     return jitnn_amd
 
 
-# ragged rows, tokens and K steps (32 past a whole 64) for tiles of 192 rows, then tiles of 256 and of 128 rows; row counts that
-# are no multiple of four
-CASES = [("Q4_0", 11003, 1056, 513), ("Q4_1", 11005, 1120, 600), ("Q8_0", 11004, 1024, 768), ("Q5_1", 10930, 1184, 515),
-         ("Q4_K", 11001, 1024, 513), ("Q5_K", 11003, 1280, 600), ("Q6_K", 11136, 1024, 701), ("Q2_K", 11007, 1024, 514),
-         ("Q8_0", 12803, 1056, 1025), ("Q8_0", 2101, 4096, 3900)]
+# ragged rows, tokens and K steps (32 past a whole 64), row counts that are no multiple of four; the last column: weight rows
+# per tile of the kernel on dequantised weights
+CASES = [("Q4_0", 11003, 1056, 513, 192), ("Q4_1", 11005, 1120, 600, 192), ("Q8_0", 11004, 1024, 768, 192), ("Q5_1", 10930, 1184, 515, 192),
+         ("Q4_K", 11001, 1024, 513, 192), ("Q5_K", 11003, 1280, 600, 192), ("Q6_K", 11136, 1024, 701, 192), ("Q2_K", 11007, 1024, 514, 192),
+         ("Q8_0", 2101, 4096, 3900, 192), ("Q8_0", 12803, 1056, 1025, 256), ("Q8_0", 2751, 1056, 1300, 128), ("Q6_K", 4001, 4096, 1300, 128)]
 
 
 @pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("fmt,n,k,rows", CASES)
-def test_linear_many_rows(jn, fmt, n, k, rows, bias):
+@pytest.mark.parametrize("fmt,n,k,rows,tile", CASES)
+def test_linear_many_rows(jn, fmt, n, k, rows, tile, bias):
+    from jitnn_amd import _lib as lib
     from oracle import oracle
+    assert lib.many_row_tile([(GGML_ID[fmt], n)], k, rows) == tile
     rng = np.random.default_rng(n + k + rows)
     raw = random_valid_blocks(rng, fmt, n, k)
     x = rng.standard_normal((rows, k)).astype(np.float32)
@@ -46,8 +48,8 @@ def test_linear_many_rows(jn, fmt, n, k, rows, bias):
 
 
 def test_long_prompt_equals_short_passes(jn):
-    """2900 tokens through one layer, whose q, k | v, gate | up and down launches all take the dequantised route, against the
-    same tokens in passes of 256, where none does.  Both round the same operands to FP16 and add up in FP32, in another order;
+    """2900 tokens through one layer, whose q, k | v and gate | up launches take the dequantised route (attn_o and down do not:
+    too few tiles; test_whole_layer_on_dequantised_weights has them), against the same tokens in passes of 256, where none does.  Both round the same operands to FP16 and add up in FP32, in another order;
     what differs before one rounding (2^-11) differs by one after it: the bar of one linear."""
     cfg = dict(layers=1, d_model=1024, heads=32, kv_heads=8, head_dim=64, ffn=1536, vocab=512, max_ctx=2900, rms_eps=1e-5, rope_theta=1e4)
     dec, *_ = build(jn, cfg, 4)
@@ -97,8 +99,7 @@ def test_capture_without_room_for_the_dequantised_weights(jn):
                     y.fill_(float("nan"))
                     graph.replay()
                     side.synchronize()
-                    err = float((y - eager).abs().max() / eager.abs().max())
-                    assert err <= 1e-4, (i, err)  # the same FP16 operands, 4096 products added up in FP32 in another order
+                    assert torch.equal(y, eager), i  # the same FP16 operands, the same FP32 sums
                 del graph
         except BaseException as e:  # noqa: BLE001 (handed to the test's thread)
             failed.append(e)
@@ -185,7 +186,6 @@ def test_recorded_linear_outlives_scratch_growth(jn, case):
     in_thread(work)
 
 
-# every launch of the layer takes the dequantised route at 3100 tokens
 LONG = dict(layers=1, d_model=1280, heads=16, kv_heads=2, head_dim=128, ffn=1792, vocab=512, max_ctx=3100, rms_eps=1e-5, rope_theta=1e4)
 TWO_FORMATS = {**MIX, "ffn_up": "Q5_K"}  # gate and up in one launch, but not as one product
 
@@ -203,4 +203,43 @@ def test_prompt_pass_grows_the_scratch_once(jn, mix):
         assert lib.thread_scratch()[2] == 2, lib.thread_scratch()
 
     in_thread(work)
+    dec.close()
+
+
+# rows of every weight, and values per row, 32 past a multiple of 128: whole and ragged tiles of every launch, K steps past the end
+RAGGED = {**LONG, "d_model": 1184, "ffn": 1312}
+
+
+@pytest.mark.parametrize("cfg,mix,tiles", [(LONG, MIX, (192, 128, 256, 128)), (LONG, TWO_FORMATS, (192, 128, 256, 128)),
+                                           (RAGGED, dict.fromkeys(MIX, "Q8_0"), (192, 128, 256, 128))], ids=["one_product", "two_formats", "ragged"])
+def test_whole_layer_on_dequantised_weights(jn, cfg, mix, tiles):
+    """3100 tokens (28 past whole tiles) through two layers whose four launches all take the dequantised route: q, k and v; attn_o
+    with the residual; gate and up as one product with the SwiGLU, or as two weights whose SwiGLU is formed by the preparation
+    of down's activations; down with the residual.  Against the same tokens in passes of 256, where none of them does:
+    the same FP16 operands and FP32 sums, in another order where the short passes split K, attention in other chunks, and the last
+    28 tokens on FP32-grade kernels - the bar of one linear.  The second layer's keys and values are made of every token's output of the first: whole and ragged tiles."""
+    from jitnn_amd import _lib as lib
+    d, qd, kd, ffn, T = cfg["d_model"], cfg["heads"] * cfg["head_dim"], cfg["kv_heads"] * cfg["head_dim"], cfg["ffn"], 3100
+    one = mix["ffn_gate"] == mix["ffn_up"]
+    f = {slot: GGML_ID[name] for slot, name in mix.items()}
+
+    def routes(tokens):
+        return (lib.many_row_tile([(f["attn_q"], qd), (f["attn_k"], kd), (f["attn_v"], kd)], d, tokens), lib.many_row_tile([(f["attn_o"], d)], qd, tokens, residual=True),
+                lib.many_row_tile([(f["ffn_gate"], ffn), (f["ffn_up"], ffn)], d, tokens, gate_up=one), lib.many_row_tile([(f["ffn_down"], d)], ffn, tokens, residual=True))
+
+    assert routes(T) == tiles and routes(256) == (0, 0, 0, 0)
+    dec, *_ = build(jn, {**cfg, "layers": 2}, 4, mix, "Q8_0")
+    x = np.random.default_rng(6).standard_normal((T, d)).astype(np.float32)
+    got = {}
+
+    def whole():
+        got["logits"] = dec.prefill(x, 0)
+        assert lib.thread_scratch()[2] == 2  # (one block for the operands, one for the weights: the route was not refused)
+
+    in_thread(whole)
+    kv = [*dec.kv_read(0, 0, T), *dec.kv_read(1, 0, T)]
+    for p in range(0, T, 256):
+        parts = dec.prefill(x[p:p + 256], p)
+    for a, b in zip(kv + [got["logits"]], [*dec.kv_read(0, 0, T), *dec.kv_read(1, 0, T), parts]):
+        assert np.isfinite(a).all() and norm_err(a, b) <= MFMA_BAR, norm_err(a, b)
     dec.close()
