@@ -869,7 +869,7 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
         a.tile0[i] = tile;
         if (i >= (dual ? 1 : count)) continue;
         a.y[i] = ys[i];
-        a.n[i] = a.ld[i] = ws[i]->n;
+        a.n[i] = ws[i]->n;
         _Float16 *dst = wo + (size_t)tile * plan.rt * ksteps * 512;
         wide_dequant_launch(ws[i]->fmt, stream, ws[i]->dev, dst, ws[i]->n, k, dual ? 0 : -1);
         if (dual) wide_dequant_launch(ws[1]->fmt, stream, ws[1]->dev, dst, ws[1]->n, k, 1);

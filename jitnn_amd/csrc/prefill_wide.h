@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(PW_THREADS) __attribute__((amdgpu_waves_per_eu
         if (tn >= a.tile0[1]) seg = tn >= a.tile0[2] ? 2 : 1;
         row0 = (tn - a.tile0[seg]) * TN;
     }
-    const int n = a.n[seg], ld = a.ld[seg], m = a.m, tok0 = tm * PW_TM + 16 * TT * wc + (lane & 15), r0 = 4 * (lane >> 4);
+    const int n = a.n[seg], m = a.m, tok0 = tm * PW_TM + 16 * TT * wc + (lane & 15), r0 = 4 * (lane >> 4);
     float *y = a.y[seg];
     const float *bias = a.bias, *res = a.res;
     float isc[TT];
@@ -211,10 +211,10 @@ __global__ void __launch_bounds__(PW_THREADS) __attribute__((amdgpu_waves_per_eu
                 f32x4 rv[TT];
 #pragma unroll
                 for (int j = 0; j < TT; ++j) {
-                    if constexpr (WHOLE) rv[j] = *reinterpret_cast<const f32x4 *>(res + (size_t)(tok0 + 16 * j) * ld + row);
+                    if constexpr (WHOLE) rv[j] = *reinterpret_cast<const f32x4 *>(res + (size_t)(tok0 + 16 * j) * n + row);
                     else {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) rv[j][e] = res[(size_t)min(tok0 + 16 * j, m - 1) * ld + min(row + e, n - 1)];
+                        for (int e = 0; e < 4; ++e) rv[j][e] = res[(size_t)min(tok0 + 16 * j, m - 1) * n + min(row + e, n - 1)];
                     }
                 }
 #pragma unroll
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(PW_THREADS) __attribute__((amdgpu_waves_per_eu
             }
 #pragma unroll
             for (int j = 0; j < TT; ++j) {
-                float *yp = y + (size_t)(tok0 + 16 * j) * ld + row;
+                float *yp = y + (size_t)(tok0 + 16 * j) * n + row;
                 if constexpr (WHOLE) *reinterpret_cast<f32x4 *>(yp) = v[j];
                 else {
 #pragma unroll
@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(PW_THREADS) __attribute__((amdgpu_waves_per_eu
             }
         }
     };
-    if (tm * PW_TM + PW_TM <= m && (ld & 3) == 0 && (DUAL ? (tn + 1) * (TN / 2) : row0 + TN) <= n) finish(std::true_type{});
+    if (tm * PW_TM + PW_TM <= m && (n & 3) == 0 && (DUAL ? (tn + 1) * (TN / 2) : row0 + TN) <= n) finish(std::true_type{});
     else finish(std::false_type{});
 }
 

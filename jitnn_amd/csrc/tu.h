@@ -79,9 +79,9 @@ void prefill_join_group_launch(const float *part, const PfSegments &sg, int m, u
 struct PwArgs {
     const _Float16 *wo, *xo;  // operands: [32-row block][K step of 16][512]
     const float *inv_scale;   // [m]
-    const float *bias, *res;  // [n], [m, ld]; one segment only, not DUAL
-    float *y[3];              // [m, ld]
-    int n[3], ld[3];          // rows of the weight here, floats from one output row to the next
+    const float *bias, *res;  // [n], [m, n]; one segment only, not DUAL
+    float *y[3];              // [m, n]
+    int n[3];                 // rows of the weight
     int tile0[3];             // first row tile of the segment (segments that do not exist: tiles_n)
     int tiles_n, tiles_m, m, ksteps;
 };
