@@ -765,7 +765,7 @@ int stage_reserve(size_t pinned_bytes, size_t dev_bytes) {
     return JITNN_HIP_OK;
 }
 
-// ---- thousands of rows: weights dequantised into operand order first, then a plain FP16 product (prefill_wide.h)
+// ---- more than 512 rows: weights dequantised into operand order first, then a plain FP16 product (prefill_wide.h)
 
 // The weight rows of a tile (32 rt) and the microseconds the product should take: whole rounds of one tile per CU, each
 // `step` per 32 values of K and `fixed` for its prologue and epilogue (measured on whole rounds: 4096 x 4096 x 4096 tokens
@@ -804,7 +804,10 @@ size_t row_scale_bytes(int rows) { return ((size_t)rows * 8 + 255) & ~(size_t)25
 // and 228 / 292 / 486; 11008 x 4096 Q4_0 162 / 245 / 488 and 111 / 194 / 361; 4096 x 4096 Q4_K 58 / 85 / 160 and 65 / 84 / 139;
 // Q8_0 64 / 94 / 179 and 65 / 85 / 140.  Two tiles of tokens or fewer, short rows of K and launches that split K lose
 // here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
-// estimate is good to a tenth on short launches: the margins.
+// estimate is good to a tenth on short launches: the margins.  For the 8B gate / up pair it errs against this route: at 4096
+// rows 920 us estimated there and 970 measured, 828 estimated here and 800 measured, so that with the margin it is
+// taken at 2049 - 2304, 2561 - 2816, 3073 - 3328 and 3585 - 4096 rows, where the product's last round is full enough, and not
+// wherever it would win.
 // residual: prefill_mfma_kernel leaves it to add_rows_kernel (12 bytes per output at 6.5 TB/s: 31 us for 4096 x 4096), the wide
 // kernel adds it as it stores: 4096 x 4096 Q4_K at 4096 rows 143 + 31 us there, 127 + 8 here.
 bool wide_pays(const int *fmt, const int *rows_of, int count, int k, int rows, bool dual, bool residual, int cus, WidePlan *plan) {

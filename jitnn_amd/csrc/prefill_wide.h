@@ -1,10 +1,11 @@
-// Many-row linear for long prompts (thousands of rows): y[M, N] = x[M, K] W[N, K]^T in two passes.
+// Many-row linear for long calls (more than 512 rows): y[M, N] = x[M, K] W[N, K]^T in two passes.
 //   1. wide_dequant_kernel writes the weights once per call as FP16 in matrix-core operand order (the decoders, and so the
 //      values, are those of prefill.h), 2 bytes per value into the calling thread's scratch;
 //   2. prefill_wide_kernel is then a plain FP16 product: both operands go from memory straight into LDS.
 // prefill_mfma_kernel decodes a weight once per 256 tokens, in the instruction stream of its one wave per SIMD; here a
 // weight is decoded once, and the product has no vector arithmetic left in its loop.  What the first pass costs (2.6 bytes
-// moved per value: 27 us for a Q4_K 14336 x 4096 weight) is paid back from about two thousand rows on (wide_pays).
+// moved per value: 37 us for a Q4_K 14336 x 4096 weight) is paid back where wide_pays estimates it to be: from 513 rows on for a
+// single weight that fills the chip, from 1025 (down) to 1875 (attn_o) rows on in an 8B layer, for its gate / up in ranges above 2048.
 #pragma once
 #include "common.h"
 #include "prefill.h"
@@ -19,8 +20,8 @@ constexpr int PW_TM = 256, PW_STAGES = 4, PW_THREADS = 512;
 // W [n, k] -> wo: 1 KiB pieces [32-row block][K step of 16][lane][8], lane l holding row 32 rb + l % 32, values
 // 16 ks + 8 (l / 32) .. + 7 in the order 0, 2, 1, 3 of each group of four (as x_to_operand_kernel stores the activations).
 // grid (32-row blocks, ceil(K / 1024)), a wave takes 32 rows x 256 values: the lanes of a store write 512 consecutive
-// bytes, and the loads - 32 rows a stride apart - use up their cache lines within the wave.  Bound by its stores: 5.6 TB/s
-// moved on Q4_K, 4.4 on Q6_K (a large copy: 5.2).  half >= 0: the row blocks of a gate (0) and an up (1) weight alternate in
+// bytes, and the loads - 32 rows a stride apart - use up their cache lines within the wave.  Bound by memory, four
+// fifths of it stores: 4.1 TB/s moved on Q4_K, 3.1 on Q6_K (14336 x 4096 values; a large copy: 5.2).  half >= 0: the row blocks of a gate (0) and an up (1) weight alternate in
 // pairs, as the dual form of the product wants them.  Values past the end of a row repeat its last ones and meet zeros.
 template <int FMT>
 __global__ void __launch_bounds__(256) wide_dequant_kernel(const uint8_t *__restrict__ W, _Float16 *__restrict__ wo, int n, int k, int half) {
@@ -63,9 +64,10 @@ __device__ __forceinline__ void pw_dma(const void *g, _Float16 *l) {
 //   * one barrier per step, in its middle: it says that the next step has arrived and that this one has been read.  The
 //     operands of the first half of a step's products are read under the second half of the step before, those of the second
 //     half under the first - no product waits for a read just issued.
-//   * v_mfma_f32_16x16x32_f16 and not 32x32x16: with random operands the chip is held by its power, and the smaller tile
-//     with the longer K moves half the accumulator bytes per multiply-add.  Products alone: 1825 against 1621 TFLOP/s; this
-//     kernel on 4096 x 14336 x 4096 tokens: 1345 against 1255 (on zeros, where power does not count: 1850).
+//   * v_mfma_f32_16x16x32_f16 and not 32x32x16: with operands that toggle the chip is held by its power, and the smaller tile
+//     with the longer K moves half the accumulator bytes per multiply-add.  Products alone, normal operands: 1990 against 1740
+//     TFLOP/s (zeros: 2440 and 2470).  This kernel on 4096 x 14336 x 4096 tokens: 1380, on zero activations 1840; the matrix
+//     cores are busy 82 % of its cycles, at 1.6 GHz.
 // RT = 8 where its tiles fill the device, 6 and 4 for launches whose last round would be half empty (wide_plan).  DUAL: as in
 // prefill_mfma_body; a wave's first RT / 2 tiles of rows are gate rows, the others the same rows of the up weight.
 template <bool DUAL, int RT>

@@ -10,19 +10,30 @@ from helpers import GGML_ID
 LAYER = [(65, (0, 0, 0, 0)),
          (512, (0, 0, 0, 0)),
          (513, (0, 0, 0, 0)),
-         (600, (0, 0, 0, 0)),
          (1024, (0, 0, 0, 0)),
-         (1100, (0, 0, 0, 128)),
-         (1500, (192, 0, 0, 128)),
-         (2000, (256, 128, 0, 128)),
+         (1025, (0, 0, 0, 128)),
+         (1280, (0, 0, 0, 128)),
+         (1281, (192, 0, 0, 128)),
+         (1792, (192, 0, 0, 128)),
+         (1793, (256, 0, 0, 128)),
+         (1874, (256, 0, 0, 128)),
+         (1875, (256, 128, 0, 128)),
          (2048, (256, 128, 0, 128)),
+         (2049, (256, 192, 256, 192)),
+         (2304, (256, 192, 256, 192)),
+         (2305, (256, 192, 0, 192)),
          (2560, (256, 192, 0, 192)),
+         (2561, (192, 192, 256, 192)),
+         (2816, (192, 192, 256, 192)),
+         (2817, (192, 256, 0, 256)),
          (3072, (192, 256, 0, 256)),
          (3073, (192, 256, 256, 256)),
          (3328, (192, 256, 256, 256)),
          (3329, (192, 256, 0, 256)),
          (3584, (192, 256, 0, 256)),
          (3585, (192, 256, 256, 256)),
+         (3840, (192, 256, 256, 256)),
+         (3841, (128, 256, 256, 256)),
          (4096, (128, 256, 256, 256))]
 
 
