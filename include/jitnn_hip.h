@@ -233,7 +233,7 @@ JITNN_HIP_API int jitnn_hip_gguf_tensor_read(const jitnn_hip_gguf *f, const char
  * JITNN_HIP_EUNSUPPORTED. */
 JITNN_HIP_API int jitnn_hip_gguf_tensor_upload(const jitnn_hip_gguf *f, const char *name, jitnn_hip_weight **out);
 
-/* ---- Llama-style decode step on quantised weights ----------------------------- */
+/* ---- Llama-style decode step on quantised weights --------------------------------------------- */
 
 /* The reference has no quantised Llama and no KV-cache operator; the step is the composition of its operators as
  * Llama.Block.forward defines it (jitnn-nn/src/main/java/ai/beestream/jitnn/nn/models/Llama.java:167-174,209-222)

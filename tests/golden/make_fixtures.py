@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Cut the data fixtures this repository's tests use out of the reference's test resources.
 
-Run in the build container only (the reference tree is not present on the GPU box):
+Run where the reference tree is present:
 
     python tests/golden/make_fixtures.py [/root/reference]
 

@@ -105,7 +105,7 @@ def test_decode_small_model(jn, mix_name):
 
 
 def test_decode_8b_shaped_layer(jn):
-    """One layer at the 8B shape of BASELINE config 5 (d_model 4096, 32/8 heads of 128, FFN 14336, context 512) with a
+    """One layer at the 8B shape (d_model 4096, 32/8 heads of 128, FFN 14336, context 512) with a
     cut-down vocabulary, Q4_K_M mix."""
     cfg = dict(layers=1, d_model=4096, heads=32, kv_heads=8, head_dim=128, ffn=14336, vocab=2048, max_ctx=513, rms_eps=1e-5, rope_theta=5e5)
     dec, layers, out_norm, out_w = build(jn, cfg, 9)

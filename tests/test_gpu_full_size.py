@@ -1,4 +1,4 @@
-"""The BASELINE configurations at their full sizes.  The oracle is a scalar FP64 loop (a third of a second per 58 M
+"""The benchmark's linears at their full sizes.  The oracle is a scalar FP64 loop (a third of a second per 58 M
 weights and activation row), so at these sizes the whole matrix is checked through properties that do not depend on
 the size - linearity in x, unit vectors give columns of the dequantised matrix, a batch agrees with its rows taken
 one at a time, the many-row path agrees with the GEMV path - and directly against the oracle on a sample of rows
@@ -10,7 +10,7 @@ from helpers import BLOCK, GGML_ID, norm_err, random_valid_blocks
 
 pytestmark = pytest.mark.gpu
 
-CONFIGS = [  # (format, n, k, batch sizes): BASELINE configs 1-4, and the 16 / 40 / 64 rows bench.py times on configs 1-3's matrices
+CONFIGS = [  # (format, n, k, batch sizes): the benchmark's four weights, and the 16 / 40 / 64 rows bench.py times on the first three
     ("Q8_0", 4096, 4096, (1, 40)),
     ("Q4_0", 11008, 4096, (1, 4, 40)),
     ("Q4_K", 14336, 4096, (1, 2, 8, 16, 40, 64)),
@@ -36,7 +36,7 @@ def rows_of(raw, fmt, k, sel):
 
 
 def baseline_weight(fmt, n, k, seed):
-    """The BASELINE configurations' weight: FP32 [n, k] drawn from N(0, 0.02) and quantised to fmt - Q8_0 with the
+    """A weight of the benchmark: FP32 [n, k] drawn from N(0, 0.02) and quantised to fmt - Q8_0 with the
     reference's own quantiser as the oracle restates it (Quant.java:102-118), the others with quantizers.py; drawn
     and quantised on the GPU by torch in row chunks (set-up only: the bytes then go to the oracle and the library)."""
     import torch
