@@ -3,7 +3,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--quick]
 
-Headline workload (BASELINE.json configs[2], batch 1): Q4_K GEMV, weight 14336x4096 drawn from N(0, 0.02)
+Headline workload (batch 1): Q4_K GEMV, weight 14336x4096 drawn from N(0, 0.02)
 and quantised to Q4_K, activation N(0, 1) [1, 4096].  One "step" is one GEMV launch through the C ABI
 (jitnn_hip_linear_dev) with weights, activations and outputs resident in HBM.  Consecutive steps rotate over
 16 distinct copies of the weight (528 MB > the 256 MB Infinity Cache) so that every step streams its weight
@@ -13,7 +13,9 @@ Prints ONE JSON line: metric/value = achieved GB/s of algorithmic bytes (weight 
 the wall-clock of the timed region; "roofline" prices the same bytes against the kernel's average launch
 duration measured with HIP events on the launch stream; "cpu_baseline" is the CPU oracle (a C restatement of
 the reference's scalar host loop, Gguf.MatVec.reference) timed on this box's host cores on the same weights
-and activations; "configs" holds the other BASELINE configurations, measured the same way with fewer steps.
+and activations; "configs" holds the other weights and batch sizes, measured the same way with fewer steps.
+The line is kept short (nested figures to five digits; no launch-shape sweep, no descriptions of the samples): the whole
+record, as one JSON object, goes to stderr.
 """
 from __future__ import annotations
 
@@ -345,7 +347,7 @@ def wrap(lib, fmt, t, n, k):
 
 
 def bench_decode(torch, lib, steps, warmup):
-    """32 layers, d_model 4096, 32/8 heads of 128, FFN 14336, vocab 128256, Q4_K_M mix (Q4_K; Q6_K for
+    """The decode step of the Llama-8B shape: 32 layers, d_model 4096, 32/8 heads of 128, FFN 14336, vocab 128256, Q4_K_M mix (Q4_K; Q6_K for
     attn_v, ffn_down, output), FP32 KV cache pre-filled with N(0,1) at context 512, one token per step.  Every layer
     has its own copy of the weights in HBM (the values of layer 0 repeated: the step streams 4.9 GB)."""
     import jitnn_amd
@@ -633,6 +635,25 @@ def bench_codec(torch, lib, with_cpu):
     return out
 
 
+# what only the whole record holds of the measurements beside the headline
+DETAIL = {"workload", "steps", "bytes_per_step", "us_per_step_wall_regions", "sample", "copies", "bytes_per_call", "roofline_launches_timed",
+          "pure_read_GBps", "GBps_events", "us_per_step_events", "dequantize_ms", "pack_and_gemm_ms", "unit", "kind", "cores"}
+
+
+def brief(line: dict) -> dict:
+    """The record as one short line: the headline whole but for its launch-shape sweep, the other measurements without DETAIL,
+    figures below the top level to five digits."""
+    def cut(o, drop):
+        if isinstance(o, float):
+            return float(f"{o:.5g}")
+        if isinstance(o, dict):
+            return {k: cut(v, drop) for k, v in o.items() if k not in drop}
+        return o
+
+    others = ("configs", "decode", "prefill", "codec")
+    return {k: cut(v, DETAIL if k in others else {"pure_read_sweep"}) if isinstance(v, dict) else v for k, v in line.items()}
+
+
 def main() -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -728,7 +749,7 @@ def main() -> int:
         "vs_baseline": None,
         "dtype": "f32",
         "data": "synthetic",
-        "config": {"workload": "Q4_K GEMV 14336x4096 batch 1 (BASELINE configs[2]), weights N(0,0.02) quantised to Q4_K, x N(0,1); "
+        "config": {"workload": "Q4_K GEMV 14336x4096 batch 1, weights N(0,0.02) quantised to Q4_K, x N(0,1); "
                                "16 weight copies rotated per step (528 MB > 256 MB Infinity Cache)",
                    "bytes_per_step": head_bytes, "device": info["name"], "compute_units": info["compute_units"],
                    "cache_resident_GBps": head_bytes * 2000 / hot_ev / 1e9, "parity_norm_err": head["parity_norm_err"],
@@ -747,7 +768,8 @@ def main() -> int:
         "prefill": prefill,
         "codec": codec,
     }
-    print(json.dumps(line))
+    print(json.dumps(line), file=sys.stderr, flush=True)
+    print(json.dumps(brief(line)))
     return 0
 
 
