@@ -78,7 +78,7 @@ JITNN_HIP_API int jitnn_hip_thread_release(void);
 /* The calling thread's many-row scratch, in bytes of device memory: what its calls use now, and what was outgrown but is
  * kept because a stream capture was given it (a recorded graph goes on using the address it was recorded with; less than
  * what is in use, and given back by jitnn_hip_thread_release, after which such graphs must not run).  *allocations: how often
- * it was allocated or grown since then.  Any out pointer may be NULL; needs no device. */
+ * it was allocated or grown since the thread's start or its last release.  Any out pointer may be NULL; needs no device. */
 JITNN_HIP_API int jitnn_hip_thread_scratch(long long *held, long long *kept_for_graphs, int *allocations);
 
 /* ---- block formats (no device needed) ------------------------------------------------------------ */
