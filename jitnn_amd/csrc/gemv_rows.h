@@ -176,12 +176,14 @@ struct RStaged {
         for (int i = 0; i < FULL; ++i) r.c[i] = ld128<ALIGN>(q + 64 * i);
         if constexpr (REST > 0) r.c[FULL] = ld128<ALIGN>(q + p.rest);  // (lanes past 16 REST repeat rows: the same lines)
     }
-    // -> this lane's row (lane & 15 of the tile) in the wave's stage
+    // -> this lane's row (lane & 15 of the tile) in the wave's stage.  ALL_LANES: the lanes that repeat rows in the load of the odd
+    // chunks store them too (the same bytes), and nothing is conditional
+    template <bool ALL_LANES = false>
     __device__ static __forceinline__ const uint8_t *park(const Raw &r, uint8_t *stage, int lane) {
 #pragma unroll
         for (int i = 0; i < FULL; ++i) *reinterpret_cast<u32x4 *>(stage + (lane >> 2) * STRIDE + 16 * (lane & 3) + 64 * i) = r.c[i];
         if constexpr (REST > 0) {
-            if (lane < 16 * REST) *reinterpret_cast<u32x4 *>(stage + (lane / RD) * STRIDE + 16 * (4 * FULL + lane % RD)) = r.c[FULL];
+            if (ALL_LANES || lane < 16 * REST) *reinterpret_cast<u32x4 *>(stage + ((lane / RD) & 15) * STRIDE + 16 * (4 * FULL + lane % RD)) = r.c[FULL];
         }
         // the lanes of a wave run in step and LDS serves them in order: a fence for the compiler is all this needs
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -201,8 +203,7 @@ struct RTile<F_Q4_K> : RStaged<144, 144, 16> {
         u32x2 q[4];
     };
     // B[s]: sc_s * q of sub-block s; Bm: the eight mins in the first eight K slots; d, dmin of the super-block
-    __device__ static __forceinline__ void decode(const Raw &raw, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
-        const uint8_t *p = park(raw, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *p, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
         const int kq = lane >> 4;
         Fields r;
         r.h = *reinterpret_cast<const u32x4 *>(p);
@@ -236,8 +237,7 @@ struct RTile<F_Q5_K> : RStaged<176, 176, 16> {
         u32x2 qh;
         u32x2 q[4];
     };
-    __device__ static __forceinline__ void decode(const Raw &raw, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
-        const uint8_t *p = park(raw, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *p, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
         const int kq = lane >> 4;
         Fields r;
         r.h = *reinterpret_cast<const u32x4 *>(p);
@@ -291,8 +291,7 @@ struct RTile<F_Q6_K> : RStaged<210, 208, 2> {
         RStaged<210, 208, 2>::load(r, p, c);
         r.tail = ld16(p.full + (size_t)c * BYTES + p.row + 208);
     }
-    __device__ static __forceinline__ void decode(const Raw &raw, uint8_t *stage, int lane, f16x8 (&B)[16], f16x8 &Bm, float &d, float &dmin) {
-        const uint8_t *p = park(raw, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *p, uint32_t tail, int lane, f16x8 (&B)[16], f16x8 &Bm, float &d, float &dmin) {
         Fields r;
         {
             const int kq = lane >> 4;
@@ -302,7 +301,7 @@ struct RTile<F_Q6_K> : RStaged<210, 208, 2> {
             for (int n = 0; n < 2; ++n) r.qh[n] = *reinterpret_cast<const u32x2 *>(p + 128 + 32 * n + 8 * kq);
             r.sc = *reinterpret_cast<const u32x4 *>(p + 192);
         }
-        d = h2f(raw.tail);
+        d = h2f(tail);
         dmin = d;  // the offset term is 32 * sc per group: y += d * (sum sc q x - 32 sum sc S)
         // FP16 64 + b with b in bits 4..7 of a half-word, 16 + a with a in bits 6, 7 (1024 + b, as the 6-bit scales of Q4_K
         // allow, would overflow: 1024 * 128)
@@ -355,8 +354,7 @@ template <>
 struct RTile<F_Q4_0> : RStaged<8 * 18, 144, 2> {
     static constexpr int NOPS = 8, SUMS = 32;
     static constexpr bool BLOCK_SCALES = true, HALVES = true, MINS = false;
-    __device__ static __forceinline__ void decode(const Raw &r, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
-        const uint8_t *row = park(r, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *row, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
         const int kq = lane >> 4;
         const uint32_t mg = magic1024();
         const f16x2 off = splat2(-1032.f);  // -1024 of the exponent trick, -8 of the format
@@ -376,8 +374,7 @@ template <>
 struct RTile<F_Q4_1> : RStaged<8 * 20, 176, 4> {
     static constexpr int NOPS = 8, SUMS = 32;
     static constexpr bool BLOCK_SCALES = true, HALVES = true, MINS = true;
-    __device__ static __forceinline__ void decode(const Raw &r, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
-        const uint8_t *row = park(r, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *row, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
         const int kq = lane >> 4;
         const uint32_t mg = magic1024();
         const f16x2 off = splat2(-1024.f);
@@ -402,8 +399,7 @@ template <>
 struct RTile<F_Q8_0> : RStaged<8 * 34, 272, 2> {
     static constexpr int NOPS = 8, SUMS = 32;
     static constexpr bool BLOCK_SCALES = true, HALVES = false, MINS = false;
-    __device__ static __forceinline__ void decode(const Raw &r, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
-        const uint8_t *row = park(r, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *row, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
         const int kq = lane >> 4;
         const uint32_t mg = magic1024();
         const f16x2 off = splat2(-1152.f);  // -1024 of the exponent trick, -128 of the sign flip below
@@ -427,8 +423,7 @@ template <>
 struct RTile<F_Q5_1> : RStaged<8 * 24, 208, 16> {
     static constexpr int NOPS = 8, SUMS = 32;
     static constexpr bool BLOCK_SCALES = true, HALVES = true, MINS = true;
-    __device__ static __forceinline__ void decode(const Raw &r, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
-        const uint8_t *row = park(r, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *row, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
         const int kq = lane >> 4;
         const uint32_t mg = magic1024();
         const f16x2 off = splat2(-1024.f);
@@ -467,15 +462,14 @@ struct RTile<F_Q2_K> : RStaged<84, 80, 4> {
         RStaged<84, 80, 4>::load(r, p, c);
         r.tail = ld32<4>(p.full + (size_t)c * BYTES + p.row + 80);
     }
-    __device__ static __forceinline__ void decode(const Raw &raw, uint8_t *stage, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
-        const uint8_t *p = park(raw, stage, lane);
+    __device__ static __forceinline__ void decode(const uint8_t *p, uint32_t tail, int lane, f16x8 (&B)[8], f16x8 &Bm, float &d, float &dmin) {
         const int kq = lane >> 4;
         const u32x4 sc = *reinterpret_cast<const u32x4 *>(p);
         u32x2 q[2];
 #pragma unroll
         for (int n = 0; n < 2; ++n) q[n] = *reinterpret_cast<const u32x2 *>(p + 16 + 32 * n + 8 * kq);
-        d = h2f(raw.tail);
-        dmin = h2f(raw.tail >> 16);
+        d = h2f(tail);
+        dmin = h2f(tail >> 16);
         const uint32_t mg = magic1024();
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -587,10 +581,10 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_rows_kernel(const uint8_t *__
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 if constexpr (R::BLOCK_SCALES) {
-                    R::decode(raw[t], stage + t * R::STAGE_BYTES, lane, B[t], Bm[t], dblk[t]);
+                    R::decode(R::park(raw[t], stage + t * R::STAGE_BYTES, lane), raw[t].tail, lane, B[t], Bm[t], dblk[t]);
                 } else {
                     float dm;
-                    R::decode(raw[t], stage + t * R::STAGE_BYTES, lane, B[t], Bm[t], d[t], dm);
+                    R::decode(R::park(raw[t], stage + t * R::STAGE_BYTES, lane), raw[t].tail, lane, B[t], Bm[t], d[t], dm);
                     dmin64[t] = dm * 64.f;
                 }
             }

@@ -1,5 +1,7 @@
-// gemv_rows_kernel: the formats it is built for.
-#include "gemv_rows.h"
+// gemv_rows_kernel: the formats it is built for, and which launches are gemv_held_kernel's instead.
+#include <algorithm>
+
+#include "gemv_held.h"
 #include "tu.h"
 
 namespace jitnn {
@@ -24,6 +26,22 @@ static int tiles_per_wave(int fmt, int n, int k, int rows, unsigned max_blocks) 
     bool half = fmt == F_Q6_K && rows > 16 && k >= 8192;
     if (rows > 32 && k >= 4096 && (fmt == F_Q4_K || fmt == F_Q5_K || fmt == F_Q6_K || fmt == F_Q4_1)) half = true;
     return pairs >= max_blocks || (half && 2 * pairs >= max_blocks) ? 2 : 1;
+}
+
+struct RowsGeo {
+    int tiles, batches, shares;  // tiles per wave, batches of them, workgroups that share out the groups of rows of one
+};
+static RowsGeo rows_geometry(int fmt, int n, int k, int rows, unsigned max_blocks) {
+    const int T = tiles_per_wave(fmt, n, k, rows, max_blocks), nbatch = ((n + 15) / 16 + T - 1) / T, groups = (rows + 7) / 8;
+    // Few tiles: the groups of activation rows are shared out over as many workgroups per tile as the device has room for -
+    // each decodes the tile's weights again (the device would idle otherwise) and writes whole outputs of its own rows.
+    // 1024 x 4096 at 40 rows: Q6_K 30.0 -> 19.4 us, Q4_K 17.5 -> 13.5; twice as many workgroups as CUs: 23.4, 13.9.
+    int gy = 1;
+    if ((unsigned)nbatch * 2 <= max_blocks) {
+        const int cap = (int)(max_blocks / (unsigned)nbatch), gper = (groups + cap - 1) / cap;
+        gy = (groups + gper - 1) / gper;
+    }
+    return {T, nbatch, gy};
 }
 
 template <int FMT>
@@ -88,16 +106,9 @@ static void launch(unsigned max_blocks, hipStream_t s, const uint8_t *W, const v
     const int groups = (rows + 7) / 8;
     const _Float16 *ops = reinterpret_cast<const _Float16 *>(scratch);
     const float *inv = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(scratch) + gemv_rows_ops_bytes(groups, k));
-    const int T = tiles_per_wave(FMT, n, k, rows, max_blocks), nbatch = ((n + 15) / 16 + T - 1) / T;
-    const unsigned blocks = (unsigned)nbatch < max_blocks ? (unsigned)nbatch : max_blocks;
-    // Few tiles: the groups of activation rows are shared out over as many workgroups per tile as the device has room for -
-    // each decodes the tile's weights again (the device would idle otherwise) and writes whole outputs of its own rows.
-    // 1024 x 4096 at 40 rows: Q6_K 30.0 -> 19.4 us, Q4_K 17.5 -> 13.5; twice as many workgroups as CUs: 23.4, 13.9.
-    int gy = 1;
-    if ((unsigned)nbatch * 2 <= max_blocks) {
-        const int cap = (int)(max_blocks / (unsigned)nbatch), gper = (groups + cap - 1) / cap;
-        gy = (groups + gper - 1) / gper;
-    }
+    const RowsGeo geo = rows_geometry(FMT, n, k, rows, max_blocks);
+    const int T = geo.tiles, gy = geo.shares;
+    const unsigned blocks = (unsigned)geo.batches < max_blocks ? (unsigned)geo.batches : max_blocks;
     if (T == 2) hipLaunchKernelGGL((gemv_rows_kernel<FMT, 2>), dim3(blocks, gy), dim3(GR_THREADS), gemv_rows_lds_bytes(2) + gemv_rows_stage_bytes<FMT>(2), s, W, ops, inv, n, k, rows, groups, blocks | ((unsigned)gy << 16), bias, res, y);
     else hipLaunchKernelGGL((gemv_rows_kernel<FMT, 1>), dim3(blocks, gy), dim3(GR_THREADS), gemv_rows_lds_bytes(1) + gemv_rows_stage_bytes<FMT>(1), s, W, ops, inv, n, k, rows, groups, blocks | ((unsigned)gy << 16), bias, res, y);
 }
@@ -115,6 +126,93 @@ void gemv_rows_main_launch(int fmt, unsigned max_blocks, hipStream_t s, const ui
     case F_Q2_K: launch<F_Q2_K>(max_blocks, s, W, scratch, bias, res, y, n, k, rows); break;
     default: break;
     }
+}
+
+
+KernelRef gemv_held_kernel_ref(int fmt, int groups_held) {
+    return block_values(fmt) == 256 ? gemv_held_kernel_k(fmt, groups_held) : gemv_held_kernel_q32(fmt, groups_held);
+}
+
+// Which of the two kernels takes a launch.  What each costs beyond its launches, in units of a wave's work - one decoded
+// tile of 16 rows and a 256-value column, met by its groups of rows - in us, fitted on both kernels at 276 launches (six
+// formats, ten shapes from 512 x 11008 to 14336 x 4096, 9 to 64 rows), root mean square of the estimates' errors 0.9 to 1.6 and
+// 0.5 to 0.8 us:
+//   streaming:  base + long_row k / 4096 + units (decode T + meet g + meet_tile g T), units = rounds x columns per wave, T tiles
+//   held:       base + long_row k / 4096 + join (sliced) + start G + steps (decode + meet G) + slice_mb (MB of sums / 4)
+// The held kernel wins where the streaming one has no whole round of workgroups (4096 x 14336, 14336 x 4096, rows of odd
+// numbers of columns) or decodes much per tile (Q6_K): Q6_K 4096 x 14336 at 12 / 24 / 40 rows 45.2 / 43.1 / 48.8 -> 32.0 / 34.7 /
+// 43.4, Q6_K 2000 x 6912 27.9 -> 18.3 (24 rows), Q4_K 14336 x 4096 25.4 -> 23.6, Q4_0 24000 x 2048 26.4 -> 23.5.  It loses where
+// every CU has exactly one batch, by its second launch: Q4_K 4096 x 4096 15.6 against 16.2, 8192 x 4096 17.2 against 18.7.
+struct RowsCost {
+    float s_base, s_decode, s_meet_tile, s_meet, s_long;
+    float h_base, h_join, h_start, h_decode, h_meet, h_mb, h_long;
+};
+static const RowsCost &rows_cost(int fmt) {
+    static const RowsCost q40 = {9.40f, 1.37f, 0.23f, 0.35f, -0.90f, 7.59f, 3.03f, 0.64f, 1.48f, 0.24f, 0.19f, 0.05f};
+    static const RowsCost q41 = {9.46f, 0.99f, 0.17f, 0.46f, -0.79f, 8.03f, 2.55f, 0.86f, 0.75f, 0.26f, 1.01f, 0.13f};
+    static const RowsCost q4 = {9.67f, 1.03f, 0.00f, 0.70f, -0.92f, 8.18f, 2.62f, 0.85f, 0.79f, 0.18f, 0.79f, 0.03f};
+    static const RowsCost q5 = {10.18f, 0.85f, 0.19f, 0.39f, -0.03f, 8.30f, 2.18f, 0.77f, 1.16f, 0.17f, 0.57f, 0.25f};
+    static const RowsCost q6 = {10.34f, 1.66f, -0.55f, 2.00f, -0.25f, 8.10f, 2.98f, 0.64f, 1.63f, 0.37f, 0.30f, 0.19f};
+    static const RowsCost q80 = {10.00f, 1.53f, 0.42f, 0.17f, -1.15f, 7.16f, 3.76f, 0.81f, 1.75f, 0.22f, 0.05f, -0.16f};
+    switch (fmt) {
+    case F_Q6_K: return q6;
+    case F_Q5_K: return q5;
+    case F_Q8_0: return q80;
+    case F_Q4_0: return q40;
+    case F_Q4_1: case F_Q5_1: return q41;
+    default: return q4;  // (Q4_K and Q2_K)
+    }
+}
+
+// The held kernel's launch, or groups_held = 0: the streaming kernel's.  adds: a bias or a residual, which take a join
+HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, bool adds, int cus) {
+    HeldPlan best;
+    const RowsCost &cost = rows_cost(fmt);
+    const int ncol = k / 256, ntiles = (n + 15) / 16, groups = (rows + 7) / 8;
+    HeldGeo geo;
+    geo.slices = (ncol + GR_WAVES - 1) / GR_WAVES;
+    geo.cols = (ncol + geo.slices - 1) / geo.slices;
+    geo.slices = (ncol + geo.cols - 1) / geo.cols;
+    geo.lanes = GR_WAVES / geo.cols;
+    if (geo.slices > cus || geo.slices > 4095) return best;
+    const int steps = (ntiles + geo.lanes - 1) / geo.lanes, part = geo.slices > 1 || adds ? geo.slices : 0;
+    const RowsGeo st = rows_geometry(fmt, n, k, rows, (unsigned)cus);
+    const float units = (float)((st.batches + cus - 1) / cus * ((ncol + GR_WAVES - 1) / GR_WAVES)), gper = (float)((groups + st.shares - 1) / st.shares),
+                tiles = (float)st.tiles;
+    // (the fitted lines err by a few per cent: a launch changes kernels for three)
+    float best_us = 0.97f * (cost.s_base + cost.s_long * k / 4096.f + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
+    for (int shares = 1; shares <= groups; ++shares) {
+        const int held = (groups + shares - 1) / shares;
+        if (held > GH_G_MAX || (groups + held - 1) / held != shares || geo.slices * shares > cus) continue;
+        const int per_slice = std::min({cus / (geo.slices * shares), steps, 4095}), walk = (steps + per_slice - 1) / per_slice;
+        const float us = cost.h_base + cost.h_long * k / 4096.f + (part ? cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
+                         cost.h_mb * 1e-6f * part * rows * n;
+        if (us < best_us) {
+            best_us = us;
+            geo.per_slice = (steps + walk - 1) / walk;
+            best.groups_held = held;
+            best.shares = shares;
+            best.slices = geo.slices;
+            best.per_slice = geo.per_slice;
+            best.part = part;
+            best.where = geo.packed();
+        }
+    }
+    return best;
+}
+
+void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
+                      float *y, float *part, int n, int k, int rows) {
+    int groups = (rows + 7) / 8;
+    const _Float16 *ops = reinterpret_cast<const _Float16 *>(scratch);
+    const float *inv = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(scratch) + gemv_rows_ops_bytes(groups, k));
+    const bool whole = plan.part == 0;
+    float *ky = whole ? y : part;
+    uint32_t where = plan.where;
+    const KernelRef kr = gemv_held_kernel_ref(fmt, plan.groups_held);
+    void *args[] = {&W, &ops, &inv, &n, &k, &rows, &groups, &where, &ky};
+    (void)hipLaunchKernel(kr.fn, dim3((unsigned)(plan.slices * plan.per_slice), (unsigned)plan.shares), dim3(GR_THREADS), args, kr.lds, s);
+    if (!whole) rows_join_launch(s, part, y, rows, n, plan.slices, bias, res, (unsigned)cus);
 }
 
 }  // namespace jitnn

@@ -669,6 +669,17 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     return JITNN_HIP_OK;
 }
 
+// Would workspace() give `bytes` where a kernel with less scratch will do as well: yes, unless it cannot hold them without an
+// allocation under a stream capture, or at all.
+bool workspace_at_hand(size_t bytes, hipStream_t stream, ScratchSource src) {
+    if (src == SCRATCH_STATIC) return bytes <= JITNN_HIP_SCRATCH_BYTES;
+    touch_thread_state();
+    bool waited = false;
+    void *p = g_ws.operands.try_get(bytes, stream_recording(stream), &waited);
+    if (waited) g_ws.used = false;
+    return p != nullptr;
+}
+
 // Room for `bytes` of dequantised weights, or nullptr - without an error, and without a word to the device where that size was
 // refused before: the caller then takes the kernel that decodes them as it goes, which needs none.  Between workspace(), which
 // orders both blocks on the stream (and may give this one up), and the launches.
@@ -1354,23 +1365,45 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
                       hipStream_t s, ScratchSource src, const float *swiglu_up = nullptr) {
     const int k = ws[0]->k;
     bool need[GR_LAYOUTS] = {};  // the operand layouts the weights ask for
+    const size_t one = (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255;
+    int layouts = 0;
     for (int i = 0; i < count; ++i) {
         if (ws[i]->k != k) return fail(JITNN_HIP_EINVAL, "weights of %d and %d values per row on one activation", k, ws[i]->k);
-        const KernelRef kr = gemv_rows_kernel_ref(ws[i]->fmt, ws[i]->n, k, rows, (unsigned)g.cus);
-        if (int rc = allow_lds(kr.fn, kr.lds)) return rc;
-        need[gemv_rows_layout(ws[i]->fmt)] = true;
+        bool &l = need[gemv_rows_layout(ws[i]->fmt)];
+        layouts += !l;
+        l = true;
     }
-    const size_t one = (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255;
+    // which weights take the kernel that holds the operands; its slices' sums, one weight's at a time, stand behind the operands
+    HeldPlan plan[3];
+    size_t part = 0;
+    for (int i = 0; i < count; ++i) {
+        plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, bias || residual, g.cus);
+        // (the same limit for both sources of scratch, so that both entry points take the same kernels)
+        if (one + plan[i].part_bytes(rows, ws[i]->n) > JITNN_HIP_SCRATCH_BYTES) plan[i] = HeldPlan{};
+        part = std::max(part, plan[i].part_bytes(rows, ws[i]->n));
+    }
     void *scratch = nullptr;
-    int layouts = 0;
-    for (int l = 0; l < GR_LAYOUTS; ++l) layouts += need[l];
-    if (int rc = workspace(one * layouts, s, &scratch, src)) return rc;
+    if (part && !workspace_at_hand(one * layouts + part, s, src)) {
+        for (HeldPlan &p : plan)
+            if (p.part) p = HeldPlan{};
+        part = 0;
+    }
+    if (int rc = workspace(one * layouts + part, s, &scratch, src)) return rc;
+    for (int i = 0; i < count; ++i) {
+        const KernelRef kr = plan[i].groups_held ? gemv_held_kernel_ref(ws[i]->fmt, plan[i].groups_held)
+                                                 : gemv_rows_kernel_ref(ws[i]->fmt, ws[i]->n, k, rows, (unsigned)g.cus);
+        if (int rc = allow_lds(kr.fn, kr.lds)) return rc;
+    }
     uint8_t *sc[GR_LAYOUTS] = {};
     for (int l = 0, used = 0; l < GR_LAYOUTS; ++l)
         if (need[l]) sc[l] = (uint8_t *)scratch + one * used++;
     gemv_rows_prepare_launch(s, x, swiglu_up, (void *const *)sc, k, rows);
-    for (int i = 0; i < count; ++i)
-        gemv_rows_main_launch(ws[i]->fmt, (unsigned)g.cus, s, ws[i]->dev, sc[gemv_rows_layout(ws[i]->fmt)], bias, residual, ys[i], ws[i]->n, k, rows);
+    for (int i = 0; i < count; ++i) {
+        const void *ops = sc[gemv_rows_layout(ws[i]->fmt)];
+        if (plan[i].groups_held)
+            gemv_held_launch(plan[i], ws[i]->fmt, g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], (float *)((uint8_t *)scratch + one * layouts), ws[i]->n, k, rows);
+        else gemv_rows_main_launch(ws[i]->fmt, (unsigned)g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], ws[i]->n, k, rows);
+    }
     HIP_TRY(hipGetLastError());
     return workspace_done(s, src);
 }

@@ -110,6 +110,25 @@ void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu
 void gemv_rows_main_launch(int fmt, unsigned max_blocks, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res, float *y,
                            int n, int k, int rows);
 
+// ---- gemv_held_k.hip, gemv_held_q32.hip: gemv_held_kernel<fmt>, the same products with the activation operands held in
+// registers (prepared by the same launch), K in slices whose sums rows_join_kernel adds up
+struct HeldPlan {
+    int groups_held = 0;  // groups of eight rows per workgroup; 0: this launch is gemv_rows_kernel's
+    int shares = 0;       // workgroups that share out the groups: gridDim.y
+    int slices = 0, per_slice = 0;
+    uint32_t where = 0;   // HeldGeo::packed
+    int part = 0;         // slices to be joined: 0 where the one slice is the result
+    size_t part_bytes(int rows, int n) const { return (size_t)part * rows * n * sizeof(float); }
+};
+HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, bool adds, int cus);  // adds: a bias or a residual
+KernelRef gemv_held_kernel_k(int fmt, int groups_held);
+KernelRef gemv_held_kernel_q32(int fmt, int groups_held);
+KernelRef gemv_held_kernel_ref(int fmt, int groups_held);
+// y = x W^T (+ bias [n]) (+ res [rows, n]); part: plan.part_bytes(rows, n) of scratch
+void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
+                      float *y, float *part, int n, int k, int rows);
+void rows_join_launch(hipStream_t s, const float *part, float *y, int rows, int n, int slices, const float *bias, const float *res, unsigned cus);
+
 // ---- gemv_i8.hip: gemv_i8_kernel / gemv_i8_plain_kernel<unit>: GEMV of one to four activation rows with INT8 matrix-core products on the
 // raw quants.  The argument block of the kernels (the launchers put what a wave's first loads need in front of it, as scalar
 // arguments the hardware preloads): up to three matrices of one format and row length share a launch and an activation vector (row segments
