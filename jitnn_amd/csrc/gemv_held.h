@@ -42,7 +42,7 @@ struct HeldGeo {
 // y[slice][b, row] = sum over the slice's k of W[row, k] x[b, k], for the rows b of this workgroup's G groups (blockIdx.y);
 // k a multiple of 256, n >= 16, per_slice at most the number of steps.  A bias and a residual are rows_join_kernel's: loads here would be waited for with the weights.
 template <int FMT, int G>
-__global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__restrict__ W, const _Float16 *__restrict__ ops, const float *__restrict__ inv,
+__global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__restrict__ W, const uint8_t *__restrict__ W2, const _Float16 *__restrict__ ops, const float *__restrict__ inv,
                                                                 int n, int k, int rows, int groups, const uint32_t where, float *__restrict__ y) {
     typedef RTile<FMT> R;
     constexpr int NOPS = R::NOPS;
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
     uint8_t *stage = gh_smem + 2 * (size_t)BUF * sizeof(float2) + (size_t)wave * R::STAGE_BYTES;
     constexpr int PARKED = gh_ops_in_lds(FMT, G), HELD = 9 - PARKED;  // operands of a group in LDS, in registers
     f16x8 *parked = reinterpret_cast<f16x8 *>(gh_smem + 2 * (size_t)BUF * sizeof(float2) + gemv_rows_stage_bytes<FMT>(1)) + wave * PARKED * G * 64 + lane;
-    const int ncol = k >> 8, ntiles = (n + 15) >> 4, nsteps = (ntiles + geo.lanes - 1) / geo.lanes;
+    const int ncol = k >> 8, each = (n + 15) >> 4, ntiles = W2 ? 2 * each : each, nsteps = (ntiles + geo.lanes - 1) / geo.lanes;
     const size_t rowbytes = (size_t)ncol * R::BYTES;
     const int slice = (int)blockIdx.x / geo.per_slice, first = (int)blockIdx.x - slice * geo.per_slice;
     const int c0 = slice * geo.cols, cols = min(geo.cols, ncol - c0);  // (the last slice may be short)
@@ -65,7 +65,10 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
 
     // the last tile of a ragged matrix is the last 16 rows: in bounds, its first rows computed twice, stored once
     typename R::Raw raw;
-    auto fetch = [&](int step) { R::load(raw, R::ptr(W, min(min(step * geo.lanes + tl, ntiles - 1) * 16, n - 16), rowbytes, lane), c); };
+    auto fetch = [&](int step) {
+        const int t = min(step * geo.lanes + tl, ntiles - 1), second = t >= each;
+        R::load(raw, R::ptr(second ? W2 : W, min((second ? t - each : t) * 16, n - 16), rowbytes, lane), c);
+    };
     f16x8 A[G][HELD];
     float2 iv[G];
     if (works) {
@@ -89,7 +92,7 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
     // the sums of a step, added up in wave order and stored: (tile, group) tg by wave tg % 8
     auto join = [&](int step, int buf) {
         for (int tg = wave; tg < geo.lanes * G; tg += GR_WAVES) {
-            const int t = tg / G, g = tg - t * G, tile = step * geo.lanes + t;
+            const int t = tg / G, g = tg - t * G, at = step * geo.lanes + t, second = at >= each, tile = second ? at - each : at;
             const float2 *p = red + buf * BUF + (t * geo.cols * G + g) * 64 + lane;
             float2 v[GR_WAVES];
 #pragma unroll
@@ -101,10 +104,10 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
                 sum.y += w < cols ? v[w].y : 0.f;
             }
             const int row = min(tile * 16, n - 16) + (lane & 15), b = (g0 + g) * 8 + 2 * kq;
-            if (tile < ntiles && row >= tile * 16) {  // rows of a ragged last tile that an earlier tile already wrote are skipped
-                float *at = ys + (size_t)b * n + row;
-                if (b < rows) at[0] = sum.x;
-                if (b + 1 < rows) at[n] = sum.y;
+            if (at < ntiles && row >= tile * 16) {  // rows of a ragged last tile that an earlier tile already wrote are skipped
+                float *to = ys + ((size_t)(second ? geo.slices : 0) * rows + b) * n + row;
+                if (b < rows) to[0] = sum.x;
+                if (b + 1 < rows) to[n] = sum.y;
             }
         }
     };

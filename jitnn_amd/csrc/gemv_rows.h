@@ -109,8 +109,9 @@ struct RowsPrepareOut {
     _Float16 *ops[3];  // per layout (plain, sums per 16 values, halves): nullptr = not wanted
     float *inv[3];
 };
+// slices > 1: x and up are [slices][rows, k], sums of K slices that meet here, in slice order.
 template <bool SWIGLU>
-__global__ void __launch_bounds__(64) rows_prepare_kernel(const float *__restrict__ x, const float *__restrict__ up, int rows, int k,
+__global__ void __launch_bounds__(64) rows_prepare_kernel(const float *__restrict__ x, const float *__restrict__ up, int rows, int k, int slices,
                                                            const RowsPrepareOut o) {  // (what the first loads need in front: preloaded with the wave)
     const int lane = threadIdx.x, b = lane >> 3, part = lane & 7;
     const int c = blockIdx.x, g = blockIdx.y, ncol = k >> 8;
@@ -121,12 +122,25 @@ __global__ void __launch_bounds__(64) rows_prepare_kernel(const float *__restric
 #pragma unroll
     for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const float4 *>(x + at + 32 * t);
     if constexpr (SWIGLU) {
+        float4 u[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) u[t] = *reinterpret_cast<const float4 *>(up + at + 32 * t);
+        for (int z = 1; z < slices; ++z) {
+            const size_t az = at + (size_t)z * rows * k;
+            float4 a[8], b[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) a[t] = *reinterpret_cast<const float4 *>(x + az + 32 * t);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) b[t] = *reinterpret_cast<const float4 *>(up + az + 32 * t);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                v[t] = make_float4(v[t].x + a[t].x, v[t].y + a[t].y, v[t].z + a[t].z, v[t].w + a[t].w);
+                u[t] = make_float4(u[t].x + b[t].x, u[t].y + b[t].y, u[t].z + b[t].z, u[t].w + b[t].w);
+            }
+        }
         auto sw = [](float gt, float u) { return (gt / (1.f + __expf(-gt))) * u; };
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float4 u = *reinterpret_cast<const float4 *>(up + at + 32 * t);
-            v[t] = make_float4(sw(v[t].x, u.x), sw(v[t].y, u.y), sw(v[t].z, u.z), sw(v[t].w, u.w));
-        }
+        for (int t = 0; t < 8; ++t) v[t] = make_float4(sw(v[t].x, u[t].x), sw(v[t].y, u[t].y), sw(v[t].z, u[t].z), sw(v[t].w, u[t].w));
     }
     if (o.ops[0]) rows_prepare_column<32, false>(v, o.ops[0], o.inv[0], c, g, ncol, have, lane);
     if (o.ops[1]) rows_prepare_column<16, false>(v, o.ops[1], o.inv[1], c, g, ncol, have, lane);

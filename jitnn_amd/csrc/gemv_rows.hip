@@ -87,7 +87,7 @@ int gemv_rows_layout(int fmt) {
 
 static_assert(GR_LAYOUT_PLAIN == 0 && GR_LAYOUT_SUMS16 == 1 && GR_LAYOUT_HALVES == 2 && GR_LAYOUTS == 3, "RowsPrepareOut is indexed by layout");
 
-void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu_up, void *const *scratch, int k, int rows) {
+void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu_up, void *const *scratch, int k, int rows, int slices) {
     const int groups = (rows + 7) / 8, ncol = k / 256;
     RowsPrepareOut o{};
     for (int l = 0; l < GR_LAYOUTS; ++l) {
@@ -96,8 +96,8 @@ void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu
         o.inv[l] = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(scratch[l]) + gemv_rows_ops_bytes(groups, k));
     }
     const dim3 grid(ncol, groups);
-    if (swiglu_up) hipLaunchKernelGGL(rows_prepare_kernel<true>, grid, dim3(64), 0, s, x, swiglu_up, rows, k, o);
-    else hipLaunchKernelGGL(rows_prepare_kernel<false>, grid, dim3(64), 0, s, x, swiglu_up, rows, k, o);
+    if (swiglu_up) hipLaunchKernelGGL(rows_prepare_kernel<true>, grid, dim3(64), 0, s, x, swiglu_up, rows, k, slices, o);
+    else hipLaunchKernelGGL(rows_prepare_kernel<false>, grid, dim3(64), 0, s, x, swiglu_up, rows, k, slices, o);
 }
 
 template <int FMT>
@@ -164,29 +164,30 @@ static const RowsCost &rows_cost(int fmt) {
     }
 }
 
-// The held kernel's launch, or groups_held = 0: the streaming kernel's.  adds: a bias or a residual, which take a join
-HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, bool adds, int cus) {
+// The held kernel's launch, or groups_held = 0: the streaming kernel's.
+HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, int join, int cus, int weights) {
     HeldPlan best;
     const RowsCost &cost = rows_cost(fmt);
-    const int ncol = k / 256, ntiles = (n + 15) / 16, groups = (rows + 7) / 8;
+    const int ncol = k / 256, ntiles = (n + 15) / 16 * weights, groups = (rows + 7) / 8;
     HeldGeo geo;
     geo.slices = (ncol + GR_WAVES - 1) / GR_WAVES;
     geo.cols = (ncol + geo.slices - 1) / geo.slices;
     geo.slices = (ncol + geo.cols - 1) / geo.cols;
     geo.lanes = GR_WAVES / geo.cols;
     if (geo.slices > cus || geo.slices > 4095) return best;
-    const int steps = (ntiles + geo.lanes - 1) / geo.lanes, part = geo.slices > 1 || adds ? geo.slices : 0;
+    const int steps = (ntiles + geo.lanes - 1) / geo.lanes, part = geo.slices > 1 || join != HELD_JOIN_SLICES ? geo.slices : 0;
     const RowsGeo st = rows_geometry(fmt, n, k, rows, (unsigned)cus);
     const float units = (float)((st.batches + cus - 1) / cus * ((ncol + GR_WAVES - 1) / GR_WAVES)), gper = (float)((groups + st.shares - 1) / st.shares),
                 tiles = (float)st.tiles;
-    // (the fitted lines err by a few per cent: a launch changes kernels for three)
-    float best_us = 0.97f * (cost.s_base + cost.s_long * k / 4096.f + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
+    // (a pair of streaming launches is taken at twice one: the preparation they share is paid by their second round of CUs; the
+    // fitted lines err by a few per cent: a launch changes kernels for three)
+    float best_us = 0.97f * (float)weights * (cost.s_base + cost.s_long * k / 4096.f + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
     for (int shares = 1; shares <= groups; ++shares) {
         const int held = (groups + shares - 1) / shares;
         if (held > GH_G_MAX || (groups + held - 1) / held != shares || geo.slices * shares > cus) continue;
         const int per_slice = std::min({cus / (geo.slices * shares), steps, 4095}), walk = (steps + per_slice - 1) / per_slice;
-        const float us = cost.h_base + cost.h_long * k / 4096.f + (part ? cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
-                         cost.h_mb * 1e-6f * part * rows * n;
+        const float us = cost.h_base + cost.h_long * k / 4096.f + (part && join != HELD_JOIN_READER ? cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
+                         cost.h_mb * 1e-6f * part * rows * n * weights;
         if (us < best_us) {
             best_us = us;
             geo.per_slice = (steps + walk - 1) / walk;
@@ -201,18 +202,21 @@ HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, bool adds, int cus) {
     return best;
 }
 
-void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
-                      float *y, float *part, int n, int k, int rows) {
+void gemv_held_slices_launch(const HeldPlan &plan, int fmt, hipStream_t s, const uint8_t *W, const uint8_t *W2, const void *scratch, float *part, int n, int k,
+                             int rows) {
     int groups = (rows + 7) / 8;
     const _Float16 *ops = reinterpret_cast<const _Float16 *>(scratch);
     const float *inv = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(scratch) + gemv_rows_ops_bytes(groups, k));
-    const bool whole = plan.part == 0;
-    float *ky = whole ? y : part;
     uint32_t where = plan.where;
     const KernelRef kr = gemv_held_kernel_ref(fmt, plan.groups_held);
-    void *args[] = {&W, &ops, &inv, &n, &k, &rows, &groups, &where, &ky};
+    void *args[] = {&W, &W2, &ops, &inv, &n, &k, &rows, &groups, &where, &part};
     (void)hipLaunchKernel(kr.fn, dim3((unsigned)(plan.slices * plan.per_slice), (unsigned)plan.shares), dim3(GR_THREADS), args, kr.lds, s);
-    if (!whole) rows_join_launch(s, part, y, rows, n, plan.slices, bias, res, (unsigned)cus);
+}
+
+void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
+                      float *y, float *part, int n, int k, int rows) {
+    gemv_held_slices_launch(plan, fmt, s, W, nullptr, scratch, plan.part ? part : y, n, k, rows);
+    if (plan.part) rows_join_launch(s, part, y, rows, n, plan.slices, bias, res, (unsigned)cus);
 }
 
 }  // namespace jitnn

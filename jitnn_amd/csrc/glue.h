@@ -247,16 +247,65 @@ __global__ void __launch_bounds__(256) rms_norm_rows_kernel(const float *__restr
     for (int i = threadIdx.x; i < n; i += 256) yr[i] = xr[i] * is * w[i];
 }
 
+// The same, 16 bytes a load and a row's loads in flight at once, on rows that may still be K slices: the row is x (the residual) +
+// part[z] [rows, n] in slice order (splits of them; none: part is nullptr), which is stored to xsum on the way.  A row of 4096 values is one
+// pass of 1024 threads: bound by latency.  n a multiple of 4, pointers 16-byte aligned.
+constexpr int NR_THREADS = 1024, NR_KEEP = 2;  // quads of a row a thread keeps (rows of up to 8192 values)
+__global__ void __launch_bounds__(NR_THREADS) rms_norm_rows_join_kernel(const float *x, const float *__restrict__ part, int splits, float *xsum,
+                                                                        const float *__restrict__ w, float *__restrict__ y, int rows, int n, float eps) {
+    __shared__ float red[NR_THREADS / 64];
+    const size_t row = (size_t)blockIdx.x * n, slice = (size_t)rows * n;
+    float4 kept[NR_KEEP];
+    float s = 0.f;
+    auto take = [&](int i) {
+        float4 a = *reinterpret_cast<const float4 *>(x + row + i);
+        if (part) {
+            float4 p[8], sum;
+#pragma unroll
+            for (int z = 0; z < 8; ++z) p[z] = *reinterpret_cast<const float4 *>(part + (size_t)min(z, splits - 1) * slice + row + i);
+            sum = p[0];
+#pragma unroll
+            for (int z = 1; z < 8; ++z)
+                if (z < splits) sum = make_float4(sum.x + p[z].x, sum.y + p[z].y, sum.z + p[z].z, sum.w + p[z].w);
+            a = make_float4(sum.x + a.x, sum.y + a.y, sum.z + a.z, sum.w + a.w);
+            *reinterpret_cast<float4 *>(xsum + row + i) = a;
+        }
+        s = __builtin_fmaf(a.x, a.x, __builtin_fmaf(a.y, a.y, __builtin_fmaf(a.z, a.z, __builtin_fmaf(a.w, a.w, s))));
+        return a;
+    };
+    const int t4 = 4 * (int)threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < NR_KEEP; ++j)
+        if (t4 + 4 * NR_THREADS * j < n) kept[j] = take(t4 + 4 * NR_THREADS * j);
+    for (int i = t4 + 4 * NR_THREADS * NR_KEEP; i < n; i += 4 * NR_THREADS) (void)take(i);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NR_THREADS / 64; ++i) s += red[i];
+    const float is = 1.f / sqrtf(s / (float)n + eps);
+    auto give = [&](int i, float4 a) {
+        const float4 g = *reinterpret_cast<const float4 *>(w + i);
+        *reinterpret_cast<float4 *>(y + row + i) = make_float4(a.x * is * g.x, a.y * is * g.y, a.z * is * g.z, a.w * is * g.w);
+    };
+#pragma unroll
+    for (int j = 0; j < NR_KEEP; ++j)
+        if (t4 + 4 * NR_THREADS * j < n) give(t4 + 4 * NR_THREADS * j, kept[j]);
+    for (int i = t4 + 4 * NR_THREADS * NR_KEEP; i < n; i += 4 * NR_THREADS)  // (a thread reads back what it wrote)
+        give(i, *reinterpret_cast<const float4 *>((part ? xsum : x) + row + i));
+}
+
 // Rotary embedding of the query heads in place (q [T, heads, D]) and of the key heads on their way into the cache,
 // values copied into the cache: token t = blockIdx.x sits at position pos0 + t.  Same rotation as attn_decode_kernel.
 __global__ void __launch_bounds__(256) rope_append_rows_kernel(float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
                                                                 float *__restrict__ kcache, float *__restrict__ vcache,
                                                                 const float *__restrict__ cosv, const float *__restrict__ sinv, int heads, int kv_heads,
                                                                 int D, int pos0, int interleaved) {
-    const int t = blockIdx.x, pos = pos0 + t, half = D / 2;
+    const int t = blockIdx.x, pos = pos0 + t, half = D / 2, first = blockIdx.y * 256 + threadIdx.x, stride = gridDim.y * 256;
     const float *cp = cosv + (size_t)pos * half, *sp = sinv + (size_t)pos * half;
     float *qt = q + (size_t)t * heads * D;
-    for (int i = threadIdx.x; i < heads * half; i += 256) {
+    for (int i = first; i < heads * half; i += stride) {
         const int h = i / half, p = i - h * half;
         const int i0 = h * D + (interleaved ? 2 * p : p), i1 = h * D + (interleaved ? 2 * p + 1 : p + half);
         const float a = qt[i0], b = qt[i1], cs = cp[p], sn = sp[p];
@@ -265,14 +314,14 @@ __global__ void __launch_bounds__(256) rope_append_rows_kernel(float *__restrict
     }
     const float *kt = k + (size_t)t * kv_heads * D, *vt = v + (size_t)t * kv_heads * D;
     float *kc = kcache + (size_t)pos * kv_heads * D, *vc = vcache + (size_t)pos * kv_heads * D;
-    for (int i = threadIdx.x; i < kv_heads * half; i += 256) {
+    for (int i = first; i < kv_heads * half; i += stride) {
         const int h = i / half, p = i - h * half;
         const int i0 = h * D + (interleaved ? 2 * p : p), i1 = h * D + (interleaved ? 2 * p + 1 : p + half);
         const float a = kt[i0], b = kt[i1], cs = cp[p], sn = sp[p];
         kc[i0] = a * cs - b * sn;
         kc[i1] = a * sn + b * cs;
     }
-    for (int i = threadIdx.x; i < kv_heads * D; i += 256) vc[i] = vt[i];
+    for (int i = first; i < kv_heads * D; i += stride) vc[i] = vt[i];
 }
 
 // The same on projections that still lie in K slices (the many-row launch of q, k and v split K and left the join to this

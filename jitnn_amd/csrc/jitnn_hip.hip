@@ -1361,8 +1361,10 @@ bool rows_path(const jitnn_hip_weight *w, int rows) {
 // ys[i] = x ws[i]^T (+ bias) (+ residual [rows, n]; bias and residual with one weight only) for weights that all pass
 // rows_path: the activation operands are prepared once per granularity of block sums and shared by the weights.
 // swiglu_up: the activations are silu(x) * swiglu_up, formed by the preparation as it reads x.
+// later, defer (one weight, a residual): where the sums come in up to eight slices, they go to later and their join is left to the
+// caller, as *defer.
 int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int count, const float *x, int rows, const float *bias, const float *residual,
-                      hipStream_t s, ScratchSource src, const float *swiglu_up = nullptr) {
+                      hipStream_t s, ScratchSource src, const float *swiglu_up = nullptr, float *later = nullptr, PfPending *defer = nullptr) {
     const int k = ws[0]->k;
     bool need[GR_LAYOUTS] = {};  // the operand layouts the weights ask for
     const size_t one = (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255;
@@ -1376,8 +1378,15 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
     // which weights take the kernel that holds the operands; its slices' sums, one weight's at a time, stand behind the operands
     HeldPlan plan[3];
     size_t part = 0;
+    int later_plan = 0;  // slices whose join the caller gets
     for (int i = 0; i < count; ++i) {
-        plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, bias || residual, g.cus);
+        const bool put_off = defer && k <= 8 * 2048;  // (a slice is at most eight columns; more slices only where that is less than k / 2048)
+        plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, put_off ? HELD_JOIN_READER : bias || residual ? HELD_JOIN_ADDS : HELD_JOIN_SLICES, g.cus);
+        if (put_off && plan[i].slices > 1 && plan[i].slices <= 8) {
+            later_plan = plan[i].slices;
+            continue;
+        }
+        if (put_off) plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, HELD_JOIN_ADDS, g.cus);
         // (the same limit for both sources of scratch, so that both entry points take the same kernels)
         if (one + plan[i].part_bytes(rows, ws[i]->n) > JITNN_HIP_SCRATCH_BYTES) plan[i] = HeldPlan{};
         part = std::max(part, plan[i].part_bytes(rows, ws[i]->n));
@@ -1400,12 +1409,81 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
     gemv_rows_prepare_launch(s, x, swiglu_up, (void *const *)sc, k, rows);
     for (int i = 0; i < count; ++i) {
         const void *ops = sc[gemv_rows_layout(ws[i]->fmt)];
-        if (plan[i].groups_held)
+        if (later_plan) {
+            gemv_held_slices_launch(plan[i], ws[i]->fmt, s, ws[i]->dev, nullptr, ops, later, ws[i]->n, k, rows);
+            defer->part = later;
+            defer->res = residual;
+            defer->out = ys[i];
+            defer->splits = later_plan;
+            defer->n = ws[i]->n;
+        } else if (plan[i].groups_held)
             gemv_held_launch(plan[i], ws[i]->fmt, g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], (float *)((uint8_t *)scratch + one * layouts), ws[i]->n, k, rows);
         else gemv_rows_main_launch(ws[i]->fmt, (unsigned)g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], ws[i]->n, k, rows);
     }
     HIP_TRY(hipGetLastError());
     return workspace_done(s, src);
+}
+
+// y = res + (silu(x wg^T) * (x wu^T)) wd^T, for weights that all pass rows_path, where gate and up (one format and shape) pay as one
+// launch of the held kernel: 45 us for the two of an 8B layer at 40 tokens, whose slices used to be joined by launches of their
+// own, 4.2 us each, and now meet in the preparation of the down projection's operands.  later, defer: as for launch_rows_group.
+struct RowsFfn {
+    HeldPlan pair, down;
+    bool to_reader;  // the slices of the down projection are joined by whoever reads y next
+    size_t ops, sums, ops_down, total;  // scratch: operands of x | slices of gate and up | operands of the gated rows | slices of down
+};
+bool rows_ffn_pays(const jitnn_hip_weight *wg, const jitnn_hip_weight *wu, const jitnn_hip_weight *wd, int rows, hipStream_t s, RowsFfn *f) {
+    if (wg->fmt != wu->fmt || wg->n != wu->n || wg->k != wu->k || wd->k != wg->n) return false;
+    if (!rows_path(wg, rows) || !rows_path(wu, rows) || !rows_path(wd, rows)) return false;
+    const int n = wg->n;
+    f->pair = gemv_held_plan(wg->fmt, n, wg->k, rows, HELD_JOIN_READER, g.cus, 2);
+    if (!f->pair.groups_held) return false;
+    f->down = gemv_held_plan(wd->fmt, wd->n, n, rows, HELD_JOIN_READER, g.cus);
+    f->to_reader = f->down.slices > 1 && f->down.slices <= 8;
+    if (!f->to_reader) f->down = gemv_held_plan(wd->fmt, wd->n, n, rows, HELD_JOIN_ADDS, g.cus);
+    auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    f->ops = pad(gemv_rows_scratch_bytes(rows, wg->k));
+    f->sums = pad(2 * f->pair.part_bytes(rows, n));
+    f->ops_down = pad(gemv_rows_scratch_bytes(rows, n));
+    f->total = f->ops + f->sums + f->ops_down + (f->to_reader ? 0 : f->down.part_bytes(rows, wd->n));
+    return workspace_at_hand(f->total, s, SCRATCH_THREAD);
+}
+int launch_rows_ffn(const RowsFfn &f, const jitnn_hip_weight *wg, const jitnn_hip_weight *wu, const jitnn_hip_weight *wd, const float *x, int rows,
+                    const float *res, float *y, hipStream_t s, float *later, PfPending *defer) {
+    const int n = wg->n, k = wg->k;
+    const HeldPlan &pair = f.pair, &down = f.down;
+    const size_t ops = f.ops, sums = f.sums, ops_down = f.ops_down, total = f.total;
+    const bool to_reader = f.to_reader;
+    const KernelRef kp = gemv_held_kernel_ref(wg->fmt, pair.groups_held),
+                    kd = down.groups_held ? gemv_held_kernel_ref(wd->fmt, down.groups_held) : gemv_rows_kernel_ref(wd->fmt, wd->n, n, rows, (unsigned)g.cus);
+    if (int rc = allow_lds(kp.fn, kp.lds)) return rc;
+    if (int rc = allow_lds(kd.fn, kd.lds)) return rc;
+    void *scratch = nullptr;
+    if (int rc = workspace(total, s, &scratch)) return rc;
+    for (const jitnn_hip_weight *w : {wg, wu, wd}) count_op(ST_GEMV, (long long)w->nbytes + 4ll * rows * ((long long)w->k + w->n));
+    uint8_t *base = (uint8_t *)scratch;
+    float *gate = (float *)(base + ops), *up = gate + (size_t)pair.slices * rows * n;
+    void *in[GR_LAYOUTS] = {}, *mid[GR_LAYOUTS] = {};
+    in[gemv_rows_layout(wg->fmt)] = base;
+    mid[gemv_rows_layout(wd->fmt)] = base + ops + sums;
+    gemv_rows_prepare_launch(s, x, nullptr, in, k, rows);
+    gemv_held_slices_launch(pair, wg->fmt, s, wg->dev, wu->dev, base, gate, n, k, rows);
+    gemv_rows_prepare_launch(s, gate, up, mid, n, rows, pair.slices);
+    const void *md = base + ops + sums;
+    if (to_reader) {
+        gemv_held_slices_launch(down, wd->fmt, s, wd->dev, nullptr, md, later, wd->n, n, rows);
+        defer->part = later;
+        defer->res = res;
+        defer->out = y;
+        defer->splits = down.slices;
+        defer->n = wd->n;
+    } else if (down.groups_held) {
+        gemv_held_launch(down, wd->fmt, g.cus, s, wd->dev, md, nullptr, res, y, (float *)(base + ops + sums + ops_down), wd->n, n, rows);
+    } else {
+        gemv_rows_main_launch(wd->fmt, (unsigned)g.cus, s, wd->dev, md, nullptr, res, y, wd->n, n, rows);
+    }
+    HIP_TRY(hipGetLastError());
+    return workspace_done(s);
 }
 
 int linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, hipStream_t s, ScratchSource src) {
@@ -1817,6 +1895,25 @@ void flush_pending(PfPending &p, int rows, hipStream_t st) {
     p = PfPending{};
 }
 
+// xn = RMSNorm(x) for `rows` rows; x - the output of the linear before - may still be in K slices, which meet here.
+void norm_rows(const jitnn_hip_llama *m, const float *x, int rows, const float *nw, float *xn, hipStream_t st, PfPending *pend) {
+    PfPending join;
+    if (pend && pend->part && pend->out == x && pend->n == m->d && pend->res) {
+        join = *pend;
+        *pend = PfPending{};
+    } else if (pend) {
+        flush_pending(*pend, rows, st);
+    }
+    // (four values a load: the model's own rows are; the caller's, in front of the first layer, need not be)
+    const float *in = join.part ? join.res : x;
+    if (((uintptr_t)in & 15) != 0 || m->d % 4 != 0) {
+        if (join.part) flush_pending(join, rows, st);
+        hipLaunchKernelGGL(rms_norm_rows_kernel, dim3(rows), dim3(256), 0, st, x, nw, xn, m->d, m->eps);
+    } else {
+        hipLaunchKernelGGL(rms_norm_rows_join_kernel, dim3(rows), dim3(NR_THREADS), 0, st, in, join.part, join.splits, join.out, nw, xn, rows, m->d, m->eps);
+    }
+}
+
 // (pend: x - the output of the linear before - may still be in K slices; the shared preparation then adds them up)
 int normed_linears_rows(const jitnn_hip_llama *m, const jitnn_hip_weight *const *ws, float *const *ys, int count, const float *x, int rows,
                         const float *nw, float *xn, hipStream_t st, PfPending *pend = nullptr, PfGroupPending *gdefer = nullptr) {
@@ -1830,8 +1927,7 @@ int normed_linears_rows(const jitnn_hip_llama *m, const jitnn_hip_weight *const 
         else if (pend) flush_pending(*pend, rows, st);  // (never both: a pending join is flushed before anybody reads its row)
         return rc;
     }
-    if (pend) flush_pending(*pend, rows, st);
-    hipLaunchKernelGGL(rms_norm_rows_kernel, dim3(rows), dim3(256), 0, st, x, nw, xn, m->d, m->eps);
+    norm_rows(m, x, rows, nw, xn, st, pend);
     // the one-pass kernel for several rows prepares its activation operands once for all the weights that take it
     bool shared = count > 1;
     for (int i = 0; i < count; ++i) shared = shared && rows_path(ws[i], rows);
@@ -1856,7 +1952,7 @@ int residual_linear_rows(const jitnn_hip_weight *w, const float *x, int rows, co
     }
     if (up && rows_path(w, rows)) {  // silu(x) * up is formed by the preparation of the one-pass kernel
         count_op(ST_GEMV, (long long)w->nbytes + 4ll * rows * ((long long)w->k + w->n));
-        return launch_rows_group(&w, &y, 1, x, rows, nullptr, res, st, SCRATCH_THREAD, up);
+        return launch_rows_group(&w, &y, 1, x, rows, nullptr, res, st, SCRATCH_THREAD, up, part, defer);
     }
     if (up) {
         const long long count = (long long)rows * w->k;
@@ -1867,7 +1963,7 @@ int residual_linear_rows(const jitnn_hip_weight *w, const float *x, int rows, co
     }
     if (rows_path(w, rows)) {  // the one-pass kernel adds the residual as it stores
         count_op(ST_GEMV, (long long)w->nbytes + 4ll * rows * ((long long)w->k + w->n));
-        return launch_rows_group(&w, &y, 1, x, rows, nullptr, res, st, SCRATCH_THREAD);
+        return launch_rows_group(&w, &y, 1, x, rows, nullptr, res, st, SCRATCH_THREAD, nullptr, part, defer);
     }
     if (int rc = jitnn_hip_linear_dev(w, x, rows, nullptr, tmp, (void *)st)) return rc;
     const size_t count4 = (size_t)rows * w->n / 4;
@@ -2184,7 +2280,7 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
                                m->kc + lo, m->vc + lo, m->cosv, m->sinv, m->heads, m->kv, m->hd, pos0, m->rope_interleaved);
             gp.part = nullptr;
         } else {
-            hipLaunchKernelGGL(rope_append_rows_kernel, dim3(T), dim3(256), 0, st, q, k, v, m->kc + lo, m->vc + lo, m->cosv, m->sinv, m->heads, m->kv,
+            hipLaunchKernelGGL(rope_append_rows_kernel, dim3(T, T < 256 ? 4 : 1), dim3(256), 0, st, q, k, v, m->kc + lo, m->vc + lo, m->cosv, m->sinv, m->heads, m->kv,
                                m->hd, pos0, m->rope_interleaved);
         }
         int arc;
@@ -2208,8 +2304,14 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
         } else {
             const jitnn_hip_weight *ws[2] = {w[JITNN_HIP_W_FFN_GATE], w[JITNN_HIP_W_FFN_UP]};
             float *ys[2] = {gate, up};
-            if (int rc = normed_linears_rows(m, ws, ys, 2, xa, T, nw + d, xn, st, &pend)) return rc;
-            if (int rc = residual_linear_rows(w[JITNN_HIP_W_FFN_DOWN], gate, T, xa, xn, xb, st, up, h, m->pf[10], &pend)) return rc;
+            RowsFfn ffn;
+            if (T <= g.gemv_max_rows && rows_ffn_pays(ws[0], ws[1], w[JITNN_HIP_W_FFN_DOWN], T, st, &ffn)) {
+                norm_rows(m, xa, T, nw + d, xn, st, &pend);
+                if (int rc = launch_rows_ffn(ffn, ws[0], ws[1], w[JITNN_HIP_W_FFN_DOWN], xn, T, xa, xb, st, m->pf[10], &pend)) return rc;
+            } else {
+                if (int rc = normed_linears_rows(m, ws, ys, 2, xa, T, nw + d, xn, st, &pend)) return rc;
+                if (int rc = residual_linear_rows(w[JITNN_HIP_W_FFN_DOWN], gate, T, xa, xn, xb, st, up, h, m->pf[10], &pend)) return rc;
+            }
         }
         x = xb;
     }

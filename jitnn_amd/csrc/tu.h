@@ -105,7 +105,8 @@ size_t gemv_rows_scratch_bytes(int rows, int k);   // operands + scales of `rows
 KernelRef gemv_rows_kernel_ref(int fmt, int n, int k, int rows, unsigned max_blocks);  // the variant gemv_rows_main_launch picks for this shape
 // every layout with a scratch (scratch[GR_LAYOUTS], nullptr: not wanted) in one launch; swiglu_up != nullptr: the rows are
 // silu(x) * swiglu_up, both [rows, k]
-void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu_up, void *const *scratch, int k, int rows);
+// (slices > 1, with swiglu_up: both are [slices][rows, k], to be added up)
+void gemv_rows_prepare_launch(hipStream_t s, const float *x, const float *swiglu_up, void *const *scratch, int k, int rows, int slices = 1);
 // y = x W^T (+ bias [n]) (+ res [rows, n])
 void gemv_rows_main_launch(int fmt, unsigned max_blocks, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res, float *y,
                            int n, int k, int rows);
@@ -120,10 +121,16 @@ struct HeldPlan {
     int part = 0;         // slices to be joined: 0 where the one slice is the result
     size_t part_bytes(int rows, int n) const { return (size_t)part * rows * n * sizeof(float); }
 };
-HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, bool adds, int cus);  // adds: a bias or a residual
+// join: by a launch of its own where there are slices, for a bias or residual in any case, or by whoever reads the sums next.
+// weights: 2 - a pair of one format and shape side by side, HELD_JOIN_READER only
+constexpr int HELD_JOIN_SLICES = 0, HELD_JOIN_ADDS = 1, HELD_JOIN_READER = 2;
+HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, int join, int cus, int weights = 1);
 KernelRef gemv_held_kernel_k(int fmt, int groups_held);
 KernelRef gemv_held_kernel_q32(int fmt, int groups_held);
 KernelRef gemv_held_kernel_ref(int fmt, int groups_held);
+// part [slices][rows, n] = the slices of x W^T, behind them those of x W2^T
+void gemv_held_slices_launch(const HeldPlan &plan, int fmt, hipStream_t s, const uint8_t *W, const uint8_t *W2, const void *scratch, float *part, int n, int k,
+                             int rows);
 // y = x W^T (+ bias [n]) (+ res [rows, n]); part: plan.part_bytes(rows, n) of scratch
 void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
                       float *y, float *part, int n, int k, int rows);
