@@ -722,12 +722,12 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 //     tiles are double-buffered, one workgroup barrier per chunk; nothing about the loads is conditional (chunks past
 //     the end repeat the last one, keys past the last visible one re-read it and are masked).
 constexpr int AM_ROWS = 64, AM_CH = 64, AM_WAVES = 2 * (AM_ROWS / 16), AM_THREADS = 64 * AM_WAVES;
-template <int D>
+template <int D, int RT>
 constexpr size_t attn_prefill_mfma_lds_bytes() {
-    return (size_t)2 * ((size_t)AM_CH * (D + 8) + (size_t)D * (AM_CH + 8)) * sizeof(_Float16) + AM_WAVES * 16 * sizeof(float);  // (the
-    // tiles also hold the second halves' outputs at the end: 4 waves x (16 x D + 32) floats fit for D >= 64)
+    return (size_t)2 * ((size_t)AM_CH * (D + 8) + (size_t)D * (AM_CH + 8)) * sizeof(_Float16) + RT * AM_WAVES * 16 * sizeof(float);  // (the
+    // tiles also hold the second halves' outputs at the end: 4 RT x (16 x D + 32) floats fit for D >= 64, RT <= 2)
 }
-template <int D>
+template <int D, int RT>
 __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const float *__restrict__ q, const float *__restrict__ kcache,
                                                                  const float *__restrict__ vcache, float *__restrict__ out, int heads, int kv_heads,
                                                                  int pos0, int T, float scale) {
@@ -738,30 +738,35 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
     extern __shared__ __align__(16) float att_smem[];
     _Float16 *Kh = reinterpret_cast<_Float16 *>(att_smem);  // [2][CH][KP]
     _Float16 *Vt = Kh + 2 * CH * KP;                        // [2][D][VP]: values transposed, keys in slot order
-    float *fx = reinterpret_cast<float *>(Vt + 2 * D * VP);  // [AM_WAVES][16]: a factor per row, from score layout to output layout
+    float *fx = reinterpret_cast<float *>(Vt + 2 * D * VP);  // [AM_WAVES][RT][16]: a factor per row, from score layout to output layout
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, kq = lane >> 4;
-    const int rt = wave & 3, half = wave >> 2;  // this wave's 16 rows of the block and its half of every chunk's keys
-    const int group = heads / kv_heads, QT = AM_ROWS / group, rows = QT * group;
-    const int g = blockIdx.y;
+    const int rt = wave & 3, half = wave >> 2;  // this wave's rows of the block - tiles rt + 4 u of 16 - and its half of every chunk's keys
+    const int group = heads / kv_heads, QT = RT * AM_ROWS / group, rows = QT * group;
+    const int g = RT == 1 ? blockIdx.y : blockIdx.x;
     // early token blocks walk few keys, late ones many: half of the key/value heads take the blocks in reverse
-    const int tb = 2 * (int)blockIdx.y < kv_heads ? (int)blockIdx.x : (int)gridDim.x - 1 - (int)blockIdx.x;
+    // (RT == 2, many blocks: the longest first; the key/value head is the fast index, so that with eight of them each has an
+    // XCD and its L2 for itself)
+    const int tb = RT == 2 ? (int)gridDim.y - 1 - (int)blockIdx.y : 2 * (int)blockIdx.y < kv_heads ? (int)blockIdx.x : (int)gridDim.x - 1 - (int)blockIdx.x;
     const int t0 = tb * QT;
     const int tl = min(t0 + QT, T) - 1;        // last token of the block
     const int jlast = pos0 + tl;               // last key any row of the block sees
     const int nchunks = jlast / CH + 1;
     // ---- this lane's query row (score layout): row r of the block, as the second operand of S^T = K Q^T
-    const int r = 16 * rt + n, tq = r / group, hq = r - tq * group;
-    const bool live = r < rows && t0 + tq < T;
-    const int jmax = pos0 + t0 + tq;  // the last key the row sees
+    bool live[RT];
+    int jmax[RT];  // the last key the row sees
     const float scale2 = scale * 1.44269504088896341f;
-    f16x8 qb[DB];
-    {
-        const float *qp = q + ((size_t)(t0 + (live ? tq : 0)) * heads + g * group + (live ? hq : 0)) * D + 8 * kq;
+    f16x8 qb[RT][DB];
+#pragma unroll
+    for (int u = 0; u < RT; ++u) {
+        const int r = 16 * (rt + 4 * u) + n, tq = r / group, hq = r - tq * group;
+        live[u] = r < rows && t0 + tq < T;
+        jmax[u] = pos0 + t0 + tq;
+        const float *qp = q + ((size_t)(t0 + (live[u] ? tq : 0)) * heads + g * group + (live[u] ? hq : 0)) * D + 8 * kq;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             const float4 a = *reinterpret_cast<const float4 *>(qp + 32 * b), c = *reinterpret_cast<const float4 *>(qp + 32 * b + 4);
-            qb[b] = live ? f16x8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w, (_Float16)c.x, (_Float16)c.y, (_Float16)c.z, (_Float16)c.w}
-                         : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            qb[u][b] = live[u] ? f16x8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w, (_Float16)c.x, (_Float16)c.y, (_Float16)c.z, (_Float16)c.w}
+                               : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
         }
     }
     // ---- staging: an item is (key pair jp, values e .. e + 3).  Eight neighbouring lanes take the eight quads of a 128-byte
@@ -805,10 +810,15 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
             *reinterpret_cast<f16x2 *>(&vt[(e + 3) * VP + col]) = f16x2{(_Float16)v0.w, (_Float16)v1.w};
         }
     };
-    f32x4 o[DT];
+    f32x4 o[RT][DT];
+    float mrun[RT], lrun[RT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float mrun = -INFINITY, lrun = 0.f;
+    for (int u = 0; u < RT; ++u) {
+        mrun[u] = -INFINITY;
+        lrun[u] = 0.f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     fetch(0);
     store(0);
     fetch(1);
@@ -819,121 +829,142 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
         const _Float16 *kh = Kh + (c & 1) * CH * KP, *vt = Vt + (c & 1) * D * VP;
         const int j0 = c * CH;
         // ---- S^T: this half's two tiles of 16 keys; the lane ends up with keys j0 + 32 half + 16 t + 4 kq + i of its row
-        f32x4 st[2];
+        f32x4 st[RT][2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            st[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < RT; ++u) st[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int b = 0; b < DB; ++b) {
                 const f16x8 a = *reinterpret_cast<const f16x8 *>(&kh[(32 * half + 16 * t + n) * KP + 32 * b + 8 * kq]);
-                st[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[b], st[t], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < RT; ++u) st[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[u][b], st[u][t], 0, 0, 0);
             }
         }
         // ---- running softmax of the row, in base 2: exp(scale s - m) = exp2(scale2 s - m2).  Only the chunks that reach
         // past the first row's last key (the diagonal of the block, and everything for rows that do not exist) need the
         // mask; in the others every score counts and no -inf can appear.
-        float mc = -INFINITY;
-        const bool masked = j0 + CH - 1 > pos0 + t0 || !(t0 + QT <= T && rows == AM_ROWS);  // workgroup-uniform
-        if (masked) {
+        const bool masked = j0 + CH - 1 > pos0 + t0 || !(t0 + QT <= T && rows == RT * AM_ROWS);  // workgroup-uniform
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+        for (int u = 0; u < RT; ++u) {
+            float mc = -INFINITY;
+            if (masked) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const bool seen = live && j0 + 32 * half + 16 * t + 4 * kq + i <= jmax;
-                    st[t][i] = seen ? st[t][i] * scale2 : -INFINITY;
-                    mc = fmaxf(mc, st[t][i]);
-                }
-        } else {
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                    for (int i = 0; i < 4; ++i) {
+                        const bool seen = live[u] && j0 + 32 * half + 16 * t + 4 * kq + i <= jmax[u];
+                        st[u][t][i] = seen ? st[u][t][i] * scale2 : -INFINITY;
+                        mc = fmaxf(mc, st[u][t][i]);
+                    }
+            } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    st[t][i] *= scale2;
-                    mc = fmaxf(mc, st[t][i]);
-                }
-        }
-        mc = fmaxf(mc, __shfl_xor(mc, 16));
-        mc = fmaxf(mc, __shfl_xor(mc, 32));
-        const float mn = fmaxf(mrun, mc);  // (-inf while this half has not met a visible key of the row yet)
-        const float alpha = mrun > -INFINITY ? __builtin_amdgcn_exp2f(mrun - mn) : 0.f;
-        float ls = 0.f;
-        if (masked) {
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                    for (int i = 0; i < 4; ++i) {
+                        st[u][t][i] *= scale2;
+                        mc = fmaxf(mc, st[u][t][i]);
+                    }
+            }
+            mc = fmaxf(mc, __shfl_xor(mc, 16));
+            mc = fmaxf(mc, __shfl_xor(mc, 32));
+            const float mn = fmaxf(mrun[u], mc);  // (-inf while this half has not met a visible key of the row yet)
+            const float alpha = mrun[u] > -INFINITY ? __builtin_amdgcn_exp2f(mrun[u] - mn) : 0.f;
+            float ls = 0.f;
+            if (masked) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float pv = st[t][i] > -INFINITY ? __builtin_amdgcn_exp2f(st[t][i] - mn) : 0.f;
-                    st[t][i] = pv;
-                    ls += pv;
-                }
-        } else {
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                    for (int i = 0; i < 4; ++i) {
+                        const float pv = st[u][t][i] > -INFINITY ? __builtin_amdgcn_exp2f(st[u][t][i] - mn) : 0.f;
+                        st[u][t][i] = pv;
+                        ls += pv;
+                    }
+            } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float pv = __builtin_amdgcn_exp2f(st[t][i] - mn);
-                    st[t][i] = pv;
-                    ls += pv;
-                }
-        }
-        lrun = lrun * alpha + ls;
-        mrun = mn;
-        if (kq == 0) fx[16 * wave + n] = alpha;
-        // (the LDS operations of one wave complete in order: the read below sees the write above)
-        const f32x4 al = *reinterpret_cast<const f32x4 *>(&fx[16 * wave + 4 * kq]);
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            o[t][0] *= al[0];
-            o[t][1] *= al[1];
-            o[t][2] *= al[2];
-            o[t][3] *= al[3];
+                    for (int i = 0; i < 4; ++i) {
+                        const float pv = __builtin_amdgcn_exp2f(st[u][t][i] - mn);
+                        st[u][t][i] = pv;
+                        ls += pv;
+                    }
+            }
+            lrun[u] = lrun[u] * alpha + ls;
+            mrun[u] = mn;
+            if (kq == 0) fx[16 * (RT * wave + u) + n] = alpha;
+            // (the LDS operations of one wave complete in order: the read below sees the write above)
+            const f32x4 al = *reinterpret_cast<const f32x4 *>(&fx[16 * (RT * wave + u) + 4 * kq]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                o[u][t][0] *= al[0];
+                o[u][t][1] *= al[1];
+                o[u][t][2] *= al[2];
+                o[u][t][3] *= al[3];
+            }
         }
         // ---- O += P V over this half's 32 keys
         {
-            const f16x8 pa = {(_Float16)st[0][0], (_Float16)st[0][1], (_Float16)st[0][2], (_Float16)st[0][3],
-                              (_Float16)st[1][0], (_Float16)st[1][1], (_Float16)st[1][2], (_Float16)st[1][3]};
+            f16x8 pa[RT];
+#pragma unroll
+            for (int u = 0; u < RT; ++u)
+                pa[u] = f16x8{(_Float16)st[u][0][0], (_Float16)st[u][0][1], (_Float16)st[u][0][2], (_Float16)st[u][0][3],
+                              (_Float16)st[u][1][0], (_Float16)st[u][1][1], (_Float16)st[u][1][2], (_Float16)st[u][1][3]};
 #pragma unroll
             for (int t = 0; t < DT; ++t) {
                 const f16x8 vb = *reinterpret_cast<const f16x8 *>(&vt[(16 * t + n) * VP + 32 * half + 8 * kq]);
-                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[t], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < RT; ++u) o[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[u], vb, o[u][t], 0, 0, 0);
             }
         }
     }
     // ---- the two halves of a row meet: the waves of the second half leave maximum, sum and output in LDS (the tiles are
     // free after the last chunk), the waves of the first half combine, normalise and write.  The lane holds rows
     // 4 kq + i, values 16 t + n of the output, and - in score layout - the statistics of row n.
-    lrun += __shfl_xor(lrun, 16);
-    lrun += __shfl_xor(lrun, 32);
+#pragma unroll
+    for (int u = 0; u < RT; ++u) {
+        lrun[u] += __shfl_xor(lrun[u], 16);
+        lrun[u] += __shfl_xor(lrun[u], 32);
+    }
     __syncthreads();  // every wave is done with the tiles
-    float *xo = att_smem + rt * (16 * D + 32);  // [DT][4][64] output, then 16 maxima, 16 sums
+    float *xo0 = att_smem + rt * RT * (16 * D + 32);  // per u: [DT][4][64] output, then 16 maxima, 16 sums
     if (half == 1) {
 #pragma unroll
-        for (int t = 0; t < DT; ++t)
+        for (int u = 0; u < RT; ++u) {
+            float *xo = xo0 + u * (16 * D + 32);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xo[(t * 4 + i) * 64 + lane] = o[t][i];
-        if (kq == 0) {
-            xo[16 * D + n] = mrun;
-            xo[16 * D + 16 + n] = lrun;
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xo[(t * 4 + i) * 64 + lane] = o[u][t][i];
+            if (kq == 0) {
+                xo[16 * D + n] = mrun[u];
+                xo[16 * D + 16 + n] = lrun[u];
+            }
         }
     }
     __syncthreads();
     if (half == 0) {
-        const float m1 = xo[16 * D + n], l1 = xo[16 * D + 16 + n];
-        const float mm = fmaxf(mrun, m1);
-        const float a0 = mrun > -INFINITY ? __builtin_amdgcn_exp2f(mrun - mm) : 0.f, a1 = m1 > -INFINITY ? __builtin_amdgcn_exp2f(m1 - mm) : 0.f;
-        const float il = live ? 1.f / (lrun * a0 + l1 * a1) : 0.f;
-        if (kq == 0) {
-            fx[16 * wave + n] = a0 * il;
-            fx[16 * (wave + 4) + n] = a1 * il;
-        }
-        const f32x4 f0 = *reinterpret_cast<const f32x4 *>(&fx[16 * wave + 4 * kq]), f1 = *reinterpret_cast<const f32x4 *>(&fx[16 * (wave + 4) + 4 * kq]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int ro = 16 * rt + 4 * kq + i, to = ro / group, ho = ro - to * group;
-            if (ro < rows && t0 + to < T) {
-                float *op = out + ((size_t)(t0 + to) * heads + g * group + ho) * D + n;
+        for (int u = 0; u < RT; ++u) {
+            const float *xo = xo0 + u * (16 * D + 32);
+            const float m1 = xo[16 * D + n], l1 = xo[16 * D + 16 + n];
+            const float mm = fmaxf(mrun[u], m1);
+            const float a0 = mrun[u] > -INFINITY ? __builtin_amdgcn_exp2f(mrun[u] - mm) : 0.f, a1 = m1 > -INFINITY ? __builtin_amdgcn_exp2f(m1 - mm) : 0.f;
+            const float il = live[u] ? 1.f / (lrun[u] * a0 + l1 * a1) : 0.f;
+            float *f = fx + 16 * (RT * wave + u), *f2 = fx + 16 * (RT * (wave + 4) + u);
+            if (kq == 0) {
+                f[n] = a0 * il;
+                f2[n] = a1 * il;
+            }
+            const f32x4 f0 = *reinterpret_cast<const f32x4 *>(&f[4 * kq]), f1 = *reinterpret_cast<const f32x4 *>(&f2[4 * kq]);
 #pragma unroll
-                for (int t = 0; t < DT; ++t) op[16 * t] = o[t][i] * f0[i] + xo[(t * 4 + i) * 64 + lane] * f1[i];
+            for (int i = 0; i < 4; ++i) {
+                const int ro = 16 * (rt + 4 * u) + 4 * kq + i, to = ro / group, ho = ro - to * group;
+                if (ro < rows && t0 + to < T) {
+                    float *op = out + ((size_t)(t0 + to) * heads + g * group + ho) * D + n;
+#pragma unroll
+                    for (int t = 0; t < DT; ++t) op[16 * t] = o[u][t][i] * f0[i] + xo[(t * 4 + i) * 64 + lane] * f1[i];
+                }
             }
         }
     }

@@ -2028,6 +2028,7 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
     if (waited) g_ws.used = false;
 }
 
+constexpr int ATT_TWO_TILES = 1;
 template <int D>
 int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, const float *q, float *att, hipStream_t st) {
     const int group = m->heads / m->kv;
@@ -2037,11 +2038,19 @@ int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tok
     if (tokens > g.gemv_max_rows) {
         if constexpr (D == 64 || D == 128) {
             if (group <= AM_ROWS) {
+                const int qt2 = 2 * AM_ROWS / group, blocks2 = (tokens + qt2 - 1) / qt2;
+                if (blocks2 * m->kv >= ATT_TWO_TILES * g.cus) {
+                    constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 2>();
+                    if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 2>, lds)) return rc;
+                    hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 2>), dim3(m->kv, blocks2), dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads,
+                                       m->kv, pos0, tokens, scale);
+                    return JITNN_HIP_OK;
+                }
                 const int qt = AM_ROWS / group;
                 const dim3 grid((tokens + qt - 1) / qt, m->kv);
-                constexpr size_t lds = attn_prefill_mfma_lds_bytes<D>();
-                if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D>, lds)) return rc;
-                hipLaunchKernelGGL(attn_prefill_mfma_kernel<D>, grid, dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads, m->kv, pos0, tokens,
+                constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 1>();
+                if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 1>, lds)) return rc;
+                hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 1>), grid, dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads, m->kv, pos0, tokens,
                                    scale);
                 return JITNN_HIP_OK;
             }

@@ -1,0 +1,41 @@
+"""The attention of long prompts, 128 query rows per workgroup (attn_prefill_mfma_kernel<D, 2>), against the same prompt in
+pieces that are short enough for 64 rows per workgroup: every row meets the same chunks of keys in the same order, with the same
+FP16 operands and FP32 sums, so that what differs between the two is the route of the linears (FP16 operands, K cut elsewhere).
+The second layer's keys and values follow from the attention output of every token of the first.
+
+Tolerance: two sets of FP16-operand linears, 2e-3 of the largest magnitude each (a wrong row of the attention is off by 1e-1)."""
+import numpy as np
+import pytest
+
+from helpers import norm_err
+from test_gpu_decode import SLOTS, build
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,tokens,pos0", [
+    (32, 8, 64, 1030, 5),   # groups of four; the last block partly filled, keys in front of the prompt
+    (32, 8, 128, 1090, 0),
+    (24, 8, 64, 1400, 63),  # groups of three: 126 of a block's 128 rows, and the mask on every chunk
+    (8, 8, 128, 4000, 1),   # one query head per key / value head
+    (10, 2, 64, 3300, 0)])  # groups of five over two heads
+def test_long_prompt_in_one_pass_and_in_pieces(heads, kv_heads, head_dim, tokens, pos0):
+    import jitnn_amd as jn
+    jn.init()
+    d = 512
+    cfg = dict(layers=2, d_model=d, heads=heads, kv_heads=kv_heads, head_dim=head_dim, ffn=512, vocab=300, max_ctx=pos0 + tokens, rms_eps=1e-5, rope_theta=5e5)
+    dec, _, _, _ = build(jn, cfg, 29, {s: "Q8_0" for s in SLOTS}, "Q8_0")
+    rng = np.random.default_rng(heads + tokens)
+    x = rng.standard_normal((pos0 + tokens, d)).astype(np.float32)
+    if pos0:
+        dec.prefill(x[:pos0], 0)
+    whole = dec.prefill(x[pos0:], pos0)
+    got = dec.kv_read(1, pos0, tokens)
+    for at in range(pos0, pos0 + tokens, 400):
+        pieces = dec.prefill(x[at:min(at + 400, pos0 + tokens)], at)
+    ref = dec.kv_read(1, pos0, tokens)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert norm_err(a, b) <= 4e-3
+    assert norm_err(whole, pieces) <= 4e-3
+    dec.close()
