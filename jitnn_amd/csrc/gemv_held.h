@@ -9,7 +9,12 @@
 // tiles of 16 weight rows: it fetches and decodes its 16 x 256 piece, runs it against its G groups and leaves the sums in LDS,
 // where the workgroup's waves are added up in wave order.  An operand is read once per workgroup instead of once per pair of
 // tiles, and a wave's G chains of products are independent of one another.  Rows longer than the workgroup's columns are cut
-// into slices of K, workgroups of their own; their sums meet in rows_join_kernel, in slice order (no atomics).
+// into slices of K, workgroups of their own; their sums meet in rows_join_kernel, or in the kernel that reads them next, in slice
+// order (no atomics).
+// What bounds it: the vector instructions of a step - decoding about 170 of them per 16 x 256 tile of Q4_K, folding 10 per group;
+// 0.8 to 1.8 us by format and 0.2 to 0.4 us per group for the two waves of a SIMD - and per launch 0.6 to 0.9 us per group for the
+// operands' way into the registers.  Q4_K 14336 x 4096 at 40 rows: 20 us, seven steps.  A second step's weights under way (9 to 17
+// more registers) measured the same or, spilling, slower.
 #pragma once
 #include "gemv_rows.h"
 
@@ -27,6 +32,8 @@ __host__ __device__ constexpr size_t gemv_held_lds_bytes(int groups_held) {
            (size_t)gh_ops_in_lds(FMT, groups_held) * GR_WAVES * groups_held * 1024;
 }
 
+// whether the request for the next weights is kept from being scheduled late (36 -> 35 us, Q4_K 14336 x 4096 at 64 rows); where
+// registers are short that spills some
 __host__ __device__ constexpr bool gh_pin_fetch(int fmt, int groups_held) { return groups_held < 5 && !(fmt == F_Q6_K && groups_held == 4); }
 
 // Where the workgroups of a launch work; one dword to the kernel, with the arguments that are preloaded.

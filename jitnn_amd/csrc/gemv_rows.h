@@ -21,7 +21,8 @@
 // a stage of its own in LDS (RStaged), turns them into operands once, and runs them against every group of eight
 // activation rows.  Partial sums live in LDS per lane (the group index is a run-time value) and are added across the
 // eight waves in wave order at the end of a tile batch: a fixed summation order, no atomics.  A launch with few tiles
-// puts several workgroups on a batch, each with a share of the groups (gridDim.y).
+// puts several workgroups on a batch, each with a share of the groups (gridDim.y).  Launches that leave this kernel a part of a
+// round, or much to decode per tile, go to gemv_held_kernel (gemv_held.h).
 #pragma once
 #include "common.h"
 #include "gemv_mfma.h"
@@ -190,14 +191,12 @@ struct RStaged {
         for (int i = 0; i < FULL; ++i) r.c[i] = ld128<ALIGN>(q + 64 * i);
         if constexpr (REST > 0) r.c[FULL] = ld128<ALIGN>(q + p.rest);  // (lanes past 16 REST repeat rows: the same lines)
     }
-    // -> this lane's row (lane & 15 of the tile) in the wave's stage.  ALL_LANES: the lanes that repeat rows in the load of the odd
-    // chunks store them too (the same bytes), and nothing is conditional
-    template <bool ALL_LANES = false>
+    // -> this lane's row (lane & 15 of the tile) in the wave's stage
     __device__ static __forceinline__ const uint8_t *park(const Raw &r, uint8_t *stage, int lane) {
 #pragma unroll
         for (int i = 0; i < FULL; ++i) *reinterpret_cast<u32x4 *>(stage + (lane >> 2) * STRIDE + 16 * (lane & 3) + 64 * i) = r.c[i];
         if constexpr (REST > 0) {
-            if (ALL_LANES || lane < 16 * REST) *reinterpret_cast<u32x4 *>(stage + ((lane / RD) & 15) * STRIDE + 16 * (4 * FULL + lane % RD)) = r.c[FULL];
+            if (lane < 16 * REST) *reinterpret_cast<u32x4 *>(stage + (lane / RD) * STRIDE + 16 * (4 * FULL + lane % RD)) = r.c[FULL];
         }
         // the lanes of a wave run in step and LDS serves them in order: a fence for the compiler is all this needs
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

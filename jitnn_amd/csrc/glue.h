@@ -296,7 +296,8 @@ __global__ void __launch_bounds__(NR_THREADS) rms_norm_rows_join_kernel(const fl
         give(i, *reinterpret_cast<const float4 *>((part ? xsum : x) + row + i));
 }
 
-// Rotary embedding of the query heads in place (q [T, heads, D]) and of the key heads on their way into the cache,
+// Rotary embedding of the query heads in place (q [T, heads, D]) and of the key heads on their way into the cache (grid: tokens x
+// workgroups that share a token: with one each, 40 tokens took 7.2 us, with four 3.7),
 // values copied into the cache: token t = blockIdx.x sits at position pos0 + t.  Same rotation as attn_decode_kernel.
 __global__ void __launch_bounds__(256) rope_append_rows_kernel(float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
                                                                 float *__restrict__ kcache, float *__restrict__ vcache,
@@ -395,23 +396,25 @@ __global__ void __launch_bounds__(256) rope_append_rows_join_kernel(const float 
 //   grid (token blocks, kv_heads), 256 threads, attn_prefill_lds_bytes<D>() of dynamic LDS; out [T, heads, D].
 constexpr int ATT_ROWS = 32;  // 16 row groups of ATT_RT rows
 constexpr int ATT_RT = ATT_ROWS / 16;
-template <int D>
+template <int D, int TR>
 constexpr size_t attn_prefill_lds_bytes() {
-    return sizeof(float) * ((size_t)ATT_ROWS * D + (size_t)AttCfg<D>::CH * (D + 4) + (size_t)AttCfg<D>::CH * D + (size_t)AttCfg<D>::CH * (ATT_ROWS + 4));
+    constexpr int ROWS = 16 * TR;
+    return sizeof(float) * ((size_t)ROWS * D + (size_t)AttCfg<D>::CH * (D + 4) + (size_t)AttCfg<D>::CH * D + (size_t)AttCfg<D>::CH * (ROWS + 4));
 }
-template <int D>
+template <int D, int TR>
 __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restrict__ q, const float *__restrict__ kcache,
                                                             const float *__restrict__ vcache, float *__restrict__ out, int heads, int kv_heads, int pos0,
                                                             int T, float scale) {
-    constexpr int CH = AttCfg<D>::CH, DQ = D / 4, KN = CH / 16, DV = D / 16, KP = D + 4, PP = ATT_ROWS + 4;
+    constexpr int ROWS = 16 * TR;
+    constexpr int CH = AttCfg<D>::CH, DQ = D / 4, KN = CH / 16, DV = D / 16, KP = D + 4, PP = ROWS + 4;
     static_assert(D % 64 == 0 && CH % 16 == 0, "tiles of 16 threads");
     extern __shared__ __align__(16) float att_smem[];
-    float *Qs = att_smem;             // [ATT_ROWS][D]
-    float *Ks = Qs + ATT_ROWS * D;    // [CH][D + 4]
+    float *Qs = att_smem;             // [ROWS][D]
+    float *Ks = Qs + ROWS * D;    // [CH][D + 4]
     float *Vs = Ks + CH * KP;         // [CH][D]
-    float *Pt = Vs + CH * D;          // [CH][ATT_ROWS + 4]: probabilities, key-major
+    float *Pt = Vs + CH * D;          // [CH][ROWS + 4]: probabilities, key-major
     const int tid = threadIdx.x, rg = tid >> 4, kl = tid & 15;
-    const int group = heads / kv_heads, QT = ATT_ROWS / group, rows = QT * group;
+    const int group = heads / kv_heads, QT = ROWS / group, rows = QT * group;
     const int g = blockIdx.y;
     // two workgroups share a CU and the early token blocks have few keys to walk: the upper half of the key/value heads
     // takes the blocks in reverse, so that the pair a CU is likely to hold has one long and one short walk
@@ -419,16 +422,16 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restri
     const int t0 = tb * QT;
     const int tl = min(t0 + QT, T) - 1;                // last token of the block
     const int nchunks = (pos0 + tl + CH) / CH;         // chunks that hold keys up to its position
-    for (int i = tid; i < ATT_ROWS * DQ; i += 256) {
+    for (int i = tid; i < ROWS * DQ; i += 256) {
         const int r = i / DQ, e = (i - r * DQ) * 4, tq = r / group, h = r - tq * group;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (r < rows && t0 + tq < T) v = *reinterpret_cast<const float4 *>(q + ((size_t)(t0 + tq) * heads + g * group + h) * D + e);
         *reinterpret_cast<float4 *>(&Qs[r * D + e]) = v;
     }
-    float mrun[ATT_RT], lrun[ATT_RT];
-    float4 acc[ATT_RT][DV / 4];
+    float mrun[TR], lrun[TR];
+    float4 acc[TR][DV / 4];
 #pragma unroll
-    for (int i = 0; i < ATT_RT; ++i) {
+    for (int i = 0; i < TR; ++i) {
         mrun[i] = -INFINITY;
         lrun[i] = 0.f;
 #pragma unroll
@@ -450,21 +453,21 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restri
             *reinterpret_cast<float4 *>(&Vs[j * D + e]) = vv;
         }
         __syncthreads();
-        // ---- scores of rows ATT_RT rg .. against keys kl + 16 n
-        float sc[ATT_RT][KN];
+        // ---- scores of rows TR rg .. against keys kl + 16 n
+        float sc[TR][KN];
 #pragma unroll
-        for (int i = 0; i < ATT_RT; ++i)
+        for (int i = 0; i < TR; ++i)
 #pragma unroll
             for (int n = 0; n < KN; ++n) sc[i][n] = 0.f;
 #pragma unroll 4
         for (int d4 = 0; d4 < DQ; ++d4) {
-            float4 qv[ATT_RT], kv[KN];
+            float4 qv[TR], kv[KN];
 #pragma unroll
-            for (int i = 0; i < ATT_RT; ++i) qv[i] = *reinterpret_cast<const float4 *>(&Qs[(ATT_RT * rg + i) * D + 4 * d4]);
+            for (int i = 0; i < TR; ++i) qv[i] = *reinterpret_cast<const float4 *>(&Qs[(TR * rg + i) * D + 4 * d4]);
 #pragma unroll
             for (int n = 0; n < KN; ++n) kv[n] = *reinterpret_cast<const float4 *>(&Ks[(kl + 16 * n) * KP + 4 * d4]);
 #pragma unroll
-            for (int i = 0; i < ATT_RT; ++i)
+            for (int i = 0; i < TR; ++i)
 #pragma unroll
                 for (int n = 0; n < KN; ++n) {
                     sc[i][n] = __builtin_fmaf(qv[i].x, kv[n].x, sc[i][n]);
@@ -475,8 +478,8 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restri
         }
         // ---- running softmax of each row (its keys sit in the 16 lanes of this DPP row, and so does its output)
 #pragma unroll
-        for (int i = 0; i < ATT_RT; ++i) {
-            const int r = ATT_RT * rg + i, tq = r / group;
+        for (int i = 0; i < TR; ++i) {
+            const int r = TR * rg + i, tq = r / group;
             const bool live = r < rows && t0 + tq < T;
             float mc = -INFINITY;
 #pragma unroll
@@ -504,17 +507,17 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restri
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // ---- weighted value sums: rows ATT_RT rg .., values DV kl .. + DV - 1
+        // ---- weighted value sums: rows TR rg .., values DV kl .. + DV - 1
 #pragma unroll 4
         for (int j = 0; j < CH; ++j) {
-            float pr[ATT_RT];
+            float pr[TR];
 #pragma unroll
-            for (int i = 0; i < ATT_RT; ++i) pr[i] = Pt[j * PP + ATT_RT * rg + i];
+            for (int i = 0; i < TR; ++i) pr[i] = Pt[j * PP + TR * rg + i];
 #pragma unroll
             for (int e = 0; e < DV / 4; ++e) {
                 const float4 v = *reinterpret_cast<const float4 *>(&Vs[j * D + DV * kl + 4 * e]);
 #pragma unroll
-                for (int i = 0; i < ATT_RT; ++i) {
+                for (int i = 0; i < TR; ++i) {
                     acc[i][e].x = __builtin_fmaf(pr[i], v.x, acc[i][e].x);
                     acc[i][e].y = __builtin_fmaf(pr[i], v.y, acc[i][e].y);
                     acc[i][e].z = __builtin_fmaf(pr[i], v.z, acc[i][e].z);
@@ -524,8 +527,8 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(const float *__restri
         }
     }
 #pragma unroll
-    for (int i = 0; i < ATT_RT; ++i) {
-        const int r = ATT_RT * rg + i, tq = r / group, h = r - tq * group;
+    for (int i = 0; i < TR; ++i) {
+        const int r = TR * rg + i, tq = r / group, h = r - tq * group;
         if (r < rows && t0 + tq < T) {
             float *o = out + ((size_t)(t0 + tq) * heads + g * group + h) * D + DV * kl;
             const float il = 1.f / lrun[i];
@@ -702,12 +705,14 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 }
 
 // The same attention on the matrix cores (v_mfma_f32_16x16x32_f16, FP16 operands, FP32 accumulation and softmax), for
-// heads of 64 or 128 values.  A workgroup of eight waves takes AM_ROWS = 64 (token, query head) rows of one key/value head
-// and walks the keys in chunks of AM_CH = 64 staged once in LDS as binary16 for all of them; a wave takes 16 rows and ONE
-// HALF of every chunk's keys (waves 0-3 the first 32, waves 4-7 the last 32), keeps its own running maximum, sum and
-// output, and the two halves of a row meet once, at the end, through LDS.  What limits this kernel is the length of the
-// dependent chain a wave walks per chunk (operand reads, MFMAs, softmax, MFMAs), not any unit's throughput: 16 rows x 64
-// keys per wave took 20 us per layer at 512 tokens whether a workgroup held 64 or 128 rows.
+// heads of 64 or 128 values.  A workgroup of eight waves takes RT * AM_ROWS = 64 or 128 (token, query head) rows of one
+// key/value head and walks the keys in chunks of AM_CH = 64 staged once in LDS as binary16 for all of them; a wave takes RT
+// tiles of 16 rows and ONE HALF of every chunk's keys (waves 0-3 the first 32, waves 4-7 the last 32), keeps its own running
+// maximum, sum and output, and the two halves of a row meet once, at the end, through LDS.  What limits this kernel is what a
+// workgroup repeats per chunk for all its rows - staging and conversion of 64 keys and values, a barrier - and the dependent
+// chain of a wave (operand reads, products, softmax, products).  RT = 2 spreads both over twice the rows: every operand read
+// from LDS feeds two products, and a wave has two chains.  Kernel trace, 32 heads over 8 of 128 values, us per layer with
+// RT = 1 / 2: 1024 tokens 53 / 41, 1536 101 / 61, 2048 158 / 97, 4096 499 / 336 (310 with the lagging maximum below).
 //   * scores, transposed: S^T = K Q^T, so that a lane ends up with the scores of ONE query row (column lane % 16 of the
 //     result) against the keys 4 (lane / 16) + i of every 16-key tile - the running softmax of a row needs its chunk
 //     maximum from the three other lanes that hold the row's other keys (two shuffles), the row sum stays a per-lane
