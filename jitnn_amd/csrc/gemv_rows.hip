@@ -181,12 +181,14 @@ HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, int join, int cus, int 
                 tiles = (float)st.tiles;
     // (a pair of streaming launches is taken at twice one: the preparation they share is paid by their second round of CUs; the
     // fitted lines err by a few per cent: a launch changes kernels for three)
+    // (a reader's join costs it extra loads, and most of what the line calls the join is the way of the slices to memory: taken as
+    // free, the 4096 x 4096 projections of a 40-token prompt went to the held kernel, 12.1 against 10.4 us)
     float best_us = 0.97f * (float)weights * (cost.s_base + cost.s_long * k / 4096.f + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
     for (int shares = 1; shares <= groups; ++shares) {
         const int held = (groups + shares - 1) / shares;
         if (held > GH_G_MAX || (groups + held - 1) / held != shares || geo.slices * shares > cus) continue;
         const int per_slice = std::min({cus / (geo.slices * shares), steps, 4095}), walk = (steps + per_slice - 1) / per_slice;
-        const float us = cost.h_base + cost.h_long * k / 4096.f + (part && join != HELD_JOIN_READER ? cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
+        const float us = cost.h_base + cost.h_long * k / 4096.f + (part ? join == HELD_JOIN_READER ? 0.75f * cost.h_join : cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
                          cost.h_mb * 1e-6f * part * rows * n * weights;
         if (us < best_us) {
             best_us = us;

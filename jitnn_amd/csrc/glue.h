@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(256) rope_append_rows_join_kernel(const float 
                                                                      float *__restrict__ kcache, float *__restrict__ vcache,
                                                                      const float *__restrict__ cosv, const float *__restrict__ sinv, int heads,
                                                                      int kv_heads, int D, int pos0, int interleaved) {
-    const int t = blockIdx.x, pos = pos0 + t, half = D / 2;
+    const int t = blockIdx.x, pos = pos0 + t, half = D / 2, first = blockIdx.y * 256 + threadIdx.x, stride = gridDim.y * 256;
     const int nq = heads * D, nk = kv_heads * D;
     const size_t zq = (size_t)T * nq, zk = (size_t)T * nk;  // floats per slice
     const float *pq = part + (size_t)t * nq, *pk = part + zq * s0 + (size_t)t * nk, *pv = part + zq * s0 + zk * s1 + (size_t)t * nk;
@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(256) rope_append_rows_join_kernel(const float 
     };
     // a rotation item: four angles p .. p + 3 of one head - values (p .. p + 3, p + half .. p + half + 3), or 2 p .. 2 p + 7 in pairs
     auto rotate = [&](auto zc, const float *src, size_t zs, int splits, float *dst, int nheads) {
-        for (int i = threadIdx.x; i < nheads * (half / 4); i += 256) {
+        for (int i = first; i < nheads * (half / 4); i += stride) {
             const int h = i / (half / 4), p = 4 * (i - h * (half / 4));
             const float4 cs = *reinterpret_cast<const float4 *>(cp + p), sn = *reinterpret_cast<const float4 *>(sp + p);
             if (interleaved) {
@@ -381,7 +381,7 @@ __global__ void __launch_bounds__(256) rope_append_rows_join_kernel(const float 
     with_slices(s1, [&](auto zc) { rotate(zc, pk, zk, s1, kcache + (size_t)pos * nk, kv_heads); });
     float *vc = vcache + (size_t)pos * nk;
     with_slices(s2, [&](auto zc) {
-        for (int i = 4 * threadIdx.x; i < nk; i += 1024) *reinterpret_cast<float4 *>(vc + i) = joined(zc, pv, zk, s2, i);
+        for (int i = 4 * first; i < nk; i += 4 * stride) *reinterpret_cast<float4 *>(vc + i) = joined(zc, pv, zk, s2, i);
     });
 }
 

@@ -1363,8 +1363,11 @@ bool rows_path(const jitnn_hip_weight *w, int rows) {
 // swiglu_up: the activations are silu(x) * swiglu_up, formed by the preparation as it reads x.
 // later, defer (one weight, a residual): where the sums come in up to eight slices, they go to later and their join is left to the
 // caller, as *defer.
+// together, room, gdefer (three weights): where one of them comes in slices, all three go to `together` (room floats), one after
+// the other, a weight that has none as its one slice, and the caller joins them, as *gdefer.
 int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int count, const float *x, int rows, const float *bias, const float *residual,
-                      hipStream_t s, ScratchSource src, const float *swiglu_up = nullptr, float *later = nullptr, PfPending *defer = nullptr) {
+                      hipStream_t s, ScratchSource src, const float *swiglu_up = nullptr, float *later = nullptr, PfPending *defer = nullptr,
+                      float *together = nullptr, size_t room = 0, PfGroupPending *gdefer = nullptr) {
     const int k = ws[0]->k;
     bool need[GR_LAYOUTS] = {};  // the operand layouts the weights ask for
     const size_t one = (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255;
@@ -1379,7 +1382,19 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
     HeldPlan plan[3];
     size_t part = 0;
     int later_plan = 0;  // slices whose join the caller gets
-    for (int i = 0; i < count; ++i) {
+    bool grouped = false;
+    if (gdefer && count == 3) {
+        size_t floats = 0;
+        int most = 1;
+        for (int i = 0; i < 3; ++i) {
+            plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, HELD_JOIN_READER, g.cus);
+            const int splits = plan[i].groups_held ? plan[i].slices : 1;
+            floats += (size_t)splits * rows * ws[i]->n;
+            most = std::max(most, splits);
+        }
+        grouped = most > 1 && most <= 8 && floats <= room;
+    }
+    for (int i = 0; i < count && !grouped; ++i) {
         const bool put_off = defer && k <= 8 * 2048;  // (a slice is at most eight columns; more slices only where that is less than k / 2048)
         plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, put_off ? HELD_JOIN_READER : bias || residual ? HELD_JOIN_ADDS : HELD_JOIN_SLICES, g.cus);
         if (put_off && plan[i].slices > 1 && plan[i].slices <= 8) {
@@ -1409,7 +1424,15 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
     gemv_rows_prepare_launch(s, x, swiglu_up, (void *const *)sc, k, rows);
     for (int i = 0; i < count; ++i) {
         const void *ops = sc[gemv_rows_layout(ws[i]->fmt)];
-        if (later_plan) {
+        if (grouped) {
+            const int splits = plan[i].groups_held ? plan[i].slices : 1;
+            if (plan[i].groups_held) gemv_held_slices_launch(plan[i], ws[i]->fmt, s, ws[i]->dev, nullptr, ops, together, ws[i]->n, k, rows);
+            else gemv_rows_main_launch(ws[i]->fmt, (unsigned)g.cus, s, ws[i]->dev, ops, nullptr, nullptr, together, ws[i]->n, k, rows);
+            if (i == 0) gdefer->part = together;
+            gdefer->sg.splits[i] = splits;
+            gdefer->sg.n[i] = ws[i]->n;
+            together += (size_t)splits * rows * ws[i]->n;
+        } else if (later_plan) {
             gemv_held_slices_launch(plan[i], ws[i]->fmt, s, ws[i]->dev, nullptr, ops, later, ws[i]->n, k, rows);
             defer->part = later;
             defer->res = residual;
@@ -1933,7 +1956,8 @@ int normed_linears_rows(const jitnn_hip_llama *m, const jitnn_hip_weight *const 
     for (int i = 0; i < count; ++i) shared = shared && rows_path(ws[i], rows);
     if (shared) {
         for (int i = 0; i < count; ++i) count_op(ST_GEMV, (long long)ws[i]->nbytes + 4ll * rows * ((long long)ws[i]->k + ws[i]->n));
-        return launch_rows_group(ws, ys, count, xn, rows, nullptr, nullptr, st, SCRATCH_THREAD);
+        // (the slices in the buffer of the gate projection, which is written after they are read)
+        return launch_rows_group(ws, ys, count, xn, rows, nullptr, nullptr, st, SCRATCH_THREAD, nullptr, nullptr, nullptr, m->pf[7], (size_t)rows * m->ffn, gdefer);
     }
     for (int i = 0; i < count; ++i)
         if (int rc = jitnn_hip_linear_dev(ws[i], xn, rows, nullptr, ys[i], (void *)st)) return rc;
@@ -2296,7 +2320,7 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
             if (int rc = normed_linears_rows(m, ws, ys, 3, x, T, nw, xn, st, &pend, &gp)) return rc;
         }
         if (gp.part) {  // q, k and v still lie in K slices: the rotation adds them up as it reads them
-            hipLaunchKernelGGL(rope_append_rows_join_kernel, dim3(T), dim3(256), 0, st, gp.part, gp.sg.splits[0], gp.sg.splits[1], gp.sg.splits[2], T, q,
+            hipLaunchKernelGGL(rope_append_rows_join_kernel, dim3(T, T < 256 ? 4 : 1), dim3(256), 0, st, gp.part, gp.sg.splits[0], gp.sg.splits[1], gp.sg.splits[2], T, q,
                                m->kc + lo, m->vc + lo, m->cosv, m->sinv, m->heads, m->kv, m->hd, pos0, m->rope_interleaved);
             gp.part = nullptr;
         } else {
