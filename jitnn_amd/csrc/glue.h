@@ -712,7 +712,7 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 // workgroup repeats per chunk for all its rows - staging and conversion of 64 keys and values, a barrier - and the dependent
 // chain of a wave (operand reads, products, softmax, products).  RT = 2 spreads both over twice the rows: every operand read
 // from LDS feeds two products, and a wave has two chains.  Kernel trace, 32 heads over 8 of 128 values, us per layer with
-// RT = 1 / 2: 1024 tokens 53 / 41, 1536 101 / 61, 2048 158 / 97, 4096 499 / 336 (310 with the lagging maximum below).
+// RT = 1 / 2: 1024 tokens 53 / 41, 1536 101 / 61, 2048 158 / 97, 4096 499 / 336.
 //   * scores, transposed: S^T = K Q^T, so that a lane ends up with the scores of ONE query row (column lane % 16 of the
 //     result) against the keys 4 (lane / 16) + i of every 16-key tile - the running softmax of a row needs its chunk
 //     maximum from the three other lanes that hold the row's other keys (two shuffles), the row sum stays a per-lane
@@ -727,7 +727,6 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 //     tiles are double-buffered, one workgroup barrier per chunk; nothing about the loads is conditional (chunks past
 //     the end repeat the last one, keys past the last visible one re-read it and are masked).
 constexpr int AM_ROWS = 64, AM_CH = 64, AM_WAVES = 2 * (AM_ROWS / 16), AM_THREADS = 64 * AM_WAVES;
-constexpr float AM_LAG = 8.f;
 template <int D, int RT>
 constexpr size_t attn_prefill_mfma_lds_bytes() {
     return (size_t)2 * ((size_t)AM_CH * (D + 8) + (size_t)D * (AM_CH + 8)) * sizeof(_Float16) + RT * AM_WAVES * 16 * sizeof(float);  // (the
@@ -849,7 +848,7 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
         }
         // ---- running softmax of the row, in base 2: exp(scale s - m) = exp2(scale2 s - m2).  Only the chunks that reach
         // past the first row's last key (the diagonal of the block, and everything for rows that do not exist) need the
-        // mask; in the others every score counts and no -inf can appear; scale2 is positive, so that it may follow the maximum.
+        // mask; in the others every score counts and no -inf can appear.
         const bool masked = j0 + CH - 1 > pos0 + t0 || !(t0 + QT <= T && rows == RT * AM_ROWS);  // workgroup-uniform
 #pragma unroll
         for (int u = 0; u < RT; ++u) {
@@ -867,32 +866,18 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) mc = fmaxf(mc, st[u][t][i]);
-                mc *= scale2;
+                    for (int i = 0; i < 4; ++i) {
+                        st[u][t][i] *= scale2;
+                        mc = fmaxf(mc, st[u][t][i]);
+                    }
             }
             mc = fmaxf(mc, __shfl_xor(mc, 16));
             mc = fmaxf(mc, __shfl_xor(mc, 32));
-            // The output so far is rescaled only where a row's maximum has grown by more than AM_LAG powers of two (a wave-uniform
-            // choice): until then the probabilities stand against the maximum of then, at most 2^AM_LAG - FP16 values of the same
-            // relative precision, fewer of them subnormal.  Most chunks past the first keep the factor's exponential, its trip
-            // through LDS and the products with the output.
-            if (__any(mc > mrun[u] + AM_LAG)) {
-                const float mn = fmaxf(mrun[u], mc);
-                const float alpha = mrun[u] > -INFINITY ? __builtin_amdgcn_exp2f(mrun[u] - mn) : 0.f;
-                lrun[u] *= alpha;
-                mrun[u] = mn;
-                if (kq == 0) fx[16 * (RT * wave + u) + n] = alpha;
-                // (the LDS operations of one wave complete in order: the read below sees the write above)
-                const f32x4 al = *reinterpret_cast<const f32x4 *>(&fx[16 * (RT * wave + u) + 4 * kq]);
-#pragma unroll
-                for (int t = 0; t < DT; ++t) {
-                    o[u][t][0] *= al[0];
-                    o[u][t][1] *= al[1];
-                    o[u][t][2] *= al[2];
-                    o[u][t][3] *= al[3];
-                }
-            }
-            const float mn = mrun[u];  // (-inf while this half has not met a visible key of the row yet)
+            // (Rescaling only once the maximum has grown by 2^8 takes 336 to 310 us at 4096 tokens, but the largest weight of a row is
+            // then no longer exactly 1 in FP16: 2 to 7 % more error against FP64.  Only where it has grown at all: the same bits, and
+            // the branch costs more than it saves, 2 to 4 % at one tile per wave.)
+            const float mn = fmaxf(mrun[u], mc);  // (-inf while this half has not met a visible key of the row yet)
+            const float alpha = mrun[u] > -INFINITY ? __builtin_amdgcn_exp2f(mrun[u] - mn) : 0.f;
             float ls = 0.f;
             if (masked) {
 #pragma unroll
@@ -908,12 +893,23 @@ __global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const flo
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[u][t][i], scale2, -mn));
+                        const float pv = __builtin_amdgcn_exp2f(st[u][t][i] - mn);
                         st[u][t][i] = pv;
                         ls += pv;
                     }
             }
-            lrun[u] += ls;
+            lrun[u] = lrun[u] * alpha + ls;
+            mrun[u] = mn;
+            if (kq == 0) fx[16 * (RT * wave + u) + n] = alpha;
+            // (the LDS operations of one wave complete in order: the read below sees the write above)
+            const f32x4 al = *reinterpret_cast<const f32x4 *>(&fx[16 * (RT * wave + u) + 4 * kq]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                o[u][t][0] *= al[0];
+                o[u][t][1] *= al[1];
+                o[u][t][2] *= al[2];
+                o[u][t][3] *= al[3];
+            }
         }
         // ---- O += P V over this half's 32 keys
         {
