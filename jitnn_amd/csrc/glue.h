@@ -732,8 +732,15 @@ constexpr size_t attn_prefill_mfma_lds_bytes() {
     return (size_t)2 * ((size_t)AM_CH * (D + 8) + (size_t)D * (AM_CH + 8)) * sizeof(_Float16) + RT * AM_WAVES * 16 * sizeof(float);  // (the
     // tiles also hold the second halves' outputs at the end: 4 RT x (16 x D + 32) floats fit for D >= 64, RT <= 2)
 }
+// Two tiles of rows per wave from how many 128-row workgroups on (64-row ones, twice as many, keep more CUs at work below): as many
+// as the device holds at once, one per CU at 128 values (199 registers), two at 64 (held to the 128 that two need: the compiler took 131
+// by itself, and with one a CU every round is half as wide).  64 values, us with one tile / two: 256 workgroups 33 / 42 (16 heads
+// over 4, 2048 tokens), 376 65 / 76 (3000), 512 107 / 87 (4096), 528 97 / 82 (32 over 4, 2100 from position 900), 1000 186 / 132 (32
+// over 8, 3970); between 376 and 512 it depends on the heads.  128 values: 176 45 / 50, 256 73 / 60 and 133 / 110 (4 key/value
+// heads), 48 / 36 (8).
+constexpr int attn_two_tiles_from(int D, int cus) { return (D == 64 ? 2 : 1) * cus; }
 template <int D, int RT>
-__global__ void __launch_bounds__(AM_THREADS) attn_prefill_mfma_kernel(const float *__restrict__ q, const float *__restrict__ kcache,
+__global__ void __launch_bounds__(AM_THREADS, D == 64 && RT == 2 ? 4 : 1) attn_prefill_mfma_kernel(const float *__restrict__ q, const float *__restrict__ kcache,
                                                                  const float *__restrict__ vcache, float *__restrict__ out, int heads, int kv_heads,
                                                                  int pos0, int T, float scale) {
     constexpr int CH = AM_CH, KP = D + 8, VP = CH + 8, DB = D / 32, DT = D / 16, DQ = D / 4;

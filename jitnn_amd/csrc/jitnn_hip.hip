@@ -2052,9 +2052,6 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
     if (waited) g_ws.used = false;
 }
 
-// Two tiles of rows per wave from one workgroup per CU on (1024 tokens of 32 heads: 53 -> 41 us); below, 64-row blocks keep more
-// CUs at work.
-constexpr int ATT_TWO_TILES = 1;
 template <int D>
 int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, const float *q, float *att, hipStream_t st) {
     const int group = m->heads / m->kv;
@@ -2065,7 +2062,7 @@ int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tok
         if constexpr (D == 64 || D == 128) {
             if (group <= AM_ROWS) {
                 const int qt2 = 2 * AM_ROWS / group, blocks2 = (tokens + qt2 - 1) / qt2;
-                if (blocks2 * m->kv >= ATT_TWO_TILES * g.cus) {
+                if (blocks2 * m->kv >= attn_two_tiles_from(D, g.cus)) {
                     constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 2>();
                     if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 2>, lds)) return rc;
                     hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 2>), dim3(m->kv, blocks2), dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads,

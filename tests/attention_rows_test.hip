@@ -183,6 +183,15 @@ static void check() {
 }
 
 int main() {
+    // what attn_two_tiles_from counts on: two workgroups of 128 rows on a CU where heads have 64 values, one where they have 128
+    printf("workgroups on a CU\n");
+    int fit64 = 0, fit128 = 0;
+    HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit64, attn_prefill_mfma_kernel<64, 2>, AM_THREADS, attn_prefill_mfma_lds_bytes<64, 2>()));
+    HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit128, attn_prefill_mfma_kernel<128, 2>, AM_THREADS, attn_prefill_mfma_lds_bytes<128, 2>()));
+    if (fit64 != attn_two_tiles_from(64, 1) || fit128 != attn_two_tiles_from(128, 1)) {
+        printf("%d and %d\n", fit64, fit128);
+        return 1;
+    }
     check<64, 1>();
     check<64, 2>();
     check<128, 1>();

@@ -1,5 +1,5 @@
-"""The attention of long prompts, 128 query rows per workgroup (attn_prefill_mfma_kernel<D, 2>), against the same prompt in
-pieces that are short enough for 64 rows per workgroup: every row meets the same chunks of keys in the same order, with the same
+"""The attention of long prompts, 128 query rows per workgroup (attn_prefill_mfma_kernel<D, 2>: from one workgroup per CU on for
+heads of 128 values, two for 64), against the same prompt in pieces that are short enough for 64 rows per workgroup: every row meets the same chunks of keys in the same order, with the same
 FP16 operands and FP32 sums, so that what differs between the two is the route of the linears (FP16 operands, K cut elsewhere).
 The second layer's keys and values follow from the attention output of every token of the first.
 
@@ -14,11 +14,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("heads,kv_heads,head_dim,tokens,pos0", [
-    (32, 8, 64, 1030, 5),   # groups of four; the last block partly filled, keys in front of the prompt
+    (32, 8, 64, 2060, 5),   # groups of four; the last block partly filled, keys in front of the prompt
     (32, 8, 128, 1090, 0),
-    (24, 8, 64, 1400, 63),  # groups of three: 126 of a block's 128 rows, and the mask on every chunk
+    (24, 8, 64, 2700, 63),  # groups of three: 126 of a block's 128 rows, and the mask on every chunk
     (8, 8, 128, 4000, 1),   # one query head per key / value head
-    (10, 2, 64, 3300, 0)])  # groups of five over two heads
+    (20, 4, 64, 3300, 0),   # groups of five over four heads
+    (32, 8, 64, 1030, 5), (24, 8, 64, 1400, 63), (10, 2, 64, 3300, 0)])  # (too few workgroups: 64 rows in the whole prompt too)
 def test_long_prompt_in_one_pass_and_in_pieces(heads, kv_heads, head_dim, tokens, pos0):
     import jitnn_amd as jn
     jn.init()
