@@ -158,6 +158,11 @@ JITNN_HIP_API long long jitnn_hip_noalloc_scratch_bytes(void);
  * runs depends on the scratch too (jitnn_hip_linear). */
 JITNN_HIP_API int jitnn_hip_many_row_tile(const int *fmts, const int *n, int count, int k, int rows, int gate_up, int residual, int compute_units);
 
+/* Which of the two kernels for 9 to 64 rows (3 to 64 of at least 12288 values; rows of whole 256-value columns) jitnn_hip_linear
+ * takes: 0 the one that streams the activations' operands - or another one, for other rows -, otherwise the slices of a row that the one
+ * that holds them adds up.  adds: with a bias.  compute_units as above. */
+JITNN_HIP_API int jitnn_hip_few_rows_slices(int fmt, int n, int k, int rows, int adds, int compute_units);
+
 /* ---- Q8_0 quantiser ----------------------------------------------------------------------------- */
 
 /* FP32 -> Q8_0 blocks (34 bytes per 32 values) with the reference quantiser's arithmetic: F.quantizeQ8 /

@@ -48,6 +48,7 @@ def _bind() -> C.CDLL:
         "jitnn_hip_linear_noalloc_dev": (i, [vp, vp, i, vp, vp, vp]),
         "jitnn_hip_noalloc_scratch_bytes": (ll, []),
         "jitnn_hip_many_row_tile": (i, [C.POINTER(i), C.POINTER(i), i, i, i, i, i, i]),
+        "jitnn_hip_few_rows_slices": (i, [i, i, i, i, i, i]),
         "jitnn_hip_thread_release": (i, []),
         "jitnn_hip_thread_scratch": (i, [C.POINTER(ll), C.POINTER(ll), C.POINTER(i)]),
         "jitnn_hip_quantize_q8_0": (i, [vp, ll, vp]),
@@ -142,6 +143,15 @@ def many_row_tile(weights, k: int, rows: int, gate_up: bool = False, residual: b
     if tile < 0:
         check(tile, "jitnn_hip_many_row_tile")
     return tile
+
+
+def few_rows_slices(fmt: int, n: int, k: int, rows: int, adds: bool = False, compute_units: int = 0) -> int:
+    """Slices of a row in the kernel that holds the activations' operands if a linear on `rows` rows takes it, 0 if it takes the
+    one that streams them (or another one, for other rows)."""
+    slices = lib.jitnn_hip_few_rows_slices(fmt, n, k, rows, adds, compute_units)
+    if slices < 0:
+        check(slices, "jitnn_hip_few_rows_slices")
+    return slices
 
 
 class _Stat(C.Structure):

@@ -133,34 +133,45 @@ KernelRef gemv_held_kernel_ref(int fmt, int groups_held) {
     return block_values(fmt) == 256 ? gemv_held_kernel_k(fmt, groups_held) : gemv_held_kernel_q32(fmt, groups_held);
 }
 
-// Which of the two kernels takes a launch.  What each costs beyond its launches, in units of a wave's work - one decoded
-// tile of 16 rows and a 256-value column, met by its groups of rows - in us, fitted on both kernels at 276 launches (six
-// formats, ten shapes from 512 x 11008 to 14336 x 4096, 9 to 64 rows), root mean square of the estimates' errors 0.9 to 1.6 and
-// 0.5 to 0.8 us:
-//   streaming:  base + long_row k / 4096 + units (decode T + meet g + meet_tile g T), units = rounds x columns per wave, T tiles
-//   held:       base + long_row k / 4096 + join (sliced) + start G + steps (decode + meet G) + slice_mb (MB of sums / 4)
-// The held kernel wins where the streaming one has no whole round of workgroups (4096 x 14336, 14336 x 4096, rows of odd
-// numbers of columns) or decodes much per tile (Q6_K): Q6_K 4096 x 14336 at 12 / 24 / 40 rows 45.2 / 43.1 / 48.8 -> 32.0 / 34.7 /
-// 43.4, Q6_K 2000 x 6912 27.9 -> 18.3 (24 rows), Q4_K 14336 x 4096 25.4 -> 23.6, Q4_0 24000 x 2048 26.4 -> 23.5.  It loses where
-// every CU has exactly one batch, by its second launch: Q4_K 4096 x 4096 15.6 against 16.2, 8192 x 4096 17.2 against 18.7.
+// Which of the two kernels takes a launch.  An estimate of each, preparation and join included, in us, from the work of a wave - one
+// decoded tile of 16 rows and a 256-value column, met by its groups of rows:
+//   streaming:  base + long_row k / 4096 + mb (MB of weights) + units (decode T + meet g + meet_tile g T), units = rounds x columns per
+//               wave, T tiles
+//   held:       base + long_row k / 4096 + mb (MB of weights) + join (sliced) + sums (MB of slices / 4) + start G + steps (decode +
+//               meet G + five (G = 5: operands in LDS))
+// Fitted at 13228 launches of both kernels (eight formats, 270 shapes of 512 to 31488 rows of 1024 to 20480 values; 9 to 64 rows, and 3 to 8
+// on long ones; profiles/linears_9_to_64_rows_both_kernels.txt) by what the choice costs: the time lost on the slower kernel, once and a
+// half for launches the held kernel slows down, a fifth of the weight on each estimate's own error.  116 of the 13228 are slower than
+// with the streaming kernel by more than 1.5 % and 27 by more than 4 (the worst by 14); the mean gain is 1.08 (Q5_1) to 1.30 (Q6_K), at
+// most 0.003 below the better kernel each time.  At 1793 launches of 40 other shapes 65 are slower by more than 1.5 %, 19 by more than 4
+// (9 at worst), mean gain 1.12.
+// The held kernel wins where the streaming one has no whole round of workgroups (4096 x 14336, 14336 x 4096, rows of odd numbers
+// of columns) or decodes much per tile (Q6_K): Q6_K 4096 x 14336 at 12 / 24 / 40 rows 45.2 / 43.1 / 48.8 -> 32.0 / 34.7 / 43.4, Q6_K
+// 2000 x 6912 27.9 -> 18.3 (24 rows), Q4_K 14336 x 4096 25.4 -> 23.6, Q4_0 24000 x 2048 26.4 -> 23.5.  It loses where every CU has
+// exactly one batch, by its second launch (Q4_K 4096 x 4096 15.6 against 16.2, 8192 x 4096 17.2 against 18.7), and with five groups in the
+// formats of 32-value blocks and minima (4096 x 8192 at 40 rows Q4_1 23.7 against 25.2, 14336 x 4096 Q5_1 35.3 against 36.8).
 struct RowsCost {
-    float s_base, s_decode, s_meet_tile, s_meet, s_long;
-    float h_base, h_join, h_start, h_decode, h_meet, h_mb, h_long;
+    float s_base, s_decode, s_meet_tile, s_meet, s_long, s_mb;
+    float h_base, h_join, h_start, h_decode, h_meet, h_sums, h_long, h_five, h_mb;
 };
 static const RowsCost &rows_cost(int fmt) {
-    static const RowsCost q40 = {9.40f, 1.37f, 0.23f, 0.35f, -0.90f, 7.59f, 3.03f, 0.64f, 1.48f, 0.24f, 0.19f, 0.05f};
-    static const RowsCost q41 = {9.46f, 0.99f, 0.17f, 0.46f, -0.79f, 8.03f, 2.55f, 0.86f, 0.75f, 0.26f, 1.01f, 0.13f};
-    static const RowsCost q4 = {9.67f, 1.03f, 0.00f, 0.70f, -0.92f, 8.18f, 2.62f, 0.85f, 0.79f, 0.18f, 0.79f, 0.03f};
-    static const RowsCost q5 = {10.18f, 0.85f, 0.19f, 0.39f, -0.03f, 8.30f, 2.18f, 0.77f, 1.16f, 0.17f, 0.57f, 0.25f};
-    static const RowsCost q6 = {10.34f, 1.66f, -0.55f, 2.00f, -0.25f, 8.10f, 2.98f, 0.64f, 1.63f, 0.37f, 0.30f, 0.19f};
-    static const RowsCost q80 = {10.00f, 1.53f, 0.42f, 0.17f, -1.15f, 7.16f, 3.76f, 0.81f, 1.75f, 0.22f, 0.05f, -0.16f};
+    static const RowsCost q40 = {8.81f, 1.33f, 0.21f, 0.36f, -0.66f, -0.04f, 7.63f, 3.16f, 0.58f, 1.47f, 0.18f, 4.09f, -0.02f, 0.30f, -0.09f};
+    static const RowsCost q41 = {8.75f, 0.63f, 0.17f, 0.51f, -0.07f, 0.02f, 8.22f, 2.75f, 0.85f, 0.97f, 0.15f, 4.23f, -0.01f, 0.53f, -0.08f};
+    static const RowsCost q51 = {9.06f, 0.84f, 0.20f, 0.39f, -0.29f, 0.05f, 8.51f, 3.76f, 0.82f, 1.31f, 0.16f, 4.42f, -0.31f, 0.38f, -0.05f};
+    static const RowsCost q80 = {8.71f, 1.64f, 0.31f, 0.25f, -1.10f, -0.00f, 6.86f, 3.85f, 0.99f, 1.67f, 0.14f, 3.05f, -0.17f, 0.14f, -0.03f};
+    static const RowsCost q2 = {9.70f, 0.46f, 0.00f, 0.76f, -0.11f, 0.02f, 7.96f, 3.42f, 0.69f, 0.94f, 0.13f, 2.17f, -0.17f, 0.24f, -0.09f};
+    static const RowsCost q4 = {9.51f, 0.64f, -0.04f, 0.81f, -0.43f, 0.03f, 7.56f, 3.78f, 0.78f, 0.91f, 0.12f, 1.91f, -0.20f, 0.40f, -0.04f};
+    static const RowsCost q5 = {9.72f, 0.62f, 0.04f, 0.67f, 0.09f, 0.03f, 8.68f, 3.34f, 0.34f, 1.24f, 0.11f, 3.73f, -0.11f, 0.48f, -0.05f};
+    static const RowsCost q6 = {11.24f, 1.21f, -0.59f, 2.01f, -0.01f, 0.05f, 8.88f, 2.77f, 0.23f, 1.80f, 0.23f, 3.59f, 0.81f, 0.34f, -0.05f};
     switch (fmt) {
     case F_Q6_K: return q6;
     case F_Q5_K: return q5;
+    case F_Q2_K: return q2;
     case F_Q8_0: return q80;
     case F_Q4_0: return q40;
-    case F_Q4_1: case F_Q5_1: return q41;
-    default: return q4;  // (Q4_K and Q2_K)
+    case F_Q4_1: return q41;
+    case F_Q5_1: return q51;
+    default: return q4;
     }
 }
 
@@ -179,17 +190,19 @@ HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, int join, int cus, int 
     const RowsGeo st = rows_geometry(fmt, n, k, rows, (unsigned)cus);
     const float units = (float)((st.batches + cus - 1) / cus * ((ncol + GR_WAVES - 1) / GR_WAVES)), gper = (float)((groups + st.shares - 1) / st.shares),
                 tiles = (float)st.tiles;
+    const float mb = (float)n * 1e-6f * (float)(k / block_values(fmt) * block_bytes(fmt));
+    // (a reader's join has no launch: half the line's join.  432 prompts of 9 to 64 tokens through 24 models, against the streaming kernel
+    // alone: the worst is 0.997 times as fast, the mean 1.20; with all of it, three quarters or a quarter 0.1 % less)
+    const float launch = join == HELD_JOIN_READER ? 0.5f : 1.f;
     // (a pair of streaming launches is taken at twice one: the preparation they share is paid by their second round of CUs; the
-    // fitted lines err by a few per cent: a launch changes kernels for three)
-    // (a reader's join costs it extra loads, and most of what the line calls the join is the way of the slices to memory: taken as
-    // free, the 4096 x 4096 projections of a 40-token prompt went to the held kernel, 12.1 against 10.4 us)
-    float best_us = 0.97f * (float)weights * (cost.s_base + cost.s_long * k / 4096.f + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
+    // estimates err by a few per cent: a launch changes kernels for three)
+    float best_us = 0.97f * (float)weights * (cost.s_base + cost.s_long * k / 4096.f + cost.s_mb * mb + units * (cost.s_decode * tiles + cost.s_meet * gper + cost.s_meet_tile * gper * tiles));
     for (int shares = 1; shares <= groups; ++shares) {
         const int held = (groups + shares - 1) / shares;
         if (held > GH_G_MAX || (groups + held - 1) / held != shares || geo.slices * shares > cus) continue;
         const int per_slice = std::min({cus / (geo.slices * shares), steps, 4095}), walk = (steps + per_slice - 1) / per_slice;
-        const float us = cost.h_base + cost.h_long * k / 4096.f + (part ? join == HELD_JOIN_READER ? 0.75f * cost.h_join : cost.h_join : 0.f) + cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held) +
-                         cost.h_mb * 1e-6f * part * rows * n * weights;
+        const float us = cost.h_base + cost.h_long * k / 4096.f + cost.h_mb * mb * weights + (part ? cost.h_join * launch + cost.h_sums * 1e-6f * part * rows * n * weights : 0.f) +
+                         cost.h_start * held + walk * (cost.h_decode + cost.h_meet * held + (held == 5 ? cost.h_five : 0.f));
         if (us < best_us) {
             best_us = us;
             geo.per_slice = (steps + walk - 1) / walk;

@@ -1358,6 +1358,14 @@ bool rows_path(const jitnn_hip_weight *w, int rows) {
            w->n >= 16;
 }
 
+// One launch of rows_path, with a join of its own where it has slices: the plan of the kernel that holds the operands, or groups_held = 0.
+size_t rows_operand_bytes(int rows, int k) { return (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255; }
+HeldPlan rows_plan(const jitnn_hip_weight *w, int rows, bool adds, int cus) {
+    const HeldPlan p = gemv_held_plan(w->fmt, w->n, w->k, rows, adds ? HELD_JOIN_ADDS : HELD_JOIN_SLICES, cus);
+    // (the same limit for both sources of scratch, so that both entry points take the same kernels)
+    return rows_operand_bytes(rows, w->k) + p.part_bytes(rows, w->n) <= JITNN_HIP_SCRATCH_BYTES ? p : HeldPlan{};
+}
+
 // ys[i] = x ws[i]^T (+ bias) (+ residual [rows, n]; bias and residual with one weight only) for weights that all pass
 // rows_path: the activation operands are prepared once per granularity of block sums and shared by the weights.
 // swiglu_up: the activations are silu(x) * swiglu_up, formed by the preparation as it reads x.
@@ -1370,7 +1378,7 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
                       float *together = nullptr, size_t room = 0, PfGroupPending *gdefer = nullptr) {
     const int k = ws[0]->k;
     bool need[GR_LAYOUTS] = {};  // the operand layouts the weights ask for
-    const size_t one = (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255;
+    const size_t one = rows_operand_bytes(rows, k);
     int layouts = 0;
     for (int i = 0; i < count; ++i) {
         if (ws[i]->k != k) return fail(JITNN_HIP_EINVAL, "weights of %d and %d values per row on one activation", k, ws[i]->k);
@@ -1396,14 +1404,12 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
     }
     for (int i = 0; i < count && !grouped; ++i) {
         const bool put_off = defer && k <= 8 * 2048;  // (a slice is at most eight columns; more slices only where that is less than k / 2048)
-        plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, put_off ? HELD_JOIN_READER : bias || residual ? HELD_JOIN_ADDS : HELD_JOIN_SLICES, g.cus);
+        if (put_off) plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, HELD_JOIN_READER, g.cus);
         if (put_off && plan[i].slices > 1 && plan[i].slices <= 8) {
             later_plan = plan[i].slices;
             continue;
         }
-        if (put_off) plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, HELD_JOIN_ADDS, g.cus);
-        // (the same limit for both sources of scratch, so that both entry points take the same kernels)
-        if (one + plan[i].part_bytes(rows, ws[i]->n) > JITNN_HIP_SCRATCH_BYTES) plan[i] = HeldPlan{};
+        plan[i] = rows_plan(ws[i], rows, bias || residual, g.cus);
         part = std::max(part, plan[i].part_bytes(rows, ws[i]->n));
     }
     void *scratch = nullptr;
@@ -1551,6 +1557,18 @@ int jitnn_hip_many_row_tile(const int *fmts, const int *n, int count, int k, int
     }
     WidePlan plan;
     return rows > g.gemv_max_rows && wide_pays(fmts, n, count, k, rows, gate_up != 0, residual != 0, compute_units, &plan) ? 32 * plan.rt : 0;
+}
+
+int jitnn_hip_few_rows_slices(int fmt, int n, int k, int rows, int adds, int compute_units) {
+    if (rows < 1 || compute_units < 0) return fail(JITNN_HIP_EINVAL, "no such launch");
+    const long long need = jitnn_hip_weight_nbytes(fmt, n, k);
+    if (need < 0) return (int)need;
+    if (compute_units == 0) {
+        if (int rc = check_ready()) return rc;
+        compute_units = g.cus;
+    }
+    const jitnn_hip_weight w{fmt, n, k, need, nullptr, false};
+    return rows_path(&w, rows) ? rows_plan(&w, rows, adds != 0, compute_units).slices : 0;
 }
 
 long long jitnn_hip_noalloc_scratch_bytes(void) { return (long long)JITNN_HIP_SCRATCH_BYTES; }
