@@ -40,7 +40,7 @@ __host__ __device__ constexpr bool gh_pin_fetch(int fmt, int groups_held) { retu
 struct HeldGeo {
     int cols;       // columns of K per workgroup, one per wave: 1..8
     int lanes;      // tiles a workgroup works on side by side: its waves are `lanes` sets of cols (cols * lanes <= 8)
-    int slices;     // slices of K: ceil(k / 256 / cols)
+    int slices;     // slices of K: ceil(k / 256 / cols); 0: the one slice of this launch, added to y
     int per_slice;  // workgroups per slice: gridDim.x = slices * per_slice
     __host__ __device__ uint32_t packed() const { return (uint32_t)cols | (uint32_t)lanes << 4 | (uint32_t)slices << 8 | (uint32_t)per_slice << 20; }
     __host__ __device__ static HeldGeo unpacked(uint32_t v) { return {(int)(v & 15u), (int)(v >> 4 & 15u), (int)(v >> 8 & 4095u), (int)(v >> 20)}; }
@@ -96,6 +96,7 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
     }
     auto operand = [&](int g, int s) { return s < HELD ? A[g][s < HELD ? s : 0] : parked[(g * PARKED + s - HELD) * 64]; };
     float *ys = y + (size_t)slice * rows * n;
+    const bool adds_up = geo.slices == 0;
     // the sums of a step, added up in wave order and stored: (tile, group) tg by wave tg % 8
     auto join = [&](int step, int buf) {
         for (int tg = wave; tg < geo.lanes * G; tg += GR_WAVES) {
@@ -113,8 +114,13 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
             const int row = min(tile * 16, n - 16) + (lane & 15), b = (g0 + g) * 8 + 2 * kq;
             if (at < ntiles && row >= tile * 16) {  // rows of a ragged last tile that an earlier tile already wrote are skipped
                 float *to = ys + ((size_t)(second ? geo.slices : 0) * rows + b) * n + row;
-                if (b < rows) to[0] = sum.x;
-                if (b + 1 < rows) to[n] = sum.y;
+                if (adds_up) {
+                    if (b < rows) to[0] += sum.x;
+                    if (b + 1 < rows) to[n] += sum.y;
+                } else {
+                    if (b < rows) to[0] = sum.x;
+                    if (b + 1 < rows) to[n] = sum.y;
+                }
             }
         }
     };

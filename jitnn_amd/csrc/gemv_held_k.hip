@@ -4,8 +4,8 @@
 namespace jitnn {
 
 // y[b, row] = sum over the K slices of part[slice][b, row], slices in order (+ bias[row]) (+ res[b, row]); count = rows * n.
-// (y, bias and res are the caller's: no alignment beyond a float's)
-__global__ void __launch_bounds__(256) rows_join_kernel(const float *__restrict__ part, float *y, int count, int n, int slices,
+// (y, bias and res are the caller's: no alignment beyond a float's; part may be y, one slice)
+__global__ void __launch_bounds__(256) rows_join_kernel(const float *part, float *y, int count, int n, int slices,
                                                          const float *__restrict__ bias, const float *res) {
     for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < count; i += (int)gridDim.x * 256) {
         float sum = 0.f;

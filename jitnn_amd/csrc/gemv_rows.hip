@@ -217,19 +217,35 @@ HeldPlan gemv_held_plan(int fmt, int n, int k, int rows, int join, int cus, int 
     return best;
 }
 
+static void held_launch(const HeldPlan &plan, int fmt, hipStream_t s, unsigned blocks, const uint8_t *W, const uint8_t *W2, const void *scratch, int first_column,
+                        uint32_t where, float *y, int n, int k, int rows) {
+    int groups = (rows + 7) / 8;
+    const _Float16 *ops = reinterpret_cast<const _Float16 *>(scratch) + (size_t)first_column * GR_OP_HALVES;
+    const float *inv = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(scratch) + gemv_rows_ops_bytes(groups, k)) + (size_t)first_column * 8;
+    const KernelRef kr = gemv_held_kernel_ref(fmt, plan.groups_held);
+    W += (size_t)first_column * (256 / block_values(fmt)) * block_bytes(fmt);
+    void *args[] = {&W, &W2, &ops, &inv, &n, &k, &rows, &groups, &where, &y};
+    (void)hipLaunchKernel(kr.fn, dim3(blocks, (unsigned)plan.shares), dim3(GR_THREADS), args, kr.lds, s);
+}
+
 void gemv_held_slices_launch(const HeldPlan &plan, int fmt, hipStream_t s, const uint8_t *W, const uint8_t *W2, const void *scratch, float *part, int n, int k,
                              int rows) {
-    int groups = (rows + 7) / 8;
-    const _Float16 *ops = reinterpret_cast<const _Float16 *>(scratch);
-    const float *inv = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(scratch) + gemv_rows_ops_bytes(groups, k));
-    uint32_t where = plan.where;
-    const KernelRef kr = gemv_held_kernel_ref(fmt, plan.groups_held);
-    void *args[] = {&W, &W2, &ops, &inv, &n, &k, &rows, &groups, &where, &part};
-    (void)hipLaunchKernel(kr.fn, dim3((unsigned)(plan.slices * plan.per_slice), (unsigned)plan.shares), dim3(GR_THREADS), args, kr.lds, s);
+    held_launch(plan, fmt, s, (unsigned)(plan.slices * plan.per_slice), W, W2, scratch, 0, plan.where, part, n, k, rows);
 }
 
 void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
                       float *y, float *part, int n, int k, int rows) {
+    if (plan.part && !part) {  // slice after slice into y: the order, and so the bits, of the join
+        HeldGeo geo = HeldGeo::unpacked(plan.where);
+        const int cols = geo.cols;
+        for (int z = 0; z < plan.slices; ++z) {
+            geo.cols = std::min(cols, k / 256 - z * cols);
+            geo.slices = z == 0;
+            held_launch(plan, fmt, s, (unsigned)plan.per_slice, W, nullptr, scratch, z * cols, geo.packed(), y, n, k, rows);
+        }
+        rows_join_launch(s, y, y, rows, n, 1, bias, res, (unsigned)cus);
+        return;
+    }
     gemv_held_slices_launch(plan, fmt, s, W, nullptr, scratch, plan.part ? part : y, n, k, rows);
     if (plan.part) rows_join_launch(s, part, y, rows, n, plan.slices, bias, res, (unsigned)cus);
 }

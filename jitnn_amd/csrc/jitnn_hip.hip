@@ -669,8 +669,8 @@ int workspace(size_t bytes, hipStream_t stream, void **out, ScratchSource src = 
     return JITNN_HIP_OK;
 }
 
-// Would workspace() give `bytes` where a kernel with less scratch will do as well: yes, unless it cannot hold them without an
-// allocation under a stream capture, or at all.
+// Would workspace() give `bytes` where the caller can do with less: yes, unless it cannot hold them without an allocation under a
+// stream capture, or at all.
 bool workspace_at_hand(size_t bytes, hipStream_t stream, ScratchSource src) {
     if (src == SCRATCH_STATIC) return bytes <= JITNN_HIP_SCRATCH_BYTES;
     touch_thread_state();
@@ -1413,11 +1413,7 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
         part = std::max(part, plan[i].part_bytes(rows, ws[i]->n));
     }
     void *scratch = nullptr;
-    if (part && !workspace_at_hand(one * layouts + part, s, src)) {
-        for (HeldPlan &p : plan)
-            if (p.part) p = HeldPlan{};
-        part = 0;
-    }
+    if (part && !workspace_at_hand(one * layouts + part, s, src)) part = 0;  // (slice after slice into the output then: the same bits)
     if (int rc = workspace(one * layouts + part, s, &scratch, src)) return rc;
     for (int i = 0; i < count; ++i) {
         const KernelRef kr = plan[i].groups_held ? gemv_held_kernel_ref(ws[i]->fmt, plan[i].groups_held)
@@ -1446,7 +1442,7 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
             defer->splits = later_plan;
             defer->n = ws[i]->n;
         } else if (plan[i].groups_held)
-            gemv_held_launch(plan[i], ws[i]->fmt, g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], (float *)((uint8_t *)scratch + one * layouts), ws[i]->n, k, rows);
+            gemv_held_launch(plan[i], ws[i]->fmt, g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], part ? (float *)((uint8_t *)scratch + one * layouts) : nullptr, ws[i]->n, k, rows);
         else gemv_rows_main_launch(ws[i]->fmt, (unsigned)g.cus, s, ws[i]->dev, ops, bias, residual, ys[i], ws[i]->n, k, rows);
     }
     HIP_TRY(hipGetLastError());

@@ -131,7 +131,7 @@ KernelRef gemv_held_kernel_ref(int fmt, int groups_held);
 // part [slices][rows, n] = the slices of x W^T, behind them those of x W2^T
 void gemv_held_slices_launch(const HeldPlan &plan, int fmt, hipStream_t s, const uint8_t *W, const uint8_t *W2, const void *scratch, float *part, int n, int k,
                              int rows);
-// y = x W^T (+ bias [n]) (+ res [rows, n]); part: plan.part_bytes(rows, n) of scratch
+// y = x W^T (+ bias [n]) (+ res [rows, n]); part: plan.part_bytes(rows, n) of scratch, or nullptr: the same bits, a launch per slice
 void gemv_held_launch(const HeldPlan &plan, int fmt, int cus, hipStream_t s, const uint8_t *W, const void *scratch, const float *bias, const float *res,
                       float *y, float *part, int n, int k, int rows);
 void rows_join_launch(hipStream_t s, const float *part, float *y, int rows, int n, int slices, const float *bias, const float *res, unsigned cus);

@@ -126,3 +126,56 @@ def test_noalloc_linear_rejects_what_does_not_fit(jn):
     rc = lib.lib.jitnn_hip_linear_noalloc_dev(w.handle, vp(x), rows, None, vp(y), None)
     assert rc == lib.EINVAL and "scratch" in lib.last_error()
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("fmt,n,k,rows,slices,bias", [
+    ("Q4_K", 14336, 4096, 24, 2, True), ("Q6_K", 4096, 14336, 37, 7, False), ("Q6_K", 20000, 2304, 40, 2, True),
+    ("Q2_K", 6001, 4352, 33, 3, False), ("Q4_0", 9001, 2816, 25, 2, True), ("Q5_1", 12003, 5888, 40, 3, False), ("Q6_K", 7601, 14336, 5, 7, True)])
+def test_captured_linear_without_room_for_its_slices(jn, fmt, n, k, rows, slices, bias):
+    """9 to 64 rows (and 5 of long ones) in the kernel that adds up slices of a row, recorded on a thread whose scratch holds the
+    operands but not the slices: the same bits as the entry point that allocates nothing and as an eager call.  Short last slices (17
+    columns in three, 23 in three, 11 in two), ragged tiles, rows that fill no group of eight."""
+    import threading
+    from jitnn_amd import _lib as lib
+    assert lib.few_rows_slices(GGML_ID[fmt], n, k, rows, adds=bias) == slices
+    rng = np.random.default_rng(n)
+    w = jn.Tensor.quantized(jn.DType[fmt], random_valid_blocks(rng, fmt, n, k), n, k)
+    small = jn.Tensor.quantized(jn.DType[fmt], random_valid_blocks(rng, fmt, 16, k), 16, k)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x, b = torch.randn(rows, k, device="cuda", generator=g), torch.randn(n, device="cuda", generator=g) if bias else None
+    ref = run(lib, "jitnn_hip_linear_noalloc_dev", w, x, b, n)
+    assert torch.isfinite(ref).all() and torch.equal(run(lib, "jitnn_hip_linear_dev", w, x, b, n), ref)
+    failed = []
+
+    def work():
+        try:
+            side = torch.cuda.Stream()
+            y, ys = torch.empty_like(ref), torch.empty(rows, 16, device="cuda")
+
+            def call(weight, out, bias):
+                lib.check(lib.lib.jitnn_hip_linear_dev(weight.handle, vp(x), rows, vp(bias) if bias is not None else None, vp(out), C.c_void_p(side.cuda_stream)), "linear")
+
+            with torch.cuda.stream(side):
+                call(small, ys, None)  # room for the operands of these rows
+                side.synchronize()
+                held = lib.thread_scratch()[0]
+                assert 0 < held < 4 * slices * rows * n
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    call(w, y, b)
+                for i in range(3):
+                    y.fill_(float("nan"))
+                    call(small, ys, None)  # (the scratch is used in between)
+                    graph.replay()
+                    side.synchronize()
+                    assert torch.equal(y, ref), i
+                assert lib.thread_scratch() == (held, 0, 1)
+                del graph
+        except BaseException as e:  # noqa: BLE001 (handed to the test's thread)
+            failed.append(e)
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    if failed:
+        raise failed[0]
