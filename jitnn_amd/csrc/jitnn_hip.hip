@@ -2037,12 +2037,12 @@ int ensure_prefill(jitnn_hip_llama *m, int tokens) {
 }
 
 // Grows the thread's scratch once, to what the largest launch of a prompt pass over dequantised weights takes, instead of
-// step by step along the first layer (every growth waits for the device).
+// step by step along the first layer (every growth waits for the device).  Where there is no room the launches ask, each for its own.
 void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
-    if (tokens <= g.gemv_max_rows || stream_recording(st)) return;
+    if (stream_recording(st)) return;
     size_t most_weights = 0, most_operands = 0;
     WidePlan p;
-    for (int l = 0; l < m->layers; ++l) {
+    for (int l = 0; l < m->layers && tokens > g.gemv_max_rows; ++l) {
         const jitnn_hip_weight *const *w = m->w + (size_t)l * 7;
         auto want = [&](int which, int count, bool dual, bool residual) {
             if (!wide_pays(w + which, count, tokens, dual, residual, &p)) return;
@@ -2055,14 +2055,9 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
         want(JITNN_HIP_W_FFN_GATE, 2, prefill_dual_ok(w[JITNN_HIP_W_FFN_GATE], w[JITNN_HIP_W_FFN_UP]), false);
         want(JITNN_HIP_W_FFN_DOWN, 1, false, true);
     }
-    bool waited = false;  // (where there is no room the launches ask, each for its own)
-    if (most_weights) {
-        touch_thread_state();
-        g_ws.operands.ask_again();
-        g_ws.weights.ask_again();
-        (void)g_ws.operands.try_get(most_operands, false, &waited);
-        (void)g_ws.weights.try_get(most_weights, false, &waited);
-    }
+    bool waited = false;
+    touch_thread_state();
+    start_pass(g_ws.operands, g_ws.weights, most_operands, most_weights, &waited);
     if (waited) g_ws.used = false;
 }
 

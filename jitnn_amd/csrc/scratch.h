@@ -104,4 +104,14 @@ public:
     }
 };
 
+// The start of a prompt pass: sizes that were refused are asked for again by whoever needs them, and where the pass knows its largest
+// launches (0: it does not) both blocks move to their sizes at once, not step by step.
+template <class Block>
+void start_pass(Block &operands, Block &weights, size_t operand_bytes, size_t weight_bytes, bool *waited) {
+    operands.ask_again();
+    weights.ask_again();
+    if (operand_bytes) (void)operands.try_get(operand_bytes, false, waited);
+    if (weight_bytes) (void)weights.try_get(weight_bytes, false, waited);
+}
+
 }  // namespace jitnn

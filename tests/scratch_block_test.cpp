@@ -140,6 +140,28 @@ static void refused_growth_keeps_the_block() {
     CHECK(live.empty());
 }
 
+// A prompt pass asks again for what was refused, also one whose launches need nothing ahead (a prompt of few tokens).
+static void a_pass_asks_again() {
+    fresh();
+    Block operands, weights;
+    bool waited = false;
+    room = 10 * MiB;
+    CHECK(!operands.try_get(11 * MiB, false, &waited) && !weights.try_get(12 * MiB, false, &waited));
+    room = 100 * MiB;
+    const int before = asked;
+    CHECK(!operands.try_get(11 * MiB, false, &waited) && !weights.try_get(12 * MiB, false, &waited) && asked == before);
+    jitnn::start_pass(operands, weights, 0, 0, &waited);
+    CHECK(asked == before && operands.try_get(11 * MiB, false, &waited) && weights.try_get(12 * MiB, false, &waited));
+    jitnn::start_pass(operands, weights, 20 * MiB, 30 * MiB, &waited);
+    CHECK(operands.capacity() == 20 * MiB && weights.capacity() == 30 * MiB && waited);
+    room = 60 * MiB;
+    jitnn::start_pass(operands, weights, 40 * MiB, 0, &waited);  // no room: the block stays
+    CHECK(operands.capacity() == 20 * MiB && live.size() == 2);
+    operands.release_all();
+    weights.release_all();
+    CHECK(live.empty());
+}
+
 // A call that cannot do without gives up the old block where there is no room for both, but never one a graph may hold.
 static void needed_growth_gives_up_the_block() {
     fresh();
@@ -161,6 +183,7 @@ int main() {
     RUN(retired_blocks_are_bounded);
     RUN(refused_release_is_not_lost);
     RUN(refused_growth_keeps_the_block);
+    RUN(a_pass_asks_again);
     RUN(needed_growth_gives_up_the_block);
     return 0;
 }
