@@ -1403,7 +1403,9 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
         grouped = most > 1 && most <= 8 && floats <= room;
     }
     for (int i = 0; i < count && !grouped; ++i) {
-        const bool put_off = defer && k <= 8 * 2048;  // (a slice is at most eight columns; more slices only where that is less than k / 2048)
+        // (a slice is at most eight columns; more slices only where that is less than k / 2048.  The kernels that join read the residual 16
+        // bytes at a time: the caller's rows, in front of the first layer, need not be aligned to that)
+        const bool put_off = defer && k <= 8 * 2048 && ((uintptr_t)residual & 15) == 0;
         if (put_off) plan[i] = gemv_held_plan(ws[i]->fmt, ws[i]->n, k, rows, HELD_JOIN_READER, g.cus);
         if (put_off && plan[i].slices > 1 && plan[i].slices <= 8) {
             later_plan = plan[i].slices;
@@ -1941,10 +1943,10 @@ void norm_rows(const jitnn_hip_llama *m, const float *x, int rows, const float *
     } else if (pend) {
         flush_pending(*pend, rows, st);
     }
-    // (four values a load: the model's own rows are; the caller's, in front of the first layer, need not be)
+    // (four values a load: the model's own rows are aligned to that; the caller's, in front of the first layer, need not be)
     const float *in = join.part ? join.res : x;
-    if (((uintptr_t)in & 15) != 0 || m->d % 4 != 0) {
-        if (join.part) flush_pending(join, rows, st);
+    if (((uintptr_t)in & 15) != 0) {
+        flush_pending(join, rows, st);  // (slices of a many-row launch, whose preparation reads such rows 16 bytes at a time too)
         hipLaunchKernelGGL(rms_norm_rows_kernel, dim3(rows), dim3(256), 0, st, x, nw, xn, m->d, m->eps);
     } else {
         hipLaunchKernelGGL(rms_norm_rows_join_kernel, dim3(rows), dim3(NR_THREADS), 0, st, in, join.part, join.splits, join.out, nw, xn, rows, m->d, m->eps);

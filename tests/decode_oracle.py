@@ -40,7 +40,7 @@ def decode_ref(cfg, layers, out_norm, out_w, kcache, vcache, x, pos, threads: in
     return lin(out_w, oracle.rms_norm(x, out_norm, eps))
 
 
-def prefill_ref(cfg, layers, out_norm, out_w, kcache, vcache, x, pos0):
+def prefill_ref(cfg, layers, out_norm, out_w, kcache, vcache, x, pos0, rope_interleaved: bool = False):
     """The same stack on T tokens at positions pos0 .. pos0 + T - 1, layer by layer, every token exactly as decode_ref
     would treat it (token t attends positions 0 .. pos0 + t).  The linears are taken as FP64 products with the oracle's
     dequantised weights (bit-exact against the reference's fixtures) rounded to FP32 - the definition of
@@ -59,8 +59,8 @@ def prefill_ref(cfg, layers, out_norm, out_w, kcache, vcache, x, pos0):
     T = x.shape[0]
     for li, L in enumerate(layers):
         n = oracle.rms_norm(x, L["attn_norm"], eps)
-        q = oracle.rope(lin(L["attn_q"], n).reshape(T, heads, hd), theta, pos0, False, True)
-        k = oracle.rope(lin(L["attn_k"], n).reshape(T, kv, hd), theta, pos0, False, True)
+        q = oracle.rope(lin(L["attn_q"], n).reshape(T, heads, hd), theta, pos0, rope_interleaved, True)
+        k = oracle.rope(lin(L["attn_k"], n).reshape(T, kv, hd), theta, pos0, rope_interleaved, True)
         v = lin(L["attn_v"], n).reshape(T, kv, hd)
         kcache[li, pos0:pos0 + T], vcache[li, pos0:pos0 + T] = k, v
         att = np.empty((T, heads * hd), dtype=np.float32)
