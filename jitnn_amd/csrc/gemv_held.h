@@ -1,4 +1,4 @@
-// 9..64 activation rows against raw GGUF blocks with the ACTIVATION operands held in registers: the main kernel of
+// 9..64 activation rows (3..64 of rows of 12288 values and more) against raw GGUF blocks with the ACTIVATION operands held in registers: the main kernel of
 // gemv_rows.h (same operands from rows_prepare_kernel, same decoders RTile, same FP32-grade products) with the roles of what
 // stays and what streams exchanged.
 //

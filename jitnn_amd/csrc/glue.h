@@ -385,16 +385,16 @@ __global__ void __launch_bounds__(256) rope_append_rows_join_kernel(const float 
     });
 }
 
-// Causal attention of a block of consecutive tokens: the (token, query head) pairs of one key/value head - ATT_ROWS
-// rows, i.e. ATT_ROWS / group tokens - walk the keys in chunks of CH, each chunk staged once in LDS for all of them; row
+// Causal attention of a block of consecutive tokens: the (token, query head) pairs of one key/value head - 16 TR rows, TR 1 or 2,
+// i.e. 16 TR / group tokens - walk the keys in chunks of CH, each chunk staged once in LDS for all of them; row
 // r = tq * group + h sees key j when j <= pos0 + t0 + tq.  q is already rotated, every key comes from the cache.
-// Register tiles instead of one LDS read per multiply-add: a thread owns ATT_RT rows x CH/16 keys of the scores and ATT_RT rows
+// Register tiles instead of one LDS read per multiply-add: a thread owns TR rows x CH/16 keys of the scores and TR rows
 // x D/16 values of the output.  The 16 threads of a DPP row hold all keys of their rows and all of these rows'
 // output, so the running softmax (maximum, sum, rescaling of the output so far) stays inside the row of lanes: two DPP
 // reductions per chunk, the probabilities handed from the score tile to the value tile through LDS without a
 // workgroup barrier, no partial results in memory and no merge pass.
-//   grid (token blocks, kv_heads), 256 threads, attn_prefill_lds_bytes<D>() of dynamic LDS; out [T, heads, D].
-constexpr int ATT_ROWS = 32;  // 16 row groups of ATT_RT rows
+//   grid (token blocks, kv_heads), 256 threads, attn_prefill_lds_bytes<D, TR>() of dynamic LDS; out [T, heads, D].
+constexpr int ATT_ROWS = 32;  // 16 row groups of ATT_RT rows: the larger block
 constexpr int ATT_RT = ATT_ROWS / 16;
 template <int D, int TR>
 constexpr size_t attn_prefill_lds_bytes() {
@@ -722,7 +722,7 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 //     ARE its eight slots of the first operand of P V, when the values are laid out in LDS in that slot order
 //     (transposed, [d][slot]).  No probability goes through LDS;
 //   * the factor that rescales a row's output so far is handed from the lanes that know it (score layout: lane % 16 =
-//     row) to the lanes that hold the output (rows 4 (lane / 16) + i) through 64 bytes of LDS per wave;
+//     row) to the lanes that hold the output (rows 4 (lane / 16) + i) through 64 bytes of LDS per wave and tile;
 //   * keys and values of the chunk after next are requested into registers while the current one is multiplied; the LDS
 //     tiles are double-buffered, one workgroup barrier per chunk; nothing about the loads is conditional (chunks past
 //     the end repeat the last one, keys past the last visible one re-read it and are masked).

@@ -2097,7 +2097,9 @@ int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tok
         if (int rc = allow_lds((const void *)attn_prefill_h_kernel<D>, lds)) return rc;
         hipLaunchKernelGGL(attn_prefill_h_kernel<D>, grid, dim3(256), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads, m->kv, pos0, tokens, scale);
     } else {
-        // few tokens: blocks of half the rows on twice the CUs (40 tokens of 32 heads over 8: 40 blocks, 14.1 us per layer, -> 80, 11.5)
+        // few tokens: blocks of half the rows on twice the CUs (40 tokens of 32 heads over 8: 40 blocks, 14.1 us per layer, -> 80, 11.5).
+        // With more blocks than that it depends on head size and context: 160 blocks of 32 rows 3 to 25 % slower than 320 of 16, but at
+        // 128 values and 352 blocks 16.0 against 21.9 us (64 tokens of 160 heads over 16), 204 against 328 from position 900.
         if (2 * grid.x * grid.y <= (unsigned)g.cus) {
             const int qt1 = 16 / group;
             constexpr size_t lds = attn_prefill_lds_bytes<D, 1>();

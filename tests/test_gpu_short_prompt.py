@@ -59,10 +59,32 @@ def test_short_prompt_with_long_rows(jn, mix, ffn, interleaved, prompts):
         torch.cuda.synchronize()
         dec.prefill_dev(buf.data_ptr() + 4 * off, pos0, tokens, logits.data_ptr())
         torch.cuda.synchronize()
-        ref = prefill_ref(cfg, layers, out_norm, out_w, kc, vc, x, pos0, interleaved)
-        errs = [norm_err(logits.cpu().numpy(), ref)]
-        for li in range(2):
-            k, v = dec.kv_read(li, pos0, tokens)
-            errs += [norm_err(k, kc[li, pos0:pos0 + tokens]), norm_err(v, vc[li, pos0:pos0 + tokens])]
-        assert max(errs) <= 2e-5, (tokens, pos0, errs)
+        check(dec, cfg, layers, out_norm, out_w, kc, vc, x, pos0, logits.cpu().numpy(), interleaved)
+    dec.close()
+
+
+def check(dec, cfg, layers, out_norm, out_w, kc, vc, x, pos0, logits, interleaved=False):
+    ref = prefill_ref(cfg, layers, out_norm, out_w, kc, vc, x, pos0, interleaved)
+    errs = [norm_err(logits, ref)]
+    for li in range(2):
+        k, v = dec.kv_read(li, pos0, len(x))
+        errs += [norm_err(k, kc[li, pos0:pos0 + len(x)]), norm_err(v, vc[li, pos0:pos0 + len(x)])]
+    assert max(errs) <= 2e-5, (len(x), pos0, errs)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,tokens,o_slices", [(128, 8, 64, 64, 4), (128, 8, 128, 40, 8), (80, 5, 64, 64, 3)])
+def test_short_prompt_with_many_heads(jn, heads, kv_heads, head_dim, tokens, o_slices):
+    """More than half as many blocks of 32 query rows as compute units: the attention of short prompts in such blocks, where a prompt on fewer heads
+    takes blocks of 16; and attn_o in up to eight slices, the most the norm adds up.  Groups of sixteen, keys in front of the prompt."""
+    cfg = dict(layers=2, d_model=512, heads=heads, kv_heads=kv_heads, head_dim=head_dim, ffn=512, vocab=200, max_ctx=75, rms_eps=1e-5, rope_theta=1e4)
+    assert 2 * -(-tokens // (32 // (heads // kv_heads))) * kv_heads > jn.device_info()["compute_units"]
+    assert slices(cfg, Q6_K, tokens)[3] == o_slices
+    dec, layers, out_norm, out_w = build(jn, cfg, 17, Q6_K, "Q6_K")
+    rng = np.random.default_rng(heads)
+    kc, vc = (np.zeros((2, 75, kv_heads, head_dim), dtype=np.float32) for _ in range(2))
+    kc[:, :11], vc[:, :11] = rng.standard_normal((2, 2, 11, kv_heads, head_dim))
+    for li in range(2):
+        dec.kv_write(li, 0, kc[li, :11], vc[li, :11])
+    x = rng.standard_normal((tokens, 512)).astype(np.float32)
+    check(dec, cfg, layers, out_norm, out_w, kc, vc, x, 11, dec.prefill(x, 11))
     dec.close()
