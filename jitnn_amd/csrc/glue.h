@@ -712,7 +712,7 @@ __global__ void __launch_bounds__(256) attn_prefill_h_kernel(const float *__rest
 // workgroup repeats per chunk for all its rows - staging and conversion of 64 keys and values, a barrier - and the dependent
 // chain of a wave (operand reads, products, softmax, products).  RT = 2 spreads both over twice the rows: every operand read
 // from LDS feeds two products, and a wave has two chains.  Kernel trace, 32 heads over 8 of 128 values, us per layer with
-// RT = 1 / 2: 1024 tokens 53 / 41, 1536 101 / 61, 2048 158 / 97, 4096 499 / 336.
+// RT = 1 / 2: 1024 tokens 56 / 43, 1536 99 / 64, 2048 160 / 96, 4096 522 / 318.
 //   * scores, transposed: S^T = K Q^T, so that a lane ends up with the scores of ONE query row (column lane % 16 of the
 //     result) against the keys 4 (lane / 16) + i of every 16-key tile - the running softmax of a row needs its chunk
 //     maximum from the three other lanes that hold the row's other keys (two shuffles), the row sum stays a per-lane
@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(AM_THREADS, D == 64 && RT == 2 ? 4 : 1) attn_p
             }
             mc = fmaxf(mc, __shfl_xor(mc, 16));
             mc = fmaxf(mc, __shfl_xor(mc, 32));
-            // (Rescaling only once the maximum has grown by 2^8 takes 336 to 310 us at 4096 tokens, but the largest weight of a row is
+            // (Rescaling only once the maximum has grown by 2^8 is 6 % faster at 4096 tokens, but the largest weight of a row is
             // then no longer exactly 1 in FP16: 2 to 7 % more error against FP64.  Only where it has grown at all: the same bits, and
             // the branch costs more than it saves, 2 to 4 % at one tile per wave.)
             const float mn = fmaxf(mrun[u], mc);  // (-inf while this half has not met a visible key of the row yet)

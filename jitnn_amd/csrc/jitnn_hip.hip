@@ -1452,7 +1452,7 @@ int launch_rows_group(const jitnn_hip_weight *const *ws, float *const *ys, int c
 }
 
 // y = res + (silu(x wg^T) * (x wu^T)) wd^T, for weights that all pass rows_path, where gate and up (one format and shape) pay as one
-// launch of the held kernel: 45 us for the two of an 8B layer at 40 tokens, whose slices used to be joined by launches of their
+// launch of the held kernel: 37 us for the two of an 8B layer at 40 tokens, whose slices used to be joined by launches of their
 // own, 4.2 us each, and now meet in the preparation of the down projection's operands.  later, defer: as for launch_rows_group.
 struct RowsFfn {
     HeldPlan pair, down;
