@@ -139,12 +139,25 @@ __device__ __forceinline__ float4 dequant4(const uint8_t *w, size_t i) {
     return make_float4(o[0], o[1], o[2], o[3]);
 }
 
+// Quad f of y.  STREAM: past the caches' replacement (nontemporal), for outputs beyond DQ_STREAM_BYTES, which the 32 MiB of L2s do not
+// hold for their reader anyway.  Stored plainly they stay in the 256 MiB Infinity Cache as dirty lines that the next weight's
+// stores wait for: three outputs in turn, Q4_K 14336 x 4096 70 -> 42 us, Q6_K 4096 x 14336 57 -> 45, Q8_0 9472 x 6144 56 -> 46; with
+// the quantiser's own streaming below, both kernels 123 -> 97, 108 -> 101 and 106 -> 101 us.  A reader with plain loads
+// finds less of it cached: a torch.sum behind it is as much slower on the last two (118 -> 120 us for both), and more where most of the output
+// would have been cached (109 -> 132 us on the first).
+constexpr size_t DQ_STREAM_BYTES = (size_t)32 << 20;
+template <bool STREAM>
+__device__ __forceinline__ void dequant_store(float *__restrict__ y, size_t f, float4 v) {
+    if constexpr (STREAM) __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(y) + f);
+    else reinterpret_cast<float4 *>(y)[f] = v;
+}
+
 // Q6_K: a lane's four values need bytes from four fields of the block, and four narrow load instructions per wave and
 // 1 KiB of output keep the CU's one address unit busier than the memory behind it.  A wave takes a whole block - 64
 // quads - instead: thirteen lanes fetch its 208 bytes as 16-byte pieces and a fourteenth its last 16 bytes for the two of d
 // (one load instruction, nothing read past the block), the pieces are parted through the wave's own LDS region, and every lane
 // decodes its quad from there with the same expressions.
-template <int FMT>
+template <int FMT, bool STREAM>
 __global__ void __launch_bounds__(256) dequant_kernel(const uint8_t *__restrict__ w, float *__restrict__ y, size_t quads) {
     if constexpr (FMT == F_Q6_K) {
         __shared__ __align__(16) uint8_t stage[4][224];
@@ -160,14 +173,14 @@ __global__ void __launch_bounds__(256) dequant_kernel(const uint8_t *__restrict_
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // (the lanes of a wave run in step, LDS serves them in order)
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            reinterpret_cast<float4 *>(y)[blk * 64 + lane] = dequant4<FMT>(stage[wave], (size_t)lane * 4);
+            dequant_store<STREAM>(y, blk * 64 + lane, dequant4<FMT>(stage[wave], (size_t)lane * 4));
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     } else {
         for (size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x; f < quads; f += (size_t)gridDim.x * blockDim.x) {
-            reinterpret_cast<float4 *>(y)[f] = dequant4<FMT>(w, f * 4);
+            dequant_store<STREAM>(y, f, dequant4<FMT>(w, f * 4));
         }
     }
 }
@@ -297,7 +310,8 @@ __device__ __forceinline__ void quantize_q8_0_block(const float *__restrict__ xb
 // away from zero.  So: a candidate from one FP32 multiplication (off by one at most), set right by the signs of
 // fma(r + 1/2, d, -|x|) and fma(r - 1/2, d, -|x|) - an FMA rounds the exact value once, its sign is the exact sign.
 // Blocks with a value that is not finite or beyond 2^100, or a maximum below 2^-100 (d near or in the subnormals), take
-// the reference's expression itself.  grid: any; 256 threads.
+// the reference's expression itself.  Input and output pass once: nontemporal, so that they leave the Infinity Cache to others (with the
+// dequantiser's output as input, dequant_store).  grid: any; 256 threads.
 constexpr int Q8Q_NI = 4, Q8Q_BLOCKS = 8 * Q8Q_NI;  // 16-byte loads per lane and blocks per wave and turn
 static __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restrict__ x, uint8_t *__restrict__ q, size_t blocks) {
     constexpr int NI = Q8Q_NI, NB = Q8Q_BLOCKS;
@@ -315,8 +329,10 @@ static __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *
         float4 v[NI];
         bool odd = false;  // a value outside the range the short form is proven for
 #pragma unroll
-        for (int i = 0; i < NI; ++i)  // block 8 i + sub of the wave's, values 4 part .. 4 part + 3; all requests before the first use,
-            v[i] = *reinterpret_cast<const float4 *>(xw + (8 * i + sub < nb ? 256 * i + 4 * lane : 4 * part));  // none conditional
+        for (int i = 0; i < NI; ++i) {  // block 8 i + sub of the wave's, values 4 part .. 4 part + 3; all requests before the first use, none conditional
+            const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(xw + (8 * i + sub < nb ? 256 * i + 4 * lane : 4 * part)));
+            v[i] = make_float4(a.x, a.y, a.z, a.w);
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             if (8 * i + sub >= nb) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -365,7 +381,7 @@ static __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *
         wave_sync();
         uint8_t *qw = q + w0 * 34;  // a multiple of NB blocks: 4-byte aligned whenever q is
         if (nb == NB && (reinterpret_cast<uintptr_t>(qw) & 3) == 0) {
-            for (int j = lane; j < NB * 34 / 4; j += 64) reinterpret_cast<uint32_t *>(qw)[j] = reinterpret_cast<const uint32_t *>(out_s[wave])[j];
+            for (int j = lane; j < NB * 34 / 4; j += 64) __builtin_nontemporal_store(reinterpret_cast<const uint32_t *>(out_s[wave])[j], reinterpret_cast<uint32_t *>(qw) + j);
         } else {
             for (int j = lane; j < nb * 34; j += 64) qw[j] = out_s[wave][j];
         }

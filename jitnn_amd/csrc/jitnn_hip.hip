@@ -1096,7 +1096,8 @@ void launch_dequant(const jitnn_hip_weight *w, float *y, hipStream_t stream) {
     size_t blocks = (quads + 255) / 256;
     const size_t cap = (size_t)g.cus * 16;
     if (blocks > cap) blocks = cap;
-    hipLaunchKernelGGL(dequant_kernel<FMT>, dim3((unsigned)blocks), dim3(256), 0, stream, w->dev, y, quads);
+    if (quads * sizeof(float4) > DQ_STREAM_BYTES) hipLaunchKernelGGL((dequant_kernel<FMT, true>), dim3((unsigned)blocks), dim3(256), 0, stream, w->dev, y, quads);
+    else hipLaunchKernelGGL((dequant_kernel<FMT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, w->dev, y, quads);
 }
 
 int check_weight_args(int fmt, long long nbytes, int n, int k, const void *blocks, jitnn_hip_weight **out) {
