@@ -9,10 +9,10 @@
 //   2. prefill_mfma_kernel: a workgroup of four waves owns a 128 (weight rows) x 256 (tokens) output tile and
 //      walks K in steps of 64.  Per step every thread dequantises 32 weights of one row from the raw blocks into a
 //      double-buffered LDS tile as FP16, and each wave issues 32 v_mfma_f32_32x32x16_f16 on its 128 x 64 slice
-//      (weight operands from LDS, each used twice; activation operands from registers loaded two steps ahead, each
-//      used four times - the shape that keeps both LDS and the vector L1 at half their bandwidth), accumulating in
-//      FP32; the raw weight bytes are requested two steps ahead and decoded after the MFMAs are issued.  The epilogue
-//      undoes the row scale and adds the bias.
+//      (weight operands from LDS, each used twice; activation operands from registers loaded one and a half steps ahead,
+//      each used four times - the shape that keeps both LDS and the vector L1 at half their bandwidth), accumulating in
+//      FP32; the raw weight bytes are requested one and a half to two steps ahead and decoded between the MFMAs of the step before
+//      theirs.  The epilogue undoes the row scale and adds the bias.
 // Both FP16 roundings are relative 2^-11, so the result stays well inside the 2e-3 bar of the MFMA path.
 #pragma once
 #include "common.h"
@@ -570,19 +570,24 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    // Software pipeline over K: the B operands of a step are requested two steps ahead (a step of 32 MFMAs per wave
-    // is shorter than a trip to memory), and so are the raw weight bytes of the 32-value formats (raw[] alternates);
-    // the 256-value formats request the blocks of the next four steps during the first of four, park them in
-    // registers (stg) and hand them to LDS during the third.  The weights of step s+1 are decoded into registers
-    // (ah) after the MFMAs of step s have been issued.  The B operands rotate through three sets, the FP16 tile
-    // through two, the staged blocks have a period of four steps: the loop is unrolled six steps (twelve for the
-    // staged formats) so that all of them are fixed registers and addresses.
+    // Software pipeline over K, one barrier per step of 64 values, in the last quarter of its MFMAs: it says that the tile of
+    // step s + 1 has been written and that of step s read.  The weights of step s + 1 are decoded and written under the first
+    // three quarters; the first operands of step s + 1 are read under the last: no MFMA waits for the write, the barrier and
+    // the read of its operands in a row, as it did with the barrier between two steps - with one wave per SIMD nobody else
+    // fills that time.  Kernel alone, us, barrier between the steps -> in the last quarter: Q6_K 14336 x 4096 at 512 rows 81 -> 75.5,
+    // Q4_K 70 -> 68 (there the chip's clock gives way under the matrix cores: four workgroups take 0.56 us a step, 224 take 0.9);
+    // four workgroups (512 rows of the weight) Q6_K 67 -> 56, Q4_K 48 -> 45.  The B operands of a half step are requested one and a half steps ahead, into the registers of the half step
+    // that has just been multiplied, and the raw weight bytes of Q4_K and the 32-value formats when their registers
+    // have been decoded, as far ahead (raw[] alternates); the staged formats request the blocks of the next four steps during the first of four, park them in registers
+    // (stg) and hand them to LDS during the third.  The loop is unrolled two steps (four for the staged formats), so that all
+    // of them are fixed registers and addresses.
     // Nothing in a step is conditional - requests past the last step repeat the last step, a half step past the end
     // of a row (K = 32 mod 64) re-reads the row's last block and meets the zeros the operand array holds there - so
     // that the compiler can count the outstanding loads exactly and a step waits only for the loads it consumes.
     f16x8 ah[4];
     PfRaw<FMT> raw[2];
-    f16x8 bq[3][2][4];
+    f16x8 bq[2][2][2][2];  // [step % 2][half][16 values of K][token block]
+    f16x8 a[2][RT];        // the weight operands of a quarter of a step's MFMAs
     // this workgroup's K steps: all of them, or slice `slice` of split_steps steps when the launch splits K (then y
     // is the slice's own [m, n] array of partial sums, to be added up by prefill_join_kernel; a slice of a staged
     // format starts on a multiple of four steps)
@@ -590,12 +595,12 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
     y += (size_t)slice * m * n;
     auto wk = [&](int s) { return min(min(s, nsteps - 1) * PF_BK + 32 * dhalf, k - 32); };  // first value this thread decodes in step s
     auto fetch_w = [&](PfRaw<FMT> &r, int s) { pf_load<FMT>(r, wrow, wk(s)); };
-    auto fetch_b = [&](f16x8(&b)[2][4], int s) {
+    auto fetch_b = [&](int set, int s, int h) {  // half h (32 values) of step s; set = s % 2
         const f16x8 *p = xb + (size_t)min(s, nsteps - 1) * 4 * 64;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) b[j][ks] = p[((size_t)j * ksteps + ks) * 64];
+            for (int ks = 0; ks < 2; ++ks) bq[set][h][ks][j] = p[((size_t)j * ksteps + 2 * h + ks) * 64];
     };
     auto decode = [&](const PfRaw<FMT> &r, int kk) {  // raw -> FP16 registers, values of each group of four in the order 0, 2, 1, 3
         if constexpr (FMT == F_Q4_K || FMT == F_Q5_K || FMT == F_Q6_K) {
@@ -642,83 +647,110 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
             }
         }
     };
-    // one K step: publish the decoded weights, request the loads of step s+2, multiply, decode step s+1.  ph = s % 4.
-    auto step = [&](int s, int ph, int buf, f16x8(&bcur)[2][4], f16x8(&bfar)[2][4], PfRaw<FMT> &rfar, const PfRaw<FMT> &rnext) {
-        {
-            f16x8 *da = reinterpret_cast<f16x8 *>(&As[buf][drow * PF_LD + 32 * dhalf]);
+    auto store_tile = [&](int buf) {
+        f16x8 *da = reinterpret_cast<f16x8 *>(&As[buf][drow * PF_LD + 32 * dhalf]);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) da[c] = ah[c];
-        }
-        __syncthreads();  // the one barrier of the step: the other buffer was read before the previous one
-        PfRaw<FMT> rl;
+        for (int c = 0; c < 4; ++c) da[c] = ah[c];
+    };
+    auto meet = [&] {  // this wave's LDS accesses are done, and everybody's (loads from memory stay under way: lgkmcnt(0) only)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // quarter u of a step: 16 values of K.  Lane l supplies row l % 32 of a block, values 8 (l / 32) .. + 7 of the 16.
+    auto read_a = [&](int buf, int u) {
+        const _Float16 *ap = &As[buf][(lane & 31) * PF_LD + 8 * (lane >> 5)];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) a[u & 1][i] = *reinterpret_cast<const f16x8 *>(ap + 32 * rblock(i) * PF_LD + 16 * u);
+    };
+    auto mul = [&](int set, int u) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bq[set][u >> 1][u & 1][j], a[u & 1][i], acc[i][j], 0, 0, 0);
+    };
+    // staged formats: the fields of step s's weights, read from LDS under the last quarter of step s - 2
+    auto load_fields = [&](PfRaw<FMT> &r, int s, int ph) {
+        if constexpr (STAGED) pf_load_lds<FMT>(r, Rs + ((s >> 2) & 1) * RBUF + drow * Stage::RP, 64 * (ph & 3) + 32 * dhalf);
+    };
+    // one K step.  ph = s % 4 (staged formats), p = s % 2: constants where it is called.
+    auto step = [&](int s, int ph, int p) {
+        constexpr int G = RT * 2;  // MFMAs of a quarter
+        fetch_b(p ^ 1, s + 1, 1);
         if constexpr (STAGED) {
-            // the staged buffer of steps 4 S .. 4 S + 3 is number S % 2: written during step 4 S - 2, read (for the
-            // decode of the step after) during steps 4 S - 1 .. 4 S + 2, every pair a barrier apart
+            // the staged buffer of steps 4 S .. 4 S + 3 is number S % 2: written during step 4 S - 2 and read from the last quarter of
+            // that step, behind its barrier, to the last quarter of step 4 S + 1
             if (ph == 0) stage_fetch((s >> 2) + 1);
             if (ph == 2) stage_store(((s >> 2) + 1) & 1);
-            pf_load_lds<FMT>(rl, Rs + (((s + 1) >> 2) & 1) * RBUF + drow * Stage::RP, 64 * ((ph + 1) & 3) + 32 * dhalf);
+            decode(raw[p ^ 1], 64 * ((ph + 1) & 3) + 32 * dhalf);
         } else {
-            fetch_w(rfar, s + 2);
+            decode(raw[p ^ 1], wk(s + 1));
+            fetch_w(raw[p ^ 1], s + 3);
         }
-        fetch_b(bfar, s + 2);
-        // ---- 4 k-substeps of 16: lane l supplies row l%32, halves 8*(l/32) .. +8 of the substep.  The weight operands
-        // of a substep are read from LDS while the MFMAs of the one before run (one wave per SIMD: nobody else hides
-        // the LDS latency).
-        const _Float16 *ap = &As[buf][(lane & 31) * PF_LD + 8 * (lane >> 5)];
-        f16x8 a[2][RT];
 #pragma unroll
-        for (int i = 0; i < RT; ++i) a[0][i] = *reinterpret_cast<const f16x8 *>(ap + 32 * rblock(i) * PF_LD);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if (ks < 3) {
-#pragma unroll
-                for (int i = 0; i < RT; ++i) a[(ks + 1) & 1][i] = *reinterpret_cast<const f16x8 *>(ap + 32 * rblock(i) * PF_LD + 16 * (ks + 1));
-            }
-#pragma unroll
-            for (int i = 0; i < RT; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bcur[j][ks], a[ks & 1][i], acc[i][j], 0, 0, 0);
+        for (int u = 0; u < 3; ++u) {
+            read_a(p, u + 1);
+            mul(p, u);
         }
-        if constexpr (STAGED) decode(rl, 64 * ((ph + 1) & 3) + 32 * dhalf);
-        else decode(rnext, wk(s + 1));
-        // One wave per SIMD: nobody else fills the matrix pipe while this wave decodes, or the VALU while it multiplies.
-        // Ask the scheduler for the interleaving by hand: 32 times one MFMA and a few decode instructions, every other
-        // time also one LDS operand read and one of the step's global loads.  The loads are spread over the step on
-        // purpose: issued in one burst after the barrier, the four waves' requests queue up at the CU's one
-        // address unit and the waves stall at the issue while the matrix pipe idles.
-        __builtin_amdgcn_sched_group_barrier(0x100, RT + Stage::NRAW, 0);
+        store_tile(p ^ 1);
+        // One wave per SIMD: nobody else fills the matrix pipe while this wave decodes, or the VALU while it multiplies.  Ask the
+        // scheduler for the interleaving by hand: an MFMA and a few decode instructions, the operand reads of the next
+        // quarter first, then the step's requests, spread out: issued in one burst, the four waves' requests queue up at the
+        // CU's one address unit and the waves stall at the issue while the matrix pipe idles.
 #pragma unroll
-        for (int i = 0; i < 8 * RT; ++i) {
+        for (int i = 0; i < 3 * G; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, RT == 4 ? 4 : 8, 0);  // (the decode of a step is as long whatever RT is)
-            if (i % 2 == 0 && i < 6 * RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            if (RT == 2 || i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            if (i % G < RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, RT == 4 ? 5 : 10, 0);  // (the decode of a step is as long whatever RT is)
+            if (i % G >= RT || i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            if (i >= 3 * G - 4) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        meet();
+        __builtin_amdgcn_sched_barrier(0);
+        read_a(p ^ 1, 0);
+        load_fields(raw[p], s + 2, ph + 2);
+        fetch_b(p, s + 2, 0);
+        mul(p, 3);
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, RT == 4 ? 1 : 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
+    // step sbeg's tile, and what the first step expects under way.  (sbeg is a multiple of four where the format is staged)
+    fetch_b(0, sbeg, 0);
+    fetch_b(0, sbeg, 1);
     if constexpr (STAGED) {
         stage_fetch(sbeg >> 2);
         stage_store((sbeg >> 2) & 1);
-        __syncthreads();
-        pf_load_lds<FMT>(raw[0], Rs + ((sbeg >> 2) & 1) * RBUF + drow * Stage::RP, 32 * dhalf);
-        fetch_b(bq[0], sbeg);
-        fetch_b(bq[1], sbeg + 1);
+        meet();
+        load_fields(raw[0], sbeg, 0);
+        load_fields(raw[1], sbeg + 1, 1);
         decode(raw[0], 32 * dhalf);
     } else {
         fetch_w(raw[0], sbeg);
-        fetch_b(bq[0], sbeg);
         fetch_w(raw[1], sbeg + 1);
-        fetch_b(bq[1], sbeg + 1);
         decode(raw[0], wk(sbeg));
+        fetch_w(raw[0], sbeg + 2);
     }
-    constexpr int UNR = STAGED ? 12 : 6;  // lcm of the rotation periods: 3 operand sets, 2 tiles (and raw sets), 4 steps per staged block
+    fetch_b(1, sbeg + 1, 0);
+    store_tile(0);
+    meet();
+    read_a(0, 0);
+    constexpr int UNR = STAGED ? 4 : 2;
     int s0 = sbeg;
     for (; s0 + UNR <= nsteps; s0 += UNR) {
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) step(s0 + u, u & 3, u & 1, bq[u % 3], bq[(u + 2) % 3], raw[u & 1], raw[(u + 1) & 1]);
+        for (int u = 0; u < UNR; ++u) step(s0 + u, u, u & 1);
     }
 #pragma unroll
     for (int u = 0; u < UNR - 1; ++u)
-        if (s0 + u < nsteps) step(s0 + u, u & 3, u & 1, bq[u % 3], bq[(u + 2) % 3], raw[u & 1], raw[(u + 1) & 1]);
+        if (s0 + u < nsteps) step(s0 + u, u, u & 1);
     // ---- epilogue.  The activations went in as the first MFMA operand, so an accumulator holds a 32 (tokens) x 32
     // (weight rows) block of y: element r is token 8*(r/4) + 4*(lane/32) + r%4, weight row lane%32 - the 32 lanes of a
     // half wave store 32 consecutive floats of one token's output row.  The 32 token scales of the lane are read

@@ -1,0 +1,45 @@
+"""Linears of more than 64 rows at the edges of the kernel that decodes as it goes (prefill.h): one to five steps of K, half a step at the
+end of a row, one row past a tile of rows or tokens, both wave layouts (up to 128 rows and beyond) - against FP64 on the oracle's dequantised weights.
+
+Tolerance: weights and activations are rounded to FP16 once each, and the K-quants' scale products once more: at most 3 x 2^-11 of
+each product, 1.5e-3 of the sum of their magnitudes, which bounds every output."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import GGML_ID, random_valid_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def linear(fmt, n, k, rows, bias, seed=0):
+    import jitnn_amd
+    from jitnn_amd import _lib as lib
+    from oracle import oracle
+    jitnn_amd.init()
+    rng = np.random.default_rng([seed, n, k, rows])
+    raw = random_valid_blocks(rng, fmt, n, k)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32) if bias else None
+    w = jitnn_amd.Tensor.quantized(jitnn_amd.DType[fmt], raw, n, k)
+    xd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda() if bias else None
+    out = []
+    for name in ("jitnn_hip_linear_dev", "jitnn_hip_linear_noalloc_dev"):
+        y = torch.full((rows * n + 4,), float("nan"), device="cuda")
+        lib.check(getattr(lib.lib, name)(w.handle, xd.data_ptr(), rows, bd.data_ptr() if bias else None, y.data_ptr(), None), name)
+        torch.cuda.synchronize()
+        assert torch.isnan(y[rows * n:]).all()
+        out.append(y[:rows * n].reshape(rows, n).cpu().numpy())
+    wd = oracle.dequantize(GGML_ID[fmt], raw, n * k).reshape(n, k).astype(np.float64)
+    x64 = x.astype(np.float64)
+    ref = x64 @ wd.T + (b.astype(np.float64) if bias else 0.0)
+    bound = 1.5e-3 * (np.abs(x64) @ np.abs(wd).T) + 1e-6 * np.abs(ref).max()
+    assert (np.abs(out[0] - ref) <= bound).all()
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("rows", [65, 129, 257])
+@pytest.mark.parametrize("fmt,k", [("Q4_0", 32), ("Q4_0", 96), ("Q4_1", 64), ("Q4_1", 160), ("Q8_0", 128), ("Q8_0", 224), ("Q8_0", 320), ("Q5_1", 96),
+                                   ("Q4_K", 256), ("Q5_K", 256), ("Q5_K", 512), ("Q6_K", 256), ("Q6_K", 768)])
+def test_short_rows_of_k(fmt, k, rows):
+    linear(fmt, 132, k, rows, False)
