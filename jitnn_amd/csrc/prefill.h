@@ -371,7 +371,7 @@ __device__ __forceinline__ void pf_decode(const PfRaw<FMT> &r, int k0, float (&o
     }
 }
 
-// Half-precision decoders for the two formats of a Q4_K_M model: the quants become exact FP16 integers without a
+// Half-precision decoders.  The K-quants of a Q4_K_M or Q5_K_M model: the quants become exact FP16 integers without a
 // conversion instruction (a byte OR-ed under the exponent 0x6400 is 1024 + byte; the 1024, and Q6_K's 32, come off
 // with one exact packed add), and the block scale is applied with packed FP16 arithmetic, two weights per
 // instruction.  Pairs come out as (byte 0, byte 2), (byte 1, byte 3) of each dword of quants: the 0, 2, 1, 3 order
@@ -482,6 +482,70 @@ __device__ __forceinline__ void pf_decode_h<F_Q6_K>(const PfRaw<F_Q6_K> &r, int 
         o[c] = __builtin_bit_cast(f16x8, out);
     }
 }
+
+// The 32-value formats: d times a quant, and for Q4_1 and Q5_1 the offset with it, in one FP16 rounding - the value that the FP32
+// decoder above rounds to FP16 (a quant of at most eight bits times an FP16 scale is exact in FP32; with an offset that one rounds twice).
+// q + 1024 leaves the 1024 in one exact packed add; a high nibble, 1024 + 16 q where it stands, in one exact packed FMA.
+template <>
+__device__ __forceinline__ void pf_decode_h<F_Q4_0>(const PfRaw<F_Q4_0> &r, int, f16x8 (&o)[4]) {
+    const uint32_t mg = pf_magic(), dd = (r.d & 0xffffu) * 0x00010001u;
+    const f16x2 d2 = pf_pair(dd), lo = {(_Float16)-1032.f, (_Float16)-1032.f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, hi = {(_Float16)-72.f, (_Float16)-72.f};
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        u32x4 a, b;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t w = r.q[2 * c + t], s = w >> 8;
+            a[2 * t] = pf_bits((pf_pair((w & 0x000f000fu) | mg) + lo) * d2);      // low nibbles of bytes 0, 2
+            a[2 * t + 1] = pf_bits((pf_pair((s & 0x000f000fu) | mg) + lo) * d2);  // of bytes 1, 3
+            b[2 * t] = pf_bits(__builtin_elementwise_fma(pf_pair((w & 0x00f000f0u) | mg), sixteenth, hi) * d2);
+            b[2 * t + 1] = pf_bits(__builtin_elementwise_fma(pf_pair((s & 0x00f000f0u) | mg), sixteenth, hi) * d2);
+        }
+        o[c] = __builtin_bit_cast(f16x8, a);
+        o[2 + c] = __builtin_bit_cast(f16x8, b);
+    }
+}
+
+template <>
+__device__ __forceinline__ void pf_decode_h<F_Q4_1>(const PfRaw<F_Q4_1> &r, int, f16x8 (&o)[4]) {
+    const uint32_t mg = pf_magic(), dd = (r.dm & 0xffffu) * 0x00010001u, mm = (r.dm >> 16) * 0x00010001u;
+    const f16x2 d2 = pf_pair(dd), m2 = pf_pair(mm), lo = {(_Float16)-1024.f, (_Float16)-1024.f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, hi = {(_Float16)-64.f, (_Float16)-64.f};
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        u32x4 a, b;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t w = r.q[2 * c + t], s = w >> 8;
+            a[2 * t] = pf_bits(__builtin_elementwise_fma(pf_pair((w & 0x000f000fu) | mg) + lo, d2, m2));
+            a[2 * t + 1] = pf_bits(__builtin_elementwise_fma(pf_pair((s & 0x000f000fu) | mg) + lo, d2, m2));
+            b[2 * t] = pf_bits(__builtin_elementwise_fma(__builtin_elementwise_fma(pf_pair((w & 0x00f000f0u) | mg), sixteenth, hi), d2, m2));
+            b[2 * t + 1] = pf_bits(__builtin_elementwise_fma(__builtin_elementwise_fma(pf_pair((s & 0x00f000f0u) | mg), sixteenth, hi), d2, m2));
+        }
+        o[c] = __builtin_bit_cast(f16x8, a);
+        o[2 + c] = __builtin_bit_cast(f16x8, b);
+    }
+}
+
+template <>
+__device__ __forceinline__ void pf_decode_h<F_Q8_0>(const PfRaw<F_Q8_0> &r, int, f16x8 (&o)[4]) {
+    const uint32_t mg = pf_magic(), dd = (r.d & 0xffffu) * 0x00010001u;
+    const f16x2 d2 = pf_pair(dd), off = {(_Float16)-1152.f, (_Float16)-1152.f};  // -1024, and -128 of the sign flip
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        u32x4 a;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int e = 2 * c + t;
+            const uint32_t w = (e < 4 ? r.q0[e] : r.q1[e - 4]) ^ 0x80808080u;
+            a[2 * t] = pf_bits((pf_pair((w & 0x00ff00ffu) | mg) + off) * d2);
+            a[2 * t + 1] = pf_bits((pf_pair(((w >> 8) & 0x00ff00ffu) | mg) + off) * d2);
+        }
+        o[c] = __builtin_bit_cast(f16x8, a);
+    }
+}
+
+// whether a format has a packed decoder; the others go through FP32
+__host__ __device__ constexpr bool pf_packed(int fmt) { return fmt != F_Q5_1 && fmt != F_Q2_K; }
 
 // The 256-value formats reach LDS in two hops.  A thread's 32 weights of a step are a few 16-byte fields scattered
 // over its row's block, so fetching them straight from global memory makes every load instruction of a wave touch
@@ -603,7 +667,7 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
             for (int ks = 0; ks < 2; ++ks) bq[set][h][ks][j] = p[((size_t)j * ksteps + 2 * h + ks) * 64];
     };
     auto decode = [&](const PfRaw<FMT> &r, int kk) {  // raw -> FP16 registers, values of each group of four in the order 0, 2, 1, 3
-        if constexpr (FMT == F_Q4_K || FMT == F_Q5_K || FMT == F_Q6_K) {
+        if constexpr (pf_packed(FMT)) {
             pf_decode_h<FMT>(r, kk, ah);
         } else {
             float v[32];
@@ -678,6 +742,9 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
     // one K step.  ph = s % 4 (staged formats), p = s % 2: constants where it is called.
     auto step = [&](int s, int ph, int p) {
         constexpr int G = RT * 2;  // MFMAs of a quarter
+        // decode instructions behind each of 24 MFMAs.  Measured 1 to 5: level for most formats, 5 best where a decode is long; Q4_1,
+        // with the shortest, 2 (11008 x 4096 at 512 rows 61 against 67 us)
+        constexpr int DV = FMT == F_Q4_1 ? 2 : 5;
         fetch_b(p ^ 1, s + 1, 1);
         if constexpr (STAGED) {
             // the staged buffer of steps 4 S .. 4 S + 3 is number S % 2: written during step 4 S - 2 and read from the last quarter of
@@ -703,7 +770,7 @@ __device__ __forceinline__ void prefill_mfma_body(const uint8_t *__restrict__ W,
         for (int i = 0; i < 3 * G; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             if (i % G < RT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, RT == 4 ? 5 : 10, 0);  // (the decode of a step is as long whatever RT is)
+            __builtin_amdgcn_sched_group_barrier(0x002, DV * 4 / RT, 0);  // (the decode of a step is as long whatever RT is)
             if (i % G >= RT || i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             if (i >= 3 * G - 4) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
         }

@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(256) wide_dequant_kernel(const uint8_t *__rest
         if (s0 + i >= nsteps) break;
         const int kk = min((s0 + i) * PF_BK + 32 * dhalf, k - 32);
         f16x8 o[4];
-        if constexpr (FMT == F_Q4_K || FMT == F_Q5_K || FMT == F_Q6_K) {
+        if constexpr (pf_packed(FMT)) {
             pf_decode_h<FMT>(raw[i], kk, o);
         } else {
             float v[32];
