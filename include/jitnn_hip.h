@@ -133,7 +133,8 @@ JITNN_HIP_API int jitnn_hip_dequantize_dev(const jitnn_hip_weight *w, float *y_d
  * into LDS; the other, for more than 512 rows and at least 1024 values per weight row where an estimate finds it faster,
  * multiplies weights that a pass before it has dequantised into the calling thread's scratch (at most 512 MiB).  Where that
  * scratch cannot grow - no memory, or the stream is being captured - the first one runs.  Both round the same values to
- * FP16 and give the same bits.
+ * FP16 and give the same bits.  The first one cuts K into up to eight slices where its tiles leave compute units idle; where the
+ * scratch cannot grow to hold their sums it takes fewer, and adds the same products up in another order.
  * JITNN_HIP_GEMV_MAX_ROWS in the environment moves the switch. */
 JITNN_HIP_API int jitnn_hip_linear(const jitnn_hip_weight *w, const float *x_host, int rows, const float *bias_host, float *y_host);
 JITNN_HIP_API int jitnn_hip_linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, void *stream);

@@ -254,7 +254,7 @@ int xreg_args(const XregCall &c, XregArgs &a) {
 
 // The INT8 matrix-core kernel (gemv_i8.h) takes what the register-resident kernels take of the K-quants, and rows of up
 // to 16384 values.
-constexpr int PREFILL_MIN_SLICE = 8;  // fewest K steps (of 64 values) a slice of a split many-row launch may have
+constexpr int PREFILL_MIN_SLICE = 8;  // fewest K steps (of 64 values) a slice of a launch of several many-row weights may have
 
 // Its row groups are four rows: at least four rows in all, and the segments of a shared launch whole groups; its buffer
 // loads address a matrix with 32 bits.
@@ -895,6 +895,39 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
     return workspace_done(stream);
 }
 
+// Whole tiles for every compute unit, or K in slices that a second kernel adds up: how many (1 to 8) a single weight of the kernel that
+// decodes as it goes takes.  The estimate, in us: whole rounds of workgroups at 0.4 + `step` per 64 values of K (three quarters of it where
+// the narrow wave layout serves up to 128 rows), the slices' way to memory and back, and their join - a launch of its own unless the
+// next kernel reads them.  Fitted on 116 launches of six formats (256 to 18000 rows of 512 to 14336 values, 65 to 1000 activation
+// rows) at 1 to 8 slices: 6 % off in the mean, and its choice 0.4 % slower than the best count, where doubling the slices as long as they
+// fit the device twice over was 4.1 %.  Q8_0 8704 x 6592 at 170 rows 61.6 -> 49.8 us (three slices, not two), Q6_K 3074 x 12544 at 711 rows
+// 115.8 -> 96.7; the worst of them Q4_K 8704 x 6656 at 415 rows, 82.9 -> 88.0.
+double many_row_step_us(int fmt) {
+    switch (fmt) {
+    case F_Q4_0: case F_Q4_K: return 0.68;
+    case F_Q5_K: return 0.79;
+    case F_Q4_1: case F_Q8_0: return 0.82;
+    default: return 0.91;
+    }
+}
+int many_row_slices(int fmt, int n, int k, int rows, bool joined_by_reader, int cus) {
+    const int tiles = (n + PF_BN - 1) / PF_BN * ((rows + PF_BM - 1) / PF_BM), nsteps = (k + PF_BK - 1) / PF_BK, unit = block_values(fmt) == 256 ? 4 : 1;
+    const double step = many_row_step_us(fmt) * (rows <= PF_NARROW_ROWS ? 0.72 : 1.0), mb = 4e-6 * rows * n;
+    int best = 1;
+    double best_us = 0;
+    for (int s = 1; s <= 8; ++s) {
+        const int each = ((nsteps + s - 1) / s + unit - 1) / unit * unit;
+        if (s > 1 && (each < 2 || (nsteps + each - 1) / each != s)) continue;  // (a count that whole blocks leave slices empty)
+        const int rounds = (int)(((long long)tiles * s + cus - 1) / cus);
+        const double us = rounds * (0.4 + step * each) + (s > 1 ? 0.4 * s * mb + (joined_by_reader ? 0.5 : 4.0) : 0.2 * mb);
+        if (best_us == 0 || us < (best == 1 ? 0.98 : 1.0) * best_us) {
+            best = s;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 // More rows than the GEMV kernels take: FP16 activations in operand order + dequantise-to-LDS MFMA kernel.
 // `count` weights of one row length share the activations x [rows, k] (prepared once): ys[i] = x ws[i]^T (+ bias, one
 // weight only).  norm_w != nullptr: the RMSNorm in front of the linears is fused into the preparation (rows of at most
@@ -922,7 +955,8 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
     if (residual && (count != 1 || !tmp || ws[0]->n % 4 != 0)) return fail(JITNN_HIP_EINVAL, "a residual needs one weight, rows of whole quads and a buffer");
     const int k = ws[0]->k;
     WidePlan plan;
-    if (src == SCRATCH_THREAD && wide_pays(ws, count, rows, false, residual != nullptr, &plan)) {
+    const bool wide = wide_pays(ws, count, rows, false, residual != nullptr, &plan);
+    if (wide && src == SCRATCH_THREAD) {
         const int rc = launch_prefill_wide(plan, ws, ys, count, false, x, rows, bias, norm_w, eps, stream, residual, swiglu_up, pend);
         if (rc != WIDE_NO_ROOM) return rc;
     }
@@ -959,11 +993,18 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
             tiles += tiles_of(ws[q]);
             nsum += (size_t)ws[q]->n;
         }
-        // A launch that would leave most CUs idle (few, large tiles) splits K: every slice of at least 8 steps writes its
-        // own partial y, a second kernel adds the slices in order.
+        // A launch that would leave CUs idle (few, large tiles) splits K: every slice writes its own partial y, a second kernel - or
+        // the one that reads y next - adds the slices in order.  Several weights: twice as many slices as long as those fit the device twice.
         int splits = 1;
         if (nsum % 4 == 0 && ws[i]->n % 4 == 0) {
             while (splits < 8 && tiles * mtiles * splits * 2 <= g.cus && nsteps / (splits * 2) >= PREFILL_MIN_SLICE) splits *= 2;
+        }
+        if (l.count == 1 && !wide) {  // (wide: the bits of the kernel that this one stands in for)
+            // One weight, with scratch to spare: the count that the estimate likes best, for outputs of any length.  (The same limit for both
+            // sources of scratch, so that both entry points give the same bits; a stream capture that finds less at hand keeps the count above.)
+            const int want = many_row_slices(ws[i]->fmt, ws[i]->n, k, rows, defer != nullptr, g.cus);
+            const size_t need = operand_bytes(rows, k) + row_scale_bytes(rows) + (want > 1 ? (size_t)want * rows * ws[i]->n * 4 : 0);
+            if (need <= JITNN_HIP_SCRATCH_BYTES && workspace_at_hand(need, stream, src)) splits = want;
         }
         int wgs = tiles * mtiles * splits;
         l.part_bytes = 0;
@@ -1036,9 +1077,7 @@ int launch_prefill_group(const jitnn_hip_weight *const *ws, float *const *ys, in
             defer->splits = l.splits[0];
             defer->n = w->n;
         } else if (split) {
-            const size_t count4 = (size_t)rows * w->n / 4;
-            const unsigned blocks = (unsigned)std::min<size_t>((count4 + 255) / 256, (size_t)g.cus * 8);
-            prefill_join_launch(part, bias, residual, ys[l.first], count4, w->n, l.splits[0], blocks, stream);
+            prefill_join_launch(part, bias, residual, ys[l.first], rows, w->n, l.splits[0], (unsigned)g.cus * 8, stream);
         } else if (residual) {
             const size_t count4 = (size_t)rows * w->n / 4;
             const unsigned blocks = (unsigned)std::min<size_t>((count4 + 255) / 256, (size_t)g.cus * 8);
@@ -1929,9 +1968,7 @@ long long model_weight_bytes(const jitnn_hip_llama *m) {
 // The join of a linear's K slices that a caller deferred and nobody could fuse: prefill_join_kernel after all.
 void flush_pending(PfPending &p, int rows, hipStream_t st) {
     if (!p.part) return;
-    const size_t count4 = (size_t)rows * p.n / 4;
-    const unsigned blocks = (unsigned)std::min<size_t>((count4 + 255) / 256, (size_t)g.cus * 8);
-    prefill_join_launch(p.part, nullptr, p.res, p.out, count4, p.n, p.splits, blocks, st);
+    prefill_join_launch(p.part, nullptr, p.res, p.out, rows, p.n, p.splits, (unsigned)g.cus * 8, st);
     p = PfPending{};
 }
 

@@ -930,33 +930,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 }
 
 // y[tok, row] = sum over the K slices of part[z][tok, row] (+ bias[row]) (+ res[tok, row]), slices in order: the second half of a
-// split-K launch.  count4 = m * n / 4 (n is a multiple of 4 whenever the launch splits).
-static __global__ void __launch_bounds__(256) prefill_join_kernel(const float *__restrict__ part, const float *__restrict__ bias,
-                                                                   const float *__restrict__ res, float *__restrict__ y, size_t count4, int n, int splits) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count4; i += (size_t)gridDim.x * 256) {
-        float4 a = reinterpret_cast<const float4 *>(part)[i];
-        for (int z = 1; z < splits; ++z) {
-            const float4 b = reinterpret_cast<const float4 *>(part)[(size_t)z * count4 + i];
-            a.x += b.x;
-            a.y += b.y;
-            a.z += b.z;
-            a.w += b.w;
-        }
-        if (bias) {
-            const float4 b = *reinterpret_cast<const float4 *>(bias + (i * 4) % (size_t)n);
-            a.x += b.x;
-            a.y += b.y;
-            a.z += b.z;
-            a.w += b.w;
-        }
-        if (res) {  // a residual [m, n] rides along (the layers of a model: y = x + W a)
-            const float4 b = reinterpret_cast<const float4 *>(res)[i];
-            a.x += b.x;
-            a.y += b.y;
-            a.z += b.z;
-            a.w += b.w;
-        }
-        reinterpret_cast<float4 *>(y)[i] = a;
+// split-K launch.  V: float4 where n is a multiple of four, float for rows of any length (4 bytes a lane, whole lines a wave); count =
+// m n / (values per V).
+__device__ __forceinline__ float join_add(float a, float b) { return a + b; }
+__device__ __forceinline__ float4 join_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+template <class V>
+__global__ void __launch_bounds__(256) prefill_join_kernel(const V *__restrict__ part, const V *__restrict__ bias, const V *__restrict__ res,
+                                                           V *__restrict__ y, size_t count, int row_values, int splits) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t)gridDim.x * 256) {
+        V a = part[i];
+        for (int z = 1; z < splits; ++z) a = join_add(a, part[(size_t)z * count + i]);
+        if (bias) a = join_add(a, bias[i % (size_t)row_values]);
+        if (res) a = join_add(a, res[i]);  // a residual [m, n] rides along (the layers of a model: y = x + W a)
+        y[i] = a;
     }
 }
 

@@ -1,4 +1,6 @@
 // prefill_mfma_kernel for the 32-value formats (Q5_1 among them), the activation preparation and the join of K slices.
+#include <algorithm>
+
 #include "prefill.h"
 #include "tu.h"
 
@@ -48,9 +50,13 @@ void prefill_prepare_launch(const float *x, float *scale, float *inv_scale, _Flo
     }
 }
 
-void prefill_join_launch(const float *part, const float *bias, const float *res, float *y, size_t count4, int n, int splits, unsigned blocks,
-                         hipStream_t s) {
-    hipLaunchKernelGGL(prefill_join_kernel, dim3(blocks), dim3(256), 0, s, part, bias, res, y, count4, n, splits);
+void prefill_join_launch(const float *part, const float *bias, const float *res, float *y, int m, int n, int splits, unsigned max_blocks, hipStream_t s) {
+    const size_t count = (size_t)m * n / (n % 4 == 0 ? 4 : 1);
+    const dim3 grid((unsigned)std::min<size_t>((count + 255) / 256, max_blocks));
+    if (n % 4 == 0)
+        hipLaunchKernelGGL(prefill_join_kernel<float4>, grid, dim3(256), 0, s, reinterpret_cast<const float4 *>(part), reinterpret_cast<const float4 *>(bias),
+                           reinterpret_cast<const float4 *>(res), reinterpret_cast<float4 *>(y), count, n / 4, splits);
+    else hipLaunchKernelGGL(prefill_join_kernel<float>, grid, dim3(256), 0, s, part, bias, res, y, count, n, splits);
 }
 
 void prefill_join_group_launch(const float *part, const PfSegments &sg, int m, unsigned blocks, hipStream_t s) {

@@ -68,8 +68,8 @@ struct PfGroupPending {
 // (pend != nullptr: x is ignored, the rows come from *pend - with norm_w and rows the preparation normalises only)
 void prefill_prepare_launch(const float *x, float *scale, float *inv_scale, _Float16 *xo, int rows, int k, int mblocks, const float *norm_w, float eps,
                             const float *swiglu_up, hipStream_t s, const PfPending *pend = nullptr);
-void prefill_join_launch(const float *part, const float *bias, const float *res, float *y, size_t count4, int n, int splits, unsigned blocks,
-                         hipStream_t s);
+// y [m, n] = the slices part[splits][m, n] in order (+ bias [n]) (+ res [m, n])
+void prefill_join_launch(const float *part, const float *bias, const float *res, float *y, int m, int n, int splits, unsigned max_blocks, hipStream_t s);
 // the join of a launch of several segments: part = per segment splits[i] arrays [m, n[i]], one segment after the other
 void prefill_join_group_launch(const float *part, const PfSegments &sg, int m, unsigned blocks, hipStream_t s);
 
