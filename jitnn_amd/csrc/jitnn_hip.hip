@@ -20,6 +20,7 @@
 #include <sys/syscall.h>
 #include <unistd.h>
 
+#include "attn_packed.h"
 #include "dequant.h"
 #include "gemv.h"
 #include "gemv_mfma.h"
@@ -1883,6 +1884,8 @@ struct jitnn_hip_llama {
     // many-token (prefill) buffers, [pf_cap, ...] each, allocated by the first prefill call and grown when a longer one comes
     int pf_cap;
     float *pf[11];  // xn, q, k, v, att, xa, xb, gate, up, h, the K slices of a linear whose join is deferred (8 x d per token)
+    _Float16 *packed;  // keys and values of one layer as attn_packed_kernel reads them, up to max_ctx positions: allocated by the first long prompt
+    bool packed_refused;
     int rope_interleaved;  // 0: rotate-half pairs (i, i + D/2); 1: pairs (2i, 2i + 1)
     // token embedding table [vocab, d] in ggml type embd_fmt (F32 = 0, F16 = 1 or a block format), owned
     uint8_t *embd;
@@ -2101,14 +2104,41 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
     if (waited) g_ws.used = false;
 }
 
+// Room for a layer's packed keys and values, for the life of the model (a 64th part of its FP32 cache at 32 layers): false where there is
+// none, or none may be allocated.
+bool packed_room(jitnn_hip_llama *m, hipStream_t st) {
+    if (m->packed || m->packed_refused) return m->packed != nullptr;
+    if (stream_recording(st)) return false;
+    if (hipMalloc(&m->packed, ap_bytes(m->hd, m->kv, m->max_ctx)) != hipSuccess) {
+        (void)hipGetLastError();
+        m->packed = nullptr;
+        m->packed_refused = true;
+    }
+    return m->packed != nullptr;
+}
+// Whether the attention of a prompt pass takes the packed form.
+bool attention_packed(const jitnn_hip_llama *m, int pos0, int tokens) {
+    if (tokens <= g.gemv_max_rows || (m->hd != 64 && m->hd != 128) || m->heads / m->kv > AP_ROWS) return false;
+    const int qt = AP_ROWS / (m->heads / m->kv), blocks = (tokens + qt - 1) / qt;
+    return attn_packed_pays(m->hd, blocks * m->kv, pos0 + tokens, g.cus);
+}
+
 template <int D>
-int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, const float *q, float *att, hipStream_t st) {
+int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, bool packed, const float *q, float *att, hipStream_t st) {
     const int group = m->heads / m->kv;
     const size_t lo = (size_t)layer * m->max_ctx * m->kv * m->hd;
     const float scale = 1.0f / sqrtf((float)D);
     // prompts beyond the GEMV range have FP16-operand linears on both sides of the attention: FP16 operands here too
     if (tokens > g.gemv_max_rows) {
         if constexpr (D == 64 || D == 128) {
+            if (packed) {
+                const int qt = AP_ROWS / group, keys = pos0 + tokens, chunks = (keys + AP_CH - 1) / AP_CH;
+                if (int rc = allow_lds((const void *)attn_packed_kernel<D>, ap_lds_bytes(D))) return rc;
+                hipLaunchKernelGGL(attn_pack_kernel<D>, dim3(chunks, m->kv), dim3(AP_THREADS), 0, st, m->kc + lo, m->vc + lo, m->packed, m->kv, keys);
+                hipLaunchKernelGGL(attn_packed_kernel<D>, dim3(m->kv, (tokens + qt - 1) / qt), dim3(AP_THREADS), ap_lds_bytes(D), st, q, m->packed, att, m->heads, m->kv,
+                                   pos0, tokens, chunks, scale);
+                return JITNN_HIP_OK;
+            }
             if (group <= AM_ROWS) {
                 const int qt2 = 2 * AM_ROWS / group, blocks2 = (tokens + qt2 - 1) / qt2;
                 if (blocks2 * m->kv >= attn_two_tiles_from(D, g.cus)) {
@@ -2225,6 +2255,7 @@ int jitnn_hip_llama_free(jitnn_hip_llama *m) {
         if (b) (void)hipFree(b);
     for (float *b : m->pf)
         if (b) (void)hipFree(b);
+    if (m->packed) (void)hipFree(m->packed);
     if (m->embd) (void)hipFree(m->embd);
     if (m->tok_dev) (void)hipFree(m->tok_dev);
     if (m->tok_pin) (void)hipHostFree(m->tok_pin);
@@ -2353,6 +2384,7 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
     StatNest nest;
     const int d = m->d, T = tokens, qd = m->heads * m->hd;
     prefill_reserve(m, T, st);
+    const bool packed = attention_packed(m, pos0, T) && packed_room(m, st);
     float *xn = m->pf[0], *q = m->pf[1], *k = m->pf[2], *v = m->pf[3], *att = m->pf[4], *xa = m->pf[5], *xb = m->pf[6], *gate = m->pf[7],
           *up = m->pf[8], *h = m->pf[9];
     const float *x = x_dev;
@@ -2377,10 +2409,10 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
         }
         int arc;
         switch (m->hd) {
-        case 64: arc = launch_attention_rows<64>(m, l, pos0, T, q, att, st); break;
-        case 128: arc = launch_attention_rows<128>(m, l, pos0, T, q, att, st); break;
-        case 192: arc = launch_attention_rows<192>(m, l, pos0, T, q, att, st); break;
-        default: arc = launch_attention_rows<256>(m, l, pos0, T, q, att, st); break;
+        case 64: arc = launch_attention_rows<64>(m, l, pos0, T, packed, q, att, st); break;
+        case 128: arc = launch_attention_rows<128>(m, l, pos0, T, packed, q, att, st); break;
+        case 192: arc = launch_attention_rows<192>(m, l, pos0, T, packed, q, att, st); break;
+        default: arc = launch_attention_rows<256>(m, l, pos0, T, packed, q, att, st); break;
         }
         if (arc) return arc;
         // xa = x + Wo att, xb = xa + W2 (silu(W1 n) * (W3 n)), n = RMSNorm(xa)
