@@ -127,7 +127,8 @@ JITNN_HIP_API int jitnn_hip_dequantize_dev(const jitnn_hip_weight *w, float *y_d
  * core/ops/Quant.java:66-80,147-187).  rows >= 1; bias may be NULL.
  * Up to 64 rows run the GEMV kernels at FP32-grade accuracy (error ~1e-6 of the largest output): FP32 arithmetic for
  * one and two rows, FP16 hi/lo splits of the activations on the matrix cores for more - 3 to 8 rows in one launch, 9 to
- * 64 rows in one pass over the weights (rows of whole 256-value columns; else in passes of 8), in one of two kernels that the shape
+ * 64 rows in one pass over the weights (rows of whole 256-value columns; of Q4_0, Q4_1 and Q8_0 rows their whole columns, the rest in a
+ * kernel of its own; else, or without scratch for it, in passes of 8), in one of two kernels that the shape
  * alone chooses (jitnn_hip_few_rows_slices; where the second one's scratch cannot grow it takes a launch per slice of a row, and
  * gives the same bits); more rows (prefill) run on the matrix cores (FP16 operands, FP32 accumulation, error < 2e-3) in one of two kernels: one decodes the weights on their way
  * into LDS; the other, for more than 512 rows and at least 1024 values per weight row where an estimate finds it faster,

@@ -47,7 +47,7 @@ struct HeldGeo {
 };
 
 // y[slice][b, row] = sum over the slice's k of W[row, k] x[b, k], for the rows b of this workgroup's G groups (blockIdx.y);
-// k a multiple of 256, n >= 16, per_slice at most the number of steps.  A bias and a residual are rows_join_kernel's: loads here would be waited for with the weights.
+// k a multiple of 256 - or, blocks of 32 values, the whole columns of any row of those -, n >= 16, per_slice at most the number of steps.  A bias and a residual are rows_join_kernel's: loads here would be waited for with the weights.
 template <int FMT, int G>
 __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__restrict__ W, const uint8_t *__restrict__ W2, const _Float16 *__restrict__ ops, const float *__restrict__ inv,
                                                                 int n, int k, int rows, int groups, const uint32_t where, float *__restrict__ y) {
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_held_kernel(const uint8_t *__
     constexpr int PARKED = gh_ops_in_lds(FMT, G), HELD = 9 - PARKED;  // operands of a group in LDS, in registers
     f16x8 *parked = reinterpret_cast<f16x8 *>(gh_smem + 2 * (size_t)BUF * sizeof(float2) + gemv_rows_stage_bytes<FMT>(1)) + wave * PARKED * G * 64 + lane;
     const int ncol = k >> 8, each = (n + 15) >> 4, ntiles = W2 ? 2 * each : each, nsteps = (ntiles + geo.lanes - 1) / geo.lanes;
-    const size_t rowbytes = (size_t)ncol * R::BYTES;
+    const size_t rowbytes = (size_t)(k / block_values(FMT)) * block_bytes(FMT);
     const int slice = (int)blockIdx.x / geo.per_slice, first = (int)blockIdx.x - slice * geo.per_slice;
     const int c0 = slice * geo.cols, cols = min(geo.cols, ncol - c0);  // (the last slice may be short)
     const int tl = wave / geo.cols, c = c0 + wave - tl * geo.cols;

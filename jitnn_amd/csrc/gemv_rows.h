@@ -517,7 +517,8 @@ __host__ __device__ constexpr size_t gemv_rows_stage_bytes(int tiles_per_wave) {
     return (size_t)GR_WAVES * tiles_per_wave * RTile<FMT>::STAGE_BYTES;
 }
 
-// y[b, row] = sum_k W[row, k] x[b, k] (+ bias[row]) (+ res[b, row]) for b < rows <= 8 * groups; k a multiple of 256, n >= 16.
+// y[b, row] = sum_k W[row, k] x[b, k] (+ bias[row]) (+ res[b, row]) for b < rows <= 8 * groups; k a multiple of 256 (Q4_0, Q4_1, Q8_0: the sum over
+// the whole 256-value columns of a row of any number of blocks), n >= 16.
 //   ops / inv: the output of rows_prepare_kernel<RTile<FMT>::SUMS> for the same x.  grid: up to one workgroup per batch of T tiles of 16
 //   weight rows (the host caps it at one per compute unit) x shares of the groups of activation rows; GR_THREADS threads;
 //   gemv_rows_lds_bytes() + gemv_rows_stage_bytes() of dynamic LDS.
@@ -541,7 +542,7 @@ __global__ void __launch_bounds__(GR_THREADS) gemv_rows_kernel(const uint8_t *__
     // (staged formats: behind accl, per wave and tile the sixteen rows of the column being decoded)
     uint8_t *stage = gr_smem + gemv_rows_lds_bytes(T) + gemv_rows_stage_bytes<FMT>(T) / GR_WAVES * wave;
     const int ncol = k >> 8, ntiles = (n + 15) >> 4, nbatch = (ntiles + T - 1) / T;
-    const size_t rowbytes = (size_t)ncol * R::BYTES;
+    const size_t rowbytes = (size_t)(k / block_values(FMT)) * block_bytes(FMT);
     // gridDim.y > 1 (matrices with few tiles): workgroup y takes the groups [gper y, gper y + gper) of activation rows - it
     // decodes the same weights as its neighbours and writes whole outputs of its own rows, nothing meets across workgroups
     if (grid_y > 1) {

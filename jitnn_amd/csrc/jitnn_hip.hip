@@ -24,6 +24,7 @@
 #include "dequant.h"
 #include "gemv.h"
 #include "gemv_mfma.h"
+#include "gemv_tail.h"
 #include "gguf_file.h"
 #include "glue.h"
 #include "prefill.h"
@@ -1399,6 +1400,16 @@ bool rows_path(const jitnn_hip_weight *w, int rows) {
            w->n >= 16;
 }
 
+// The same for rows of 32-value blocks that are not whole columns: the whole ones in one pass, the rest by gemv_tail_kernel, instead of
+// passes of eight rows, which stream the weight once each.  us, passes against this: Q4_1 5120 x 11456 at 5 / 9 / 40 / 64 rows 57 / 70 / 308 / 492
+// and 26 / 29 / 44 / 55, Q8_0 8000 x 5088 48 / 68 / 276 / 441 and 29 / 32 / 43 / 55, Q4_0 2048 x 2272 at 5 / 8 / 9 / 40 16 / 18 / 23 / 88 and 17.5 / 17.5 /
+// 17 / 20, Q4_0 4096 x 1504 at 9 / 11 / 16 16.4 / 16.7 / 21.0 and 17.3 / 17.8 / 17.7, Q8_0 2672 x 1056 at 8 / 9 9.6 / 17.4 and 14.0 / 14.1.
+bool rows_ragged_path(const jitnn_hip_weight *w, int rows) {
+    if (w->fmt != F_Q4_0 && w->fmt != F_Q4_1 && w->fmt != F_Q8_0) return false;
+    const int rows_min = w->k >= 12288 ? 3 : w->k >= 3072 ? 5 : w->k >= 2048 || w->fmt == F_Q8_0 ? 9 : 13;
+    return w->k % 256 != 0 && w->k > 256 && rows >= rows_min && rows <= 64 && rows <= g.gemv_max_rows && w->n >= 16;
+}
+
 // One launch of rows_path, with a join of its own where it has slices: the plan of the kernel that holds the operands, or groups_held = 0.
 size_t rows_operand_bytes(int rows, int k) { return (gemv_rows_scratch_bytes(rows, k) + 255) & ~(size_t)255; }
 HeldPlan rows_plan(const jitnn_hip_weight *w, int rows, bool adds, int cus) {
@@ -1554,6 +1565,16 @@ int launch_rows_ffn(const RowsFfn &f, const jitnn_hip_weight *wg, const jitnn_hi
     return workspace_done(s);
 }
 
+int launch_gemv_tail(const jitnn_hip_weight *w, const float *x, int rows, float *y, hipStream_t s) {
+    const int blocks = w->k % 256 / 32;
+    const size_t lds = gemv_tail_lds_bytes(rows, blocks);
+    auto kernel = w->fmt == F_Q4_0 ? gemv_tail_kernel<F_Q4_0> : w->fmt == F_Q4_1 ? gemv_tail_kernel<F_Q4_1> : gemv_tail_kernel<F_Q8_0>;
+    if (int rc = allow_lds((const void *)kernel, lds)) return rc;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((w->n + GT_ROWS - 1) / GT_ROWS)), dim3(GT_THREADS), lds, s, w->dev, x, y, w->n, w->k, rows, blocks);
+    HIP_TRY(hipGetLastError());
+    return JITNN_HIP_OK;
+}
+
 int linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, hipStream_t s, ScratchSource src) {
     if (!w || !x_dev || !y_dev) return fail(JITNN_HIP_EINVAL, "weight, input or output is NULL");
     if (rows < 1) return fail(JITNN_HIP_EINVAL, "rows = %d", rows);
@@ -1563,6 +1584,11 @@ int linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const fl
     if (many) return launch_prefill(w, x_dev, rows, bias_dev, y_dev, s, src);
     // several rows, rows of whole 256-value columns: every row meets the weights in one pass over them (gemv_rows.h)
     if (rows_path(w, rows)) return launch_rows_group(&w, &y_dev, 1, x_dev, rows, bias_dev, nullptr, s, src);
+    // (no scratch at hand - a stream capture before the first eager call, no memory: the passes of eight, which need none)
+    if (rows_ragged_path(w, rows) && workspace_at_hand(rows_operand_bytes(rows, w->k), s, src)) {
+        if (int rc = launch_rows_group(&w, &y_dev, 1, x_dev, rows, bias_dev, nullptr, s, src)) return rc;
+        return launch_gemv_tail(w, x_dev, rows, y_dev, s);
+    }
     for (int r0 = 0; r0 < rows; r0 += 8) {
         const int nb = rows - r0 < 8 ? rows - r0 : 8;
         if (int rc = launch_gemv(w, x_dev + (size_t)r0 * w->k, nb, bias_dev, y_dev + (size_t)r0 * w->n, s)) return rc;
