@@ -30,6 +30,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const float *__restrict__
 // the value to the cache, grouped-query attention over the s = pos + 1 cached positions
 // (F.scaledDotProductAttentionBTHD with F.repeatHeads, F.java:588-624; ops/FlashAttention.java:538-626: query head
 // h reads key/value head h / group).
+//   (Long caches take attn_split_kernel, attn_split.h, where the heads allow.)
 //   grid (chunks, kv_heads): a workgroup stages CH keys and values of one kv head in LDS (the cache chunk is read
 //   once for the whole group of query heads), computes the group's scores from LDS, each chunk's softmax statistics
 //   and unnormalised weighted value sum, and leaves them in `part` for attn_merge_kernel.

@@ -21,6 +21,7 @@
 #include <unistd.h>
 
 #include "attn_packed.h"
+#include "attn_split.h"
 #include "dequant.h"
 #include "gemv.h"
 #include "gemv_mfma.h"
@@ -1922,13 +1923,42 @@ struct jitnn_hip_llama {
 
 namespace {
 
+using AttnDecodeKernel = void (*)(const float *, const float *, const float *, float *, float *, float *, uint32_t, uint32_t);
+template <int D, int P>
+AttnDecodeKernel attn_split_of(int group) {
+    switch (group) {
+    case 1: return attn_split_kernel<D, 1, P>;
+    case 2: return attn_split_kernel<D, 2, P>;
+    case 3: return attn_split_kernel<D, 3, P>;
+    default: return attn_split_kernel<D, 4, P>;
+    }
+}
+
+// Passes of 8 keys per wave that one token's attention takes in attn_split_kernel, 0: attn_decode_kernel.  Both with their merge and what one
+// waits for the other, us per layer more than the shortest cache takes, attn_decode_kernel / 2 / 4 passes: 32 heads of 128 values
+// over 8, 700 keys 1.0 / 1.0 / 1.8, 1000 1.6 / 1.1 / 2.1, 1400 3.7 / 1.8 / 2.5 (more than 32 chunks: the merge takes its longer form), 2000
+// 4.5 / 2.3 / 2.9, 3000 6.2 / 6.1 / 4.4, 4000 10.0 / 7.8 / 5.8, 8000 20.0 / 16.1 / 14.9; 8 over 8, 1000 1.4 / 0.7 / 0.5, 4000 9.1 / 6.0 / 3.7; 32
+// heads of 64 values over 8, 1000 0.5 / 0.4 / 0.7, 4000 4.0 / 3.3 / 2.2.  Two passes while their workgroups have a CU each.
+int attn_split_passes(int D, int group, int kv, int keys, int cus) {
+    if ((D != 64 && D != 128) || group > AS_GMAX || keys < 1024) return 0;
+    return (keys + as_keys(2) - 1) / as_keys(2) * kv <= cus ? 2 : 4;
+}
+
 template <int D>
 void launch_attention(const jitnn_hip_llama *m, int layer, int pos, hipStream_t st) {
-    const int chunks = (pos + 1 + AttCfg<D>::CH - 1) / AttCfg<D>::CH;
     const size_t lo = (size_t)layer * m->max_ctx * m->kv * m->hd;
+    AttnDecodeKernel kernel = attn_decode_kernel<D>;
+    int keys = AttCfg<D>::CH;  // of a chunk
+    if constexpr (D == 64 || D == 128) {
+        if (const int passes = attn_split_passes(D, m->heads / m->kv, m->kv, pos + 1, g.cus)) {
+            kernel = passes == 2 ? attn_split_of<D, 2>(m->heads / m->kv) : attn_split_of<D, 4>(m->heads / m->kv);
+            keys = as_keys(passes);
+        }
+    }
+    const int chunks = (pos + keys) / keys;
     // (q, k, v: one buffer, see jitnn_hip_llama_create)
-    hipLaunchKernelGGL(attn_decode_kernel<D>, dim3(chunks, m->kv), dim3(256), 0, st, m->q, m->cosv, m->sinv, m->kc + lo, m->vc + lo, m->part,
-                       (uint32_t)m->heads | ((uint32_t)m->kv << 16), (uint32_t)pos | (m->rope_interleaved ? 0x80000000u : 0u));
+    hipLaunchKernelGGL(kernel, dim3(chunks, m->kv), dim3(256), 0, st, m->q, m->cosv, m->sinv, m->kc + lo, m->vc + lo, m->part, (uint32_t)m->heads | ((uint32_t)m->kv << 16),
+                       (uint32_t)pos | (m->rope_interleaved ? 0x80000000u : 0u));
     constexpr int NPL = 1024 / D < 8 ? 1024 / D : 8;  // long contexts: more threads per value share the chunks
     if (chunks > 32) hipLaunchKernelGGL((attn_merge_kernel<D, NPL>), dim3(m->heads), dim3(NPL * D), 0, st, m->part, m->att, chunks);
     else hipLaunchKernelGGL((attn_merge_kernel<D, 2>), dim3(m->heads), dim3(2 * D), 0, st, m->part, m->att, chunks);
