@@ -815,9 +815,12 @@ size_t row_scale_bytes(int rows) { return ((size_t)rows * 8 + 255) & ~(size_t)25
 // the estimate of both passes against that of prefill_mfma_kernel, which takes rounds of 128-row tiles (dual: 64 rows of each
 // weight) by 256 tokens at `step` us per 64 values of K.  Measured, both routes, activation preparation included (us):
 // 14336 x 4096 Q4_K, 1024 / 2048 / 4096 rows 139 / 268 / 496 there and 137 / 256 / 484 here; 4096 x 14336 Q6_K 169 / 298 / 612
-// and 228 / 292 / 486; 11008 x 4096 Q4_0 162 / 245 / 488 and 111 / 194 / 361; 4096 x 4096 Q4_K 58 / 85 / 160 and 65 / 84 / 139;
-// Q8_0 64 / 94 / 179 and 65 / 85 / 140.  Two tiles of tokens or fewer, short rows of K and launches that split K lose
-// here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
+// and 228 / 292 / 486; 4096 x 4096 Q4_K 58 / 85 / 160 and 65 / 84 / 139; Q8_0 64 / 94 / 179 and 65 / 85 / 140.
+// Up to 1024 rows Q4_0, Q4_1 and Q5_K have the steps that lost least on 326 linears and 61 prompts of 4 layers, timed with both routes since
+// prefill_mfma_kernel decodes them in packed FP16 under its products (beyond, where only whole prompts were timed, 1.06 stands): Q4_0 linears
+// 0.5 % behind the faster route in the mean and not 1.3.  Of Q4_0, here -> there: 4352 x 12800 at 886 rows 170 -> 146 us, 14336 x 4096 at 900
+// 139 -> 125, 800 tokens of four 4096-wide layers 2244 -> 2136; the most it costs: Q5_K 14336 x 4096 at 1024 rows, 135 -> 138 us.
+// Two tiles of tokens or fewer, short rows of K and launches that split K lose here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
 // estimate is good to a tenth on short launches: the margins.  For the 8B gate / up pair it errs against this route: at 4096
 // rows 920 us estimated there and 970 measured, 828 estimated here and 800 measured, so that with the margin it is
 // taken at 2049 - 2304, 2561 - 2816, 3073 - 3328 and 3585 - 4096 rows, where the product's last round is full enough, and not
@@ -835,7 +838,7 @@ bool wide_pays(const int *fmt, const int *rows_of, int count, int k, int rows, b
         if (i == 0 || !dual) n[i] = rows_of[i];
         tiles += (rows_of[i] + PF_BN - 1) / PF_BN;
         dequant += 3.0 + (f == F_Q6_K ? 0.62e-6 : 0.45e-6) * rows_of[i] * (double)k;
-        step = std::max(step, f == F_Q4_K ? 0.87 : f == F_Q6_K ? 1.17 : 1.06);
+        step = std::max(step, f == F_Q4_K ? 0.87 : f == F_Q6_K ? 1.17 : rows > 1024 ? 1.06 : f == F_Q4_0 ? 0.92 : f == F_Q4_1 || f == F_Q5_K ? 0.98 : 1.06);
     }
     *plan = wide_plan(n, dual ? 1 : count, k, mtiles, dual, cus);
     if (wide_weight_bytes(*plan, k) > WIDE_MAX_BYTES) return false;

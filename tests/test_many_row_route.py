@@ -66,3 +66,12 @@ def test_misuse():
                            ([(k4, 64), (k4, 64)], 256, dict(residual=True)), ([(k4, 64)] * 4, 256, {})):
         with pytest.raises(ValueError):
             many_row_tile(weights, k, 2000, compute_units=256, **kw)
+
+
+@pytest.mark.parametrize("fmt,n,k,rows,tile", [
+    ("Q4_0", 14336, 4096, 512, 0), ("Q4_0", 14336, 4096, 900, 0), ("Q4_1", 14336, 4096, 900, 0), ("Q5_K", 14336, 4096, 900, 0),
+    ("Q8_0", 14336, 4096, 900, 256), ("Q4_0", 4352, 12800, 886, 0), ("Q4_0", 14336, 4096, 1024, 0), ("Q4_0", 4096, 14336, 2048, 128), ("Q8_0", 4352, 12800, 886, 128)])
+def test_formats_decoded_in_packed_fp16(fmt, n, k, rows, tile):
+    """Up to 1024 rows Q4_0, Q4_1 and Q5_K stay with the kernel that decodes as it goes where Q8_0, whose decode is longer, does not."""
+    from jitnn_amd._lib import many_row_tile
+    assert many_row_tile([(GGML_ID[fmt], n)], k, rows, compute_units=256) == tile
