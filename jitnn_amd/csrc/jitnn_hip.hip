@@ -907,7 +907,9 @@ int launch_prefill_wide(const WidePlan &plan, const jitnn_hip_weight *const *ws,
 // next kernel reads them.  Fitted on 116 launches of six formats (256 to 18000 rows of 512 to 14336 values, 65 to 1000 activation
 // rows) at 1 to 8 slices: 6 % off in the mean, and its choice 0.4 % slower than the best count, where doubling the slices as long as they
 // fit the device twice over was 4.1 %.  Q8_0 8704 x 6592 at 170 rows 61.6 -> 49.8 us (three slices, not two), Q6_K 3074 x 12544 at 711 rows
-// 115.8 -> 96.7; the worst of them Q4_K 8704 x 6656 at 415 rows, 82.9 -> 88.0.
+// 115.8 -> 96.7.  A device that whole tiles keep more than half busy slows its clock when the rest joins in: there the estimate has to see 8 %
+// (90 launches of 101 to 255 tiles: 0.26 % behind the best count, at worst 2.1, where 2 % gave 0.32 and 5.8; Q4_K 9472 x 6144 at
+// 361 rows 86 us in three slices, 83 whole; Q6_K 6912 deep, 8495 at 323, 104 -> 97 in three).
 double many_row_step_us(int fmt) {
     switch (fmt) {
     case F_Q4_0: case F_Q4_K: return 0.68;
@@ -926,7 +928,7 @@ int many_row_slices(int fmt, int n, int k, int rows, bool joined_by_reader, int 
         if (s > 1 && (each < 2 || (nsteps + each - 1) / each != s)) continue;  // (a count that whole blocks leave slices empty)
         const int rounds = (int)(((long long)tiles * s + cus - 1) / cus);
         const double us = rounds * (0.4 + step * each) + (s > 1 ? 0.4 * s * mb + (joined_by_reader ? 0.5 : 4.0) : 0.2 * mb);
-        if (best_us == 0 || us < (best == 1 ? 0.98 : 1.0) * best_us) {
+        if (best_us == 0 || us < (best > 1 ? 1.0 : 2 * tiles > cus ? 0.92 : 0.98) * best_us) {
             best = s;
             best_us = us;
         }
