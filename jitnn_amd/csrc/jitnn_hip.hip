@@ -1917,7 +1917,6 @@ struct jitnn_hip_llama {
     int pf_cap;
     float *pf[11];  // xn, q, k, v, att, xa, xb, gate, up, h, the K slices of a linear whose join is deferred (8 x d per token)
     _Float16 *packed;  // keys and values of one layer as attn_packed_kernel reads them, up to max_ctx positions: allocated by the first long prompt
-    bool packed_refused;
     int rope_interleaved;  // 0: rotate-half pairs (i, i + D/2); 1: pairs (2i, 2i + 1)
     // token embedding table [vocab, d] in ggml type embd_fmt (F32 = 0, F16 = 1 or a block format), owned
     uint8_t *embd;
@@ -2166,14 +2165,12 @@ void prefill_reserve(const jitnn_hip_llama *m, int tokens, hipStream_t st) {
 }
 
 // Room for a layer's packed keys and values, for the life of the model (a 64th part of its FP32 cache at 32 layers): false where there is
-// none, or none may be allocated.
+// none, or none may be allocated; the next prompt pass asks again.
 bool packed_room(jitnn_hip_llama *m, hipStream_t st) {
-    if (m->packed || m->packed_refused) return m->packed != nullptr;
-    if (stream_recording(st)) return false;
+    if (m->packed || stream_recording(st)) return m->packed != nullptr;
     if (hipMalloc(&m->packed, ap_bytes(m->hd, m->kv, m->max_ctx)) != hipSuccess) {
         (void)hipGetLastError();
         m->packed = nullptr;
-        m->packed_refused = true;
     }
     return m->packed != nullptr;
 }
