@@ -117,6 +117,9 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
     // (64 and 128 values, 600 to 2048 tokens, scores of three widths) the output is off by 0.89 to 1.016 times, 0.989 in the mean, what it
     // is off by in attn_prefill_mfma_kernel, whose two running maxima per row make two weights of a row exact; without it 1.004 times.
     // 3 % of the kernel's time.
+    // q comes times 1 / sqrt(D) and log2(e): scores in base-2 units, whose largest less itself is 0 at any magnitude.  (Scaled behind the
+    // product, by an FMA with the rounded maximum, it is the rounding of that: beyond 2^28 a weight past what FP16 holds.)
+    const float scale2 = scale * 1.44269504088896341f;
     f16x8 qb[RT][DB], ql[RT];
 #pragma unroll
     for (int u = 0; u < RT; ++u) {
@@ -127,7 +130,9 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             const float *qp = q + at[u] + 32 * b + 8 * kq;
-            const float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
+            float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
+            x = make_float4(x.x * scale2, x.y * scale2, x.z * scale2, x.w * scale2);
+            y = make_float4(y.x * scale2, y.y * scale2, y.z * scale2, y.w * scale2);
             qb[u][b] = live[u] ? f16x8{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w, (_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w}
                                : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
             if (b == 0) {
@@ -137,7 +142,6 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
             }
         }
     }
-    const float scale2 = scale * 1.44269504088896341f;
     f32x4 o[RT][DT];
     float mrun[RT], lrun[RT];  // the row's maximum so far (base 2), this lane's share of its sum
 #pragma unroll
@@ -185,14 +189,14 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
                     if constexpr (MASK) st[u][t][i] = j0 + 16 * t + 4 * kq + i <= jmax[u] ? st[u][t][i] : -INFINITY;
                     mc = fmaxf(mc, st[u][t][i]);
                 }
-            const float mn = fmaxf(mrun[u], ap_max4(mc) * scale2);  // (scale > 0)
+            const float mn = fmaxf(mrun[u], ap_max4(mc));
             const float alpha = mrun[u] > -INFINITY ? __builtin_amdgcn_exp2f(mrun[u] - mn) : 0.f;
             mrun[u] = mn;
 #pragma unroll
             for (int t = 0; t < KT; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[u][t][i], scale2, -mn));
+                    float p = __builtin_amdgcn_exp2f(st[u][t][i] - mn);
                     if constexpr (MASK) p = st[u][t][i] > -INFINITY ? p : 0.f;  // (a row without a visible key: -inf minus -inf)
                     st[u][t][i] = p;
                 }

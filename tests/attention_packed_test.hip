@@ -130,6 +130,47 @@ static bool later_blocks_do_not_reach_earlier_ones() {
     return rows_match<D>(c, attention<D>(c), 32);
 }
 
+// Scores around 2^32 (positive queries and keys up to 3e4): a row's weight lies on its best key alone, and its output is that key's value as
+// FP16 holds it.  A score is off by less than 2^-10 of itself (FP16 queries, FP32 sums): rows whose best two are closer than 2^-9 are left out.
+template <int D>
+static bool large_scores() {
+    printf("%d values, scores around 2^32\n", D);
+    fflush(stdout);
+    Case c = random_case<D>(4, 2, 70, 75, false);
+    std::mt19937 gen(D);
+    std::uniform_real_distribution<float> spread(0.5f, 1.f), rank(0.25f, 1.f);
+    for (float &x : c.q) x = 3e4f * spread(gen);
+    for (size_t i = 0; i < c.k.size(); i += D) {
+        const float r = rank(gen);
+        for (int e = 0; e < D; ++e) c.k[i + e] = (float)(_Float16)(3e4f * r * spread(gen));
+    }
+    const std::vector<float> out = attention<D>(c);
+    int clear = 0;
+    for (int t = 0; t < c.tokens; ++t)
+        for (int h = 0; h < c.heads; ++h) {
+            int best = 0;
+            double top = 0, second = 0;
+            for (int j = 0; j <= c.pos0 + t; ++j) {
+                double a = 0;
+                for (int e = 0; e < D; ++e) a += (double)c.q[((size_t)t * c.heads + h) * D + e] * c.k[((size_t)j * c.kv + h / 2) * D + e];
+                if (a > top) best = j;
+                second = std::max(second, std::min(a, top));
+                top = std::max(top, a);
+            }
+            if (top - second < 0x1p-9 * top) continue;
+            ++clear;
+            for (int e = 0; e < D; ++e) {
+                const float got = out[((size_t)t * c.heads + h) * D + e], want = (float)(_Float16)c.v[((size_t)best * c.kv + h / 2) * D + e];
+                if (!(fabsf(got - want) <= 1e-6f * fabsf(want))) {
+                    printf("token %d head %d value %d: %.7f, not %.7f\n", t, h, e, got, want);
+                    return false;
+                }
+            }
+        }
+    if (clear < c.tokens) printf("%d rows of %d with a clear best key\n", clear, c.tokens * c.heads);
+    return clear >= c.tokens;
+}
+
 int main() {
     bool ok = true;
     for (int grow = 0; grow < 2; ++grow) {
@@ -137,6 +178,7 @@ int main() {
         ok = ok && run<64>(8, 2, 0, 64, grow) && run<64>(3, 1, 62, 91, grow) && run<64>(4, 4, 130, 130, grow) && run<64>(16, 1, 64, 9, grow);
     }
     ok = ok && later_blocks_do_not_reach_earlier_ones<128>() && later_blocks_do_not_reach_earlier_ones<64>();
+    ok = ok && large_scores<128>() && large_scores<64>();
     printf(ok ? "all hold\n" : "FAILED\n");
     return ok ? 0 : 1;
 }
