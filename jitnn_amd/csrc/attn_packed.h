@@ -20,14 +20,16 @@ constexpr size_t ap_lds_bytes(int D) { return 2 * ap_chunk_halves(D) * sizeof(_F
 // the packed keys and values of `keys` positions
 constexpr size_t ap_bytes(int D, int kv_heads, int keys) { return (size_t)kv_heads * ((keys + AP_CH - 1) / AP_CH) * ap_chunk_halves(D) * sizeof(_Float16); }
 
-// Whether the packing pays, for `blocks` workgroups of 128 rows and that many keys.  Kernel trace, us per layer, with
-// attn_prefill_mfma_kernel / packing + this; 128 values: 4096 tokens of 32 heads over 8 (1024 workgroups) 285 to 304 / 10 + 174 to 181, 3000 tokens
-// (750) 172 / 9 + 106, 2048 (512) 84 / 7 + 61, 1500 (376) 61 / 7 + 45, 1024 (256) 38 / 6 + 30, 720 (184) 32.3 / 6.6 + 22.8; 640 (160) 26.3 / 6.4 +
-// 21.6, 512 (128) 18.4 / 6.3 + 18.1.  Between 128 and 176 the other kernel's blocks, of 64 rows there, need a second place on some CUs, which
-// costs the more the more keys there are: 600 tokens from position 900 (152) 67 / 6.5 + 40.8, 2200 tokens of 8 heads over 4 (140) 59.4 / 6.6 + 51.
-// 64 values: 1024 workgroups 155 / 6 + 114, 376 84 / 5.6 + 60; 256 to 260 50 / 5 + 39, 38 / 5.7 + 40.6, 40.5 / 5 + 39.7.
-constexpr bool attn_packed_pays(int D, int blocks, int keys, int cus) {
-    return D == 64 ? 4 * blocks >= 5 * cus : 16 * blocks >= 11 * cus || (2 * blocks > cus && keys >= 1024);
+// Whether the packing pays, for `blocks` workgroups of 128 rows.  Whole prompts of six layers, us per layer, with it / with the form of
+// attn_prefill_mfma_kernel that runs otherwise.  128 values, 32 heads over 8: 4096 tokens (1024 workgroups) 1066 / 1134, 3000 (752) 881 / 915,
+// 2048 (512) 562 / 561, 1536 (384) 479 / 472, 1024 (256) 330 / 327, 900 (232) 318 / 327, 720 (184) 284 / 285; 16 over 4, 3000 (376) 389 / 397;
+// 8 over 8, 3000 (192) 262 / 283; 8 over 4, 3000 (188) 231 / 245.  From 128 to 176 the other kernel's blocks, of 64 rows there, need a
+// second place on some CUs, which costs where all blocks walk about the same number of keys: 600 tokens from position 900 (152) 299 / 321,
+// 560 from 3000 (144) 341 / 402, 1200 from 900 (152, 16 over 4) 226 / 228, but 2200 from 900 (140, 8 over 4) 218 / 211, 2500 from 0 (160)
+// 208 / 202, 640 from 0 (160) 278 / 275; 512 from 2000 (128) 276 / 275.
+// 64 values: 1024 workgroups 458 / 481, 528 299 / 308, 376 213 / 220, 328 to 340 205 / 209, 192 / 203 and 195 / 197; 256 to 304 173 / 169, 193 / 191, 181 / 177.
+constexpr bool attn_packed_pays(int D, int blocks, int pos0, int tokens, int cus) {
+    return D == 64 ? 4 * blocks >= 5 * cus : 16 * blocks >= 11 * cus || (2 * blocks > cus && 4 * pos0 >= 3 * tokens);
 }
 
 // kcache, vcache [keys, kv_heads, D] -> packed[kv head][chunk]:
@@ -113,32 +115,30 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
     bool live[RT];
     int jmax[RT];  // the last key the row sees
     size_t at[RT];  // the row's place in q and out
-    // ql: what rounding to FP16 left of the first 32 values.  It joins the scores of the first D / 64 tiles of a chunk's keys: against FP64
-    // (64 and 128 values, 600 to 2048 tokens, scores of three widths) the output is off by 0.89 to 1.016 times, 0.989 in the mean, what it
-    // is off by in attn_prefill_mfma_kernel, whose two running maxima per row make two weights of a row exact; without it 1.004 times.
-    // 3 % of the kernel's time.
     // q comes times 1 / sqrt(D) and log2(e): scores in base-2 units, whose largest less itself is 0 at any magnitude.  (Scaled behind the
     // product, by an FMA with the rounded maximum, it is the rounding of that: beyond 2^28 a weight past what FP16 holds.)
+    // It comes in two parts, qb + ql, 22 bits.  Against FP64 (64 and 128 values, 600 to 2048 tokens, queries of width 1, 3 and 8) the output is
+    // off by 0.86 to 0.90, 0.77 to 0.80 and 0.75 to 0.80 times what it is off by in attn_prefill_mfma_kernel; with one part 1.004 times in the
+    // mean - that kernel's two running maxima per row make two weights of a row exact.  The products with ql take 22 of 203 us (4096 tokens, 32
+    // heads over 8 of 128 values); heads of 64 values lose nothing by them but at the longest prompts (127 against 117 us there).
     const float scale2 = scale * 1.44269504088896341f;
-    f16x8 qb[RT][DB], ql[RT];
+    f16x8 qb[RT][DB], ql[RT][DB];
 #pragma unroll
     for (int u = 0; u < RT; ++u) {
         const int r = 16 * (RT * wave + u) + n, tq = r / group, hq = r - tq * group;
         live[u] = r < rows && t0 + tq < T;
         jmax[u] = pos0 + t0 + tq;
         at[u] = ((size_t)(t0 + (live[u] ? tq : 0)) * heads + g * group + (live[u] ? hq : 0)) * D;
+        const float f = live[u] ? scale2 : 0.f;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             const float *qp = q + at[u] + 32 * b + 8 * kq;
-            float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
-            x = make_float4(x.x * scale2, x.y * scale2, x.z * scale2, x.w * scale2);
-            y = make_float4(y.x * scale2, y.y * scale2, y.z * scale2, y.w * scale2);
-            qb[u][b] = live[u] ? f16x8{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w, (_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w}
-                               : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (b == 0) {
-                const float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+            const float4 x = *reinterpret_cast<const float4 *>(qp), y = *reinterpret_cast<const float4 *>(qp + 4);
+            const float v[8] = {x.x * f, x.y * f, x.z * f, x.w * f, y.x * f, y.y * f, y.z * f, y.w * f};
 #pragma unroll
-                for (int i = 0; i < 8; ++i) ql[u][i] = live[u] ? (_Float16)(f[i] - (float)qb[u][0][i]) : (_Float16)0.f;
+            for (int i = 0; i < 8; ++i) {
+                qb[u][b][i] = (_Float16)v[i];
+                ql[u][b][i] = (_Float16)(v[i] - (float)qb[u][b][i]);
             }
         }
     }
@@ -172,10 +172,8 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
                 const f16x8 a = kp[(t * DB + b) * 64];
 #pragma unroll
                 for (int u = 0; u < RT; ++u) st[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[u][b], st[u][t], 0, 0, 0);
-                if (b == 0 && t < D / 64) {  // (an eighth of the products with q)
 #pragma unroll
-                    for (int u = 0; u < RT; ++u) st[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u], st[u][t], 0, 0, 0);
-                }
+                for (int u = 0; u < RT; ++u) st[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[u][b], st[u][t], 0, 0, 0);
             }
         }
         f16x8 pa[RT][2];

@@ -2178,7 +2178,7 @@ bool packed_room(jitnn_hip_llama *m, hipStream_t st) {
 bool attention_packed(const jitnn_hip_llama *m, int pos0, int tokens) {
     if (tokens <= g.gemv_max_rows || (m->hd != 64 && m->hd != 128) || m->heads / m->kv > AP_ROWS) return false;
     const int qt = AP_ROWS / (m->heads / m->kv), blocks = (tokens + qt - 1) / qt;
-    return attn_packed_pays(m->hd, blocks * m->kv, pos0 + tokens, g.cus);
+    return attn_packed_pays(m->hd, blocks * m->kv, pos0, tokens, g.cus);
 }
 
 template <int D>

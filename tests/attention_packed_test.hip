@@ -57,11 +57,11 @@ static std::vector<float> attention(const Case &c) {
     return out;
 }
 
-// Row by row against FP64.  A score is off by at most d = (2^-10 + 2^-22 + 2^-20) sum |q_e k_e| / sqrt(D) (two FP16 operands, FP32 sums), so
+// Row by row against FP64.  A score is off by at most d = `off` sum |q_e k_e| / sqrt(D) (2^-10 + 2^-22 + 2^-20: two FP16 operands, FP32 sums), so
 // the weights, after normalisation, by factors within exp(+-2 d); a weight and a value round by 2^-11 each; 1e-5 for the FP32 sums
 // and the exponentials.  Against the sum of |weight value|.
 template <int D>
-static bool rows_match(const Case &c, const std::vector<float> &out, int tokens) {
+static bool rows_match(const Case &c, const std::vector<float> &out, int tokens, double off = 0x1p-10 + 0x1p-22 + 0x1p-20) {
     const int group = c.heads / c.kv;
     for (int t = 0; t < tokens; ++t)
         for (int h = 0; h < c.heads; ++h) {
@@ -77,7 +77,7 @@ static bool rows_match(const Case &c, const std::vector<float> &out, int tokens)
                 s[j] = a / sqrt((double)D);
                 size = std::max(size, b / sqrt((double)D));
             }
-            const double top = *std::max_element(s.begin(), s.end()), d = (0x1p-10 + 0x1p-22 + 0x1p-20) * size;
+            const double top = *std::max_element(s.begin(), s.end()), d = off * size;
             for (double &x : s) sum += x = exp(x - top);
             for (int e = 0; e < D; ++e) {
                 double want = 0, mag = 0;
@@ -130,6 +130,18 @@ static bool later_blocks_do_not_reach_earlier_ones() {
     return rows_match<D>(c, attention<D>(c), 32);
 }
 
+// Wide scores on keys that FP16 holds as they are: the queries' 22 bits are what is left to be off by, d = (2^-22 + 2^-20) sum |q_e k_e| /
+// sqrt(D) - whichever place a key has in its chunk.
+template <int D>
+static bool queries_in_two_parts() {
+    printf("%d values, queries of 22 bits\n", D);
+    fflush(stdout);
+    Case c = random_case<D>(4, 2, 3, 140, false);
+    for (float &x : c.q) x *= 32.f;
+    for (float &x : c.k) x = (float)(_Float16)x;
+    return rows_match<D>(c, attention<D>(c), c.tokens, 0x1p-22 + 0x1p-20);
+}
+
 // Scores around 2^32 (positive queries and keys up to 3e4): a row's weight lies on its best key alone, and its output is that key's value as
 // FP16 holds it.  A score is off by less than 2^-10 of itself (FP16 queries, FP32 sums): rows whose best two are closer than 2^-9 are left out.
 template <int D>
@@ -178,6 +190,7 @@ int main() {
         ok = ok && run<64>(8, 2, 0, 64, grow) && run<64>(3, 1, 62, 91, grow) && run<64>(4, 4, 130, 130, grow) && run<64>(16, 1, 64, 9, grow);
     }
     ok = ok && later_blocks_do_not_reach_earlier_ones<128>() && later_blocks_do_not_reach_earlier_ones<64>();
+    ok = ok && queries_in_two_parts<128>() && queries_in_two_parts<64>();
     ok = ok && large_scores<128>() && large_scores<64>();
     printf(ok ? "all hold\n" : "FAILED\n");
     return ok ? 0 : 1;
