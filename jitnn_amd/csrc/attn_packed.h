@@ -84,7 +84,7 @@ __device__ __forceinline__ float ap_max4(float v) {
 //   * a chunk is two runs of 1 KiB operands in memory and in LDS: every LDS read is 64 lanes x 16 consecutive bytes and feeds both tiles.
 //     (Reads scheduled four to six ahead of their products by hand: level to 10 % slower - it keeps the compiler from laying the
 //     exponentials of one tile under the other's products.)
-//   * one barrier per chunk: it says that the chunk has arrived and that the buffer of the one before is free, which the request for the
+//   * one barrier per chunk, behind a wait for both counters: it says that the chunk has arrived and that the buffer of the one before has been read, which the request for the
 //     next chunk then fills - two workgroups a CU work under each other's barriers.
 // The last keys a row does not see are masked in the chunks that reach past the block's first token, with their values cleared past its
 // last token: what a later block's token holds (infinities, NaN) does not reach this one.
@@ -155,7 +155,9 @@ __global__ void __launch_bounds__(AP_THREADS, D == 64 ? 3 : 2) attn_packed_kerne
     const int masked_from = (pos0 + t0 + 1) / CH;
     auto chunk = [&](int c, auto with_mask) {
         constexpr bool MASK = decltype(with_mask)::value;
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of chunk c has arrived
+        // vmcnt(0): this wave's share of chunk c has arrived; lgkmcnt(0): it has read what it needs of chunk c - 1, whose buffer the others
+        // fill behind the barrier (the products have taken those reads by then: no time)
+        __builtin_amdgcn_s_waitcnt(0x0070);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
