@@ -124,4 +124,14 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
+// The power of two that brings a largest magnitude into [2^13, 2^14) on its way to FP16: 1 for zero and what is not finite, and at most
+// 2^126, so that it and its inverse are normal numbers - the largest of a row below 2^-112 stays below 2^13, where FP16 still holds
+// whatever bits such a row has.
+__device__ __forceinline__ float half_scale(float amax) {
+    if (!(amax > 0.f && amax < INFINITY)) return 1.f;
+    int e;
+    frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
+    return ldexpf(1.f, min(14 - e, 126));
+}
+
 }  // namespace jitnn

@@ -352,12 +352,7 @@ __device__ __forceinline__ void mf_build_operands(const float4 (&v)[8], bool hav
 #pragma unroll
     for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[t].x), fabsf(v[t].y)), fmaxf(fabsf(v[t].z), fabsf(v[t].w))));
     amax = group_max8(amax);
-    float scale = 1.f;
-    if (amax > 0.f && amax < 3.0e38f) {
-        int e;
-        frexpf(amax, &e);             // amax = f * 2^e, f in [0.5, 1)
-        scale = ldexpf(1.f, 14 - e);  // largest scaled magnitude in [2^13, 2^14)
-    }
+    float scale = half_scale(amax);
     const float myinv = 1.f / scale;
 #pragma unroll
     for (int i = 0; i < 4; ++i) inv[i] = __shfl(myinv, ((4 * kq + i) & 7) * 8);  // C rows 4 kq + i belong to activation row (4 kq + i) & 7

@@ -55,12 +55,7 @@ __device__ __forceinline__ void rows_prepare_column(const float4 (&v)[8], _Float
 #pragma unroll
     for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[t].x), fabsf(v[t].y)), fmaxf(fabsf(v[t].z), fabsf(v[t].w))));
     amax = group_max8(amax);
-    float scale = 1.f;
-    if (amax > 0.f && amax < 3.0e38f) {
-        int e;
-        frexpf(amax, &e);             // amax = f * 2^e, f in [0.5, 1)
-        scale = ldexpf(1.f, 14 - e);  // largest scaled magnitude in [2^13, 2^14)
-    }
+    float scale = half_scale(amax);
     const float myinv = 1.f / scale;
     if (!have) scale = 0.f;
     uint8_t *base = reinterpret_cast<uint8_t *>(ops + ((size_t)g * ncol + c) * GR_OP_HALVES);

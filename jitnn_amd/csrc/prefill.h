@@ -29,7 +29,7 @@ constexpr int PF_NARROW_ROWS = 128;  // calls of at most this many rows: two 32-
 // position of value i (0..3) of a group of four in the FP16 operands: 0, 2, 1, 3
 __host__ __device__ constexpr int pf_perm4(int i) { return ((i & 1) << 1) | (i >> 1); }
 
-// One workgroup per activation row: amax -> scale = 2^(13 - floor(log2 amax)) and 1/scale for the epilogue.
+// One workgroup per activation row: amax -> scale (half_scale) and 1/scale for the epilogue.
 static __global__ void __launch_bounds__(256) x_row_scale_kernel(const float *__restrict__ x, float *__restrict__ scale, float *__restrict__ inv_scale,
                                                            int k) {
     __shared__ float red[4];
@@ -43,12 +43,7 @@ static __global__ void __launch_bounds__(256) x_row_scale_kernel(const float *__
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    float sc = 1.f;
-    if (m > 0.f && m < 3.0e38f) {
-        int e;
-        frexpf(m, &e);  // m = f * 2^e, f in [0.5, 1)
-        sc = ldexpf(1.f, 14 - e);
-    }
+    const float sc = half_scale(m);
     if (threadIdx.x == 0) {
         scale[blockIdx.x] = sc;
         inv_scale[blockIdx.x] = 1.f / sc;
@@ -192,12 +187,7 @@ __global__ void __launch_bounds__(256) x_prepare_kernel(const float *__restrict_
     if ((t & 63) == 0) red[t >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    float sc = 1.f;
-    if (amax > 0.f && amax < 3.0e38f) {
-        int e;
-        frexpf(amax, &e);
-        sc = ldexpf(1.f, 14 - e);
-    }
+    const float sc = half_scale(amax);
     if (t == 0 && tok < m) inv_scale[tok] = 1.f / sc;
     f16x8 *dst = reinterpret_cast<f16x8 *>(xo) + (size_t)(tok >> 5) * ksteps * 64 + (tok & 31);
 #pragma unroll
