@@ -45,7 +45,8 @@ __host__ __device__ constexpr size_t gemv_rows_lds_bytes(int tiles_per_wave) { r
 // kq = 0 = sum of sub-block j of the scaled row / 64, the other lanes zero.  GS == 16 (Q6_K, whose scales cover 16 values):
 // slot j of the lanes kq = 0 and slot j - 8 of the lanes kq = 1 = sum of the 16-value group j / 64, sixteen groups.
 // HALVES (the 4-bit 32-value formats, whose byte i holds values i and i + 16 of a block): lane group kq holds values
-// 4 kq .. 4 kq + 3 and 16 + 4 kq .. + 3 of the sub-block instead of 8 kq .. 8 kq + 7, each four in the order 0 2 1 3.
+// 4 kq .. 4 kq + 3 and 16 + 4 kq .. + 3 of the sub-block instead of 8 kq .. 8 kq + 7, each four in the order 0 2 1 3; and the block sums stand
+// in operand 8 three times, times 4 in the lanes kq = 1 and 2 (RTile<F_Q4_1>).
 // The work of one wave: column c of group g, the lane's eight quads v of its row already loaded (and normalised / gated).
 template <int GS, bool HALVES>
 __device__ __forceinline__ void rows_prepare_column(const float4 (&v)[8], _Float16 *__restrict__ ops, float *__restrict__ inv, int c, int g, int ncol,
@@ -86,9 +87,16 @@ __device__ __forceinline__ void rows_prepare_column(const float4 (&v)[8], _Float
     sm *= 0.015625f;
     const _Float16 shi = (_Float16)sm, slo = (_Float16)(sm - (float)shi);
     _Float16 *sop = reinterpret_cast<_Float16 *>(base + 8 * 1024);
-    if (lane >= (GS == 32 ? 16 : 32)) *reinterpret_cast<u32x4 *>(base + 8 * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+    if (lane >= (GS == 16 ? 32 : HALVES ? 48 : 16)) *reinterpret_cast<u32x4 *>(base + 8 * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
     sop[(2 * b) * 8 + part] = shi;
     sop[(2 * b + 1) * 8 + part] = slo;
+    if constexpr (HALVES) {  // (below 2^15)
+#pragma unroll
+        for (int z = 1; z < 3; ++z) {
+            sop[(16 * z + 2 * b) * 8 + part] = shi * (_Float16)4.f;
+            sop[(16 * z + 2 * b + 1) * 8 + part] = slo * (_Float16)4.f;
+        }
+    }
     if constexpr (GS == 16) {
         sm2 *= 0.015625f;
         const _Float16 thi = (_Float16)sm2, tlo = (_Float16)(sm2 - (float)thi);
@@ -385,7 +393,7 @@ struct RTile<F_Q4_1> : RStaged<8 * 20, 176, 4> {
     __device__ static __forceinline__ void decode(const uint8_t *row, uint32_t, int lane, f16x8 (&B)[8], f16x8 &Bm, float (&dblk)[8]) {
         const int kq = lane >> 4;
         const uint32_t mg = magic1024();
-        const f16x2 off = splat2(-1024.f);
+        const f16x2 off = splat2(-1032.f);  // -1024 of the exponent trick, and the quants around zero: -8 .. 7
         uint32_t dm[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
@@ -395,10 +403,13 @@ struct RTile<F_Q4_1> : RStaged<8 * 20, 176, 4> {
             dm[s] = ld32<4>(row + 20 * s);
             dblk[s] = h2f(dm[s]);
         }
-        // the offsets m of the eight blocks against the block sums of x: slot s of the lanes kq = 0, FP16 as they are
+        // The offsets of the eight blocks against the block sums of x, slot s: m in the lanes kq = 0, d - against sums times 4 - in the lanes
+        // kq = 1 and 2, FP16 as they are.  Their products meet in one sum as m + 8 d, half a d in a weight around zero, where sixteen times that
+        // would have to go off again against the sums of quants from 0 to 15.
+        const uint32_t sel = kq == 0 ? 0x07060302u : 0x05040100u, keep = kq < 3 ? 0xffffffffu : 0u;
         u32x4 mb;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mb[j] = kq == 0 ? (dm[2 * j] >> 16) | (dm[2 * j + 1] & 0xffff0000u) : 0u;
+        for (int j = 0; j < 4; ++j) mb[j] = __builtin_amdgcn_perm(dm[2 * j + 1], dm[2 * j], sel) & keep;
         Bm = __builtin_bit_cast(f16x8, mb);
     }
 };

@@ -9,7 +9,7 @@ namespace jitnn {
 constexpr int GT_ROWS = 16, GT_B = 4, GT_THREADS = 256;  // weight rows of a workgroup, activation rows of a thread (64 in all at most)
 __host__ __device__ constexpr size_t gemv_tail_lds_bytes(int rows, int blocks) { return (size_t)(rows + GT_ROWS) * (8 * blocks + 1) * sizeof(float4); }
 
-// y[b, row] += sum over the last `blocks` (1..7) blocks of W [n, k], in FP32: the dequantiser's values, one FMA each, in order of k.
+// y[b, row] += sum over the last `blocks` (1..7) blocks of W [n, k], in FP32: the dequantiser's values, one FMA each, in four sums.
 // The tails of the workgroup's weight rows, dequantised once, and of the activations wait in LDS, rows an odd number of quads apart, so that
 // the rows a wave reads at a time lie in different banks; a thread takes one weight row and GT_B activation rows.
 // Bound by the narrow loads of the blocks: 9.8 us for 14336 weight rows, 7 blocks and 16 activation rows, 12 for 8000 rows of Q8_0 and 40; with
@@ -35,21 +35,21 @@ __global__ void __launch_bounds__(GT_THREADS) gemv_tail_kernel(const uint8_t *__
     const float4 *wp = ws + r * pitch, *xp[GT_B];
 #pragma unroll
     for (int i = 0; i < GT_B; ++i) xp[i] = xs + min(b0 + i, rows - 1) * pitch;
-    float acc[GT_B] = {};
+    float4 acc[GT_B] = {};
     for (int q = 0; q < quads; ++q) {
         const float4 w = wp[q];
 #pragma unroll
         for (int i = 0; i < GT_B; ++i) {
             const float4 v = xp[i][q];
-            acc[i] = __builtin_fmaf(w.x, v.x, acc[i]);
-            acc[i] = __builtin_fmaf(w.y, v.y, acc[i]);
-            acc[i] = __builtin_fmaf(w.z, v.z, acc[i]);
-            acc[i] = __builtin_fmaf(w.w, v.w, acc[i]);
+            acc[i].x = __builtin_fmaf(w.x, v.x, acc[i].x);
+            acc[i].y = __builtin_fmaf(w.y, v.y, acc[i].y);
+            acc[i].z = __builtin_fmaf(w.z, v.z, acc[i].z);
+            acc[i].w = __builtin_fmaf(w.w, v.w, acc[i].w);
         }
     }
 #pragma unroll
     for (int i = 0; i < GT_B; ++i)
-        if (b0 + i < rows) y[(size_t)(b0 + i) * n + n0 + r] += acc[i];
+        if (b0 + i < rows) y[(size_t)(b0 + i) * n + n0 + r] += (acc[i].x + acc[i].y) + (acc[i].z + acc[i].w);
 }
 
 }  // namespace jitnn

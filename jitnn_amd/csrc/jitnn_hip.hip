@@ -1410,6 +1410,8 @@ bool rows_path(const jitnn_hip_weight *w, int rows) {
 // passes of eight rows, which stream the weight once each.  us, passes against this: Q4_1 5120 x 11456 at 5 / 9 / 40 / 64 rows 57 / 70 / 308 / 492
 // and 26 / 29 / 44 / 55, Q8_0 8000 x 5088 48 / 68 / 276 / 441 and 29 / 32 / 43 / 55, Q4_0 2048 x 2272 at 5 / 8 / 9 / 40 16 / 18 / 23 / 88 and 17.5 / 17.5 /
 // 17 / 20, Q4_0 4096 x 1504 at 9 / 11 / 16 16.4 / 16.7 / 21.0 and 17.3 / 17.8 / 17.7, Q8_0 2672 x 1056 at 8 / 9 9.6 / 17.4 and 14.0 / 14.1.
+// Against FP64 (weights around zero, 288 to 14304 values, 3 to 64 rows; 2-norm) the passes' FP32 arithmetic is 2.4e-7 to 3.7e-7 off, this,
+// whose sums are shorter, 0.49 (Q8_0), 0.52 (Q4_0) and 0.58 (Q4_1) times as much in the mean from nine rows on, nowhere more.
 bool rows_ragged_path(const jitnn_hip_weight *w, int rows) {
     if (w->fmt != F_Q4_0 && w->fmt != F_Q4_1 && w->fmt != F_Q8_0) return false;
     const int rows_min = w->k >= 12288 ? 3 : w->k >= 3072 ? 5 : w->k >= 2048 || w->fmt == F_Q8_0 ? 9 : 13;

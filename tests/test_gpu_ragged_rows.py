@@ -47,6 +47,32 @@ def test_ragged_rows_match_the_oracle(fmt, n, k, rows, bias):
     assert np.array_equal(out[0], out[1])
 
 
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q4_1", "Q8_0"])
+@pytest.mark.parametrize("k,rows,few", [(480, 24, 8), (1056, 16, 8), (2272, 40, 8), (5088, 24, 4), (11456, 40, 4), (14304, 10, 2)])
+def test_no_further_off_than_in_passes(fmt, k, rows, few):
+    """The same rows a few at a time take the kernels that multiply in FP32: in one pass the call is at most as far from FP64 (2-norm over 40000
+    outputs and more), on weights around zero, where the offsets of Q4_1 and the sums of its quants all but cancel."""
+    import jitnn_amd
+    from jitnn_amd import _lib as lib
+    from oracle import oracle
+    jitnn_amd.init()
+    n = 4000
+    rng = np.random.default_rng([k, rows])
+    raw = random_valid_blocks(rng, fmt, n, k)
+    if fmt == "Q4_1":
+        blocks = raw.reshape(-1, 20)
+        blocks[:, 2:4] = (-7.5 * blocks[:, :2].copy().view(np.float16).astype(np.float32)).astype(np.float16).view(np.uint8)
+    w = jitnn_amd.Tensor.quantized(jitnn_amd.DType[fmt], raw, n, k)
+    x = torch.randn(rows, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(k))
+    whole, parts = torch.empty(rows, n, device="cuda"), torch.empty(rows, n, device="cuda")
+    call(lib, "jitnn_hip_linear_dev", w, x, None, whole)
+    for r in range(0, rows, few):
+        call(lib, "jitnn_hip_linear_dev", w, x[r:r + few], None, parts[r:r + few])
+    torch.cuda.synchronize()
+    ref = x.double() @ torch.from_numpy(oracle.dequantize(GGML_ID[fmt], raw, n * k).reshape(n, k)).cuda().double().T
+    assert (whole - ref).norm() <= (parts - ref).norm()
+
+
 def test_captured_without_scratch():
     """A thread whose first call is recorded has no scratch: the passes of eight rows, the same products in FP32-grade arithmetic of another kind."""
     import jitnn_amd
