@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(64 * AS_WAVES, 2) attn_split_kernel(const floa
         for (int u = 1; u < AS_WAVES; ++u) m = fmaxf(m, sm[u][h]);
 #pragma unroll
         for (int u = 0; u < AS_WAVES; ++u) {
-            const float f = __expf(sm[u][h] - m);
+            const float f = sm[u][h] > -INFINITY ? __expf(sm[u][h] - m) : 0.f;  // (a workgroup whose scores are all -inf: -inf minus -inf)
             l += sl[u][h] * f;
             a += red[u][h][d] * f;
         }

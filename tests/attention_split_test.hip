@@ -138,6 +138,57 @@ static bool run(int pos, bool interleaved, float width) {
     return ok;
 }
 
+// All scores of one workgroup's keys are -inf (their FP32 dot products overflow): those keys have no weight, as in attn_decode_kernel, and
+// the others the weights they have without them.  Unrotated (angle zero); 1e-5 of the sum of |weight value|, the scores are at most 30.
+template <int D, int G, int P>
+static bool keys_without_weight() {
+    constexpr int heads = KV * G, first = 2 * as_keys(P), last = first + as_keys(P), pos = last + 40, chunks = pos / as_keys(P) + 1;
+    printf("%d values, %d heads over %d, %d keys per workgroup, one of them without weight\n", D, heads, KV, as_keys(P));
+    fflush(stdout);
+    std::mt19937 gen(D + P);
+    std::normal_distribution<float> normal;
+    std::vector<float> qkv((size_t)(heads + 2 * KV) * D), cosv((size_t)MAX_CTX * D / 2, 1.f), sinv(cosv.size(), 0.f), k((size_t)MAX_CTX * KV * D), v(k.size());
+    for (size_t i = 0; i < qkv.size(); ++i) qkv[i] = i < (size_t)heads * D ? 0.5f + 0.5f * fabsf(normal(gen)) : normal(gen);
+    for (size_t i = 0; i < k.size(); ++i) {
+        const int j = (int)(i / ((size_t)KV * D));
+        k[i] = j >= first && j < last ? -3e38f : normal(gen);
+        v[i] = normal(gen);
+    }
+    float *qd = device(qkv), *cd = device(cosv), *sd = device(sinv), *kd = device(k), *vd = device(v), *part, *out;
+    HIP(hipMalloc(&part, (size_t)heads * chunks * (D + 2) * 4));
+    HIP(hipMalloc(&out, (size_t)heads * D * 4));
+    hipLaunchKernelGGL((attn_split_kernel<D, G, P>), dim3(chunks, KV), dim3(256), 0, 0, qd, cd, sd, kd, vd, part, (uint32_t)heads | ((uint32_t)KV << 16), (uint32_t)pos);
+    hipLaunchKernelGGL((attn_merge_kernel<D, 2>), dim3(heads), dim3(2 * D), 0, 0, part, out, chunks);
+    HIP(hipGetLastError());
+    HIP(hipDeviceSynchronize());
+    std::vector<float> got((size_t)heads * D);
+    HIP(hipMemcpy(got.data(), out, got.size() * 4, hipMemcpyDeviceToHost));
+    for (void *p : {(void *)qd, (void *)cd, (void *)sd, (void *)kd, (void *)vd, (void *)part, (void *)out}) HIP(hipFree(p));
+    std::copy(qkv.begin() + (size_t)heads * D, qkv.begin() + (size_t)(heads + KV) * D, k.begin() + (size_t)pos * KV * D);
+    std::copy(qkv.begin() + (size_t)(heads + KV) * D, qkv.end(), v.begin() + (size_t)pos * KV * D);
+    for (int h = 0; h < heads; ++h) {
+        std::vector<double> w(pos + 1), sum(D), mag(D);
+        double all = 0;
+        for (int j = 0; j <= pos; ++j) {
+            double a = 0;
+            for (int e = 0; e < D; ++e) a += (double)qkv[(size_t)h * D + e] * k[((size_t)j * KV + h / G) * D + e];
+            all += w[j] = exp(a / sqrt((double)D));
+        }
+        for (int j = 0; j <= pos; ++j)
+            for (int e = 0; e < D; ++e) {
+                const double p = w[j] / all * v[((size_t)j * KV + h / G) * D + e];
+                sum[e] += p;
+                mag[e] += fabs(p);
+            }
+        for (int e = 0; e < D; ++e)
+            if (!(fabs(got[(size_t)h * D + e] - sum[e]) <= 1e-5 * mag[e])) {
+                printf("head %d value %d: %.7f, not %.7f\n", h, e, got[(size_t)h * D + e], sum[e]);
+                return false;
+            }
+    }
+    return true;
+}
+
 template <int D, int G>
 static bool positions() {
     bool ok = true;
@@ -149,8 +200,9 @@ static bool positions() {
 }
 
 int main() {
-    const bool ok = positions<128, 1>() && positions<128, 2>() && positions<128, 3>() && positions<128, 4>() && positions<64, 1>() && positions<64, 2>() &&
+    bool ok = positions<128, 1>() && positions<128, 2>() && positions<128, 3>() && positions<128, 4>() && positions<64, 1>() && positions<64, 2>() &&
                     positions<64, 3>() && positions<64, 4>();
+    ok = ok && keys_without_weight<128, 4, 2>() && keys_without_weight<128, 2, 4>() && keys_without_weight<64, 3, 2>() && keys_without_weight<64, 1, 4>();
     printf(ok ? "all hold\n" : "FAILED\n");
     return ok ? 0 : 1;
 }
