@@ -45,6 +45,8 @@ __global__ void __launch_bounds__(AP_THREADS) attn_pack_kernel(const float *__re
     __shared__ float vs[AP_CH][D + 4];  // the chunk's values, read along the rows and written along the columns
     const int c = blockIdx.x, g = blockIdx.y, j0 = c * AP_CH;
     f16x8 *out = reinterpret_cast<f16x8 *>(packed + ((size_t)g * gridDim.x + c) * ap_chunk_halves(D));
+    // (a finite key beyond FP16 is the largest FP16 holds: as infinity it would meet a query's two parts, of either sign, as inf - inf)
+    auto key = [](float x) { return (_Float16)(fabsf(x) < INFINITY ? fminf(fmaxf(x, -65504.f), 65504.f) : x); };
     auto row = [&](int j) { return ((size_t)min(j0 + j, keys - 1) * kv_heads + g) * D; };
     for (int i = threadIdx.x; i < AP_CH * D / 4; i += AP_THREADS) {
         const int j = i / (D / 4), e = 4 * (i % (D / 4));
@@ -54,7 +56,7 @@ __global__ void __launch_bounds__(AP_THREADS) attn_pack_kernel(const float *__re
         const int lane = p & 63, n = lane & 15, kq = lane >> 4, b = (p >> 6) % DB, t = (p >> 6) / DB;
         const float *k = kcache + row(16 * t + n) + 32 * b + 8 * kq;
         const float4 x = *reinterpret_cast<const float4 *>(k), y = *reinterpret_cast<const float4 *>(k + 4);
-        out[p] = f16x8{(_Float16)x.x, (_Float16)x.y, (_Float16)x.z, (_Float16)x.w, (_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w};
+        out[p] = f16x8{key(x.x), key(x.y), key(x.z), key(x.w), key(y.x), key(y.y), key(y.z), key(y.w)};
     }
     __syncthreads();
     for (int p = threadIdx.x; p < PIECES; p += AP_THREADS) {

@@ -142,6 +142,27 @@ static bool queries_in_two_parts() {
     return rows_match<D>(c, attention<D>(c), c.tokens, 0x1p-22 + 0x1p-20);
 }
 
+// Keys beyond what FP16 holds, against the queries' signs: no weight lies on them, whatever their size.
+template <int D>
+static bool keys_beyond_fp16() {
+    printf("%d values, keys of -7e4\n", D);
+    fflush(stdout);
+    Case c = random_case<D>(4, 2, 70, 75, false);
+    for (float &x : c.q) x = 0.1f + fabsf(x);
+    std::vector<float> out[2];
+    for (int i = 0; i < 2; ++i) {
+        for (int j : {3, 40, 63, 64, 100, 130})
+            for (int e = 0; e < c.kv * D; ++e) c.k[(size_t)j * c.kv * D + e] = i ? -7e4f : -6e4f;
+        out[i] = attention<D>(c);
+    }
+    for (size_t i = 0; i < out[0].size(); ++i)
+        if (!(out[0][i] == out[1][i])) {
+            printf("output %zu: %.6f, not %.6f\n", i, out[1][i], out[0][i]);
+            return false;
+        }
+    return true;
+}
+
 // Scores around 2^32 (positive queries and keys up to 3e4): a row's weight lies on its best key alone, and its output is that key's value as
 // FP16 holds it.  A score is off by less than 2^-10 of itself (FP16 queries, FP32 sums): rows whose best two are closer than 2^-9 are left out.
 template <int D>
@@ -191,6 +212,7 @@ int main() {
     }
     ok = ok && later_blocks_do_not_reach_earlier_ones<128>() && later_blocks_do_not_reach_earlier_ones<64>();
     ok = ok && queries_in_two_parts<128>() && queries_in_two_parts<64>();
+    ok = ok && keys_beyond_fp16<128>() && keys_beyond_fp16<64>();
     ok = ok && large_scores<128>() && large_scores<64>();
     printf(ok ? "all hold\n" : "FAILED\n");
     return ok ? 0 : 1;
