@@ -139,13 +139,16 @@ __device__ __forceinline__ float4 dequant4(const uint8_t *w, size_t i) {
     return make_float4(o[0], o[1], o[2], o[3]);
 }
 
-// Quad f of y.  STREAM: past the caches' replacement (nontemporal), for outputs beyond DQ_STREAM_BYTES, which the 32 MiB of L2s do not
-// hold for their reader anyway.  Stored plainly they stay in the 256 MiB Infinity Cache as dirty lines that the next weight's
-// stores wait for: three outputs in turn, Q4_K 14336 x 4096 70 -> 42 us, Q6_K 4096 x 14336 57 -> 45, Q8_0 9472 x 6144 56 -> 46; with
-// the quantiser's own streaming below, both kernels 123 -> 97, 108 -> 101 and 106 -> 101 us.  A reader with plain loads
-// finds less of it cached: a torch.sum behind it is as much slower on the last two (118 -> 120 us for both), and more where most of the output
-// would have been cached (109 -> 132 us on the first).
-constexpr size_t DQ_STREAM_BYTES = (size_t)32 << 20;
+// Quad f of y.  STREAM: past the caches' replacement (nontemporal), for outputs beyond DQ_STREAM_BYTES, which the 256 MiB Infinity Cache does
+// not hold together with the weight and what a reader makes of them.  Stored plainly they stay there as dirty lines that later stores
+// wait for.  Three outputs in turn, plain -> streamed, us, the dequantiser alone / with the Q8_0 quantiser behind it / a product with 8 rows /
+// a conversion to FP16 / a copy / a torch.sum: Q4_K 14336 x 4096 (224 MiB) 71 -> 42, 119 -> 99, 115 -> 111, 120 -> 121, 161 -> 153, 111 -> 125;
+// Q6_K 4096 x 14336 56 -> 45, 105 -> 102, 112 -> 99, 110 -> 113, 147 -> 142, 118 -> 120; Q4_K 16384 x 8192 (512 MiB) 161 -> 98, 271 -> 225,
+// 280 -> 243, 314 -> 286, 370 -> 351, 312 -> 280.  A reader whose speed hangs on the cache loses in between: the sum of one and the same
+// 224 MiB output again and again 85 -> 109, its scaling in place 127 -> 142 in turn.  Smaller outputs are left to the caches: streamed, Q4_K
+// 8192 x 4096 (128 MiB) again and again takes 66 us for 55 with a sum behind it, 55 for 49 with a product, 60 for 62 with the quantiser, and
+// Q8_0 4096 x 4096 (64 MiB) 41 for 35, 34 for 30 and 32 for 34.
+constexpr size_t DQ_STREAM_BYTES = (size_t)192 << 20;
 template <bool STREAM>
 __device__ __forceinline__ void dequant_store(float *__restrict__ y, size_t f, float4 v) {
     if constexpr (STREAM) __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(y) + f);
@@ -310,8 +313,9 @@ __device__ __forceinline__ void quantize_q8_0_block(const float *__restrict__ xb
 // away from zero.  So: a candidate from one FP32 multiplication (off by one at most), set right by the signs of
 // fma(r + 1/2, d, -|x|) and fma(r - 1/2, d, -|x|) - an FMA rounds the exact value once, its sign is the exact sign.
 // Blocks with a value that is not finite or beyond 2^100, or a maximum below 2^-100 (d near or in the subnormals), take
-// the reference's expression itself.  Input and output pass once: nontemporal, so that they leave the Infinity Cache to others (with the
-// dequantiser's output as input, dequant_store).  grid: any; 256 threads.
+// the reference's expression itself.  Input and output pass once: nontemporal, so that they leave the Infinity Cache to others (behind the
+// dequantiser's plain stores, plain -> nontemporal: 16 MiB of values 13.3 -> 13.1 us for both kernels, 32 MiB 19.6 -> 19.0, 64 MiB 36.7 -> 32.5, 128 MiB
+// 75 -> 58, 172 MiB 95 -> 76).  grid: any; 256 threads.
 constexpr int Q8Q_NI = 4, Q8Q_BLOCKS = 8 * Q8Q_NI;  // 16-byte loads per lane and blocks per wave and turn
 static __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restrict__ x, uint8_t *__restrict__ q, size_t blocks) {
     constexpr int NI = Q8Q_NI, NB = Q8Q_BLOCKS;

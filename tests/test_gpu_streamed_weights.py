@@ -1,4 +1,4 @@
-"""The dequantiser's streamed stores (outputs beyond 32 MiB) beside its plain ones, on the device: the largest output that is stored
+"""The dequantiser's streamed stores (outputs beyond 192 MiB) beside its plain ones, on the device: the largest output that is stored
 plainly and the smallest that is streamed, the same bits as the oracle's, and the Q8_0 quantiser reading them from there in stream order."""
 import ctypes as C
 
@@ -18,7 +18,7 @@ def test_dequantised_on_the_device_then_quantised(fmt, extra):
     from jitnn_amd import _lib
     from oracle import oracle
     jitnn_amd.init()
-    n, k = (1 << 23) // 256 + extra, 256
+    n, k = (192 << 18) // 256 + extra, 256
     raw = random_valid_blocks(np.random.default_rng(n), fmt, n, k)
     w = jitnn_amd.Tensor.quantized(jitnn_amd.DType[fmt], raw, n, k)
     y = torch.full((n * k + 4,), -7.0, device="cuda")
