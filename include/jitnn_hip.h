@@ -297,6 +297,24 @@ JITNN_HIP_API int jitnn_hip_llama_decode_dev(jitnn_hip_llama *m, const float *x_
 JITNN_HIP_API int jitnn_hip_llama_prefill(jitnn_hip_llama *m, const float *x_host, int pos0, int tokens, float *logits_host);
 JITNN_HIP_API int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0, int tokens, float *logits_dev, void *stream);
 
+/* The attention of a prompt pass: up to 64 tokens in FP32; longer ones with FP16 operands and FP32 sums - heads of 64 and 128 values on the
+ * matrix cores, 64 or 128 query rows per workgroup, the longest prompts on a copy of a layer's keys and values packed as FP16 operands. */
+#define JITNN_HIP_ATTN_FP32 0
+#define JITNN_HIP_ATTN_DOT2 1
+#define JITNN_HIP_ATTN_MFMA_64 2
+#define JITNN_HIP_ATTN_MFMA_128 3
+#define JITNN_HIP_ATTN_PACKED 4
+/* Which of them a pass takes.  packing: whether the model has, or may have, room for the packed copy.  compute_units 0: the device's;
+ * otherwise no device is needed. */
+JITNN_HIP_API int jitnn_hip_prompt_attention(int heads, int kv_heads, int head_dim, int pos0, int tokens, int packing, int compute_units);
+/* The packed copy (4 bytes per position, key/value head and value of a head) belongs to the model and is allocated by the first pass that
+ * wants it.  A pass that cannot have it - no memory, or its stream is being captured before any eager pass wanted it - takes the kernel it
+ * would take otherwise; the next one asks again.  Keys and values are rounded to FP16 in both, the queries to 22 bits with the copy and 11
+ * without, and the sums are in another order: results differ within the FP16 operands' error.  allow 0: this model's passes do without. */
+JITNN_HIP_API int jitnn_hip_llama_set_packing(jitnn_hip_llama *m, int allow);
+/* What the model's last prompt pass took; JITNN_HIP_EINVAL before the first. */
+JITNN_HIP_API int jitnn_hip_llama_last_attention(const jitnn_hip_llama *m);
+
 /* ---- generation loop ------------------------------------------------------------------------------------------------ */
 
 /* Text generation from a GGUF model is jitnn-llm's Llm.generate (jitnn-llm/src/main/java/ai/beestream/jitnn/llm/Llm.java:64-93),

@@ -76,6 +76,9 @@ def _bind() -> C.CDLL:
         "jitnn_hip_llama_decode": (i, [vp, vp, i, vp]),
         "jitnn_hip_llama_decode_dev": (i, [vp, vp, i, vp, vp]),
         "jitnn_hip_llama_prefill": (i, [vp, vp, i, i, vp]),
+        "jitnn_hip_prompt_attention": (i, [i, i, i, i, i, i, i]),
+        "jitnn_hip_llama_set_packing": (i, [vp, i]),
+        "jitnn_hip_llama_last_attention": (i, [vp]),
         "jitnn_hip_llama_set_rope_interleaved": (i, [vp, i]),
         "jitnn_hip_llama_set_embedding": (i, [vp, i, vp, ll]),
         "jitnn_hip_llama_embed_dev": (i, [vp, vp, i, vp, vp]),
@@ -143,6 +146,17 @@ def many_row_tile(weights, k: int, rows: int, gate_up: bool = False, residual: b
     if tile < 0:
         check(tile, "jitnn_hip_many_row_tile")
     return tile
+
+
+ATTN_FP32, ATTN_DOT2, ATTN_MFMA_64, ATTN_MFMA_128, ATTN_PACKED = range(5)
+
+
+def prompt_attention(heads: int, kv_heads: int, head_dim: int, pos0: int, tokens: int, packing: bool = True, compute_units: int = 0) -> int:
+    """Which attention (ATTN_*) a prompt pass takes, with or without room for packed keys and values."""
+    how = lib.jitnn_hip_prompt_attention(heads, kv_heads, head_dim, pos0, tokens, packing, compute_units)
+    if how < 0:
+        check(how, "jitnn_hip_prompt_attention")
+    return how
 
 
 def few_rows_slices(fmt: int, n: int, k: int, rows: int, adds: bool = False, compute_units: int = 0) -> int:

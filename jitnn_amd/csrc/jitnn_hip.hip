@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1919,6 +1920,8 @@ struct jitnn_hip_llama {
     int pf_cap;
     float *pf[11];  // xn, q, k, v, att, xa, xb, gate, up, h, the K slices of a linear whose join is deferred (8 x d per token)
     _Float16 *packed;  // keys and values of one layer as attn_packed_kernel reads them, up to max_ctx positions: allocated by the first long prompt
+    bool no_packing;    // the caller's wish: packed stays as it is and unused
+    int attention;      // the PromptAttention of the last prompt pass, -1: there was none
     int rope_interleaved;  // 0: rotate-half pairs (i, i + D/2); 1: pairs (2i, 2i + 1)
     // token embedding table [vocab, d] in ggml type embd_fmt (F32 = 0, F16 = 1 or a block format), owned
     uint8_t *embd;
@@ -2176,51 +2179,60 @@ bool packed_room(jitnn_hip_llama *m, hipStream_t st) {
     }
     return m->packed != nullptr;
 }
-// Whether the attention of a prompt pass takes the packed form.
-bool attention_packed(const jitnn_hip_llama *m, int pos0, int tokens) {
-    if (tokens <= g.gemv_max_rows || (m->hd != 64 && m->hd != 128) || m->heads / m->kv > AP_ROWS) return false;
-    const int qt = AP_ROWS / (m->heads / m->kv), blocks = (tokens + qt - 1) / qt;
-    return attn_packed_pays(m->hd, blocks * m->kv, pos0, tokens, g.cus);
+// The kernels that the attention of a prompt pass may take.  Prompts beyond the GEMV range have FP16-operand linears on both sides of it:
+// FP16 operands there too.
+enum PromptAttention {
+    ATTN_FP32 = JITNN_HIP_ATTN_FP32,          // attn_prefill_kernel
+    ATTN_DOT2 = JITNN_HIP_ATTN_DOT2,          // attn_prefill_h_kernel
+    ATTN_MFMA_64 = JITNN_HIP_ATTN_MFMA_64,    // attn_prefill_mfma_kernel<D, 1>
+    ATTN_MFMA_128 = JITNN_HIP_ATTN_MFMA_128,  // attn_prefill_mfma_kernel<D, 2>
+    ATTN_PACKED = JITNN_HIP_ATTN_PACKED,      // attn_packed_kernel (with room for the packed keys and values)
+};
+PromptAttention prompt_attention(int hd, int heads, int kv, int pos0, int tokens, bool room, int cus) {
+    const int group = heads / kv;
+    if (tokens <= g.gemv_max_rows) return ATTN_FP32;
+    if ((hd != 64 && hd != 128) || group > AM_ROWS) return ATTN_DOT2;
+    static_assert(AP_ROWS == 2 * AM_ROWS, "one count of blocks for both");
+    const int qt = AP_ROWS / group, blocks = (tokens + qt - 1) / qt * kv;
+    // (a head's chunks behind one buffer descriptor of less than 2 GiB)
+    if (room && attn_packed_pays(hd, blocks, pos0, tokens, cus) && ap_bytes(hd, 1, pos0 + tokens) < (size_t)1 << 31) return ATTN_PACKED;
+    return blocks >= attn_two_tiles_from(hd, cus) ? ATTN_MFMA_128 : ATTN_MFMA_64;
 }
 
 template <int D>
-int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, bool packed, const float *q, float *att, hipStream_t st) {
+int launch_attention_rows(const jitnn_hip_llama *m, int layer, int pos0, int tokens, PromptAttention how, const float *q, float *att, hipStream_t st) {
     const int group = m->heads / m->kv;
     const size_t lo = (size_t)layer * m->max_ctx * m->kv * m->hd;
     const float scale = 1.0f / sqrtf((float)D);
-    // prompts beyond the GEMV range have FP16-operand linears on both sides of the attention: FP16 operands here too
-    if (tokens > g.gemv_max_rows) {
-        if constexpr (D == 64 || D == 128) {
-            if (packed) {
-                const int qt = AP_ROWS / group, keys = pos0 + tokens, chunks = (keys + AP_CH - 1) / AP_CH;
-                if (int rc = allow_lds((const void *)attn_packed_kernel<D>, ap_lds_bytes(D))) return rc;
-                hipLaunchKernelGGL(attn_pack_kernel<D>, dim3(chunks, m->kv), dim3(AP_THREADS), 0, st, m->kc + lo, m->vc + lo, m->packed, m->kv, keys);
-                hipLaunchKernelGGL(attn_packed_kernel<D>, dim3(m->kv, (tokens + qt - 1) / qt), dim3(AP_THREADS), ap_lds_bytes(D), st, q, m->packed, att, m->heads, m->kv,
-                                   pos0, tokens, chunks, scale);
-                return JITNN_HIP_OK;
-            }
-            if (group <= AM_ROWS) {
-                const int qt2 = 2 * AM_ROWS / group, blocks2 = (tokens + qt2 - 1) / qt2;
-                if (blocks2 * m->kv >= attn_two_tiles_from(D, g.cus)) {
-                    constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 2>();
-                    if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 2>, lds)) return rc;
-                    hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 2>), dim3(m->kv, blocks2), dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads,
-                                       m->kv, pos0, tokens, scale);
-                    return JITNN_HIP_OK;
-                }
-                const int qt = AM_ROWS / group;
-                const dim3 grid((tokens + qt - 1) / qt, m->kv);
-                constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 1>();
-                if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 1>, lds)) return rc;
-                hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 1>), grid, dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads, m->kv, pos0, tokens,
-                                   scale);
-                return JITNN_HIP_OK;
-            }
+    if constexpr (D == 64 || D == 128) {
+        if (how == ATTN_PACKED) {
+            const int qt = AP_ROWS / group, keys = pos0 + tokens, chunks = (keys + AP_CH - 1) / AP_CH;
+            if (int rc = allow_lds((const void *)attn_packed_kernel<D>, ap_lds_bytes(D))) return rc;
+            hipLaunchKernelGGL(attn_pack_kernel<D>, dim3(chunks, m->kv), dim3(AP_THREADS), 0, st, m->kc + lo, m->vc + lo, m->packed, m->kv, keys);
+            hipLaunchKernelGGL(attn_packed_kernel<D>, dim3(m->kv, (tokens + qt - 1) / qt), dim3(AP_THREADS), ap_lds_bytes(D), st, q, m->packed, att, m->heads, m->kv,
+                               pos0, tokens, chunks, scale);
+            return JITNN_HIP_OK;
+        }
+        if (how == ATTN_MFMA_128) {
+            const int qt = 2 * AM_ROWS / group;
+            constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 2>();
+            if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 2>, lds)) return rc;
+            hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 2>), dim3(m->kv, (tokens + qt - 1) / qt), dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att,
+                               m->heads, m->kv, pos0, tokens, scale);
+            return JITNN_HIP_OK;
+        }
+        if (how == ATTN_MFMA_64) {
+            const int qt = AM_ROWS / group;
+            constexpr size_t lds = attn_prefill_mfma_lds_bytes<D, 1>();
+            if (int rc = allow_lds((const void *)attn_prefill_mfma_kernel<D, 1>, lds)) return rc;
+            hipLaunchKernelGGL((attn_prefill_mfma_kernel<D, 1>), dim3((tokens + qt - 1) / qt, m->kv), dim3(AM_THREADS), lds, st, q, m->kc + lo, m->vc + lo, att,
+                               m->heads, m->kv, pos0, tokens, scale);
+            return JITNN_HIP_OK;
         }
     }
     const int qt = ATT_ROWS / group;
     const dim3 grid((tokens + qt - 1) / qt, m->kv);
-    if (tokens > g.gemv_max_rows) {
+    if (how == ATTN_DOT2) {
         constexpr size_t lds = attn_prefill_h_lds_bytes<D>();
         if (int rc = allow_lds((const void *)attn_prefill_h_kernel<D>, lds)) return rc;
         hipLaunchKernelGGL(attn_prefill_h_kernel<D>, grid, dim3(256), lds, st, q, m->kc + lo, m->vc + lo, att, m->heads, m->kv, pos0, tokens, scale);
@@ -2264,6 +2276,7 @@ int jitnn_hip_llama_create(int layers, int d_model, int heads, int kv_heads, int
     *m = jitnn_hip_llama{};
     m->layers = layers; m->d = d_model; m->heads = heads; m->kv = kv_heads; m->hd = head_dim; m->ffn = ffn; m->vocab = vocab;
     m->max_ctx = max_ctx; m->eps = rms_eps; m->theta = rope_theta;
+    m->attention = -1;
     m->w = new (std::nothrow) const jitnn_hip_weight *[(size_t)layers * 7]();
     m->chunks_max = (max_ctx + 15) / 16;  // the smallest key chunk any head size uses
     const size_t cache = (size_t)layers * max_ctx * kv_heads * head_dim;
@@ -2444,7 +2457,9 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
     StatNest nest;
     const int d = m->d, T = tokens, qd = m->heads * m->hd;
     prefill_reserve(m, T, st);
-    const bool packed = attention_packed(m, pos0, T) && packed_room(m, st);
+    PromptAttention how = prompt_attention(m->hd, m->heads, m->kv, pos0, T, !m->no_packing, g.cus);
+    if (how == ATTN_PACKED && !packed_room(m, st)) how = prompt_attention(m->hd, m->heads, m->kv, pos0, T, false, g.cus);
+    m->attention = how;
     float *xn = m->pf[0], *q = m->pf[1], *k = m->pf[2], *v = m->pf[3], *att = m->pf[4], *xa = m->pf[5], *xb = m->pf[6], *gate = m->pf[7],
           *up = m->pf[8], *h = m->pf[9];
     const float *x = x_dev;
@@ -2469,10 +2484,10 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
         }
         int arc;
         switch (m->hd) {
-        case 64: arc = launch_attention_rows<64>(m, l, pos0, T, packed, q, att, st); break;
-        case 128: arc = launch_attention_rows<128>(m, l, pos0, T, packed, q, att, st); break;
-        case 192: arc = launch_attention_rows<192>(m, l, pos0, T, packed, q, att, st); break;
-        default: arc = launch_attention_rows<256>(m, l, pos0, T, packed, q, att, st); break;
+        case 64: arc = launch_attention_rows<64>(m, l, pos0, T, how, q, att, st); break;
+        case 128: arc = launch_attention_rows<128>(m, l, pos0, T, how, q, att, st); break;
+        case 192: arc = launch_attention_rows<192>(m, l, pos0, T, how, q, att, st); break;
+        default: arc = launch_attention_rows<256>(m, l, pos0, T, how, q, att, st); break;
         }
         if (arc) return arc;
         // xa = x + Wo att, xb = xa + W2 (silu(W1 n) * (W3 n)), n = RMSNorm(xa)
@@ -2511,6 +2526,28 @@ int jitnn_hip_llama_prefill_dev(jitnn_hip_llama *m, const float *x_dev, int pos0
 }
 
 // ---- generation loop: embedding lookup, greedy choice, prompt + token-by-token decode --------------------------------
+
+int jitnn_hip_prompt_attention(int heads, int kv_heads, int head_dim, int pos0, int tokens, int packing, int compute_units) {
+    if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0 || heads / kv_heads > ATT_GMAX || (head_dim != 64 && head_dim != 128 && head_dim != 192 && head_dim != 256) ||
+        pos0 < 0 || tokens < 1 || pos0 > INT_MAX - tokens || compute_units < 0)
+        return fail(JITNN_HIP_EINVAL, "no such prompt");
+    if (compute_units == 0) {
+        if (int rc = check_ready()) return rc;
+        compute_units = g.cus;
+    }
+    return prompt_attention(head_dim, heads, kv_heads, pos0, tokens, packing != 0, compute_units);
+}
+
+int jitnn_hip_llama_set_packing(jitnn_hip_llama *m, int allow) {
+    if (!m) return fail(JITNN_HIP_EINVAL, "model is NULL");
+    m->no_packing = !allow;
+    return JITNN_HIP_OK;
+}
+
+int jitnn_hip_llama_last_attention(const jitnn_hip_llama *m) {
+    if (!m) return fail(JITNN_HIP_EINVAL, "model is NULL");
+    return m->attention < 0 ? fail(JITNN_HIP_EINVAL, "no prompt pass yet") : m->attention;
+}
 
 int jitnn_hip_llama_set_rope_interleaved(jitnn_hip_llama *m, int interleaved) {
     if (!m) return fail(JITNN_HIP_EINVAL, "model is NULL");

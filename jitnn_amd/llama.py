@@ -87,6 +87,17 @@ class LlamaDecoder:
         """Rotary pairs (2i, 2i + 1) instead of the default (i, i + head_dim / 2): the two forms of Rope (core/ops/Rope.java:126-150)."""
         _lib.check(_lib.lib.jitnn_hip_llama_set_rope_interleaved(self._h, 1 if on else 0), "jitnn_hip_llama_set_rope_interleaved")
 
+    def set_packing(self, allow: bool) -> None:
+        """Whether prompt passes may keep a layer's keys and values packed as FP16 operands (the default), in a buffer of the model."""
+        _lib.check(_lib.lib.jitnn_hip_llama_set_packing(self._h, 1 if allow else 0), "jitnn_hip_llama_set_packing")
+
+    def last_attention(self) -> int:
+        """The attention (_lib.ATTN_*) that the last prompt pass took."""
+        how = _lib.lib.jitnn_hip_llama_last_attention(self._h)
+        if how < 0:
+            _lib.check(how, "jitnn_hip_llama_last_attention")
+        return how
+
     def set_embedding(self, ggml_type: int, table) -> None:
         """The token embedding table [vocab, d_model] as raw bytes of ggml type F32 (0), F16 (1) or a block format."""
         raw = np.ascontiguousarray(table).view(np.uint8).reshape(-1)
