@@ -202,8 +202,8 @@ __global__ void __launch_bounds__(256) x_prepare_kernel(const float *__restrict_
 }
 
 // 32 consecutive weights of a row, starting at value k0 (k0 % 32 == 0), in two phases so that the loads of the next
-// K step can be in flight while the matrix cores work on the current one: pf_load fetches the raw bytes, pf_decode
-// turns them into FP32 values in the dequantiser's arithmetic.
+// K step can be in flight while the matrix cores work on the current one: pf_load fetches the raw bytes, pf_decode_h
+// turns them into FP16, or pf_decode into FP32 values in the dequantiser's arithmetic.
 template <int FMT>
 struct PfRaw;
 template <>
@@ -273,28 +273,13 @@ __device__ __forceinline__ void pf_load(PfRaw<FMT> &r, const uint8_t *row, int k
     }
 }
 
+// whether a format has a packed decoder (pf_decode_h); Q5_1 and Q2_K go through FP32 (pf_decode)
+__host__ __device__ constexpr bool pf_packed(int fmt) { return fmt != F_Q5_1 && fmt != F_Q2_K; }
+
 template <int FMT>
 __device__ __forceinline__ void pf_decode(const PfRaw<FMT> &r, int k0, float (&o)[32]) {
-    if constexpr (FMT == F_Q4_0 || FMT == F_Q4_1) {
-        float d, m = 0.f;
-        if constexpr (FMT == F_Q4_0) {
-            d = h2f(r.d);
-        } else {
-            d = h2f(r.dm);
-            m = h2f(r.dm >> 16);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t byte = (r.q[i >> 2] >> (8 * (i & 3))) & 0xffu;
-            if constexpr (FMT == F_Q4_0) {
-                o[i] = (float)((int)(byte & 15u) - 8) * d;
-                o[16 + i] = (float)((int)(byte >> 4) - 8) * d;
-            } else {
-                o[i] = (float)(byte & 15u) * d + m;
-                o[16 + i] = (float)(byte >> 4) * d + m;
-            }
-        }
-    } else if constexpr (FMT == F_Q5_1) {  // (q_low + 16 bit e of qh) d + m (GgufKernels.java:155-163)
+    static_assert(!pf_packed(FMT), "Q5_1 and Q2_K");
+    if constexpr (FMT == F_Q5_1) {  // (q_low + 16 bit e of qh) d + m (GgufKernels.java:155-163)
         const float d = h2f(r.dm), m = h2f(r.dm >> 16);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -303,7 +288,7 @@ __device__ __forceinline__ void pf_decode(const PfRaw<FMT> &r, int k0, float (&o
             o[i] = lo + m;
             o[16 + i] = hi + m;
         }
-    } else if constexpr (FMT == F_Q2_K) {  // d (scale nibble) q - dmin (min nibble), a scale byte per 16 values (GgufKernels.java:166-175)
+    } else {  // d (scale nibble) q - dmin (min nibble), a scale byte per 16 values (GgufKernels.java:166-175)
         const int j = ((k0 & 127) >> 5);
         const float d = h2f(r.dd), dmin = h2f(r.dd >> 16);
         const float ds0 = d * (float)(r.sc & 15u), m0 = dmin * (float)((r.sc >> 4) & 15u);
@@ -314,50 +299,6 @@ __device__ __forceinline__ void pf_decode(const PfRaw<FMT> &r, int k0, float (&o
             const float a = (i < 16 ? ds0 : ds1) * (float)((w >> (8 * (i & 3) + 2 * j)) & 3u);
             o[i] = a - (i < 16 ? m0 : m1);
         }
-    } else if constexpr (FMT == F_Q8_0) {
-        const float d = h2f(r.d);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const uint32_t w = i < 16 ? r.q0[i >> 2] : r.q1[(i - 16) >> 2];
-            o[i] = d * (float)(int)(int8_t)((w >> (8 * (i & 3))) & 0xffu);
-        }
-    } else if constexpr (FMT == F_Q4_K || FMT == F_Q5_K) {
-        const int e = k0 & 255, j = e >> 6, half = (e >> 5) & 1, sub = 2 * j + half;
-        int sc, mn;
-        {
-            const uint32_t s0 = r.h.y, s1 = r.h.z, s2 = r.h.w;
-            const int sh = 8 * (sub & 3);
-            if (sub < 4) {
-                sc = (s0 >> sh) & 63;
-                mn = (s1 >> sh) & 63;
-            } else {
-                sc = ((s2 >> sh) & 15) | (((s0 >> sh) >> 6 & 3) << 4);
-                mn = ((s2 >> sh) >> 4 & 15) | (((s1 >> sh) >> 6 & 3) << 4);
-            }
-        }
-        const float ds = h2f(r.h.x) * (float)sc, m = h2f(r.h.x >> 16) * (float)mn;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const uint32_t w = i < 16 ? r.q0[i >> 2] : r.q1[(i - 16) >> 2];
-            uint32_t q = (w >> (8 * (i & 3) + 4 * half)) & 15u;
-            if constexpr (FMT == F_Q5_K) {
-                const uint32_t hw = i < 16 ? r.qh0[i >> 2] : r.qh1[(i - 16) >> 2];
-                q += 16u * ((hw >> (8 * (i & 3) + sub)) & 1u);
-            }
-            o[i] = ds * (float)q - m;
-        }
-    } else {  // F_Q6_K
-        const int kk = ((k0 & 255) >> 5) & 3;
-        const float d = h2f(r.d);
-        const float a0 = d * (float)(int)(int8_t)(r.sc & 0xffu), a1 = d * (float)(int)(int8_t)(r.sc >> 8);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const uint32_t lw = i < 16 ? r.l0[i >> 2] : r.l1[(i - 16) >> 2];
-            const uint32_t hw = i < 16 ? r.h0[i >> 2] : r.h1[(i - 16) >> 2];
-            const int low = (lw >> (8 * (i & 3) + (kk < 2 ? 0 : 4))) & 15;
-            const int hb = (hw >> (8 * (i & 3) + 2 * kk)) & 3;
-            o[i] = (i < 16 ? a0 : a1) * (float)(low + 16 * hb - 32);
-        }
     }
 }
 
@@ -365,8 +306,8 @@ __device__ __forceinline__ void pf_decode(const PfRaw<FMT> &r, int k0, float (&o
 // conversion instruction (a byte OR-ed under the exponent 0x6400 is 1024 + byte; the 1024, and Q6_K's 32, come off
 // with one exact packed add), and the block scale is applied with packed FP16 arithmetic, two weights per
 // instruction.  Pairs come out as (byte 0, byte 2), (byte 1, byte 3) of each dword of quants: the 0, 2, 1, 3 order
-// the activations are stored in.  Rounding: the scale product d*sc is rounded to FP16 once more than in the FP32
-// decoder, still far inside the 2e-3 bar of this path.
+// the activations are stored in.  Rounding: the scale product d*sc is rounded to FP16 before it meets the quant, once more than
+// the dequantiser's value, still far inside the 2e-3 bar of this path.
 typedef union { uint32_t u; f16x2 h; } pf_h2;
 
 __device__ __forceinline__ f16x2 pf_pair(uint32_t u) { pf_h2 t; t.u = u; return t.h; }
@@ -473,8 +414,8 @@ __device__ __forceinline__ void pf_decode_h<F_Q6_K>(const PfRaw<F_Q6_K> &r, int 
     }
 }
 
-// The 32-value formats: d times a quant, and for Q4_1 and Q5_1 the offset with it, in one FP16 rounding - the value that the FP32
-// decoder above rounds to FP16 (a quant of at most eight bits times an FP16 scale is exact in FP32; with an offset that one rounds twice).
+// The 32-value formats but Q5_1: d times a quant, and for Q4_1 the offset with it, in one FP16 rounding - the dequantiser's FP32 value
+// rounded to FP16 (a quant of at most eight bits times an FP16 scale is exact in FP32; with an offset that one rounds twice).
 // q + 1024 leaves the 1024 in one exact packed add; a high nibble, 1024 + 16 q where it stands, in one exact packed FMA.
 template <>
 __device__ __forceinline__ void pf_decode_h<F_Q4_0>(const PfRaw<F_Q4_0> &r, int, f16x8 (&o)[4]) {
@@ -534,9 +475,6 @@ __device__ __forceinline__ void pf_decode_h<F_Q8_0>(const PfRaw<F_Q8_0> &r, int,
     }
 }
 
-// whether a format has a packed decoder; the others go through FP32
-__host__ __device__ constexpr bool pf_packed(int fmt) { return fmt != F_Q5_1 && fmt != F_Q2_K; }
-
 // The 256-value formats reach LDS in two hops.  A thread's 32 weights of a step are a few 16-byte fields scattered
 // over its row's block, so fetching them straight from global memory makes every load instruction of a wave touch
 // 32 to 64 cache lines (one or two per row), and the CU's one vector L1 spends more cycles on tag look-ups than the
@@ -546,13 +484,13 @@ __host__ __device__ constexpr bool pf_packed(int fmt) { return fmt != F_Q5_1 && 
 // 16-byte reads, and every field a decoder reads with one 16-byte load is 16-byte aligned relative to the block);
 // each step's decoder then reads its fields from there.
 template <int FMT>
-struct PfStage { static constexpr bool ON = false; static constexpr int NB = 16, CPR = 1, RP = 16, TAIL = 0, ALIGN = 16, NRAW = 0; };
+struct PfStage { static constexpr bool ON = false; static constexpr int NB = 16, CPR = 1, RP = 16, TAIL = 0, ALIGN = 16; };
 template <>
-struct PfStage<F_Q4_K> { static constexpr bool ON = false; static constexpr int NB = 144, CPR = 9, RP = 144, TAIL = 0, ALIGN = 16, NRAW = 3; };
+struct PfStage<F_Q4_K> { static constexpr bool ON = false; static constexpr int NB = 144, CPR = 9, RP = 144, TAIL = 0, ALIGN = 16; };
 template <>
-struct PfStage<F_Q5_K> { static constexpr bool ON = true; static constexpr int NB = 176, CPR = 11, RP = 176, TAIL = 0, ALIGN = 16, NRAW = 5; };
+struct PfStage<F_Q5_K> { static constexpr bool ON = true; static constexpr int NB = 176, CPR = 11, RP = 176, TAIL = 0, ALIGN = 16; };
 template <>
-struct PfStage<F_Q6_K> { static constexpr bool ON = true; static constexpr int NB = 210, CPR = 13, RP = 240, TAIL = 1, ALIGN = 2, NRAW = 6; };
+struct PfStage<F_Q6_K> { static constexpr bool ON = true; static constexpr int NB = 210, CPR = 13, RP = 240, TAIL = 1, ALIGN = 2; };
 
 // dynamic LDS of prefill_mfma_kernel<FMT>: the FP16 weight tile of two steps, then the staged raw blocks of two
 // groups of four steps
