@@ -128,8 +128,8 @@ JITNN_HIP_API int jitnn_hip_dequantize_dev(const jitnn_hip_weight *w, float *y_d
  * Up to 64 rows run the GEMV kernels at FP32-grade accuracy (error ~1e-6 of the largest output): FP32 arithmetic for
  * one and two rows, FP16 hi/lo splits of the activations on the matrix cores for more - 3 to 8 rows in one launch, 9 to
  * 64 rows in one pass over the weights (rows of whole 256-value columns; of Q4_0, Q4_1 and Q8_0 rows their whole columns, the rest in a
- * kernel of its own; else, or without scratch for it, in passes of 8), in one of two kernels that the shape
- * alone chooses (jitnn_hip_few_rows_slices; where the second one's scratch cannot grow it takes a launch per slice of a row, and
+ * kernel of its own; else, or without scratch for it, in passes of 8: FP32-grade too, not the same bits), in one of two kernels that the
+ * shape alone chooses (jitnn_hip_few_rows_slices says which for rows of whole columns; where the second one's scratch cannot grow it takes a launch per slice of a row, and
  * gives the same bits); more rows (prefill) run on the matrix cores (FP16 operands, FP32 accumulation, error < 2e-3) in one of two kernels: one decodes the weights on their way
  * into LDS; the other, for more than 512 rows and at least 1024 values per weight row where an estimate finds it faster,
  * multiplies weights that a pass before it has dequantised into the calling thread's scratch (at most 512 MiB).  Where that
@@ -141,7 +141,9 @@ JITNN_HIP_API int jitnn_hip_linear(const jitnn_hip_weight *w, const float *x_hos
 JITNN_HIP_API int jitnn_hip_linear_dev(const jitnn_hip_weight *w, const float *x_dev, int rows, const float *bias_dev, float *y_dev, void *stream);
 
 /* jitnn_hip_linear_dev for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments, same results bit for bit; the
+ * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments; same results bit for bit as
+ * jitnn_hip_linear_dev with its scratch at hand (a call that cannot have it, for want of memory or because its stream is being captured
+ * before an eager call of that size, may add up in another order; see there).  The
  * same kernels too, except that weights are never dequantised ahead of the product (long calls can take longer here).  Where
  * jitnn_hip_linear_dev takes the scratch of a many-row launch (FP16 activations in operand order, their row
  * scales, the partial sums of K slices) from a buffer of the calling thread that it may have to allocate or grow, this
@@ -162,7 +164,8 @@ JITNN_HIP_API long long jitnn_hip_noalloc_scratch_bytes(void);
 JITNN_HIP_API int jitnn_hip_many_row_tile(const int *fmts, const int *n, int count, int k, int rows, int gate_up, int residual, int compute_units);
 
 /* Which of the two kernels for 9 to 64 rows (3 to 64 of at least 12288 values; rows of whole 256-value columns) jitnn_hip_linear
- * takes: 0 the one that streams the activations' operands - or another one, for other rows -, otherwise the slices of a row that the one
+ * takes: 0 the one that streams the activations' operands - or another one, for other rows, those of 32-value blocks that are no whole
+ * columns among them, whose whole columns take either -, otherwise the slices of a row that the one
  * that holds them adds up.  adds: with a bias.  compute_units as above. */
 JITNN_HIP_API int jitnn_hip_few_rows_slices(int fmt, int n, int k, int rows, int adds, int compute_units);
 

@@ -26,6 +26,8 @@ __device__ __forceinline__ float as_ror8(float v) { return __int_as_float(__buil
 //   * all keys and values of a wave are requested before the first is used: 128 KiB per workgroup (P = 4, 128 values).
 //   * the eight partial sums of a value meet in registers, two at a time in swapped lane halves (each step halves the registers), the
 //     four waves in LDS.
+// Groups of up to four: a query head of 128 values takes 16 registers of a lane and its sums 16 more, so that eight heads alone would fill the
+// 256 that two workgroups to a CU leave, with 64 or 128 for keys and values still to come.
 // Keys past the new token repeat its row; their scores are masked, their values cleared.
 // Bound by the cache's way from memory, one round trip for all of it: 4000 positions of 8 key/value heads of 128 values (32.8 MB), with its
 // merge, 4.2 us per layer less than attn_decode_kernel (whose three workgroups per CU stage a chunk in LDS and wait for it in step), the

@@ -815,17 +815,19 @@ size_t row_scale_bytes(int rows) { return ((size_t)rows * 8 + 255) & ~(size_t)25
 // Whether `count` weights of one row length (dual: a gate and an up weight) are worth dequantising first for `rows` rows:
 // the estimate of both passes against that of prefill_mfma_kernel, which takes rounds of 128-row tiles (dual: 64 rows of each
 // weight) by 256 tokens at `step` us per 64 values of K.  Measured, both routes, activation preparation included (us):
-// 14336 x 4096 Q4_K, 1024 / 2048 / 4096 rows 139 / 268 / 496 there and 137 / 256 / 484 here; 4096 x 14336 Q6_K 169 / 298 / 612
-// and 228 / 292 / 486; 4096 x 4096 Q4_K 58 / 85 / 160 and 65 / 84 / 139; Q8_0 64 / 94 / 179 and 65 / 85 / 140.
+// 14336 x 4096 Q4_K, 1024 / 2048 / 4096 rows 139 / 262 / 490 there and 140 / 254 / 489 here; 4096 x 14336 Q6_K 159 / 277 / 555
+// and 232 / 290 / 478; 4096 x 4096 Q4_K 57 / 84 / 160 and 68 / 85 / 140; Q8_0 63 / 90 / 171 and 69 / 86 / 141; 11008 x 4096 Q4_0 122 / 199 / 398
+// and 112 / 205 / 375.  (The steps of Q4_K, Q6_K and Q8_0 are older than the kernel there: they were fitted when its barrier stood between two
+// steps.  Where that errs: Q6_K 4096 x 14336 at 2048 rows is taken here, and Q8_0 4096 x 4096 is not.)
 // Up to 1024 rows Q4_0, Q4_1 and Q5_K have the steps that lost least on 326 linears and 61 prompts of 4 layers, timed with both routes since
 // prefill_mfma_kernel decodes them in packed FP16 under its products (beyond, where only whole prompts were timed, 1.06 stands): Q4_0 linears
-// 0.5 % behind the faster route in the mean and not 1.3.  Of Q4_0, here -> there: 4352 x 12800 at 886 rows 170 -> 146 us, 14336 x 4096 at 900
-// 139 -> 125, 800 tokens of four 4096-wide layers 2244 -> 2136; the most it costs: Q5_K 14336 x 4096 at 1024 rows, 135 -> 138 us.
-// Two tiles of tokens or fewer, short rows of K and launches that split K lose here, whatever the estimate (8448 x 512 at 4096 rows 90 and 80, but at 2048 55 and 59; 1024 x 4096 at 1024 37 and 63), and the
-// estimate is good to a tenth on short launches: the margins.  For the 8B gate / up pair it errs against this route: at 4096
-// rows 920 us estimated there and 970 measured, 828 estimated here and 800 measured, so that with the margin it is
-// taken at 2049 - 2304, 2561 - 2816, 3073 - 3328 and 3585 - 4096 rows, where the product's last round is full enough, and not
-// wherever it would win.
+// 0.5 % behind the faster route in the mean and not 1.3.  Of Q4_0, here -> there: 4352 x 12800 at 886 rows 172 -> 148 us, 14336 x 4096 at 900
+// 140 -> 128, 800 tokens of four 4096-wide layers 2244 -> 2136; Q5_K 14336 x 4096 at 1024 rows is level, 137 us.
+// Two tiles of tokens or fewer, short rows of K and launches that split K lose here, whatever the estimate (1024 x 4096 at 1024 36 and 63; at 1024 values it turns, 8448 x 1024 at 2048 rows 72 and 69, at 4096 120 and 102), and the
+// estimate is good to a tenth on short launches: the margins.  For the 8B gate / up pair it errs against this route: with the margin it is
+// taken at 2049 - 2304, 2561 - 2816, 3073 - 3328 and 3585 - 4096 rows, where the product's last round is full enough (whole prompts, us per layer,
+// there / here: 2304 tokens 1275 / 1225, 2816 1513 / 1438, 3328 1774 / 1664, 4096 2081 / 1950), and not wherever it would win (1300 919 / 889, 1536
+// 949 / 932, 2560 1379 / 1341, 3072 1655 / 1595; level at 1792 and 2048, 51, 7 and 11 us slower at 600, 800 and 1024).
 // residual: prefill_mfma_kernel leaves it to add_rows_kernel (12 bytes per output at 6.5 TB/s: 31 us for 4096 x 4096), the wide
 // kernel adds it as it stores: 4096 x 4096 Q4_K at 4096 rows 143 + 31 us there, 127 + 8 here.
 bool wide_pays(const int *fmt, const int *rows_of, int count, int k, int rows, bool dual, bool residual, int cus, WidePlan *plan) {
