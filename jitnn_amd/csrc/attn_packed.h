@@ -27,6 +27,8 @@ constexpr size_t ap_bytes(int D, int kv_heads, int keys) { return (size_t)kv_hea
 // second place on some CUs, which costs where all blocks walk about the same number of keys: 600 tokens from position 900 (152) 299 / 321,
 // 560 from 3000 (144) 341 / 402, 1200 from 900 (152, 16 over 4) 226 / 228, but 2200 from 900 (140, 8 over 4) 218 / 211, 2500 from 0 (160)
 // 208 / 202, 640 from 0 (160) 278 / 275; 512 from 2000 (128) 276 / 275.
+// From 256 to 511, where the other kernel has 128 rows too, the two are level (24 prompts: 2.2 % slower to 2.1 % faster, 0.2 % slower in the
+// mean): packed, for its smaller error.
 // 64 values: 1024 workgroups 458 / 481, 528 299 / 308, 376 213 / 220, 328 to 340 205 / 209, 192 / 203 and 195 / 197; 256 to 304 173 / 169, 193 / 191, 181 / 177.
 constexpr bool attn_packed_pays(int D, int blocks, int pos0, int tokens, int cus) {
     return D == 64 ? 4 * blocks >= 5 * cus : 16 * blocks >= 11 * cus || (2 * blocks > cus && 4 * pos0 >= 3 * tokens);
