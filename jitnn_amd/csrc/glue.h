@@ -739,7 +739,8 @@ constexpr size_t attn_prefill_mfma_lds_bytes() {
 // over 4, 2048 tokens), 376 65 / 76 (3000), 512 107 / 87 (4096), 528 97 / 82 (32 over 4, 2100 from position 900), 1000 186 / 132 (32
 // over 8, 3970); between 376 and 512 it depends on the heads.  128 values: 176 45 / 50, 256 73 / 60 and 133 / 110 (4 key/value
 // heads), 48 / 36 (8).
-// (Such prompts take attn_packed_kernel, attn_packed.h, which is faster still; two tiles here are for a model without room for its packed keys.)
+// (Such prompts take attn_packed_kernel, attn_packed.h, which is level or faster and less far off; two tiles here are for a model without room
+// for its packed keys, or told to do without.)
 constexpr int attn_two_tiles_from(int D, int cus) { return (D == 64 ? 2 : 1) * cus; }
 template <int D, int RT>
 __global__ void __launch_bounds__(AM_THREADS, D == 64 && RT == 2 ? 4 : 1) attn_prefill_mfma_kernel(const float *__restrict__ q, const float *__restrict__ kcache,
